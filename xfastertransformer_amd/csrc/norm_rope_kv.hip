@@ -302,11 +302,13 @@ __global__ __launch_bounds__(64) void rope_kv_kernel(RopeKvParams p) {
 // leave as 16-byte runs.  Blocks the new tokens only partly fill (the first and the last of an append) fall back to
 // element stores for the values: the other slots of the tile belong to tokens already there.  Same arithmetic and the
 // same rounding points as the per-token kernel.  D = 128, bf16 rows, [maxPos, 64] tables, fused q | k | v rows.
+// cosT == nullptr: a plain append (the grid then holds the key / value heads only; the per-token kernel launches a wave a
+// query head and token that has nothing to do: 4 x 2000 tokens, 32 + 8 heads 75.9 us).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <bool INT8>
 __global__ __launch_bounds__(256) void rope_kv_block_kernel(RopeKvParams p, int nblk) {
     __shared__ __attribute__((aligned(16))) unsigned char tile[128 * 32 * 2];
-    const int head = blockIdx.x;
+    const int head = p.cosT ? blockIdx.x : p.qHeads + blockIdx.x;
     const int b = blockIdx.y / nblk, wb = blockIdx.y % nblk;
     int past = p.past;
     if (p.past_dev) {
@@ -328,17 +330,23 @@ __global__ __launch_bounds__(256) void rope_kv_block_kernel(RopeKvParams p, int 
     const size_t tok = (size_t)b * p.S + (live ? t - past : t_lo - past);
     const uint16_t *row = (const uint16_t *)p.qkv + tok * p.stride + (size_t)head * 128;
     const u32x4 rlo = *(const u32x4 *)(row + 8 * c), rhi = *(const u32x4 *)(row + 64 + 8 * c);
-    const float *ct = p.cosT + (size_t)(live ? t : t_lo) * 64 + 8 * c, *st = p.sinT + (size_t)(live ? t : t_lo) * 64 + 8 * c;
-    const f32x4 c0 = *(const f32x4 *)ct, c1 = *(const f32x4 *)(ct + 4), s0 = *(const f32x4 *)st, s1 = *(const f32x4 *)(st + 4);
     float lo[8], hi[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const uint32_t wl = rlo[e >> 1], wh = rhi[e >> 1];
-        const float a = bf16_to_f32((uint16_t)(e & 1 ? wl >> 16 : wl)), bb = bf16_to_f32((uint16_t)(e & 1 ? wh >> 16 : wh));
-        const float cs = e < 4 ? c0[e & 3] : c1[e & 3], sn = e < 4 ? s0[e & 3] : s1[e & 3];
-        // reference: fmsub(q, cos, qHalf*sin) ; fmadd(qHalf, cos, q*sin)
-        lo[e] = fmaf(a, cs, -(bb * sn));
-        hi[e] = fmaf(bb, cs, a * sn);
+        lo[e] = bf16_to_f32((uint16_t)(e & 1 ? wl >> 16 : wl)), hi[e] = bf16_to_f32((uint16_t)(e & 1 ? wh >> 16 : wh));
+    }
+    if (p.cosT) {
+        const float *ct = p.cosT + (size_t)(live ? t : t_lo) * 64 + 8 * c, *st = p.sinT + (size_t)(live ? t : t_lo) * 64 + 8 * c;
+        const f32x4 c0 = *(const f32x4 *)ct, c1 = *(const f32x4 *)(ct + 4), s0 = *(const f32x4 *)st, s1 = *(const f32x4 *)(st + 4);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float a = lo[e], bb = hi[e];
+            const float cs = e < 4 ? c0[e & 3] : c1[e & 3], sn = e < 4 ? s0[e & 3] : s1[e & 3];
+            // reference: fmsub(q, cos, qHalf*sin) ; fmadd(qHalf, cos, q*sin)
+            lo[e] = fmaf(a, cs, -(bb * sn));
+            hi[e] = fmaf(bb, cs, a * sn);
+        }
     }
     if (isq) {
         if (live) {
@@ -586,10 +594,10 @@ int xfthip_rope_tables_create(int dim, int maxPos, int base, float scalingFactor
 static int launch_rope(const RopeKvParams &p, int tokens, hipStream_t stream) {
     const int half = p.D / 2;
     // many tokens of fused bf16 rows into a cache: the block form (see rope_kv_block_kernel for what it assumes)
-    if (p.kv.k && p.S >= 16 && p.D == 128 && p.dtype == XFTHIP_BF16 && p.cosT && !p.table_full && !p.positions && !p.key &&
+    if (p.kv.k && p.S >= 16 && p.D == 128 && p.dtype == XFTHIP_BF16 && !p.table_full && !p.positions && !p.key &&
             p.stride % 8 == 0 && ((uintptr_t)p.qkv & 15) == 0 && ((uintptr_t)p.cosT & 15) == 0 && ((uintptr_t)p.sinT & 15) == 0) {
         const int nblk = (p.S + 31) / 32 + 1; // cache blocks an append of S tokens can touch
-        dim3 grid(p.qHeads + p.kvHeads, p.B * nblk);
+        dim3 grid((p.cosT ? p.qHeads : 0) + p.kvHeads, p.B * nblk);
         if (p.kv.int8) hipLaunchKernelGGL(rope_kv_block_kernel<true>, grid, dim3(256), 0, stream, p, nblk);
         else hipLaunchKernelGGL(rope_kv_block_kernel<false>, grid, dim3(256), 0, stream, p, nblk);
         XFT_CHECK_HIP(hipGetLastError());
