@@ -114,6 +114,21 @@ def test_paged_prefill_matches_oracle(xh, orc, qH, kvH, lens, block_size):
     assert err <= 2e-2 and _cos(got, ref) >= 0.9999
 
 
+@pytest.mark.parametrize("B,qH,kvH,block_size,max_ctx", [(2, 40, 2, 5, 200), (1, 8, 8, 3, 33), (4, 16, 4, 16, 129), (70, 8, 1, 16, 500), (2, 68, 4, 7, 1500)])
+def test_paged_decode_column_groups(xh, orc, B, qH, kvH, block_size, max_ctx):
+    """Groups of more than 16 query heads (two column groups, the second of one or four columns), one head a group, block sizes that
+    are no power of two, contexts one token past a 32-token block, and enough (sequence, head) pairs for an unsplit context."""
+    test_paged_decode_matches_oracle(xh, orc, B, qH, kvH, block_size, max_ctx)
+
+
+@pytest.mark.parametrize("qH,kvH,lens,block_size", [(32, 4, [33, 500, 1, 700, 65], 16), (16, 4, [31, 32, 33, 64, 96, 97], 5), (8, 8, [40] * 70, 16),
+                                                    (24, 3, [600, 200, 450, 20, 7], 16), (4, 2, [3, 90, 17], 4)])
+def test_paged_prefill_side_by_side(xh, orc, qH, kvH, lens, block_size):
+    """Sequences that share a launch: unequal lengths about the 32-token block, more sequences than a launch takes, (sequence, KV head)
+    pairs that do not divide among eight, and so little work that the 16-column form runs."""
+    test_paged_prefill_matches_oracle(xh, orc, qH, kvH, lens, block_size)
+
+
 def test_invoke_attention_serving_loop(orc):
     """xft::invokeAttention on host buffers: prefill of two sequences, then decode steps that append to
     the paged cache; outputs against the oracle and the caller's cache arrays kept current."""

@@ -158,7 +158,7 @@ enum ScratchPurpose {
     kScratchW8a8Codes, // quantised activation rows of xfthip_gemm_w8a8_from_bf16
     kScratchW8a8Stats,
     kScratchPagedParts, // context splits of xfthip_paged_attention_decode
-    kScratchPagedQkv, // fused q|k|v rows of xfthip_paged_attention_prefill
+    kScratchPagedKv, // FP16 keys and values of xfthip_paged_attention_prefill
     kScratchPurposes
 };
 int stream_scratch(ScratchPurpose purpose, hipStream_t stream, size_t bytes, bool zero_new, void **out);

@@ -7,29 +7,28 @@
 //
 // Decode (one new token per sequence), as crossAttention does per (sequence, head): the new key and
 // value rows go to their slots first, then scores = q . K^T in fp32 over context + 1 tokens,
-// softmax(scale * scores) in fp32, out = P . V in fp32, narrowed to bf16.  HBM-bound with one query
-// row, so the products run on the vector ALUs: 16 lanes share a token (8 dims each, one 128-bit
-// load per lane), a wave covers 4 tokens per load, (max, sum, out) run as an online softmax per
-// lane group and are merged through LDS; long contexts are split over workgroups whose partials a
-// second kernel merges in a fixed order.
+// softmax(scale * scores) in fp32, out = P . V in fp32, narrowed to bf16.  HBM-bound: the query heads
+// that share a key / value head are the columns of matrix products (paged_decode_kernel), so that the
+// cache is read once a group; long contexts are split over workgroups whose partials a second kernel
+// merges in a fixed order.
 // Where this build departs from the reference's text: sequence b uses query / key / value row b
 // (the reference reads row 0 for every sequence: no batch offset at attention_kernels.cpp:51,61,
 // right only for batch_size = 1) and query head i uses KV head i / (q_heads / kv_heads) (the
 // reference indexes the KV head with the query head, right only without grouped heads).
 //
 // Prefill: causal self-attention of every sequence over its own new tokens (the reference's
-// selfAttention call), through this library's FP16-cache attention kernel on a scratch cache, and
-// every token's key / value row stored to its slot (slot_mapping holds one entry per token; the
-// reference's closures, marked "TODO: debug and fix", pass only slot_mapping[b]).
-#include <map>
-#include <mutex>
+// selfAttention call), through this library's FP16-cache attention kernels on a scratch copy of the
+// keys and values, and every token's key / value row stored to its slot (slot_mapping holds one entry
+// per token; the reference's closures, marked "TODO: debug and fix", pass only slot_mapping[b]).
+// All sequences of a call go through the same launches.
+#include <algorithm>
+#include <vector>
 
-#include "common.h"
+#include "attention_dev.h"
+#include "attention_prefill.h"
 
 namespace xfthip {
 namespace {
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct PagedParams {
     uint16_t *out; // bf16 [batch, o_stride]
@@ -56,126 +55,321 @@ __global__ __launch_bounds__(256) void paged_store_kernel(uint16_t *kc, uint16_t
     }
 }
 
-__device__ inline void unpack8(const u32x4 &w, float (&f)[8]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        f[2 * i] = __uint_as_float(w[i] << 16);
-        f[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
-    }
-}
+union BFrag {
+    bf16x8 v;
+    uint32_t u[4];
+    u32x4 q;
+};
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
-// grid (nsplit, q_heads, batch), 256 threads.  head_size = 128.
-__global__ __launch_bounds__(256) void paged_decode_kernel(PagedParams p) {
-    constexpr int D = 128, U = 4;
-    __shared__ float s_m[16], s_l[16], s_o[16][D];
-    const int split = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int grp = lane >> 4, sub = lane & 15; // token phase, dims 8 sub .. 8 sub + 7
-    const int kvh = hq / (p.q_heads / p.kv_heads);
+// grid (nsplit, kv_heads * column groups, batch), 256 threads.  head_size = 128.
+// The columns of a workgroup are up to 16 query heads of one key / value head; a wave takes every fourth 32-token block of
+// the workgroup's part of the context.
+//   S^T[token][col] = K . Q^T: v_mfma_f32_16x16x32_bf16, A = key rows straight from the cache (products of bf16 values
+//     in fp32, as before), lane (cl, g) holds dims 32 s + 8 g .. + 7 of token row cl in step s
+//   O^T[dim][col] += V^T . P^T: the A operand wants 8 tokens of one dim a lane.  A lane loads dims 8 cl .. + 7 of 8 tokens
+//     (whole 256-byte rows across 16 lanes), turns its 8 x 8 values round with 32 byte permutes and so holds the operands
+//     of 8 products whose row r stands for dim 8 r + j - no LDS, no exchange.  Lane group g takes the tokens 4 g .. + 3 of
+//     both 16-token score tiles, the ones whose probabilities it holds.
+// The probabilities stay at 16 bits of mantissa and more: each goes in as the sum of two bf16 values (upper half, rounded
+// rest), one product each; sums of probabilities are those of the fp32 values.
+// The next block's keys are requested once this block's scores are done, its values once this block's are turned; the
+// cache rows of the block after that (a table look-up a lane) a block earlier.
+// Bound by the cache's trip from HBM.  32 sequences of 2100 .. 4100 tokens, 32 query / 8 KV heads, 408 MB:
+// 86 us, 4.7 TB/s (244 us with a workgroup a query head on the vector ALUs, every head of a group reading the cache again).  212
+// registers, two workgroups a CU; held to three, 63 of them spill.
+__global__ __launch_bounds__(256, 2) void paged_decode_kernel(PagedParams p) {
+    constexpr int D = 128;
+    __shared__ float s_m[4][16], s_l[4][16], s_o[4][16][D + 4];
+    const int split = blockIdx.x, b = blockIdx.z;
+    const int kvh = blockIdx.y % p.kv_heads, cg = blockIdx.y / p.kv_heads;
+    const int G = p.q_heads / p.kv_heads, cols = min(16, G - cg * 16);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, cl = lane & 15;
     // tokens to attend to, the new one included (never more than the table describes)
     const int n = min(max(p.ctx[b], 0) + 1, p.table_stride * p.block_size);
-    // tokens of this split: whole 16-token rounds
-    const int rounds = (n + 15) / 16;
-    const int r0 = (int)((long)rounds * split / p.nsplit), r1 = (int)((long)rounds * (split + 1) / p.nsplit);
+    const int nblk = (n + 31) >> 5;
+    const int b0 = (int)((long)nblk * split / p.nsplit), b1 = (int)((long)nblk * (split + 1) / p.nsplit);
     const int *table = p.tables + (size_t)b * p.table_stride;
-    const size_t row = (size_t)p.kv_heads * D;
+    const size_t row_bytes = (size_t)p.kv_heads * D * 2;
+    const char *kbase = (const char *)p.kc + kvh * (D * 2) + g * 16;
+    const char *vbase = (const char *)p.vc + kvh * (D * 2) + cl * 16;
 
-    float q[8];
-    unpack8(*(const u32x4 *)(p.q + (size_t)b * p.q_stride + hq * D + sub * 8), q);
-    float m = -INFINITY, l = 0.0f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int r = r0; r < r1; r += U) {
-        u32x4 kk[U], vv[U];
-        bool ok[U];
+    // cache row of token 32 blk + (lane & 31); past the end the last token's (a valid row, masked below)
+    auto row_of = [&](int blk) {
+        const int t = min(32 * blk + (lane & 31), n - 1);
+        const int at = t / p.block_size;
+        return min(max(table[at], 0), p.block_num - 1) * p.block_size + (t - at * p.block_size); // a bad table entry reads a valid block
+    };
+    BFrag kf[2][4], vf[8], qf[4];
+    auto load_keys = [&](int rows) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int t = (r + u) * 16 + wave * 4 + grp;
-            ok[u] = r + u < r1 && t < n;
-            const int tc = ok[u] ? t : 0; // masked lanes read token 0 (always present) and drop it
-            const int blk = min(max(table[tc / p.block_size], 0), p.block_num - 1); // a bad table entry reads a valid block
-            const size_t at = ((size_t)blk * p.block_size + tc % p.block_size) * row + kvh * D + sub * 8;
-            kk[u] = *(const u32x4 *)(p.kc + at);
-            vv[u] = *(const u32x4 *)(p.vc + at);
+        for (int a = 0; a < 2; ++a) {
+            const char *src = kbase + (size_t)__shfl(rows, 16 * a + cl, 64) * row_bytes;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) kf[a][s].q = *(const u32x4 *)(src + 64 * s);
         }
+    };
+    auto load_values = [&](int rows) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            float kf[8], vf[8];
-            unpack8(kk[u], kf);
-            float s = 0.0f;
+        for (int i = 0; i < 8; ++i) vf[i].q = *(const u32x4 *)(vbase + (size_t)__shfl(rows, 16 * (i >> 2) + 4 * g + (i & 3), 64) * row_bytes);
+    };
+    int blk = b0 + wave;
+    int rows_next = 0;
+    if (blk < b1) {
+        const int rows = row_of(blk);
+        load_keys(rows);
+        load_values(rows);
+        rows_next = row_of(min(blk + 4, nblk - 1));
+    }
+    {
+        const uint16_t *qrow = p.q + (size_t)b * p.q_stride + (size_t)(kvh * G + cg * 16 + min(cl, cols - 1)) * D + 8 * g;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s = fmaf(q[i], kf[i], s);
-            s += __shfl_xor(s, 1, 64);
-            s += __shfl_xor(s, 2, 64);
-            s += __shfl_xor(s, 4, 64);
-            s += __shfl_xor(s, 8, 64);
-            if (!ok[u]) continue; // uniform over the 16 lanes of a token
-            s *= p.scale;
-            const float mn = fmaxf(m, s);
-            const float c = __expf(m - mn), e = __expf(s - mn); // exp(-inf) = 0 on the first token
-            unpack8(vv[u], vf);
-            l = l * c + e;
+        for (int s = 0; s < 4; ++s) qf[s].q = *(const u32x4 *)(qrow + 32 * s);
+    }
+    float m = -INFINITY, l = 0.0f;
+    f32x4 o[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) o[i] = fmaf(e, vf[i], o[i] * c);
-            m = mn;
+    for (int j = 0; j < 8; ++j) o[j] = f32x4 {0.f, 0.f, 0.f, 0.f};
+    for (; blk < b1; blk += 4) {
+        const bool more = blk + 4 < b1; // (uniform over the wave)
+        f32x4 sc[2];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            sc[a] = f32x4 {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) sc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[a][s].v, qf[s].v, sc[a], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) load_keys(rows_next);
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- online softmax: this lane's column, tokens 16 a + 4 g + r of the block ----
+        float bmax = -INFINITY;
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const bool seen = 32 * blk + 16 * a + 4 * g + r < n;
+                sc[a][r] = seen ? sc[a][r] * p.scale : -INFINITY;
+                bmax = fmaxf(bmax, sc[a][r]);
+            }
+        bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
+        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
+        const float m_new = fmaxf(m, bmax);
+        const float ref = m_new == -INFINITY ? 0.0f : m_new; // (nothing but minus infinity so far: exp() gives zeros)
+        const float alpha = __expf(m - ref);
+        m = m_new;
+        float e[8], psum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            e[i] = __expf(sc[i >> 2][i & 3] - ref);
+            psum += e[i];
+        }
+        l = l * alpha + psum;
+        BFrag hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float x = e[2 * i], y = e[2 * i + 1];
+            hi.u[i] = __builtin_amdgcn_perm(f2u(y), f2u(x), 0x07060302u);
+            const f32x2_t rest = {x - u2f(f2u(x) & 0xFFFF0000u), y - u2f(f2u(y) & 0xFFFF0000u)};
+            lo.u[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, bf16x2_t));
+        }
+        // ---- values: 8 tokens x 8 dims turned round, then O^T ----
+        BFrag vt[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                vt[j].u[i] = __builtin_amdgcn_perm(vf[2 * i + 1].u[j >> 1], vf[2 * i].u[j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) {
+            load_values(rows_next);
+            rows_next = row_of(min(blk + 8, nblk - 1));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            o[j] = o[j] * alpha;
+            o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[j].v, lo.v, o[j], 0, 0, 0);
+            o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[j].v, hi.v, o[j], 0, 0, 0);
         }
     }
-    // merge the 16 (wave, phase) partials of the workgroup
-    const int slot = wave * 4 + grp;
-    if (sub == 0) s_m[slot] = m, s_l[slot] = l;
+    // ---- merge the four waves; row 4 g + r of product j is dim 8 (4 g + r) + j ----
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (g == 0) s_m[wave][cl] = m, s_l[wave][cl] = l;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) s_o[slot][sub * 8 + i] = o[i];
+    for (int r = 0; r < 4; ++r) {
+        float *dst = &s_o[wave][cl][8 * (4 * g + r)];
+        *(f32x4 *)dst = f32x4 {o[0][r], o[1][r], o[2][r], o[3][r]};
+        *(f32x4 *)(dst + 4) = f32x4 {o[4][r], o[5][r], o[6][r], o[7][r]};
+    }
     __syncthreads();
-    if (threadIdx.x < D) {
-        float mm = -INFINITY;
-        for (int s = 0; s < 16; ++s) mm = fmaxf(mm, s_m[s]);
+    for (int v = threadIdx.x; v < cols * D; v += 256) {
+        const int col = v / D, d = v % D, hq = kvh * G + cg * 16 + col;
+        const float mm = fmaxf(fmaxf(s_m[0][col], s_m[1][col]), fmaxf(s_m[2][col], s_m[3][col]));
         float ll = 0.0f, acc = 0.0f;
-        for (int s = 0; s < 16; ++s) {
-            const float f = s_m[s] == -INFINITY ? 0.0f : __expf(s_m[s] - mm);
-            ll = fmaf(s_l[s], f, ll);
-            acc = fmaf(s_o[s][threadIdx.x], f, acc);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float f = s_m[w][col] == -INFINITY ? 0.0f : __expf(s_m[w][col] - mm);
+            ll = fmaf(s_l[w][col], f, ll);
+            acc = fmaf(s_o[w][col][d], f, acc);
         }
-        float *dst = p.part + (((size_t)b * p.q_heads + hq) * p.nsplit + split) * (D + 2);
-        if (threadIdx.x == 0) dst[0] = mm, dst[1] = ll;
-        dst[2 + threadIdx.x] = acc;
+        if (p.nsplit == 1) {
+            p.out[(size_t)b * p.o_stride + hq * D + d] = f32_to_bf16_ref(acc / ll);
+        } else {
+            float *dst = p.part + (((size_t)b * p.q_heads + hq) * p.nsplit + split) * (D + 2);
+            if (d == 0) dst[0] = mm, dst[1] = ll;
+            dst[2 + d] = acc;
+        }
     }
 }
 
-// grid (q_heads, batch), 128 threads: fixed-order merge of the splits, normalisation, bf16 output
+// grid (q_heads, batch), 128 threads: fixed-order merge of at most 32 splits, normalisation, bf16 output.  All the partials a
+// thread needs are requested together: one round trip whatever the number of splits.
+constexpr int kMaxSplits = 32;
 __global__ __launch_bounds__(128) void paged_merge_kernel(PagedParams p) {
     constexpr int D = 128;
-    const int hq = blockIdx.x, b = blockIdx.y;
+    __shared__ float s_m[kMaxSplits], s_l[kMaxSplits];
+    const int hq = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
     const float *src = p.part + ((size_t)b * p.q_heads + hq) * p.nsplit * (D + 2);
-    float mm = -INFINITY;
-    for (int s = 0; s < p.nsplit; ++s) mm = fmaxf(mm, src[(size_t)s * (D + 2)]);
-    float ll = 0.0f, acc = 0.0f;
-    for (int s = 0; s < p.nsplit; ++s) {
-        const float ms = src[(size_t)s * (D + 2)];
-        const float f = ms == -INFINITY ? 0.0f : __expf(ms - mm);
-        ll = fmaf(src[(size_t)s * (D + 2) + 1], f, ll);
-        acc = fmaf(src[(size_t)s * (D + 2) + 2 + threadIdx.x], f, acc);
+    if (d < p.nsplit) {
+        const float2 ml = *(const float2 *)(src + (size_t)d * (D + 2));
+        s_m[d] = ml.x, s_l[d] = ml.y;
     }
-    p.out[(size_t)b * p.o_stride + hq * D + threadIdx.x] = f32_to_bf16_ref(acc / ll);
+    float acc = 0.0f, ll = 0.0f, mm = -INFINITY;
+    float t[kMaxSplits];
+#pragma unroll
+    for (int s = 0; s < kMaxSplits; ++s) t[s] = s < p.nsplit ? src[(size_t)s * (D + 2) + 2 + d] : 0.0f;
+    __syncthreads();
+    for (int s = 0; s < p.nsplit; ++s) mm = fmaxf(mm, s_m[s]);
+#pragma unroll
+    for (int s = 0; s < kMaxSplits; ++s)
+        if (s < p.nsplit) {
+            const float f = s_m[s] == -INFINITY ? 0.0f : __expf(s_m[s] - mm);
+            ll = fmaf(s_l[s], f, ll);
+            acc = fmaf(t[s], f, acc);
+        }
+    p.out[(size_t)b * p.o_stride + hq * D + d] = f32_to_bf16_ref(acc / ll);
 }
 
-// q | k | v rows of one sequence -> one fused [tokens, (qH + 2 kvH) * D] bf16 buffer
-__global__ __launch_bounds__(256) void paged_fuse_qkv_kernel(uint16_t *qkv, const uint16_t *q, const uint16_t *k, const uint16_t *v,
-        int q_stride, int kv_stride, int q_elems, int kv_elems) {
-    const int tok = blockIdx.x;
-    uint16_t *dst = qkv + (size_t)tok * (q_elems + 2 * kv_elems);
-    for (int i = threadIdx.x * 8; i < q_elems; i += blockDim.x * 8) *(u32x4 *)(dst + i) = *(const u32x4 *)(q + (size_t)tok * q_stride + i);
-    for (int i = threadIdx.x * 8; i < kv_elems; i += blockDim.x * 8) {
-        *(u32x4 *)(dst + q_elems + i) = *(const u32x4 *)(k + (size_t)tok * kv_stride + i);
-        *(u32x4 *)(dst + q_elems + kv_elems + i) = *(const u32x4 *)(v + (size_t)tok * kv_stride + i);
-    }
-}
-
-// Scratch of the paged entry points, grow-only, one set per stream: the context splits and the fused q|k|v rows come
-// from stream_scratch, the FP16 scratch cache of the prefill from the table below.
-struct PrefillCache {
-    xfthip_kvcache_t cache = nullptr;
-    int heads = 0, seq = 0;
+// ---- prefill: the sequences of a call side by side ---------------------------------------------------------------
+// Sequence i of a launch: tokens from row row0[i] on (row0[i + 1] - row0[i] of them), 32-token blocks from blk0[i] on in the
+// scratch copy (which holds blk0[n] blocks a head).  grp0 (attention): workgroups of an XCD in front of (sequence, KV head) pairs
+// 8 k .. 8 k + 7, used with more than one sequence.  By value: no copy in front of the launch.
+constexpr int kSeqs = 64, kGroups = 256;
+struct SeqBatch {
+    int n;
+    int row0[kSeqs], rows[kSeqs], blk0[kSeqs + 1];
+    int grp0[kGroups + 1];
 };
-std::mutex g_mu;
-std::map<hipStream_t, PrefillCache> g_prefill_cache;
+
+__device__ inline int seq_of_block(const SeqBatch &s, int blk) {
+    int lo = 0, hi = s.n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (s.blk0[mid] <= blk) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// One workgroup a (KV head, 32-token block): a token's key and value row go to its slot as they are, to the scratch copy in FP16,
+// the values turned into the [dim][32 slots] tile the attention kernels read (kvcache.h).  Slots of a block past the sequence's
+// end are zero: what lies there is multiplied by a probability of zero.
+// (6 sequences of 750 .. 1500 tokens, 32 query / 8 KV heads: the slots' store, a fused q | k | v copy, an append and an attention launch a
+// sequence took 11 + 28 + 6 x (14 + 43) us, 366 the call; one store and one attention launch 143.  3 x 60 tokens 38 -> 13 us.)
+__global__ __launch_bounds__(256) void paged_prefill_store_kernel(SeqBatch s, KvView kv, uint16_t *kc, uint16_t *vc, const uint16_t *k, const uint16_t *v,
+        const int *slots, int kv_stride, int slot_num) {
+    __shared__ __attribute__((aligned(16))) uint16_t tile[128 * 32];
+    const int kvh = blockIdx.y, blk = blockIdx.x, i = seq_of_block(s, blk);
+    const int t0 = 32 * (blk - s.blk0[i]), tl = threadIdx.x >> 3, c = threadIdx.x & 7;
+    const bool live = t0 + tl < s.rows[i];
+    const size_t tok = (size_t)s.row0[i] + t0 + tl;
+    u32x4 x[4]; // keys 8 c .. and 64 + 8 c .., values the same
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = u32x4 {0u, 0u, 0u, 0u};
+    if (live) {
+        const uint16_t *kr = k + tok * kv_stride + kvh * 128 + 8 * c, *vr = v + tok * kv_stride + kvh * 128 + 8 * c;
+        x[0] = *(const u32x4 *)kr, x[1] = *(const u32x4 *)(kr + 64), x[2] = *(const u32x4 *)vr, x[3] = *(const u32x4 *)(vr + 64);
+        const int slot = slots[tok];
+        if (slot >= 0 && slot < slot_num) { // a slot outside the cache is dropped, never written
+            const size_t dst = ((size_t)slot * kv.H + kvh) * 128 + 8 * c;
+            *(u32x4 *)(kc + dst) = x[0], *(u32x4 *)(kc + dst + 64) = x[1];
+            *(u32x4 *)(vc + dst) = x[2], *(u32x4 *)(vc + dst + 64) = x[3];
+        }
+    }
+    uint16_t h[4][8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) h[e][j] = f32_to_fp16_bits(u2f(j & 1 ? x[e][j >> 1] & 0xFFFF0000u : x[e][j >> 1] << 16));
+    uint16_t *kd = (uint16_t *)kv.k + ((size_t)kvh * kv.S + 32 * blk + tl) * 128 + 8 * c;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        u32x4 w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = (uint32_t)h[e][2 * j] | ((uint32_t)h[e][2 * j + 1] << 16);
+        *(u32x4 *)(kd + 64 * e) = w;
+    }
+    const int slot_in = v_slot(tl);
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) tile[(64 * e + 8 * c + j) * 32 + slot_in] = h[2 + e][j];
+    __syncthreads();
+    u32x4 *vd = (u32x4 *)((uint16_t *)kv.v + ((size_t)kvh * (kv.S / 32) + blk) * 128 * 32);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) vd[threadIdx.x + 256 * e] = ((const u32x4 *)tile)[threadIdx.x + 256 * e];
+}
+
+// the parameters of sequence i of a batch
+__device__ inline AttnParams seq_params(const AttnParams &all, const SeqBatch &s, int i) {
+    AttnParams p = all;
+    p.S = s.rows[i];
+    p.CG = (p.S * p.G + 15) / 16;
+    p.q += (size_t)s.row0[i] * p.qStride;
+    p.out = (uint16_t *)p.out + (size_t)s.row0[i] * p.oStride;
+    p.kv.k = (uint16_t *)p.kv.k + (size_t)s.blk0[i] * 32 * 128;
+    p.kv.v = (uint16_t *)p.kv.v + (size_t)s.blk0[i] * 32 * 128;
+    return p;
+}
+
+// attn_prefill32_kernel over the sequences: (sequence, KV head) pairs go to the XCDs in turn, an XCD walks the column groups of one
+// pair, longest history first, before it starts the next
+__global__ __launch_bounds__(256, 2) void paged_prefill_attn_kernel(AttnParams all, SeqBatch s) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[3 * 16384];
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    int group, at;
+    if (s.n == 1) {
+        const int ncg = (s.rows[0] * all.G + 127) / 128;
+        group = slot / ncg, at = slot % ncg;
+    } else {
+        int lo = 0, hi = (s.n * all.kv.H + 7) / 8 - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (s.grp0[mid] <= slot) lo = mid;
+            else hi = mid - 1;
+        }
+        group = lo, at = slot - s.grp0[lo];
+    }
+    const int pair = group * 8 + xcd, i = pair / all.kv.H;
+    if (i >= s.n) return;
+    const AttnParams p = seq_params(all, s, i);
+    const int ncg = (p.S * p.G + 127) / 128;
+    if (at >= ncg) return; // (a longer sequence shares the group)
+    attn_prefill32_unit<4, 1, false>(p, pair % all.kv.H, ncg - 1 - at, 0, lds);
+}
+
+// attn_kernel over the sequences, each walked by one workgroup a column group: grid (KV heads x the longest's column groups, sequences)
+__global__ __launch_bounds__(256, 3) void paged_prefill_few_kernel(AttnParams all, SeqBatch s) {
+    __shared__ AttnLds<4> lds;
+    const AttnParams p = seq_params(all, s, blockIdx.y);
+    const int cg = blockIdx.x / all.kv.H;
+    if (cg >= p.CG) return;
+    attn_unit<false, 4, false>(p, 0, blockIdx.x % all.kv.H, cg, 0, lds, [] { __syncthreads(); });
+}
 
 int check_common(const void *out, const void *q, const void *k, const void *v, int q_heads, int kv_heads, int head_size, int q_stride,
         int kv_stride, int o_stride, const void *kc, const void *vc, int block_size) {
@@ -206,15 +400,19 @@ extern "C" int xfthip_paged_attention_decode(void *out, const void *q, const voi
             max_context / block_size + 1, table_stride);
     XFT_REQUIRE(block_num > 0, "xfthip_paged_attention_decode: bad block count");
     hipStream_t st = (hipStream_t)stream;
-    // enough workgroups to fill the device, at least 64 tokens a split
-    int nsplit = (4 * device_cu_count() + batch * q_heads - 1) / (batch * q_heads);
-    const int cap = (max_context + 1 + 63) / 64;
+    // One workgroup a CU, at least one 32-token block a wave (1, 2 or 4 workgroups a CU: 1 x 1000 tokens, 8 KV heads 10.3 / 11.7 / 11.6 us,
+    // 64 x 500, 4 KV heads 15.0 / 17.5 / 19.1, 1 x 9000 16.8 / 16.8 / 16.9, 32 x 4100 86.6 / 87.2 / 85.2; 64 splits in place of 32 cost
+    // 1 x 9000 2.5 us)
+    const int colgroups = (q_heads / kv_heads + 15) / 16, units = batch * kv_heads * colgroups;
+    int nsplit = (device_cu_count() + units - 1) / units;
+    const int cap = (max_context + 1 + 127) / 128;
     if (nsplit > cap) nsplit = cap;
-    if (nsplit > 64) nsplit = 64;
+    if (nsplit > kMaxSplits) nsplit = kMaxSplits;
     if (nsplit < 1) nsplit = 1;
     const size_t need = (size_t)batch * q_heads * nsplit * 130;
     void *part = nullptr;
-    if (int rc = stream_scratch(kScratchPagedParts, st, need * sizeof(float), false, &part)) return rc;
+    if (nsplit > 1)
+        if (int rc = stream_scratch(kScratchPagedParts, st, need * sizeof(float), false, &part)) return rc;
     PagedParams p = {};
     p.out = (uint16_t *)out, p.q = (const uint16_t *)q, p.kc = (const uint16_t *)kcache, p.vc = (const uint16_t *)vcache;
     p.tables = block_tables, p.ctx = context_lens, p.part = (float *)part;
@@ -222,8 +420,8 @@ extern "C" int xfthip_paged_attention_decode(void *out, const void *q, const voi
     p.block_size = block_size, p.block_num = block_num, p.nsplit = nsplit, p.scale = scale;
     hipLaunchKernelGGL(paged_store_kernel, dim3(batch), dim3(256), 0, st, (uint16_t *)kcache, (uint16_t *)vcache, (const uint16_t *)k,
             (const uint16_t *)v, slot_mapping, kv_stride, kv_heads * 128, block_num * block_size);
-    hipLaunchKernelGGL(paged_decode_kernel, dim3(nsplit, q_heads, batch), dim3(256), 0, st, p);
-    hipLaunchKernelGGL(paged_merge_kernel, dim3(q_heads, batch), dim3(128), 0, st, p);
+    hipLaunchKernelGGL(paged_decode_kernel, dim3(nsplit, kv_heads * colgroups, batch), dim3(256), 0, st, p);
+    if (nsplit > 1) hipLaunchKernelGGL(paged_merge_kernel, dim3(q_heads, batch), dim3(128), 0, st, p);
     XFT_CHECK_HIP(hipGetLastError());
     return 0;
 }
@@ -235,46 +433,61 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
     XFT_REQUIRE(batch > 0 && token_lens_host && slot_mapping && block_num > 0, "xfthip_paged_attention_prefill: bad argument");
     XFT_REQUIRE(o_stride % 8 == 0, "xfthip_paged_attention_prefill: o_stride must be a multiple of 8 elements");
     hipStream_t st = (hipStream_t)stream;
-    int total = 0, longest = 0;
-    for (int b = 0; b < batch; ++b) {
+    for (int b = 0; b < batch; ++b)
         XFT_REQUIRE(token_lens_host[b] > 0, "xfthip_paged_attention_prefill: sequence %d has %d tokens", b, token_lens_host[b]);
-        total += token_lens_host[b];
-        if (token_lens_host[b] > longest) longest = token_lens_host[b];
+    // launches of up to kSeqs sequences (and kGroups groups of 8 (sequence, KV head) pairs), the longest first
+    const int per_launch = std::max(1, std::min(kSeqs, kGroups * 8 / kv_heads - 1));
+    std::vector<int> order(batch), first(batch);
+    for (int b = 0, at = 0; b < batch; at += token_lens_host[b], ++b) order[b] = b, first[b] = at;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return token_lens_host[x] > token_lens_host[y]; });
+    size_t most = 0; // 32-token blocks of the largest launch
+    for (int b = 0; b < batch; b += per_launch) {
+        size_t blocks = 0;
+        for (int i = b; i < batch && i < b + per_launch; ++i) blocks += (token_lens_host[order[i]] + 31) / 32;
+        most = std::max(most, blocks);
     }
-    const int q_elems = q_heads * 128, kv_elems = kv_heads * 128, fused = q_elems + 2 * kv_elems;
-    void *fused_rows = nullptr;
-    if (int rc = stream_scratch(kScratchPagedQkv, st, (size_t)total * fused * 2, false, &fused_rows)) return rc;
-    uint16_t *g_qkv = (uint16_t *)fused_rows;
-    xfthip_kvcache_t g_cache = nullptr;
-    {
-        std::lock_guard<std::mutex> lk(g_mu);
-        PrefillCache &pc = g_prefill_cache[st];
-        if (pc.cache == nullptr || pc.heads != kv_heads || pc.seq < longest) {
-            if (pc.cache) {
-                XFT_CHECK_HIP(hipDeviceSynchronize());
-                (void)xfthip_kvcache_destroy(pc.cache);
-                pc.cache = nullptr;
-            }
-            const int seq = ((longest + 255) / 256) * 256;
-            if (int rc = xfthip_kvcache_create(XFTHIP_FP16, 1, kv_heads, seq, 128, &pc.cache)) return rc;
-            pc.heads = kv_heads, pc.seq = seq;
+    void *scratch = nullptr;
+    if (int rc = stream_scratch(kScratchPagedKv, st, most * 32 * kv_heads * 128 * 4, false, &scratch)) return rc;
+    const int G = q_heads / kv_heads;
+    for (int b = 0; b < batch; b += per_launch) {
+        SeqBatch s = {};
+        s.n = std::min(per_launch, batch - b);
+        long waves = 0; // of 16 columns
+        for (int i = 0; i < s.n; ++i) {
+            const int S = token_lens_host[order[b + i]];
+            s.row0[i] = first[order[b + i]], s.rows[i] = S, s.blk0[i + 1] = s.blk0[i] + (S + 31) / 32;
+            waves += (long)kv_heads * (((long)S * G + 15) / 16);
         }
-        g_cache = pc.cache;
-    }
-    hipLaunchKernelGGL(paged_store_kernel, dim3(total), dim3(256), 0, st, (uint16_t *)kcache, (uint16_t *)vcache, (const uint16_t *)k,
-            (const uint16_t *)v, slot_mapping, kv_stride, kv_elems, block_num * block_size);
-    hipLaunchKernelGGL(paged_fuse_qkv_kernel, dim3(total), dim3(256), 0, st, g_qkv, (const uint16_t *)q, (const uint16_t *)k,
-            (const uint16_t *)v, q_stride, kv_stride, q_elems, kv_elems);
-    XFT_CHECK_HIP(hipGetLastError());
-    int first = 0;
-    for (int b = 0; b < batch; ++b) {
-        const int S = token_lens_host[b];
-        uint16_t *rows = g_qkv + (size_t)first * fused;
-        if (int rc = xfthip_rope_kvstore(g_cache, rows, XFTHIP_BF16, fused, 1, S, q_heads, nullptr, nullptr, 0, nullptr, stream)) return rc;
-        if (int rc = attention_launch(g_cache, rows, fused, (uint16_t *)out + (size_t)first * o_stride, o_stride, XFTHIP_BF16, 1, S, q_heads,
-                    scale, 0, nullptr, 0, st, nullptr, false))
-            return rc;
-        first += S;
+        const int blocks = s.blk0[s.n];
+        KvView kv = {};
+        kv.B = 1, kv.H = kv_heads, kv.S = 32 * blocks, kv.D = 128;
+        kv.k = scratch, kv.v = (uint16_t *)scratch + (size_t)32 * blocks * kv_heads * 128;
+        hipLaunchKernelGGL(paged_prefill_store_kernel, dim3(blocks, kv_heads), dim3(256), 0, st, s, kv, (uint16_t *)kcache, (uint16_t *)vcache,
+                (const uint16_t *)k, (const uint16_t *)v, slot_mapping, kv_stride, block_num * block_size);
+        if (s.n == 1) {
+            // one sequence: the rules of attention over a contiguous cache, splits of a short one's keys among them
+            xfthip_kvcache cache = {};
+            cache.kv = kv, cache.maxSeq = s.rows[0];
+            XFT_CHECK_HIP(hipGetLastError());
+            if (int rc = attention_launch(&cache, (const uint16_t *)q + (size_t)s.row0[0] * q_stride, q_stride,
+                        (uint16_t *)out + (size_t)s.row0[0] * o_stride, o_stride, XFTHIP_BF16, 1, s.rows[0], q_heads, scale, 0, nullptr, 0, st, nullptr, false))
+                return rc;
+            continue;
+        }
+        AttnParams p = {};
+        p.kv = kv, p.q = (const uint16_t *)q, p.qStride = q_stride, p.out = out, p.oStride = o_stride, p.out_dtype = XFTHIP_BF16;
+        p.B = 1, p.G = G, p.scale = scale, p.nsplit = 1;
+        if (waves >= 4L * device_cu_count()) { // the rule of attention_launch, over all sequences
+            const int groups = (s.n * kv_heads + 7) / 8;
+            for (int g = 0; g < groups; ++g) { // (the sequences are sorted: the group's first pair belongs to its longest)
+                const int ncg = (int)(((long)s.rows[g * 8 / kv_heads] * G + 127) / 128);
+                s.grp0[g + 1] = s.grp0[g] + ncg;
+            }
+            hipLaunchKernelGGL(paged_prefill_attn_kernel, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
+        } else {
+            hipLaunchKernelGGL(paged_prefill_few_kernel, dim3(kv_heads * ((s.rows[0] * G + 15) / 16), s.n), dim3(256), 0, st, p, s);
+        }
+        XFT_CHECK_HIP(hipGetLastError());
     }
     return 0;
 }
