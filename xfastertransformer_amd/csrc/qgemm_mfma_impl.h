@@ -50,28 +50,29 @@ __device__ inline float silu_big(float x) {
 // KIND: weight kind; WN: 32-column tiles per wave (4 waves per block split the columns);
 // WM: 32-row activation tiles per block (shared by the waves through LDS); NEED_SUM: accumulate
 // row sums of A for the zero-point term; KTAIL: K is not a whole number of tiles.
-template <int KIND>
+template <int KIND, bool DIRECT = false>
 struct StepTraits;
-template <>
-struct StepTraits<XFTHIP_W_INT8> {
+template <bool DIRECT>
+struct StepTraits<XFTHIP_W_INT8, DIRECT> {
     // a lane of half h takes the whole 16-byte chunks of k groups h and 2 + h (one 128-bit load each):
     // the k index of an MFMA is only a summation index, so lane half h of micro-step (g, sb) stands for
     // k = 32 g + 16 h + 8 sb .. + 7 in both operands
     static constexpr int KTILE = 64, GROUPS = 2, SUB = 2, WREGS = 4, PACKED_K = 64;
 };
-template <>
-struct StepTraits<XFTHIP_W_UINT4> {
+template <bool DIRECT>
+struct StepTraits<XFTHIP_W_UINT4, DIRECT> {
     // 16 bytes per lane per k group, 2 MFMAs.  A step covers half a packed tile (two of its four k groups): with the
     // whole 128-deep tile a step the three activation buffers of a 128-row block take 104 KB of LDS, one workgroup a CU
     static constexpr int KTILE = 64, GROUPS = 2, SUB = 2, WREGS = 4, PACKED_K = 128;
 };
-template <>
-struct StepTraits<XFTHIP_W_NF4> {
+template <bool DIRECT>
+struct StepTraits<XFTHIP_W_NF4, DIRECT> {
     static constexpr int KTILE = 64, GROUPS = 2, SUB = 2, WREGS = 4, PACKED_K = 128;
 };
-template <>
-struct StepTraits<XFTHIP_W_BF16> {
-    static constexpr int KTILE = 32, GROUPS = 2, SUB = 1, WREGS = 4, PACKED_K = 32;
+template <bool DIRECT>
+struct StepTraits<XFTHIP_W_BF16, DIRECT> {
+    // DIRECT: a step takes two packed tiles, so that the activation rows are the 128 bytes its LDS layout is made of
+    static constexpr int KTILE = DIRECT ? 64 : 32, GROUPS = DIRECT ? 4 : 2, SUB = 1, WREGS = 4, PACKED_K = 32;
 };
 
 // Row blocks a band: 8, or, with a device-side row count, only as many as the rows the host expects fill: the
@@ -101,6 +102,10 @@ __host__ __device__ inline int band_rows(const SkinnyParams &p) {
 // one workgroup a CU - weights four tiles ahead in five register sets, six LDS tiles requested five steps ahead - was
 // built and measured no faster, 921 / 919 against 953 / 956 TFLOP/s on 2048 x 4096 x 4096 and 2048 x 4096 x 11008:
 // a lone wave a SIMD is not waiting for memory there, it issues its widening and its MFMAs one after the other.)
+// BF16 weights (nothing to widen, twice the bytes of INT8): steps of two packed tiles, two register sets reloaded behind
+// the products that read them (RELOAD), 250 registers.  Against the 128 x 256 tile staged through registers (one
+// workgroup a CU): 2048 x 11008 x 4096 206 -> 168 us (1.10 PFLOP/s), 4096 x 28672 x 4096 with SwiGLU 1043 -> 798 us
+// (1.21 PFLOP/s), 4096 x 4096 x 4096 136 -> 120 us, 2048 x 4096 x 14336 248 -> 217 us (two K groups).
 //
 // KG = 2 (DIRECT only): the form for launches of at most one block a CU.  Eight waves a workgroup: waves 0..3 take the
 // first half of K, waves 4..7 the second, each group with LDS tiles and a pipeline of its own (the step barriers are
@@ -109,9 +114,9 @@ __host__ __device__ inline int band_rows(const SkinnyParams &p) {
 // through LDS, which runs the epilogue.
 template <int KIND, int WN, int WM, bool NEED_SUM, bool KTAIL, bool DEVROWS = false, bool DIRECT = false, int WSETS = 3, int KG = 1>
 __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_mfma_kernel(SkinnyParams p, int nblocks_n, int nblocks_m) {
-    using T = StepTraits<KIND>;
+    using T = StepTraits<KIND, DIRECT>;
     constexpr int KTILE = T::KTILE, GROUPS = T::GROUPS, SUB = T::SUB, WREGS = T::WREGS;
-    constexpr int PACKED_K = T::PACKED_K, STEPS_PER_TILE = PACKED_K / KTILE; // k of a packed 1-KiB tile; steps that share one
+    constexpr int PACKED_K = T::PACKED_K, STEPS_PER_TILE = PACKED_K >= KTILE ? PACKED_K / KTILE : 1; // k of a packed 1-KiB tile; steps that share one
     constexpr int ROWS = 32 * WM;
     constexpr int ROWB = DIRECT ? KTILE * 2 : KTILE * 2 + 16; // LDS row pitch in bytes (padded when staged through registers)
     static_assert(!DIRECT || (KTILE == 64 && !KTAIL && !DEVROWS && ROWS % 32 == 0), "direct-to-LDS form: 64-deep steps, whole k tiles, host-side row count");
@@ -276,8 +281,12 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     // weight register sets: tile j in set j % WSETS, loaded WSETS - 1 steps ahead.  Three for the large tiles (MFMA
     // bound; the registers are the accumulators'); six for the 32- and 64-row tiles, whose launches are bound by
     // the weights' trip from HBM - with two tiles in flight a step of such a workgroup waited most of a round trip
-    static_assert(WSETS % 3 == 0 && (!DIRECT || WSETS == 3), "the activation side of the pipeline walks three buffers");
-    constexpr int WD = WSETS - 1;
+    // RELOAD (BF16, DIRECT): two sets; a set's registers take the tile two steps on as soon as the products of a micro-step
+    // have read them.  Three sets of the 64 bytes a lane loads a step would not leave room for two workgroups a CU.
+    constexpr bool RELOAD = WSETS == 2;
+    static_assert(RELOAD == (DIRECT && KIND == XFTHIP_W_BF16), "two weight sets: the direct BF16 form");
+    static_assert(RELOAD || (WSETS % 3 == 0 && (!DIRECT || WSETS == 3)), "the activation side of the pipeline walks three buffers");
+    constexpr int WD = RELOAD ? 2 : WSETS - 1;
     uint32_t wreg[WSETS][GROUPS][WN][WREGS];
     u32x4 areg[3][ALOADS];
     const int kt_n = (p.K + KTILE - 1) / KTILE;
@@ -291,8 +300,8 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
                 const u32x4 v = *(const u32x4 *)(wbase[t] + (size_t)kt * 1024 + (2 * gq + h) * 256);
                 wreg[buf][gq][t][0] = v[0]; wreg[buf][gq][t][1] = v[1]; wreg[buf][gq][t][2] = v[2]; wreg[buf][gq][t][3] = v[3];
             } else if constexpr (KIND == XFTHIP_W_BF16) {
-                // chunk g = 2 s + h holds k = 8 g .. 8 g + 7
-                const u32x4 v = *(const u32x4 *)(wbase[t] + (size_t)kt * 1024 + (2 * gq + h) * 256);
+                // chunk g = 2 s + h holds k = 8 g .. 8 g + 7 (DIRECT: of the step's first or second packed tile)
+                const u32x4 v = *(const u32x4 *)(wbase[t] + ((size_t)kt * (KTILE / PACKED_K) + gq / 2) * 1024 + (2 * (gq & 1) + h) * 256);
                 wreg[buf][gq][t][0] = v[0]; wreg[buf][gq][t][1] = v[1]; wreg[buf][gq][t][2] = v[2]; wreg[buf][gq][t][3] = v[3];
             } else {
                 const u32x4 v = *(const u32x4 *)(wbase[t] + (size_t)(kt / STEPS_PER_TILE) * 1024 + ((kt % STEPS_PER_TILE) * GROUPS + gq) * 256);
@@ -427,7 +436,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     MFrag wcur_hi, wcur_lo;
     // the explicit interleave below pays for the BF16 kind (no widening work to hide: +5 %) and costs
     // the INT8 kind 6 % on 128 x 128 tiles, where the compiler's own order is better
-    constexpr bool SGB = KIND == XFTHIP_W_BF16;
+    constexpr bool SGB = KIND == XFTHIP_W_BF16 && !DIRECT;
     // VALU instructions one widening takes (a hint for the instruction interleave below)
     constexpr int VW = KIND == XFTHIP_W_INT8 ? 12 : KIND == XFTHIP_W_UINT4 ? 9 : KIND == XFTHIP_W_NF4 ? 6 : 0;
     constexpr int VPER = (VW + WM - 1) / WM;
@@ -440,7 +449,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
 #pragma unroll
         for (int ms = 0; ms < MICRO; ++ms) {
             const int gq = ms / SUB, sb = ms % SUB;
-            if (sb == 0) load_w_part(w_load, kt_cur + WD, gq);
+            if (sb == 0 && !RELOAD) load_w_part(w_load, kt_cur + WD, gq);
             if (ms % A_EVERY == 0) {
                 if constexpr (DIRECT) {
                     direct_a_part(lds_req, kt_cur + 3, ms / A_EVERY);
@@ -500,6 +509,11 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
                     }
                 }
             }
+            if constexpr (RELOAD) {
+                __builtin_amdgcn_sched_barrier(0);
+                load_w_part(w_load, kt_cur + WD, gq);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
     };
 
@@ -541,7 +555,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
 #define XFT_STEP(s)                                        \
     {                                                      \
         if constexpr (DIRECT) {                            \
-            compute((s), ((s) + 1) % 3, ((s) + 2) % 3, 0, 0, kt, kt & 3, (kt + 1) & 3, (kt + 3) & 3); \
+            compute((s) % WSETS, ((s) + 1) % WSETS, ((s) + WD) % WSETS, 0, 0, kt, kt & 3, (kt + 1) & 3, (kt + 3) & 3); \
             XFT_FENCE();                                   \
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(REQS_PER_STEP) : "memory"); \
         } else {                                           \
@@ -560,6 +574,11 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
         if (kt < kt_n) XFT_STEP(2)
         if (kt < kt_n) XFT_STEP(3)
         if (kt < kt_n) XFT_STEP(4)
+    } else if constexpr (RELOAD) {
+        while (kt + 2 <= kt_n) {
+            XFT_STEP(0) XFT_STEP(1)
+        }
+        if (kt < kt_n) XFT_STEP(0)
     } else {
         while (kt + 3 <= kt_n) {
             XFT_STEP(0) XFT_STEP(1) XFT_STEP(2)
@@ -799,8 +818,8 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
 template <int KIND, int WN, int WM, bool NEED_SUM, bool KTAIL, bool DEVROWS = false, bool DIRECT = false, int KG = 1>
 static int launch_big2(const SkinnyParams &p, hipStream_t stream) {
     // six weight tiles in flight for the 32- and 64-row tiles (see the kernel), three for the others
-    constexpr int WSETS = (!DIRECT && WN == 1 && WM <= 2) ? 6 : 3;
-    using T = StepTraits<KIND>;
+    constexpr int WSETS = DIRECT && KIND == XFTHIP_W_BF16 ? 2 : (!DIRECT && WN == 1 && WM <= 2) ? 6 : 3;
+    using T = StepTraits<KIND, DIRECT>;
     constexpr int ROWS = 32 * WM, ROWB = DIRECT ? T::KTILE * 2 : T::KTILE * 2 + 16;
     const int n32 = (p.NTILES + 1) / 2;
     const int nblocks_n = (n32 + 4 * WN - 1) / (4 * WN);
@@ -844,15 +863,17 @@ static int launch_big(const SkinnyParams &p, hipStream_t stream) {
         }
     }
     if (p.K % StepTraits<KIND>::KTILE != 0) return launch_big2<KIND, WN, WM, NEED_SUM, true>(p, stream);
-    if constexpr (WN == 2 && WM == 4 && KIND != XFTHIP_W_BF16) {
+    if constexpr (WN == 2 && WM == 4) {
         // whole k tiles: the 128 x 256 tile takes its activations straight into LDS, two workgroups a CU
         // (the kernel keeps a lane's byte offset into the activations in 32 bits)
-        if ((size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32)) {
+        using TD = StepTraits<KIND, true>;
+        const int span = p.ksplit > 1 ? p.split_ktiles * TD::PACKED_K : p.K; // (a K part: whole steps as well)
+        if ((size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32) && p.K % TD::KTILE == 0 && span % TD::KTILE == 0) {
             // at most one block a CU: two K groups a workgroup give every SIMD a second wave (see the kernel)
             const long wgs = (long)(((p.NTILES + 1) / 2 + 4 * WN - 1) / (4 * WN)) * ((p.M + 32 * WM - 1) / (32 * WM));
             // (2048 rows x 4096 columns, K = 4096 / 11008: INT8 963 / 993 against 926 / 934 TFLOP/s on the same box, UINT4
             // 859 / 954 against 812 / 926, NF4 519 / 569 against 492 / 532)
-            if (wgs <= device_cu_count() && p.ksplit <= 1 && p.K % (2 * StepTraits<KIND>::PACKED_K) == 0)
+            if (wgs <= device_cu_count() && p.ksplit <= 1 && p.K % (2 * (TD::PACKED_K > TD::KTILE ? TD::PACKED_K : TD::KTILE)) == 0)
                 return launch_big2<KIND, WN, WM, NEED_SUM, false, false, true, 2>(p, stream);
             return launch_big2<KIND, WN, WM, NEED_SUM, false, false, true>(p, stream);
         }
