@@ -149,6 +149,67 @@ def test_mfma_gateup_silu_vs_oracle(xh, orc, kind, M):
     dw.free()
 
 
+def _random_weight(xh, orc, rng, kind, K, N, gateup=False):
+    """Packed weight, its values in 64 bits and the size of what the kernel adds up (bound below), by code."""
+    scale = rng.uniform(0.5e-2, 1.5e-2, N).astype(np.float32)
+    flags = xh.WF_GATEUP if gateup else xh.WF_NONE
+    if kind == "bf16":
+        W = orc.round_bf16(rng.standard_normal((K, N), dtype=np.float32) * 0.05)
+        return xh.Weight(xh.W_BF16, K, N, orc.to_bf16(W), flags=flags), W.astype(np.float64), np.abs(W).astype(np.float64)
+    if kind.startswith("int8"):
+        q = rng.integers(-127, 128, (K, N)).astype(np.int8)
+        zero = (rng.standard_normal(N) * 0.05).astype(np.float32) if kind == "int8z" else None
+        W = q * scale.astype(np.float64) + (0.0 if zero is None else zero.astype(np.float64))
+        return xh.Weight(xh.W_INT8, K, N, q, scale, zero, flags=flags), W, np.abs(q) * scale.astype(np.float64) + (0.0 if zero is None else np.abs(zero))
+    u = rng.integers(0, 16, (K, N)).astype(np.uint8)
+    packed = (u[:, 0::2] | (u[:, 1::2] << 4)).astype(np.uint8)
+    if kind == "uint4":
+        zero = (-7.5 * scale).astype(np.float32)
+        # (the matrix units multiply 128 + code, the row sums take 128 off again)
+        return xh.Weight(xh.W_UINT4, K, N, packed, scale, zero, flags=flags), u * scale.astype(np.float64) + zero, (144.0 + u) * scale + np.abs(zero)
+    w = xh.Weight(xh.W_NF4, K, N, packed, scale, flags=flags)
+    W = w.dequant().astype(np.float64)  # (pinned bit for bit above)
+    return w, W, np.abs(W)
+
+
+# more shapes than the tiles of qgemm_mfma, so that every one is taken somewhere with a ragged last block: 32 and 64 rows with K in parts,
+# 128 x 128 and 128 x 256 with one and two K groups and with K in parts, bands of one to eight row blocks
+@pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])
+@pytest.mark.parametrize("M,K,N", [(33, 8192, 3088), (97, 4096, 1040), (129, 1024, 12304), (200, 4096, 6160), (450, 11008, 2064), (641, 8192, 4112), (700, 4096, 4112),
+                                   (1285, 4096, 4112), (2100, 1024, 6160), (1161, 2048, 2832), (300, 4160, 2064), (770, 2048, 80)])
+def test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N):
+    """Bound: K + 8 additions and the epilogue's few operations in fp32, each off by 2^-24 of what has been added up so far at most; NF4 values
+    go in as two bf16 parts, off by 2^-17."""
+    rng = np.random.default_rng(M + K + N)
+    w, W, size = _random_weight(xh, orc, rng, kind, K, N)
+    A = orc.round_bf16(rng.standard_normal((M, K), dtype=np.float32))
+    got = _run_gemm(xh, w, orc.to_bf16(A), M, K, N, xh.F32)
+    bound = np.abs(A).astype(np.float64) @ size * ((K + 8) * 2.0 ** -24 + (2.0 ** -16 if kind == "nf4" else 0.0))
+    worst = float((np.abs(got - A.astype(np.float64) @ W) / bound).max())
+    print(f"case {kind} {M} x {N} x {K}: {worst:.2e} of the bound", flush=True)
+    assert worst <= 1.0
+    w.free()
+
+
+@pytest.mark.parametrize("kind", ["int8", "uint4", "nf4", "bf16"])
+@pytest.mark.parametrize("M,K,I", [(100, 1024, 1040), (700, 2048, 2064), (1285, 4096, 2064), (2100, 1024, 3088)])
+def test_mfma_gateup_every_tile_against_64_bits(xh, orc, kind, M, K, I):
+    """silu(g) u: off by what the bounds of g and u (test above) make of it, |silu'| <= 1.1, and 2^-20 of the value for the exponential."""
+    rng = np.random.default_rng(M + I)
+    w, W, size = _random_weight(xh, orc, rng, kind, K, 2 * I, gateup=True)
+    A = orc.round_bf16(rng.standard_normal((M, K), dtype=np.float32))
+    a_dev, o_dev = xh.DeviceBuffer.from_numpy(orc.to_bf16(A)), xh.DeviceBuffer(M * I * 4)
+    xh.gemm_gateup_silu(w, a_dev.ptr, M, K, o_dev.ptr, I, xh.F32)
+    xh.synchronize()
+    got = o_dev.to_numpy(np.float32, (M, I))
+    y, b = A.astype(np.float64) @ W, np.abs(A).astype(np.float64) @ size * ((K + 8) * 2.0 ** -24 + (2.0 ** -16 if kind == "nf4" else 0.0))
+    g, u = y[:, :I], y[:, I:]
+    silu = g / (1.0 + np.exp(-g))
+    bound = 1.1 * b[:, :I] * np.abs(u) + b[:, I:] * (np.abs(silu) + 1.1 * b[:, :I]) + np.abs(silu * u) * 2.0 ** -20
+    assert float((np.abs(got - silu * u) / bound).max()) <= 1.0
+    w.free()
+
+
 def test_bf16_weight_gemm_both_kernels(xh, orc):
     rng = np.random.default_rng(70)
     K, N = 512, 1000

@@ -33,6 +33,9 @@ struct SkinnyParams {
     // fp32 [M][N] into split_part + y * M * N; a second kernel adds the parts in order and applies the epilogue
     int ksplit, split_ktiles;
     float *split_part;
+    // M > 32 kernel, host-side row count: the block tile (1: 32 rows x 128 columns, 2: 64 x 128, 3: 128 x 128, 4: 128 x 256), its K groups
+    // a workgroup, whether the activations go straight into LDS (tiles 3 and 4); chosen by qgemm_mfma
+    int tile, kgroups, direct;
     // Row count known on the device only (the experts of a sparse MLP): when rows_dev is set the kernels read
     // {rows, first row of A, first row of C} from it, M is only the upper bound that sizes the grid, and m_hint
     // (0 = M) is the row count the host expects, used where it chooses between forms.  No residual epilogues.
@@ -69,6 +72,22 @@ struct SkinnyParams {
 __device__ inline float clamped_glu(float gate, float up, float limit, float alpha) {
     const float g = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
     return g / (1.0f + fast_exp(-alpha * g)) * (u + 1.0f);
+}
+
+// Row blocks are walked in bands of at most 8 (qgemm_mfma_impl.h), `units` units of work a band.  The bands are of one height, the
+// one that leaves the XCD with the most units the least to do (3072 columns in 256s, 19 row blocks: three bands of 7 are 36 units,
+// five for some XCDs, 35 blocks on 32 CUs; four of 5 are 48, six each, 30 blocks), and no band of a few rows is padded to 8 with
+// workgroups that leave at once.  Those do harm: an XCD hands its workgroups to its four shader engines in turn, whatever they
+// do there, so that 5 working ones of 8 put two on the first engine and one on each other (600 x 12288 x 4096 INT8, 240 blocks of
+// two K groups on 256 CUs: over 100 us against 65).
+__host__ __device__ inline int band_rows(int nblocks_m, int units) {
+    const int bands = (nblocks_m + 7) / 8;
+    int best = nblocks_m > 0 ? (nblocks_m + bands - 1) / bands : 1, least = (bands * units + 7) / 8 * best;
+    for (int n = bands + 1; n <= bands + 3; ++n) {
+        const int rows = (nblocks_m + n - 1) / n, load = (n * units + 7) / 8 * rows;
+        if (load < least) best = rows, least = load;
+    }
+    return best;
 }
 
 int qgemm_skinny(const PackedWeight &pw, const SkinnyParams &p, hipStream_t stream); // M <= 32

@@ -96,10 +96,84 @@ __global__ __launch_bounds__(256) void qgemm_split_finish_kernel(SkinnyParams p)
 }
 
 // Partial results of the K split: one buffer per stream and device (stream_scratch), allocated once at its upper
-// bound (a split launch has at most CUs / 2 tiles of 32 x 128 results in at most 16 parts: 33.5 MB on 256 CUs), so
+// bound (64 KB of results a CU in 4 parts: 67 MB on 256 CUs; a split that needs more is not taken), so
 // nothing is allocated or freed on a stream once its buffer exists.  Launches on one stream are ordered; launches
 // on different streams work in different buffers.
-size_t split_bound_floats() { return (size_t)16 * (device_cu_count() / 2 + 1) * 4096; }
+size_t split_bound_floats() { return (size_t)device_cu_count() * 65536; }
+
+// Which tile, how many parts of K and how many K groups a workgroup: the cheapest by a cost model of the launch.
+//   time = start + rounds of resident blocks (steps of 64 k times what a step costs with so many blocks on a CU, + pipeline fill and
+//          results) + the sum of the parts of a split K
+// A CU's blocks are those of the XCD with the most (band_rows); a partly filled round costs between the blocks of the fullest CU and
+// those of the average one, a partly filled device a little less a step than a full one.  The constants (microseconds) are a
+// least-squares fit to 35000 timings on weights that do not fit the Infinity Cache: 340 shapes of 1024 .. 28672 columns x 1024 .. 14336 deep,
+// 33 to 4096 rows, 1 to 8 parts, the five weight kinds.  What it takes is 1.01 to 1.02 times the best form's time on average over those
+// cells (1.33 at worst).  In words: the largest tile that gives most CUs a block, K split or taken in two groups where that takes it to
+// about a block a CU, and for few rows parts of K until there are two or three 32- or 64-row blocks a CU.  Against thresholds on the rows
+// (which left 700 rows x 4096 columns on 64-row tiles and split 128 rows too little) and bands padded to 8 row blocks: INT8 1.15 times as
+// fast in the geometric mean over the cells, with zero points 1.17, UINT4 1.12, NF4 1.19, BF16 1.43; 900 x 4096 x 14336 INT8 142 -> 113 us,
+// 128 x 4096 x 14336 46 -> 34, 600 x 12288 x 4096 94 -> 65, 64 x 28672 x 4096 57 -> 33.
+struct TileCost {
+    int rows, cols, kgroups, resident;
+    float fixed; // a block's pipeline fill and results
+    float step[3], more[3]; // per step of a block alone on a CU; per further resident block.  INT8 and UINT4, BF16, NF4
+};
+constexpr TileCost kTiles[] = {
+        {32, 128, 1, 4, 0.6f, {0.26f, 0.0f, 0.39f}, {0.15f, 0.0f, 0.26f}},
+        {64, 128, 1, 4, 1.2f, {0.35f, 0.56f, 0.51f}, {0.27f, 0.34f, 0.43f}},
+        {128, 128, 1, 2, 1.7f, {0.71f, 0.64f, 0.90f}, {0.26f, 0.36f, 0.65f}},
+        {128, 128, 2, 1, 4.3f, {1.0f, 1.14f, 1.38f}, {}},
+        {128, 256, 1, 2, 3.1f, {0.92f, 0.93f, 1.59f}, {0.73f, 0.77f, 1.34f}},
+        {128, 256, 2, 1, 8.7f, {1.49f, 1.8f, 2.63f}, {}},
+};
+
+constexpr float kSplitStart[3] = {3.0f, 4.0f, 3.0f}, kSplitMb[3] = {0.3f, 0.35f, 0.3f}; // launch and megabytes of a split K's sum
+
+void choose_tile(SkinnyParams &p, int kind, int ktile) {
+    const int cus = device_cu_count(), kt_n = (p.K + ktile - 1) / ktile, cls = kind == XFTHIP_W_BF16 ? 1 : kind == XFTHIP_W_NF4 ? 2 : 0;
+    // activations straight into LDS: steps of 64 k, byte offsets of 32 bits
+    const bool direct = p.K % 64 == 0 && (size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32);
+    p.tile = 2, p.kgroups = 1, p.direct = 0;
+    if (!direct && (long)((p.N + 255) / 256) * ((p.M + 127) / 128) >= cus) {
+        p.tile = 4; // staged through registers: only where it fills the device
+        return;
+    }
+    float best = 1e30f;
+    for (const TileCost &t : kTiles) {
+        if (t.rows == 32 && kind == XFTHIP_W_BF16) continue; // (not built: two bytes a weight want more rows behind them)
+        if (t.rows == 128 && !direct) continue;
+        const int row_blocks = (p.M + t.rows - 1) / t.rows, col_blocks = (p.N + t.cols - 1) / t.cols;
+        for (int want : {1, 2, 3, 4, 6, 8}) {
+            if (want > 1 && (p.gateup || p.K / want < 512)) break;
+            int part = (kt_n + want - 1) / want; // packed tiles
+            if (kind == XFTHIP_W_BF16) part = (part + 1) / 2 * 2; // (whole steps of 64)
+            const int parts = (kt_n + part - 1) / part, span = parts > 1 ? part * ktile : p.K;
+            if (parts > 1 && (size_t)parts * p.M * p.N > split_bound_floats()) break;
+            const int band = band_rows(row_blocks, col_blocks * parts), bands = (row_blocks + band - 1) / band;
+            const long blocks = ((long)bands * col_blocks * parts + 7) / 8 * 8 * band;
+            float steps = (float)((span + 63) / 64);
+            if (t.kgroups == 2) {
+                // at most a block a CU, groups of whole packed tiles (in every part), deep enough to pay for their hand-over
+                const int unit = 2 * (ktile > 64 ? ktile : 64);
+                if (blocks > cus || p.K % unit || span % unit || steps < 48) continue;
+                steps *= 0.5f;
+            }
+            const long slots = (long)cus * t.resident, full = blocks / slots, rest = blocks - full * slots;
+            float us = 7.0f + (float)full * (steps * (t.step[cls] + t.more[cls] * (float)(t.resident - 1)) + t.fixed);
+            if (rest) {
+                const float x = (float)rest / (float)cus, fullest = (float)((rest + cus - 1) / cus);
+                us += steps * (x <= 1.0f ? t.step[cls] * (0.77f + 0.23f * x) : t.step[cls] + t.more[cls] * (0.55f * fullest + 0.45f * x - 1.0f)) + t.fixed;
+            }
+            if (parts > 1) us += kSplitStart[cls] + kSplitMb[cls] * 4e-6f * (float)parts * (float)p.M * (float)p.N;
+            if (us < best) {
+                best = us;
+                p.tile = t.rows == 32 ? 1 : t.rows == 64 ? 2 : t.cols == 128 ? 3 : 4;
+                p.kgroups = t.kgroups, p.direct = t.rows == 128;
+                p.ksplit = parts > 1 ? parts : 0, p.split_ktiles = part;
+            }
+        }
+    }
+}
 
 } // namespace
 
@@ -120,14 +194,14 @@ int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t strea
     p.K = pw.K;
     p.N = pw.N;
     p.ksplit = 0, p.split_ktiles = 0, p.split_part = nullptr;
-    // Few rows against few columns and a deep K (the down projection of an expert, the output projection at a
-    // few dozen sequences): the 32-row tiles would not even give every CU a workgroup, so K is split as well.
     const int ktile = ktile_of(pw.kind), kt_n = (pw.K + ktile - 1) / ktile;
     const int cus = device_cu_count(), n32 = (pw.NTILES + 1) / 2;
-    const int rows_expected = (p.rows_dev && !p.group && p.m_hint > 0) ? p.m_hint : p.M;
-    const long tiles = (long)((n32 + 3) / 4) * ((rows_expected + 31) / 32);
-    if (!p.gateup && 2 * tiles <= cus && kt_n >= 16) {
-        long want = (2L * cus) / tiles;
+    if (!p.rows_dev) choose_tile(p, pw.kind, ktile);
+    if (p.rows_dev && !p.group && !p.gateup && kt_n >= 16) {
+        // One expert of several kinds: as many parts of K as give every CU two 32-row tiles of the rows the host expects
+        const int rows_expected = p.m_hint > 0 ? p.m_hint : p.M;
+        const long tiles = (long)((n32 + 3) / 4) * ((rows_expected + 31) / 32);
+        long want = 2 * tiles <= cus ? (2L * cus) / tiles : 0;
         want = want < kt_n / 8 ? want : kt_n / 8;
         want = want < 16 ? want : 16;
         if (want >= 2) {
@@ -143,30 +217,12 @@ int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t strea
         long want = (8L * cus + tiles64 - 1) / tiles64;
         want = want < kt_n / 8 ? want : kt_n / 8;
         want = want < 16 ? want : 16;
-        const long fit = (long)(split_bound_floats() / ((size_t)p.M * p.N));
+        const long fit = (long)(split_bound_floats() / 2 / ((size_t)p.M * p.N));
         want = want < fit ? want : fit;
         p.ksplit = 0;
         if (want >= 2) {
             p.split_ktiles = (kt_n + (int)want - 1) / (int)want;
             p.ksplit = (kt_n + p.split_ktiles - 1) / p.split_ktiles;
-        }
-    }
-    if (p.ksplit <= 1 && !p.gateup && !p.group && !p.rows_dev && p.M >= 256 && pw.K >= 8192) {
-        // A few hundred rows against few columns and a very deep K (the down projection of a 512-token prompt, 4096
-        // columns x 11008): 64-row tiles give every CU at most one workgroup with a k loop of 172 steps, 32-row tiles
-        // (two a CU) widen every weight for a single row tile.  K is split until the 64-row tiles come two a CU:
-        // 65 us with the addition of the parts against 79 (512 x 4096 x 11008).  At K = 4096 the loops are too short
-        // for the split to pay (31 us either way).
-        const long tiles64 = (long)((n32 + 3) / 4) * ((p.M + 63) / 64);
-        if (tiles64 < 2 * cus) {
-            long want = (2L * cus + tiles64 - 1) / tiles64;
-            const long fit = (long)(split_bound_floats() / ((size_t)p.M * p.N));
-            want = want < fit ? want : fit;
-            want = want < pw.K / 2048 ? want : pw.K / 2048; // parts at least 2048 deep
-            if (want >= 2) {
-                p.split_ktiles = (kt_n + (int)want - 1) / (int)want;
-                p.ksplit = (kt_n + p.split_ktiles - 1) / p.split_ktiles;
-            }
         }
     }
     if (p.ksplit > 1) {

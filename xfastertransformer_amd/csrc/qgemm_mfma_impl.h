@@ -75,20 +75,6 @@ struct StepTraits<XFTHIP_W_BF16, DIRECT> {
     static constexpr int KTILE = DIRECT ? 64 : 32, GROUPS = DIRECT ? 4 : 2, SUB = 1, WREGS = 4, PACKED_K = 32;
 };
 
-// Row blocks a band: 8, or, with a device-side row count, only as many as the rows the host expects fill: the
-// workgroups that do work then come first in the launch order and spread over the CUs; the ones past the count (which
-// leave at once) follow them instead of sitting between them.  (Host and device: the grid is sized with it.)
-template <int ROWS, bool DEVROWS>
-__host__ __device__ inline int band_rows(const SkinnyParams &p) {
-    if constexpr (DEVROWS) {
-        if (!p.group) {
-            const int want = (p.m_hint + ROWS - 1) / ROWS;
-            return want < 1 ? 1 : want < 8 ? want : 8;
-        }
-    }
-    return 8;
-}
-
 // DEVROWS: the row count (and, for a group of weights, the weight) comes from device memory (SkinnyParams::rows_dev /
 // group); a form of its own, so that the plain kernels carry none of it
 //
@@ -131,17 +117,37 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     const int kgroup = KG == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
     const int h = lane >> 5, nl = lane & 31;
     const int part_rows = p.M; // rows of a K part: the host's bound, also when the device knows fewer
-    // workgroup -> (K part, column block, row block).  Row blocks are walked in bands of 8; a unit of work is one
-    // (band, K part, column block): its 8 workgroups share the column block's weights.  Workgroup ids go round the 8
-    // XCDs in launch order, so the units are dealt out to the XCDs one by one - an XCD runs the 8 workgroups of a unit
+    // workgroup -> (K part, column block, row block).  Row blocks are walked in bands (band_rows); a unit of work is one
+    // (band, K part, column block): its workgroups share the column block's weights.  Workgroup ids go round the 8
+    // XCDs in launch order, so the units are dealt out to the XCDs one by one - an XCD runs the workgroups of a unit
     // next to each other (the weights pass through its L2 once) and its units follow each other column block by column
     // block inside a band (the band's activation rows stay in its L2 while the weights stream past them) - and the
     // XCDs carry the same load whatever the number of column blocks (43 blocks of 256 columns dealt out block by block
     // would give three XCDs 6 and five XCDs 5).
+    // Row counts on the device: the row blocks that are there are numbered, so that all workgroups past them come last.
+    int group_before = 0; // (lane e of every wave, groups) row blocks of the weights before weight e of its 64
+    if constexpr (DEVROWS) {
+        if (p.group) {
+            nblocks_m = 0;
+            for (int e0 = 0; e0 < p.group_n; e0 += 64) {
+                int n = e0 + lane < p.group_n ? (p.rows_dev[(e0 + lane) * p.rows_stride] + ROWS - 1) / ROWS : 0;
+#pragma unroll
+                for (int off = 1; off < 64; off <<= 1) {
+                    const int up = __shfl_up(n, off, 64);
+                    n += lane >= off ? up : 0;
+                }
+                group_before = n; // (inclusive; of the last 64)
+                nblocks_m += __builtin_amdgcn_readlane(n, 63);
+            }
+        } else if (p.rows_dev) {
+            p.M = p.rows_dev[0] < part_rows ? p.rows_dev[0] : part_rows;
+            nblocks_m = (p.M + ROWS - 1) / ROWS;
+        }
+    }
     int nb, mb, part;
     {
-        const int BAND = band_rows<ROWS, DEVROWS>(p);
         const int parts = p.ksplit > 1 ? p.ksplit : 1;
+        const int BAND = band_rows(nblocks_m, parts * nblocks_n);
         const int id = blockIdx.x, xcd = id & 7, slot = id >> 3; // gridDim.x is a multiple of 8
         const int nbands = (nblocks_m + BAND - 1) / BAND;
         const int units = nbands * parts * nblocks_n;
@@ -157,14 +163,20 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     if constexpr (DEVROWS) {
     if (p.group) {
         // several weights of one shape behind one launch: the row blocks of all of them are numbered in a
-        // row, weight after weight, by their device-side row counts; blocks past the last one leave
+        // row, weight after weight, by their device-side row counts
         int e = 0, first = 0;
-        for (; e < p.group_n; ++e) {
-            const int nblk = (p.rows_dev[e * p.rows_stride] + ROWS - 1) / ROWS;
-            if (mb < first + nblk) break;
-            first += nblk;
+        if (p.group_n <= 64) {
+            const unsigned long long before = __builtin_amdgcn_ballot_w64(group_before <= mb);
+            e = __builtin_popcountll(before); // (group_before is ascending over the lanes)
+            first = e ? __builtin_amdgcn_readlane(group_before, e - 1) : 0;
+        } else {
+            for (; e < p.group_n; ++e) {
+                const int nblk = (p.rows_dev[e * p.rows_stride] + ROWS - 1) / ROWS;
+                if (mb < first + nblk) break;
+                first += nblk;
+            }
         }
-        if (e == p.group_n) return;
+        if (e >= p.group_n) return;
         mb -= first;
         const int *rec = p.rows_dev + e * p.rows_stride;
         p.M = rec[0];
@@ -175,7 +187,6 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
         p.scale = p.group[e].scale;
         p.zero = p.group[e].zero;
     } else if (p.rows_dev) {
-        p.M = p.rows_dev[0] < part_rows ? p.rows_dev[0] : part_rows;
         p.A += (size_t)p.rows_dev[1] * p.lda;
         c_row = p.rows_dev[2]; // the K parts hold local rows, the kernel that adds them shifts
     }
@@ -825,10 +836,11 @@ static int launch_big2(const SkinnyParams &p, hipStream_t stream) {
     const int nblocks_n = (n32 + 4 * WN - 1) / (4 * WN);
     // a group's row blocks: every weight may end in a partly filled one
     const int nblocks_m = (p.M + ROWS - 1) / ROWS + (p.group ? p.group_n : 0);
-    // 8 workgroups a unit of (band of row blocks, K part, column block), the units dealt out to the 8 XCDs
-    const int band = band_rows<ROWS, DEVROWS>(p), parts = p.ksplit > 1 ? p.ksplit : 1;
-    const long units = (long)((nblocks_m + band - 1) / band) * parts * nblocks_n;
-    const long blocks_l = (units + 7) / 8 * 8 * band;
+    // band_rows workgroups a unit of (band of row blocks, K part, column block), the units dealt out to the 8 XCDs; a
+    // device-side row count may make up to a block a band and eight units more of a smaller number of row blocks
+    const int parts = p.ksplit > 1 ? p.ksplit : 1, band = band_rows(nblocks_m, parts * nblocks_n), nbands = (nblocks_m + band - 1) / band;
+    const long blocks_l = DEVROWS ? ((long)(nblocks_m + (nblocks_m + 7) / 8) * parts * nblocks_n + 64 + 7) / 8 * 8
+                                  : ((long)nbands * parts * nblocks_n + 7) / 8 * 8 * band;
     if (blocks_l > 0x7fffffffL) {
         set_error("qgemm_mfma: too many workgroups");
         return 2;
@@ -862,77 +874,47 @@ static int launch_big(const SkinnyParams &p, hipStream_t stream) {
             return 2;
         }
     }
-    if (p.K % StepTraits<KIND>::KTILE != 0) return launch_big2<KIND, WN, WM, NEED_SUM, true>(p, stream);
-    if constexpr (WN == 2 && WM == 4) {
-        // whole k tiles: the 128 x 256 tile takes its activations straight into LDS, two workgroups a CU
-        // (the kernel keeps a lane's byte offset into the activations in 32 bits)
-        using TD = StepTraits<KIND, true>;
-        const int span = p.ksplit > 1 ? p.split_ktiles * TD::PACKED_K : p.K; // (a K part: whole steps as well)
-        if ((size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32) && p.K % TD::KTILE == 0 && span % TD::KTILE == 0) {
-            // at most one block a CU: two K groups a workgroup give every SIMD a second wave (see the kernel)
-            const long wgs = (long)(((p.NTILES + 1) / 2 + 4 * WN - 1) / (4 * WN)) * ((p.M + 32 * WM - 1) / (32 * WM));
-            // (2048 rows x 4096 columns, K = 4096 / 11008: INT8 963 / 993 against 926 / 934 TFLOP/s on the same box, UINT4
-            // 859 / 954 against 812 / 926, NF4 519 / 569 against 492 / 532)
-            if (wgs <= device_cu_count() && p.ksplit <= 1 && p.K % (2 * (TD::PACKED_K > TD::KTILE ? TD::PACKED_K : TD::KTILE)) == 0)
-                return launch_big2<KIND, WN, WM, NEED_SUM, false, false, true, 2>(p, stream);
-            return launch_big2<KIND, WN, WM, NEED_SUM, false, false, true>(p, stream);
+    if constexpr (WM == 4) {
+        // 128-row tiles: the activations straight into LDS, two workgroups a CU, or (at most a block a CU) two K groups a workgroup: 2048
+        // rows x 4096 columns, K = 4096 / 11008, INT8 963 / 993 against 926 / 934 TFLOP/s, UINT4 859 / 954 against 812 / 926, NF4 519 / 569
+        // against 492 / 532.  Staged through registers only for a ragged K or more than 4 GB of activations (128 x 256 alone).
+        if (p.direct) return p.kgroups == 2 ? launch_big2<KIND, WN, WM, NEED_SUM, false, false, true, 2>(p, stream)
+                                            : launch_big2<KIND, WN, WM, NEED_SUM, false, false, true>(p, stream);
+        if constexpr (WN == 2) {
+            return launch_big2<KIND, WN, WM, NEED_SUM, true>(p, stream);
+        } else {
+            set_error("qgemm_mfma: the 128 x 128 tile takes its activations straight into LDS");
+            return 2;
         }
+    } else {
+        if (p.K % StepTraits<KIND>::KTILE != 0) return launch_big2<KIND, WN, WM, NEED_SUM, true>(p, stream);
+        return launch_big2<KIND, WN, WM, NEED_SUM, false>(p, stream);
     }
-    return launch_big2<KIND, WN, WM, NEED_SUM, false>(p, stream);
 }
 
 template <int KIND, bool NEED_SUM>
 static int dispatch_big_tile(const SkinnyParams &p, hipStream_t stream) {
-    const int cus = device_cu_count();
-    // Block tile = (4*WN*32 columns) x (WM*32 rows).  The choices below are the measured winners on
-    // 4096x{4096,12288,22016} and 11008x4096 weights at 512, 1024 and 2048 rows: 128-row tiles only
-    // pay once there are many row blocks to share a weight tile's trip through L2; below that,
-    // more and smaller workgroups per CU (whose k loops overlap) win by up to 1.5x.
-    const int n32 = (p.NTILES + 1) / 2;
-    // the tile is chosen for the rows the host expects; with a device-side row count p.M is only the bound
-    const int rows = (p.rows_dev && !p.group && p.m_hint > 0) ? p.m_hint : p.M;
-    const long t_large = (long)((n32 + 7) / 8) * ((rows + 127) / 128);
-    const long t_mid = (long)((n32 + 3) / 4) * ((rows + 127) / 128);
-    const long t_small = (long)((n32 + 3) / 4) * ((rows + 63) / 64);
     if (p.rows_dev) {
-        // 32- or 64-row tiles.  A group's weights with more than 32 rows each keep 64-row tiles: the 32-row ones
-        // read every weight tile twice, and with all the weights' workgroups side by side there is no CU left to fill.
+        // Device-side row counts: 32- or 64-row tiles, chosen for the rows the host expects (p.M is only the bound).  A group's weights with
+        // more than 32 rows each keep 64-row tiles: the 32-row ones read every weight tile twice, and with all the weights' workgroups side
+        // by side there is no CU left to fill.  (128-row tiles for a group whose weights expect about 64 rows each - one pass over a weight
+        // instead of a second row block for the rows past 64 - measured 574 us a sparse MLP layer against 496)
         if constexpr (KIND != XFTHIP_W_BF16) {
-            if (t_small < 2 * cus && !(p.group && p.M > 32 * p.group_n)) return launch_big<KIND, 1, 1, NEED_SUM>(p, stream);
+            const int rows = (!p.group && p.m_hint > 0) ? p.m_hint : p.M;
+            const long t_small = (long)(((p.NTILES + 1) / 2 + 3) / 4) * ((rows + 63) / 64);
+            if (t_small < 2 * device_cu_count() && !(p.group && p.M > 32 * p.group_n)) return launch_big<KIND, 1, 1, NEED_SUM>(p, stream);
         }
-        // (128-row tiles for a group whose weights expect about 64 rows each - one pass over a weight instead of a
-        // second row block for the rows past 64 - measured 574 us a sparse MLP layer against 496)
         return launch_big<KIND, 1, 2, NEED_SUM>(p, stream);
     }
-    if constexpr (KIND == XFTHIP_W_BF16) {
-        if (t_large >= cus) return launch_big<KIND, 2, 4, NEED_SUM>(p, stream);
-        if (t_mid >= cus) return launch_big<KIND, 1, 4, NEED_SUM>(p, stream);
-        return launch_big<KIND, 1, 2, NEED_SUM>(p, stream);
-    } else if constexpr (KIND == XFTHIP_W_INT8) {
-        // The 128 x 256 tile with the activations straight into LDS (two workgroups a CU) wherever it fills the
-        // device: 960 / 918 - 944 / 960 TFLOP/s on N x K = 4096x4096 / 11008x4096 / 4096x11008 at 2048 rows
-        // (1050 - 1110 at 4096 rows), against 921 / 777 / 856 on the 128 x 128 tile (two workgroups a CU, bound by the
-        // LDS port: 20 KB of operand reads and staging writes per 16 MFMAs and wave) and 750 - 760 on the 128 x 256
-        // tile staged through registers (one wave per SIMD, nothing to run while it waits).
-        // (512 rows x 22016 columns, the gate / up projection of a 512-token prompt: 117 us against 133)
-        if (rows >= 512 && t_large >= cus) return launch_big<KIND, 2, 4, NEED_SUM>(p, stream);
-        if (rows > 1024 && t_mid >= cus) return launch_big<KIND, 1, 4, NEED_SUM>(p, stream);
-    } else {
-        // 4-bit kinds: the same 128 x 256 tile (UINT4 850 / 922 / 916 TFLOP/s at 2048 rows on 4096^2, 11008 x 4096,
-        // 4096 x 11008 against 785 / 743 / 861 staged through registers, one workgroup a CU; NF4 499 / 549 / 535
-        // against 495 / 483 / 540).  The 128 x 128 tile (two workgroups a CU) measured no better than the staged
-        // 128 x 256 one (UINT4 751 / 766 / 813, NF4 515 / 512 / 551).
-        // (512 rows x 22016 columns: UINT4 119 us against 138, NF4 203 against 210)
-        if (rows >= 512 && t_large >= cus) return launch_big<KIND, 2, 4, NEED_SUM>(p, stream);
+    switch (p.tile) { // (choose_tile)
+        case 1:
+            if constexpr (KIND != XFTHIP_W_BF16) return launch_big<KIND, 1, 1, NEED_SUM>(p, stream);
+            break;
+        case 3: return launch_big<KIND, 1, 4, NEED_SUM>(p, stream);
+        case 4: return launch_big<KIND, 2, 4, NEED_SUM>(p, stream);
+        default: break;
     }
-    if constexpr (KIND != XFTHIP_W_BF16) {
-        // Few rows against a deep K (512 tokens x 4096 columns): 64-row tiles would leave one
-        // workgroup per CU, whose k loop is then a chain of load latencies; 32-row tiles put two
-        // on a CU.
-        // (the K parts of a split GEMM count as workgroups of their own)
-        if (t_small * (p.ksplit > 1 ? p.ksplit : 1) < 2 * cus) return launch_big<KIND, 1, 1, NEED_SUM>(p, stream);
-        return launch_big<KIND, 1, 2, NEED_SUM>(p, stream);
-    }
+    return launch_big<KIND, 1, 2, NEED_SUM>(p, stream);
 }
 
 } // namespace
