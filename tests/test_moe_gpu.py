@@ -152,6 +152,15 @@ def test_mixtral_mlp_bf16_experts(xh, orc, tokens, hidden, inter):
     assert np.abs(got - exp).max() < 2e-2 and _cos(got, exp) >= 0.9999
 
 
+@pytest.mark.parametrize("tokens", [400, 1030])
+def test_mixtral_mlp_many_rows_an_expert(xh, orc, tokens):
+    """100 and 257 rows an expert on average: 128-row blocks, some experts' last ones of few rows, several blocks an expert."""
+    test_mixtral_mlp_vs_oracle(xh, orc, tokens, False)
+    test_mixtral_mlp_four_bit_experts(xh, orc, 1, tokens)
+    test_mixtral_mlp_bf16_experts(xh, orc, tokens, 512, 1024)
+    test_mixtral_mlp_bf16_experts(xh, orc, tokens, 352, 736)  # (a depth that is no whole number of steps)
+
+
 @pytest.mark.parametrize("tokens", [12, 70])
 def test_mixtral_mlp_experts_of_different_layouts(xh, orc, tokens):
     """Experts that cannot share a launch (some INT8 weights carry a zero-point vector, some do not) go through the

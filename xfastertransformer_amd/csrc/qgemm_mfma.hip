@@ -2,6 +2,8 @@
 // Replaces MMHelper::compute* (reference src/utils/matmul_helper.h:565-1705) at large M, where
 // the reference switches to AMX (oneDNN) kernels.  The kernel lives in qgemm_mfma_impl.h; this
 // file picks the weight kind.
+#include <math.h>
+
 #include <mutex>
 
 #include "qgemm.h"
@@ -113,6 +115,9 @@ size_t split_bound_floats() { return (size_t)device_cu_count() * 65536; }
 // (which left 700 rows x 4096 columns on 64-row tiles and split 128 rows too little) and bands padded to 8 row blocks: INT8 1.15 times as
 // fast in the geometric mean over the cells, with zero points 1.17, UINT4 1.12, NF4 1.19, BF16 1.43; 900 x 4096 x 14336 INT8 142 -> 113 us,
 // 128 x 4096 x 14336 46 -> 34, 600 x 12288 x 4096 94 -> 65, 64 x 28672 x 4096 57 -> 33.
+// Several weights behind one launch (the experts of a sparse MLP): the same, without K groups, over the row blocks to be expected.  Against
+// 64-row tiles with K in up to 4 parts throughout: a Mixtral-8x7B layer, INT8, 400 tokens 549 -> 490 us, 1000 tokens 1060 -> 940; 8 experts
+// of width 2816 at width 2048, BF16, 6132 tokens, two layers and all else 3.28 -> 2.98 ms.
 struct TileCost {
     int rows, cols, kgroups, resident;
     float fixed; // a block's pipeline fill and results
@@ -134,7 +139,7 @@ void choose_tile(SkinnyParams &p, int kind, int ktile) {
     // activations straight into LDS: steps of 64 k, byte offsets of 32 bits
     const bool direct = p.K % 64 == 0 && (size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32);
     p.tile = 2, p.kgroups = 1, p.direct = 0;
-    if (!direct && (long)((p.N + 255) / 256) * ((p.M + 127) / 128) >= cus) {
+    if (!direct && !p.rows_dev && (long)((p.N + 255) / 256) * ((p.M + 127) / 128) >= cus) {
         p.tile = 4; // staged through registers: only where it fills the device
         return;
     }
@@ -142,7 +147,22 @@ void choose_tile(SkinnyParams &p, int kind, int ktile) {
     for (const TileCost &t : kTiles) {
         if (t.rows == 32 && kind == XFTHIP_W_BF16) continue; // (not built: two bytes a weight want more rows behind them)
         if (t.rows == 128 && !direct) continue;
-        const int row_blocks = (p.M + t.rows - 1) / t.rows, col_blocks = (p.N + t.cols - 1) / t.cols;
+        if (t.kgroups == 2 && p.rows_dev) continue; // (not built)
+        // (8 weights of 28672 x 4096 and 4096 x 14336 INT8 with 37 rows each: 386 us a layer in 32-row blocks, which read every weight tile twice,
+        // 353 in 64-row ones)
+        if (t.rows == 32 && p.group && p.M > 32 * p.group_n) continue;
+        int row_blocks = (p.M + t.rows - 1) / t.rows;
+        const int col_blocks = (p.N + t.cols - 1) / t.cols;
+        if (p.group) {
+            // expected blocks of a weight whose rows scatter normally about their share: 1 + the chances that there are more than t.rows,
+            // 2 t.rows, .. of them
+            const float each = (float)p.M / (float)p.group_n, spread = sqrtf(each) + 0.1f * each;
+            float blocks = 1.0f;
+            for (int j = t.rows; (float)j < each + 4.0f * spread; j += t.rows) blocks += 0.5f * erfcf(((float)j - each) / (1.41421356f * spread));
+            row_blocks = (int)(blocks * (float)p.group_n + 0.999f);
+        } else if (p.rows_dev && p.m_hint > 0) {
+            row_blocks = (p.m_hint + t.rows - 1) / t.rows;
+        }
         for (int want : {1, 2, 3, 4, 6, 8}) {
             if (want > 1 && (p.gateup || p.K / want < 512)) break;
             int part = (kt_n + want - 1) / want; // packed tiles
@@ -195,36 +215,7 @@ int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t strea
     p.N = pw.N;
     p.ksplit = 0, p.split_ktiles = 0, p.split_part = nullptr;
     const int ktile = ktile_of(pw.kind), kt_n = (pw.K + ktile - 1) / ktile;
-    const int cus = device_cu_count(), n32 = (pw.NTILES + 1) / 2;
-    if (!p.rows_dev) choose_tile(p, pw.kind, ktile);
-    if (p.rows_dev && !p.group && !p.gateup && kt_n >= 16) {
-        // One expert of several kinds: as many parts of K as give every CU two 32-row tiles of the rows the host expects
-        const int rows_expected = p.m_hint > 0 ? p.m_hint : p.M;
-        const long tiles = (long)((n32 + 3) / 4) * ((rows_expected + 31) / 32);
-        long want = 2 * tiles <= cus ? (2L * cus) / tiles : 0;
-        want = want < kt_n / 8 ? want : kt_n / 8;
-        want = want < 16 ? want : 16;
-        if (want >= 2) {
-            p.split_ktiles = (kt_n + (int)want - 1) / (int)want;
-            p.ksplit = (kt_n + p.split_ktiles - 1) / p.split_ktiles;
-        }
-    }
-    if (p.group && !p.gateup && kt_n >= 16) {
-        // A group's workgroups all run side by side; K is split until there are about 8 of them a CU (measured on
-        // 8 weights of 14336 x 4096 with 512 rows in all: 4 parts 497 us a layer against 523 unsplit), as far as
-        // the parts fit their buffer
-        const long tiles64 = (long)((n32 + 3) / 4) * ((p.M + 63) / 64 + p.group_n);
-        long want = (8L * cus + tiles64 - 1) / tiles64;
-        want = want < kt_n / 8 ? want : kt_n / 8;
-        want = want < 16 ? want : 16;
-        const long fit = (long)(split_bound_floats() / 2 / ((size_t)p.M * p.N));
-        want = want < fit ? want : fit;
-        p.ksplit = 0;
-        if (want >= 2) {
-            p.split_ktiles = (kt_n + (int)want - 1) / (int)want;
-            p.ksplit = (kt_n + p.split_ktiles - 1) / p.split_ktiles;
-        }
-    }
+    choose_tile(p, pw.kind, ktile);
     if (p.ksplit > 1) {
         if ((size_t)p.ksplit * p.M * p.N > split_bound_floats()) p.ksplit = 0; // cannot happen within the bound; stay correct anyway
         else if (int rc = qgemm_split_reserve(stream, &p.split_part)) return rc;

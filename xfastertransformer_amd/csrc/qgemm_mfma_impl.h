@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     constexpr int PACKED_K = T::PACKED_K, STEPS_PER_TILE = PACKED_K >= KTILE ? PACKED_K / KTILE : 1; // k of a packed 1-KiB tile; steps that share one
     constexpr int ROWS = 32 * WM;
     constexpr int ROWB = DIRECT ? KTILE * 2 : KTILE * 2 + 16; // LDS row pitch in bytes (padded when staged through registers)
-    static_assert(!DIRECT || (KTILE == 64 && !KTAIL && !DEVROWS && ROWS % 32 == 0), "direct-to-LDS form: 64-deep steps, whole k tiles, host-side row count");
+    static_assert(!DIRECT || (KTILE == 64 && !KTAIL && ROWS % 32 == 0), "direct-to-LDS form: 64-deep steps, whole k tiles");
     constexpr int CHUNKS_PER_ROW = KTILE / 8; // 16-byte chunks
     constexpr int TOTAL_CHUNKS = ROWS * CHUNKS_PER_ROW;
     constexpr int ALOADS = TOTAL_CHUNKS / 256;
@@ -269,6 +269,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
             const int r = 8 * (ALOADS * wave + i) + (lane >> 3);
             int row = m0 + r;
             row = row < p.M ? row : p.M - 1;
+            if constexpr (DEVROWS) row = p.a_rows ? p.a_rows[row] : row;
             a_off[i] = ((uint32_t)row * (uint32_t)p.lda + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2; // in bytes
         } else {
             int row = m0 + a_row0 + i * ROW_STEP;
@@ -865,13 +866,11 @@ static int launch_big2(const SkinnyParams &p, hipStream_t stream) {
 template <int KIND, int WN, int WM, bool NEED_SUM>
 static int launch_big(const SkinnyParams &p, hipStream_t stream) {
     if (p.rows_dev) {
-        // device-side row counts: built for the 32- and 64-row tiles only (dispatch_big_tile picks no other then)
-        if constexpr (WN == 1 && WM <= 2) {
+        if constexpr (WM == 4) {
+            return launch_big2<KIND, WN, WM, NEED_SUM, false, true, true>(p, stream); // (taken for whole k steps only)
+        } else {
             if (p.K % StepTraits<KIND>::KTILE != 0) return launch_big2<KIND, WN, WM, NEED_SUM, true, true>(p, stream);
             return launch_big2<KIND, WN, WM, NEED_SUM, false, true>(p, stream);
-        } else {
-            set_error("qgemm_mfma: no device-side row count for this tile");
-            return 2;
         }
     }
     if constexpr (WM == 4) {
@@ -894,18 +893,6 @@ static int launch_big(const SkinnyParams &p, hipStream_t stream) {
 
 template <int KIND, bool NEED_SUM>
 static int dispatch_big_tile(const SkinnyParams &p, hipStream_t stream) {
-    if (p.rows_dev) {
-        // Device-side row counts: 32- or 64-row tiles, chosen for the rows the host expects (p.M is only the bound).  A group's weights with
-        // more than 32 rows each keep 64-row tiles: the 32-row ones read every weight tile twice, and with all the weights' workgroups side
-        // by side there is no CU left to fill.  (128-row tiles for a group whose weights expect about 64 rows each - one pass over a weight
-        // instead of a second row block for the rows past 64 - measured 574 us a sparse MLP layer against 496)
-        if constexpr (KIND != XFTHIP_W_BF16) {
-            const int rows = (!p.group && p.m_hint > 0) ? p.m_hint : p.M;
-            const long t_small = (long)(((p.NTILES + 1) / 2 + 3) / 4) * ((rows + 63) / 64);
-            if (t_small < 2 * device_cu_count() && !(p.group && p.M > 32 * p.group_n)) return launch_big<KIND, 1, 1, NEED_SUM>(p, stream);
-        }
-        return launch_big<KIND, 1, 2, NEED_SUM>(p, stream);
-    }
     switch (p.tile) { // (choose_tile)
         case 1:
             if constexpr (KIND != XFTHIP_W_BF16) return launch_big<KIND, 1, 1, NEED_SUM>(p, stream);
