@@ -335,6 +335,8 @@ struct PageTable {
     int pages_for(int tokens) const { return (tokens / unit + kPageTokens - 1) / kPageTokens; }
 };
 
+constexpr int kLogitPieces = 4; // of a logits copy to the host
+
 // What a model from a plan adds to xfthip_model: the page pool and the state slots, scratch, the step's description.
 struct PlanState {
     xfthip_plan *plan = nullptr;
@@ -356,7 +358,8 @@ struct PlanState {
     // pinned images of what else a step copies: the rows whose logits are wanted, a decode call's slots, the page table, logits
     int *want_host = nullptr, *dec_host = nullptr, *table_pinned = nullptr;
     float *logits_pinned = nullptr;
-    int *tok_seg = nullptr, *tok_pos = nullptr, *ids = nullptr, *seg = nullptr, *dec_rows = nullptr, *want = nullptr;
+    hipEvent_t fetched[kLogitPieces - 1] = {}; // behind all pieces of the logits but the last
+    int *tok_seg = nullptr, *tok_pos = nullptr, *ids = nullptr, *seg = nullptr, *dec_rows = nullptr;
     std::vector<int> seg_off_host, seg_len_host, seg_pos_host, seg_row_host; // the step's segments
     std::vector<int> dec_list; // slots of the decode call in flight
     std::vector<int> logit_of_row; // which row of the logits a slot's last ones are in

@@ -66,6 +66,17 @@ __global__ void plan_advance_kernel(const int *seg, int seg_cap, int n, const in
     last_token[seg[b]] = ids[seg[seg_cap + b] + seg[2 * seg_cap + b] - 1];
 }
 
+// ahead of a step: its description from pinned host memory (tok_seg | tok_pos | ids, `stride` apart, T of each; 4 seg_cap segment entries behind
+// them) into the device's copy, which is laid out alike.  One launch of 4 us for four copies of 5 us each, which the first kernel waited for
+__global__ void plan_describe_kernel(const int *host, int stride, int T, int seg_ints, int *desc) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < T) {
+        const int a = host[i], b = host[(size_t)stride + i], c = host[2 * (size_t)stride + i];
+        desc[i] = a, desc[(size_t)stride + i] = b, desc[2 * (size_t)stride + i] = c;
+    }
+    if (i < seg_ints) desc[3 * (size_t)stride + i] = host[3 * (size_t)stride + i];
+}
+
 __global__ void plan_fill_kernel(int *p, int n, int v) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
@@ -448,7 +459,7 @@ int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int
     for (int i = 0; i < n; ++i)
         if (int rc = plan_reserve(m, rows[i], std::max(m->row_pos[rows[i]], 0) + lens[i])) return rc;
     if (int rc = upload_table(p, st)) return rc;
-    // the description: tok_seg | tok_pos | ids | seg (4 arrays of `slots`), one copy each way
+    // the description: tok_seg | tok_pos | ids | seg (4 arrays of `slots`)
     const int cap = p.slots, mt = c.max_tokens;
     int *hs = p.desc_host, *hp = hs + mt, *hi = hp + mt, *hg = hi + mt;
     int t = 0;
@@ -459,10 +470,8 @@ int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int
         hg[i] = rows[i], hg[cap + i] = t, hg[2 * cap + i] = lens[i], hg[3 * cap + i] = at;
         for (int k = 0; k < lens[i]; ++k, ++t) hs[t] = i, hp[t] = at + k, hi[t] = ids[t];
     }
-    XFT_CHECK_HIP(hipMemcpyAsync(p.tok_seg, hs, (size_t)T * 4, hipMemcpyHostToDevice, st));
-    XFT_CHECK_HIP(hipMemcpyAsync(p.tok_pos, hp, (size_t)T * 4, hipMemcpyHostToDevice, st));
-    XFT_CHECK_HIP(hipMemcpyAsync(p.ids, hi, (size_t)T * 4, hipMemcpyHostToDevice, st));
-    XFT_CHECK_HIP(hipMemcpyAsync(p.seg, hg, (size_t)4 * cap * 4, hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL(plan_describe_kernel, dim3((std::max((int)T, 4 * cap) + 255) / 256), dim3(256), 0, st, p.desc_host, mt, (int)T, 4 * cap, p.desc);
+    XFT_CHECK_HIP(hipGetLastError());
     const StepView view = view_of(m, n, (int)T, longest);
     if (int rc = plan_embed(embed_tables(m), view, p.ids, p.last_token, m->x, st)) return rc;
     m->len_hint = deepest;
@@ -484,6 +493,7 @@ int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int
     return 0;
 }
 
+// rows_dev: of the step's tokens, read by the card (device or pinned host memory; the stream is waited for before a pinned list changes), or null for all
 int plan_head(xfthip_model *m, const int *rows_dev, int n, int at, hipStream_t st) {
     PlanState &p = *m->plan;
     const xfthip_plan &plan = *p.plan;
@@ -496,17 +506,35 @@ int plan_head(xfthip_model *m, const int *rows_dev, int n, int at, hipStream_t s
     return plan.cfg.logit_softcap > 0.0f ? plan_softcap(logits, (size_t)n * c.vocab, plan.cfg.logit_softcap, st) : 0;
 }
 
+// Behind the head: `floats` logits into the caller's pageable memory by way of a pinned buffer, in up to kLogitPieces pieces of 512 KB or more, so
+// that the host moves one on while the card sends the next.  The stream is idle on return.  Bound by the host's way where the caller's memory is
+// fresh (16 rows of 32000, 2 MB: 48 us for the card's way, 60 to 80 for the host's, one after the other before; a decode step of 16 sequences
+// 470 -> 445 us with it and plan_describe_kernel)
+static int plan_fetch_logits(PlanState &p, const float *logits, size_t floats, float *logits_host, hipStream_t st) {
+    const size_t pieces = std::min<size_t>(std::max<size_t>(floats / (128 * 1024), 1), kLogitPieces), each = ((floats + pieces - 1) / pieces + 63) / 64 * 64;
+    for (size_t i = 0; i < pieces; ++i) {
+        const size_t at = std::min(i * each, floats), n = std::min(each, floats - at);
+        if (n == 0) continue;
+        XFT_CHECK_HIP(hipMemcpyAsync(p.logits_pinned + at, logits + at, n * 4, hipMemcpyDeviceToHost, st));
+        if (i + 1 < pieces) XFT_CHECK_HIP(hipEventRecord(p.fetched[i], st));
+    }
+    for (size_t i = 0; i < pieces; ++i) {
+        const size_t at = std::min(i * each, floats), n = std::min(each, floats - at);
+        if (i + 1 < pieces && n > 0) XFT_CHECK_HIP(hipEventSynchronize(p.fetched[i]));
+        if (i + 1 == pieces) XFT_CHECK_HIP(hipStreamSynchronize(st));
+        memcpy(logits_host + at, p.logits_pinned + at, n * 4);
+    }
+    return 0;
+}
+
 int plan_logits(xfthip_model *m, const int *list, int n, float *logits_host, hipStream_t st) {
     PlanState &p = *m->plan;
     const size_t vocab = m->cfg.vocab;
     for (int i = 0; i < n; i += p.logit_rows) {
         const int k = std::min(n - i, p.logit_rows);
         memcpy(p.want_host, list + i, (size_t)k * 4);
-        XFT_CHECK_HIP(hipMemcpyAsync(p.want, p.want_host, (size_t)k * 4, hipMemcpyHostToDevice, st));
-        if (int rc = plan_head(m, p.want, k, 0, st)) return rc;
-        XFT_CHECK_HIP(hipMemcpyAsync(p.logits_pinned, m->logits, (size_t)k * vocab * 4, hipMemcpyDeviceToHost, st));
-        XFT_CHECK_HIP(hipStreamSynchronize(st));
-        memcpy(logits_host + (size_t)i * vocab, p.logits_pinned, (size_t)k * vocab * 4);
+        if (int rc = plan_head(m, p.want_host, k, 0, st)) return rc;
+        if (int rc = plan_fetch_logits(p, m->logits, (size_t)k * vocab, logits_host + (size_t)i * vocab, st)) return rc;
     }
     return 0;
 }
@@ -517,16 +545,14 @@ int plan_prompt_pass(xfthip_model *m, const int *rows, int B, int S, const int *
     std::vector<int> lens(B, S);
     if (int rc = plan_run(m, B, rows, lens.data(), ids, st)) return rc;
     for (int b = 0; b < B; ++b) p.want_host[b] = (b + 1) * S - 1;
-    XFT_CHECK_HIP(hipMemcpyAsync(p.want, p.want_host, (size_t)B * 4, hipMemcpyHostToDevice, st));
     // (the prompts of one call sit in neighbouring slots)
-    if (int rc = plan_head(m, p.want, B, rows[0], st)) return rc;
+    if (int rc = plan_head(m, p.want_host, B, rows[0], st)) return rc;
     if (int rc = argmax_rows(m->logits + (size_t)rows[0] * c.vocab, B, c.vocab, m->ids, p.seg, nullptr, nullptr, st)) return rc;
     hipLaunchKernelGGL(plan_fill_kernel, dim3(1), dim3(64), 0, st, m->step, 1, 0);
     XFT_CHECK_HIP(hipGetLastError());
-    if (logits_host)
-        XFT_CHECK_HIP(hipMemcpyAsync(p.logits_pinned, m->logits + (size_t)rows[0] * c.vocab, (size_t)B * c.vocab * 4, hipMemcpyDeviceToHost, st));
-    XFT_CHECK_HIP(hipStreamSynchronize(st));
-    if (logits_host) memcpy(logits_host, p.logits_pinned, (size_t)B * c.vocab * 4);
+    if (logits_host) {
+        if (int rc = plan_fetch_logits(p, m->logits + (size_t)rows[0] * c.vocab, (size_t)B * c.vocab, logits_host, st)) return rc;
+    } else XFT_CHECK_HIP(hipStreamSynchronize(st));
     for (int b = 0; b < B; ++b) p.logit_of_row[rows[b]] = rows[0] + b;
     return 0;
 }
@@ -649,6 +675,8 @@ void plan_state_destroy(PlanState *p) {
     if (p->trace_buf) (void)hipFree(p->trace_buf);
     if (p->desc_host) (void)hipHostFree(p->desc_host);
     if (p->logits_pinned) (void)hipHostFree(p->logits_pinned);
+    for (hipEvent_t e : p->fetched)
+        if (e) (void)hipEventDestroy(e);
     delete p;
 }
 
@@ -1389,7 +1417,6 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
     alloc(&p->table, p->table_host.size() * 4, true);
     alloc(&p->desc, (3 * T + 4 * (size_t)max_batch) * 4, true);
     alloc(&p->dec_rows, (size_t)max_batch * 4, true);
-    alloc(&p->want, (size_t)p->logit_rows * 4, true);
     std::map<std::vector<double>, std::pair<float *, float *>> rot; // layers of the same rotation share its tables
     auto tables_of = [&](const xfthip_plan_layer &s, float **cosT, float **sinT) {
         const bool extended = s.rot_factor > 0.0;
@@ -1414,6 +1441,7 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
     }
     ok = ok && hipHostMalloc((void **)&p->desc_host, (3 * T + 5 * (size_t)max_batch + p->logit_rows + p->table_host.size()) * 4) == hipSuccess
             && hipHostMalloc((void **)&p->logits_pinned, (size_t)p->logit_rows * plan->cfg.vocab * 4) == hipSuccess;
+    for (hipEvent_t &e : p->fetched) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     p->dec_host = p->desc_host + 3 * T + 4 * (size_t)max_batch;
     p->want_host = p->dec_host + max_batch;
     p->table_pinned = p->want_host + p->logit_rows;
