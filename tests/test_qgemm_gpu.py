@@ -191,8 +191,16 @@ def test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N):
     w.free()
 
 
+# on 256 CUs: 1, 2, 3, 4 (at 17 rows and more) and 6 column tiles a block, ragged last blocks, 8 to 1 K slices, and more than 8 tiles a CU
+@pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])
+@pytest.mark.parametrize("M", [3, 13, 29])
+@pytest.mark.parametrize("K,N", [(1280, 1040), (1280, 4112), (1280, 9232), (768, 13328), (768, 18448), (768, 28672), (768, 36880), (256, 36880)])
+def test_few_rows_every_form_against_64_bits(xh, orc, kind, M, K, N):
+    test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N)
+
+
 @pytest.mark.parametrize("kind", ["int8", "uint4", "nf4", "bf16"])
-@pytest.mark.parametrize("M,K,I", [(100, 1024, 1040), (700, 2048, 2064), (1285, 4096, 2064), (2100, 1024, 3088)])
+@pytest.mark.parametrize("M,K,I", [(3, 768, 1040), (13, 768, 14336), (29, 768, 9232), (29, 768, 18448), (100, 1024, 1040), (700, 2048, 2064), (1285, 4096, 2064), (2100, 1024, 3088)])
 def test_mfma_gateup_every_tile_against_64_bits(xh, orc, kind, M, K, I):
     """silu(g) u: off by what the bounds of g and u (test above) make of it, |silu'| <= 1.1, and 2^-20 of the value for the exponential."""
     rng = np.random.default_rng(M + I)

@@ -721,9 +721,92 @@ static int dispatch_tail(const SkinnyParams &p, int kslices, hipStream_t stream)
         if (MT == 2 || p.M > 4) return launch<KIND, NT, MT, U, NEED_SUM, false, false, false, true, true>(p, kslices, stream);
         if constexpr (MT == 1) return launch<KIND, NT, MT, U, NEED_SUM, false, false, false, false, true>(p, kslices, stream);
     }
-    if (MT == 2 || p.M > 4) return launch<KIND, NT, MT, U, NEED_SUM, false, false, false, true>(p, kslices, stream);
-    if constexpr (MT == 1) return launch<KIND, NT, MT, U, NEED_SUM, false, false>(p, kslices, stream);
-    return 0;
+    set_error("qgemm_skinny: no form for this shape"); // (launch_form has the plain products)
+    return 2;
+}
+
+// The form of a plain product (no prologue, no RoPE, one weight, K of whole tiles): column tiles a block, k tiles a load batch, K slices (waves)
+struct SkinnyForm {
+    int nt, u, kslices;
+};
+
+// What sets the time is the CU with the most column tiles: blocks are spread over the CUs in turn, so that it is w = ceil(blocks / CUs) blocks of nt
+// tiles.  A tile costs least in blocks of two (an activation fragment serves both; wider blocks lose some of that to registers), a block half a
+// tile more for its sums over the waves.  All blocks of a CU run side by side: 8 waves between them keep enough loads in flight (more K
+// slices only add sums), two a block at least.  BF16 at up to 16 rows: single tiles, whose stream alone is 32 KB a block.
+// Timed over 20 shapes of 512 .. 32000 columns x 1408 .. 14336 deep, six row counts, four kinds, all forms: 0.96 .. 0.99 of the best form on
+// average.  Against two tiles (3 .. 6 at 17 .. 32 rows) in 8 slices throughout, geometric mean at up to 4 / 16 / 32 rows: UINT4 1.13 / 1.16 /
+// 1.07 times as fast, NF4 1.12 / 1.14 / 1.08, INT8 1.04 / 1.08 / 1.07, BF16 1.03 / 1.03 / 1.05; UINT4 24 x 4096 x 28672 30 -> 22 us, 6 rows
+// 25 -> 15.6, 16 x 8192 x 10240 19 -> 14.
+// More than 8 tiles a CU, where the blocks come in rounds anyway: the form that was best over 55296 .. 151936 columns (UINT4 16 x 4096 x 128256
+// 101 -> 52 us, INT8 32 rows 126 -> 101, NF4 6 rows 115 -> 74, BF16 6 rows 166 -> 152).
+template <int KIND>
+static SkinnyForm choose_form(const SkinnyParams &p) {
+    constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4;
+    const int cus = device_cu_count(), mt = p.M <= 16 ? 1 : 2;
+    auto clamped = [&](SkinnyForm f) { // a batch a slice at least
+        const int batches = p.KT / f.u;
+        if (f.kslices > batches) f.kslices = batches;
+        return f;
+    };
+    auto per_cu = [&](int nt) { return ((p.NTILES + nt - 1) / nt + cus - 1) / cus; };
+    if (p.NTILES > 8 * cus) {
+        if (mt == 2) return clamped({4, 1, FOUR ? 2 : KIND == XFTHIP_W_INT8 ? 3 : 1});
+        if (FOUR) return clamped({4, 1, 4});
+        // (BF16, 16 rows of 128256 columns: single tiles in 8 slices 199 us, 171 before, 166 in this form)
+        if (KIND == XFTHIP_W_BF16 && p.M > 8) return clamped({2, 2, 1});
+        return clamped({KIND == XFTHIP_W_INT8 || p.gateup ? 2 : 1, 2, 8});
+    }
+    int nt = p.gateup ? 2 : 1;
+    if (KIND != XFTHIP_W_BF16 || mt == 2) {
+        float least = 1e30f;
+        for (int n : {1, 2, 3, 4, 6}) {
+            if ((p.gateup && n % 2) || (n >= 4 && mt == 1)) continue;
+            const int w = per_cu(n);
+            // (17 .. 32 rows, two blocks of four tiles on a CU: well for 4-bit codes, 1.2 times the time of four blocks of two for the others)
+            const float tile = n == 1 ? 1.2f : n == 2 ? 1.0f : n == 4 && w > 1 && !FOUR ? 1.3f : 1.1f;
+            const float cost = (float)w * ((float)n * tile + 0.5f);
+            if (cost < least) least = cost, nt = n;
+        }
+    }
+    SkinnyForm f = {nt, 1, 8 / per_cu(nt)};
+    if (mt == 2) f.u = !FOUR && nt <= 3 ? 2 : 1;
+    else if (KIND == XFTHIP_W_INT8) f.u = nt == 1 ? 4 : nt == 3 ? 1 : 2;
+    else if (KIND == XFTHIP_W_BF16) f.u = 2;
+    const int least = KIND == XFTHIP_W_BF16 ? 1 : 2;
+    if (f.kslices < least) f.kslices = least;
+    return clamped(f);
+}
+
+template <int KIND, int MT, bool NEED_SUM, bool STAGE>
+static int launch_form(const SkinnyParams &p, hipStream_t stream) {
+    constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4;
+    constexpr int U1 = FOUR ? 1 : MT == 1 && KIND == XFTHIP_W_INT8 ? 4 : 2, U2 = FOUR ? 1 : 2; // (choose_form's, for one and two tiles)
+    const SkinnyForm f = choose_form<KIND>(p);
+    switch (f.nt) {
+        case 1: return launch<KIND, 1, MT, U1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+        case 2: return launch<KIND, 2, MT, U2, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+        case 3:
+            if constexpr (MT == 2) return launch<KIND, 3, MT, U2, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            else if constexpr (KIND != XFTHIP_W_BF16) return launch<KIND, 3, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            break;
+        case 4:
+            if constexpr (MT == 2) return launch<KIND, 4, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            else if constexpr (FOUR) return launch<KIND, 4, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            break;
+        case 6:
+            if constexpr (MT == 2) return launch<KIND, 6, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            break;
+    }
+    set_error("qgemm_skinny: no form of %d column tiles", f.nt);
+    return 2;
+}
+
+template <int KIND, bool NEED_SUM>
+static int dispatch_form(const SkinnyParams &p, hipStream_t stream) {
+    if (p.M > 16) return launch_form<KIND, 2, NEED_SUM, true>(p, stream);
+    if (p.M > 4) return launch_form<KIND, 1, NEED_SUM, true>(p, stream);
+    return launch_form<KIND, 1, NEED_SUM, false>(p, stream);
 }
 
 template <int KIND, int NT, int MT>
@@ -740,6 +823,12 @@ static int dispatch_sum(const SkinnyParams &p, int kslices, hipStream_t stream) 
 
 template <int KIND>
 static int dispatch_shape(const SkinnyParams &p, hipStream_t stream) {
+    if (!p.norm_x && !p.rope && !p.group && p.KT * KindTraits<KIND>::KTILE == p.K) {
+        if constexpr (KIND == XFTHIP_W_INT8) {
+            if (!p.zero) return dispatch_form<KIND, false>(p, stream);
+        }
+        return dispatch_form<KIND, KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_INT8>(p, stream);
+    }
     const int cus = device_cu_count();
     const int mt = (p.M + 15) / 16;
     // column tiles per wave: 2 when that still leaves at least 2 blocks per CU (gate/up needs pairs); with two
