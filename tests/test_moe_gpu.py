@@ -152,6 +152,16 @@ def test_mixtral_mlp_bf16_experts(xh, orc, tokens, hidden, inter):
     assert np.abs(got - exp).max() < 2e-2 and _cos(got, exp) >= 0.9999
 
 
+@pytest.mark.parametrize("tokens", [1, 2, 5, 16, 17, 32])
+def test_mixtral_mlp_few_rows_an_expert(xh, orc, tokens):
+    """Blocks of one, two and four column tiles, few and many of them on a compute unit, for up to 4, 16 and 32 rows."""
+    test_mixtral_mlp_vs_oracle(xh, orc, tokens, False)
+    test_mixtral_mlp_four_bit_experts(xh, orc, 1, tokens)
+    test_mixtral_mlp_four_bit_experts(xh, orc, 2, tokens)
+    test_mixtral_mlp_bf16_experts(xh, orc, tokens, 512, 1024)
+    test_mixtral_mlp_bf16_experts(xh, orc, tokens, 1024, 3584)
+
+
 @pytest.mark.parametrize("tokens", [400, 1030])
 def test_mixtral_mlp_many_rows_an_expert(xh, orc, tokens):
     """100 and 257 rows an expert on average: 128-row blocks, some experts' last ones of few rows, several blocks an expert."""

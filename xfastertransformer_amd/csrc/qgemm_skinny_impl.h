@@ -716,16 +716,11 @@ static int dispatch_tail(const SkinnyParams &p, int kslices, hipStream_t stream)
     if constexpr (MT == 1) {
         if (p.norm_x) return launch<KIND, NT, MT, U, NEED_SUM, false, true>(p, kslices, stream);
     }
-    // more than a few rows: activation rows loaded as contiguous runs (see STAGE)
-    if (p.group) {
-        if (MT == 2 || p.M > 4) return launch<KIND, NT, MT, U, NEED_SUM, false, false, false, true, true>(p, kslices, stream);
-        if constexpr (MT == 1) return launch<KIND, NT, MT, U, NEED_SUM, false, false, false, false, true>(p, kslices, stream);
-    }
-    set_error("qgemm_skinny: no form for this shape"); // (launch_form has the plain products)
+    set_error("qgemm_skinny: no form for this shape"); // (launch_form has the products without prologue and RoPE)
     return 2;
 }
 
-// The form of a plain product (no prologue, no RoPE, one weight, K of whole tiles): column tiles a block, k tiles a load batch, K slices (waves)
+// The form of a product without prologue and RoPE, K of whole tiles: column tiles a block, k tiles a load batch, K slices (waves)
 struct SkinnyForm {
     int nt, u, kslices;
 };
@@ -740,28 +735,42 @@ struct SkinnyForm {
 // 25 -> 15.6, 16 x 8192 x 10240 19 -> 14.
 // More than 8 tiles a CU, where the blocks come in rounds anyway: the form that was best over 55296 .. 151936 columns (UINT4 16 x 4096 x 128256
 // 101 -> 52 us, INT8 32 rows 126 -> 101, NF4 6 rows 115 -> 74, BF16 6 rows 166 -> 152).
+// Several weights behind one launch: the same over the columns of those that have rows, as many as there are rows at most.  8 weights each of
+// 28672 x 4096 and 4096 x 14336, a layer of 10 / 32 tokens: UINT4 224 / 306 -> 142 / 207 us, NF4 284 / 384 -> 200 / 280,
+// INT8 255 / 333 -> 214 / 276, BF16 400 / 501 -> 394 / 484.
 template <int KIND>
 static SkinnyForm choose_form(const SkinnyParams &p) {
     constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4;
     const int cus = device_cu_count(), mt = p.M <= 16 ? 1 : 2;
-    auto clamped = [&](SkinnyForm f) { // a batch a slice at least
-        const int batches = p.KT / f.u;
-        if (f.kslices > batches) f.kslices = batches;
-        return f;
+    const int weights = !p.group ? 1 : p.m_hint < 1 ? 1 : p.m_hint < p.group_n ? p.m_hint : p.group_n;
+    auto form = [&](int nt, int u, int kslices) { // a batch a slice at least
+        const int batches = p.KT / u;
+        kslices = kslices < 8 ? kslices : 8;
+        kslices = kslices < batches ? kslices : batches;
+        return SkinnyForm {nt, u, kslices > 1 ? kslices : 1};
     };
-    auto per_cu = [&](int nt) { return ((p.NTILES + nt - 1) / nt + cus - 1) / cus; };
-    if (p.NTILES > 8 * cus) {
-        if (mt == 2) return clamped({4, 1, FOUR ? 2 : KIND == XFTHIP_W_INT8 ? 3 : 1});
-        if (FOUR) return clamped({4, 1, 4});
+    auto per_cu = [&](int nt) { return ((p.NTILES + nt - 1) / nt * weights + cus - 1) / cus; };
+    const long tiles = (long)p.NTILES * weights;
+    // (two slices against eight: 3 % faster at K = 4096, 2 % slower at 2048)
+    if (KIND == XFTHIP_W_BF16 && p.group && mt == 1) return form(p.gateup ? 2 : 1, 4, p.gateup && p.K >= 4096 ? 2 : 8);
+    if (p.group && tiles >= 8 * cus) { // K slices by the depth
+        if (FOUR && mt == 1) return form(p.M <= 4 ? 2 : 4, 1, p.KT < 32 ? 4 : p.KT / 8);
+        if (FOUR) return form(4, 1, p.KT / 16);
+        if (KIND == XFTHIP_W_INT8) return mt == 1 ? form(2, 2, p.KT / 8) : form(2, 1, 4);
+        return form(2, 2, 2);
+    }
+    if (tiles > 8 * cus) {
+        if (mt == 2) return form(4, 1, FOUR ? 2 : KIND == XFTHIP_W_INT8 ? 3 : 1);
+        if (FOUR) return form(4, 1, 4);
         // (BF16, 16 rows of 128256 columns: single tiles in 8 slices 199 us, 171 before, 166 in this form)
-        if (KIND == XFTHIP_W_BF16 && p.M > 8) return clamped({2, 2, 1});
-        return clamped({KIND == XFTHIP_W_INT8 || p.gateup ? 2 : 1, 2, 8});
+        if (KIND == XFTHIP_W_BF16 && p.M > 8) return form(2, 2, 1);
+        return form(KIND == XFTHIP_W_INT8 || p.gateup ? 2 : 1, 2, 8);
     }
     int nt = p.gateup ? 2 : 1;
     if (KIND != XFTHIP_W_BF16 || mt == 2) {
         float least = 1e30f;
         for (int n : {1, 2, 3, 4, 6}) {
-            if ((p.gateup && n % 2) || (n >= 4 && mt == 1)) continue;
+            if ((p.gateup && n % 2) || (n >= 4 && mt == 1) || (n % 3 == 0 && p.group)) continue;
             const int w = per_cu(n);
             // (17 .. 32 rows, two blocks of four tiles on a CU: well for 4-bit codes, 1.2 times the time of four blocks of two for the others)
             const float tile = n == 1 ? 1.2f : n == 2 ? 1.0f : n == 4 && w > 1 && !FOUR ? 1.3f : 1.1f;
@@ -769,44 +778,46 @@ static SkinnyForm choose_form(const SkinnyParams &p) {
             if (cost < least) least = cost, nt = n;
         }
     }
-    SkinnyForm f = {nt, 1, 8 / per_cu(nt)};
-    if (mt == 2) f.u = !FOUR && nt <= 3 ? 2 : 1;
-    else if (KIND == XFTHIP_W_INT8) f.u = nt == 1 ? 4 : nt == 3 ? 1 : 2;
-    else if (KIND == XFTHIP_W_BF16) f.u = 2;
-    const int least = KIND == XFTHIP_W_BF16 ? 1 : 2;
-    if (f.kslices < least) f.kslices = least;
-    return clamped(f);
+    int u = 1;
+    if (FOUR) u = 1;
+    else if (mt == 2) u = nt > 3 || (KIND == XFTHIP_W_INT8 && p.group && nt == 2) ? 1 : 2;
+    else if (KIND == XFTHIP_W_INT8) u = nt == 1 ? 4 : nt == 3 ? 1 : 2;
+    else u = 2;
+    const int least = KIND == XFTHIP_W_BF16 ? 1 : 2, slices = 8 / per_cu(nt);
+    return form(nt, u, slices > least ? slices : least);
 }
 
-template <int KIND, int MT, bool NEED_SUM, bool STAGE>
+template <int KIND, int MT, bool NEED_SUM, bool STAGE, bool GROUP>
 static int launch_form(const SkinnyParams &p, hipStream_t stream) {
-    constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4;
-    constexpr int U1 = FOUR ? 1 : MT == 1 && KIND == XFTHIP_W_INT8 ? 4 : 2, U2 = FOUR ? 1 : 2; // (choose_form's, for one and two tiles)
+    // (load batches of one and two tiles as choose_form has them)
+    constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4, INT8 = KIND == XFTHIP_W_INT8;
+    constexpr int U1 = FOUR ? 1 : MT == 1 && (INT8 || GROUP) ? 4 : 2, U2 = FOUR || (INT8 && GROUP && MT == 2) ? 1 : !INT8 && GROUP && MT == 1 ? 4 : 2;
     const SkinnyForm f = choose_form<KIND>(p);
     switch (f.nt) {
-        case 1: return launch<KIND, 1, MT, U1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
-        case 2: return launch<KIND, 2, MT, U2, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+        case 1: return launch<KIND, 1, MT, U1, NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
+        case 2: return launch<KIND, 2, MT, U2, NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
         case 3:
-            if constexpr (MT == 2) return launch<KIND, 3, MT, U2, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            if constexpr (GROUP) break;
+            else if constexpr (MT == 2) return launch<KIND, 3, MT, U2, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
             else if constexpr (KIND != XFTHIP_W_BF16) return launch<KIND, 3, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
             break;
         case 4:
-            if constexpr (MT == 2) return launch<KIND, 4, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
-            else if constexpr (FOUR) return launch<KIND, 4, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            if constexpr (MT == 2 || FOUR) return launch<KIND, 4, MT, 1, NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
             break;
         case 6:
-            if constexpr (MT == 2) return launch<KIND, 6, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            if constexpr (MT == 2 && !GROUP) return launch<KIND, 6, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
             break;
     }
     set_error("qgemm_skinny: no form of %d column tiles", f.nt);
     return 2;
 }
 
-template <int KIND, bool NEED_SUM>
+template <int KIND, bool NEED_SUM, bool GROUP>
 static int dispatch_form(const SkinnyParams &p, hipStream_t stream) {
-    if (p.M > 16) return launch_form<KIND, 2, NEED_SUM, true>(p, stream);
-    if (p.M > 4) return launch_form<KIND, 1, NEED_SUM, true>(p, stream);
-    return launch_form<KIND, 1, NEED_SUM, false>(p, stream);
+    // more than a few rows: activation rows loaded as contiguous runs (see STAGE)
+    if (p.M > 16) return launch_form<KIND, 2, NEED_SUM, true, GROUP>(p, stream);
+    if (p.M > 4) return launch_form<KIND, 1, NEED_SUM, true, GROUP>(p, stream);
+    return launch_form<KIND, 1, NEED_SUM, false, GROUP>(p, stream);
 }
 
 template <int KIND, int NT, int MT>
@@ -823,11 +834,12 @@ static int dispatch_sum(const SkinnyParams &p, int kslices, hipStream_t stream) 
 
 template <int KIND>
 static int dispatch_shape(const SkinnyParams &p, hipStream_t stream) {
-    if (!p.norm_x && !p.rope && !p.group && p.KT * KindTraits<KIND>::KTILE == p.K) {
+    if (!p.norm_x && !p.rope && p.KT * KindTraits<KIND>::KTILE == p.K) {
         if constexpr (KIND == XFTHIP_W_INT8) {
-            if (!p.zero) return dispatch_form<KIND, false>(p, stream);
+            if (!p.zero) return p.group ? dispatch_form<KIND, false, true>(p, stream) : dispatch_form<KIND, false, false>(p, stream);
         }
-        return dispatch_form<KIND, KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_INT8>(p, stream);
+        constexpr bool SUM = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_INT8;
+        return p.group ? dispatch_form<KIND, SUM, true>(p, stream) : dispatch_form<KIND, SUM, false>(p, stream);
     }
     const int cus = device_cu_count();
     const int mt = (p.M + 15) / 16;
