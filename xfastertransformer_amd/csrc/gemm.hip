@@ -40,7 +40,7 @@ int gemm_rows_dev(xfthip_weight_t w, int m_max, int m_hint, const int *rows_dev,
 
 int gemm_grouped_rows_dev(const xfthip_weight_t *w, int n_group, const GroupWeight *table_dev, int rows_max, int rows_each_max,
         const int *rows_dev, int rows_stride, const void *A, int lda, void *C, int ldc, int c_dtype, hipStream_t stream, const int *a_rows,
-        float glu_limit, float glu_alpha) {
+        float glu_limit, float glu_alpha, int *parts, const float **part) {
     XFT_REQUIRE(w && n_group >= 1 && table_dev && rows_dev && rows_stride >= 3, "gemm_grouped_rows_dev: bad group arguments");
     if (int rc = check_common("gemm_grouped_rows_dev", w[0], rows_max, A, lda, C, ldc)) return rc;
     XFT_REQUIRE(rows_each_max >= 1 && rows_each_max <= rows_max, "gemm_grouped_rows_dev: bad row bounds %d / %d", rows_each_max, rows_max);
@@ -55,6 +55,7 @@ int gemm_grouped_rows_dev(const xfthip_weight_t *w, int n_group, const GroupWeig
     XFT_REQUIRE(c_dtype == XFTHIP_F32 || c_dtype == XFTHIP_BF16, "gemm_grouped_rows_dev: c_dtype must be f32 or bf16");
     const int gateup = (pw.flags & XFTHIP_WF_GATEUP) ? 1 : 0;
     XFT_REQUIRE(ldc >= (gateup ? pw.N / 2 : pw.N), "gemm_grouped_rows_dev: ldc=%d too small", ldc);
+    if (parts) *parts = 1, *part = (const float *)C;
     SkinnyParams p = {};
     p.M = rows_max;
     p.A = (const uint16_t *)A;
@@ -76,7 +77,7 @@ int gemm_grouped_rows_dev(const xfthip_weight_t *w, int n_group, const GroupWeig
         p.M = rows_each_max, p.m_hint = rows_max; // the few-row kernel: a grid row a weight, each with at most this many rows
         return qgemm_skinny(pw, p, stream);
     }
-    return qgemm_mfma(pw, p, stream);
+    return qgemm_mfma(pw, p, stream, parts, part);
 }
 
 } // namespace xfthip

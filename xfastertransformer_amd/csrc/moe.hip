@@ -1,5 +1,5 @@
-// Mixtral-style sparse MLP: router GEMM, top-2 selection with a 2-way softmax, per-expert gather,
-// SwiGLU MLP on the gathered rows and weighted scatter-add.  Replaces MixtralMLP::forward,
+// Mixtral-style sparse MLP: norm, router and top-2 selection with a 2-way softmax in one kernel, SwiGLU MLP
+// of every expert on its rows and weighted scatter-add.  Replaces MixtralMLP::forward,
 // selectTop2Experts, gatherInput and scatterOutput (reference src/layers/mlp_mixtral.h:29-291).
 // Experts run one after another in ascending order, as the reference's loop does, so every
 // token's two contributions are added in a fixed order.
@@ -10,40 +10,13 @@
 
 namespace xfthip {
 
-// logits[t][e] = sum_k xn[t][k] * Wr[k][e]; one wave per token, fp32 router weights
-// (GateTypeSelector: fp32 for quantised weight types, src/utils/type_selector.h:93-111)
-template <int E>
-__global__ __launch_bounds__(64) void router_kernel(const uint16_t *__restrict__ xn, int ld, const float *__restrict__ Wr,
-        float *__restrict__ logits, int hidden) {
-    const int t = blockIdx.x, lane = threadIdx.x;
-    float acc[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) acc[e] = 0.0f;
-    for (int k = lane; k < hidden; k += 64) {
-        const float x = bf16_to_f32(xn[(size_t)t * ld + k]);
-#pragma unroll
-        for (int e = 0; e < E; ++e) acc[e] = fmaf(x, Wr[(size_t)k * E + e], acc[e]);
-    }
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) acc[e] += __shfl_xor(acc[e], off, 64);
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) logits[(size_t)t * E + e] = acc[e];
-    }
-}
-
 // strict '>' scan: the lower index wins ties (mlp_mixtral.h:262-283); weights = softmax over the
 // two selected logits (:221-259)
-__global__ void top2_kernel(const float *__restrict__ logits, int M, int E, int *__restrict__ sel, float *__restrict__ w) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= M) return;
+__device__ inline void pick_top2(const float *logits, int E, int *sel, float *w) {
     float max1 = -INFINITY, max2 = -INFINITY;
     int idx1 = -1, idx2 = -1;
     for (int j = 0; j < E; ++j) {
-        const float v = logits[(size_t)t * E + j];
+        const float v = logits[j];
         if (v > max1) {
             max2 = max1;
             idx2 = idx1;
@@ -55,10 +28,93 @@ __global__ void top2_kernel(const float *__restrict__ logits, int M, int E, int 
         }
     }
     const float e1 = 1.0f, e2 = fast_exp(max2 - max1); // relative to the larger of the two
-    sel[2 * t] = idx1;
-    sel[2 * t + 1] = idx2;
-    w[2 * t] = e1 / (e1 + e2);
-    w[2 * t + 1] = e2 / (e1 + e2);
+    sel[0] = idx1;
+    sel[1] = idx2;
+    w[0] = e1 / (e1 + e2);
+    w[1] = e2 / (e1 + e2);
+}
+
+__global__ void top2_kernel(const float *__restrict__ logits, int M, int E, int *__restrict__ sel, float *__restrict__ w) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < M) pick_top2(logits + (size_t)t * E, E, sel + 2 * t, w + 2 * t);
+}
+
+// A token's row normed (NORM; y = bf16((x rstd) w) as rmsnorm_vec_kernel) and narrowed, its router logits sum_k xn[k] Wr[k][e] with fp32 router
+// weights (GateTypeSelector: fp32 for quantised weight types, src/utils/type_selector.h:93-111) unless they are given, and its two experts.
+// One workgroup a token, bound by a chain of load round trips: everything for the first 4096 columns is requested at once, router weights before
+// the norm is known.  The tokens' workgroups all read the same router weights: their waves start at places apart, so that they do not ask
+// the same L2 channel at a time.  In place of a norm, a router of one wave a token and a selection: 256 tokens of width 4096 6 + 33 + 5 -> 13 us
+// (4 waves a token, weights requested behind the norm: 24).
+constexpr int kRouteThreads = 1024, kRouteCols = 4; // columns a thread and round
+template <bool NORM, int E>
+__global__ __launch_bounds__(kRouteThreads) void route_kernel(const float *__restrict__ in, int in_ld, const float *__restrict__ ln, float eps,
+        uint16_t *__restrict__ xn, const float *__restrict__ Wr, const float *__restrict__ given, int *__restrict__ sel, float *__restrict__ w, int hidden) {
+    static_assert(E == 8, "a row of the router weights as two 16-byte loads");
+    constexpr int WAVES = kRouteThreads / 64;
+    __shared__ float part[WAVES], logit[WAVES][E];
+    const int t = blockIdx.x, tid = (threadIdx.x + 64 * t) & (kRouteThreads - 1), lane = tid & 63, wave = tid >> 6;
+    const float *row = in + (size_t)t * in_ld;
+    uint16_t *out = xn + (size_t)t * hidden;
+    float x[kRouteCols], g[kRouteCols];
+    float4 lo[kRouteCols], hi[kRouteCols];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < kRouteCols; ++i) {
+            const int k = k0 + i * kRouteThreads + tid, kc = k < hidden ? k : 0;
+            x[i] = k < hidden ? row[kc] : 0.0f;
+            g[i] = NORM ? ln[kc] : 1.0f;
+            if (!given) lo[i] = ((const float4 *)Wr)[2 * kc], hi[i] = ((const float4 *)Wr)[2 * kc + 1];
+        }
+    };
+    load(0);
+    float rstd = 1.0f;
+    if constexpr (NORM) {
+        float sq = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kRouteCols; ++i) sq = fmaf(x[i], x[i], sq);
+        for (int k = kRouteCols * kRouteThreads + tid; k < hidden; k += kRouteThreads) sq = fmaf(row[k], row[k], sq);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);
+        if (lane == 0) part[wave] = sq;
+        __syncthreads();
+        float total = 0.0f;
+#pragma unroll
+        for (int i = 0; i < WAVES; ++i) total += part[i];
+        rstd = 1.0f / sqrtf(total / (float)hidden + eps);
+    }
+    float acc[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] = 0.0f;
+    for (int k0 = 0; k0 < hidden; k0 += kRouteCols * kRouteThreads) {
+        if (k0) load(k0);
+#pragma unroll
+        for (int i = 0; i < kRouteCols; ++i) {
+            const int k = k0 + i * kRouteThreads + tid;
+            const uint16_t bits = f32_to_bf16_ref(NORM ? (x[i] * rstd) * g[i] : x[i]);
+            if (k < hidden) out[k] = bits;
+            if (given) continue; // (uniform)
+            const float v = k < hidden ? bf16_to_f32(bits) : 0.0f;
+            acc[0] = fmaf(v, lo[i].x, acc[0]), acc[1] = fmaf(v, lo[i].y, acc[1]), acc[2] = fmaf(v, lo[i].z, acc[2]), acc[3] = fmaf(v, lo[i].w, acc[3]);
+            acc[4] = fmaf(v, hi[i].x, acc[4]), acc[5] = fmaf(v, hi[i].y, acc[5]), acc[6] = fmaf(v, hi[i].z, acc[6]), acc[7] = fmaf(v, hi[i].w, acc[7]);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) acc[e] += __shfl_xor(acc[e], off, 64);
+        if (lane == 0) logit[wave][e] = acc[e];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float v[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            v[e] = 0.0f;
+            for (int i = 0; i < WAVES; ++i) v[e] += logit[i][e];
+            if (given) v[e] = given[(size_t)t * E + e];
+        }
+        pick_top2(v, E, sel + 2 * t, w + 2 * t);
+    }
 }
 
 // Per-expert token lists in ascending token order, in one workgroup: wave e collects expert e's tokens 64 at
@@ -132,22 +188,28 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint16_t *__rest
 
 // out[t] += eo[row of choice] * weight, the lower expert index first: the order in which the reference's
 // loop over the experts adds a token's two contributions (xft::addto: one fused multiply-add per element).
-// grid = tokens
+// grid = tokens.  eo may lie in `parts` parts of a split K, `part_stride` apart, added in order here: a pass over them (11 us at 256 tokens of
+// width 4096 in 2 parts) is not worth a launch of its own.
 // The residual comes straight from the layer's input (`in`, which may be `out` itself: a thread reads an element
 // before it writes it), so no copy of the input into the output runs first.
 __global__ __launch_bounds__(256) void combine_kernel(float *out, int ld, const float *in, int in_ld, const float *__restrict__ eo,
-        const int *__restrict__ sel, const int *__restrict__ slot_row, const float *__restrict__ w, int hidden, int wide) {
+        int parts, size_t part_stride, const int *__restrict__ sel, const int *__restrict__ slot_row, const float *__restrict__ w, int hidden, int wide) {
     const int t = blockIdx.x;
     const int first = sel[2 * t] < sel[2 * t + 1] ? 0 : 1;
     const int ga = slot_row[2 * t + first], gb = slot_row[2 * t + 1 - first];
     const float wa = w[2 * t + first], wb = w[2 * t + 1 - first];
+    auto whole = [&](const float *e, int c) {
+        float v = e[c];
+        for (int s = 1; s < parts; ++s) v += e[s * part_stride + c];
+        return v;
+    };
     if (ga < 0 || gb < 0) {
         // a choice without an expert (NaN logits) contributes nothing; not the common case, kept simple
         const float *ea = eo + (size_t)(ga < 0 ? 0 : ga) * hidden, *eb = eo + (size_t)(gb < 0 ? 0 : gb) * hidden;
         for (int c = threadIdx.x; c < hidden; c += blockDim.x) {
             float o = in[(size_t)t * in_ld + c];
-            if (ga >= 0) o = fmaf(ea[c], wa, o);
-            if (gb >= 0) o = fmaf(eb[c], wb, o);
+            if (ga >= 0) o = fmaf(whole(ea, c), wa, o);
+            if (gb >= 0) o = fmaf(whole(eb, c), wb, o);
             out[(size_t)t * ld + c] = o;
         }
         return;
@@ -158,7 +220,12 @@ __global__ __launch_bounds__(256) void combine_kernel(float *out, int ld, const 
         const float4 *src = (const float4 *)(in + (size_t)t * in_ld);
         for (int c = threadIdx.x; c < hidden / 4; c += blockDim.x) {
             float4 o = src[c];
-            const float4 a = ea[c], b = eb[c];
+            float4 a = ea[c], b = eb[c];
+            for (int s = 1; s < parts; ++s) {
+                const float4 a2 = ea[s * (part_stride / 4) + c], b2 = eb[s * (part_stride / 4) + c];
+                a.x += a2.x, a.y += a2.y, a.z += a2.z, a.w += a2.w;
+                b.x += b2.x, b.y += b2.y, b.z += b2.z, b.w += b2.w;
+            }
             o.x = fmaf(b.x, wb, fmaf(a.x, wa, o.x));
             o.y = fmaf(b.y, wb, fmaf(a.y, wa, o.y));
             o.z = fmaf(b.z, wb, fmaf(a.z, wa, o.z));
@@ -169,14 +236,8 @@ __global__ __launch_bounds__(256) void combine_kernel(float *out, int ld, const 
         const float *ea = eo + (size_t)ga * hidden, *eb = eo + (size_t)gb * hidden;
         float *dst = out + (size_t)t * ld;
         const float *src = in + (size_t)t * in_ld;
-        for (int c = threadIdx.x; c < hidden; c += blockDim.x) dst[c] = fmaf(eb[c], wb, fmaf(ea[c], wa, src[c]));
+        for (int c = threadIdx.x; c < hidden; c += blockDim.x) dst[c] = fmaf(whole(eb, c), wb, fmaf(whole(ea, c), wa, src[c]));
     }
-}
-
-__global__ void narrow_rows_kernel2(const float *__restrict__ in, int in_stride, uint16_t *__restrict__ out, int cols) {
-    const float *row = in + (size_t)blockIdx.x * in_stride;
-    uint16_t *orow = out + (size_t)blockIdx.x * cols;
-    for (int c = threadIdx.x; c < cols; c += blockDim.x) orow[c] = f32_to_bf16_ref(row[c]);
 }
 
 } // namespace xfthip
@@ -188,7 +249,7 @@ struct xfthip_moe {
     float *router = nullptr, *ln = nullptr;
     std::vector<xfthip_weight_t> gateup, down;
     uint16_t *xn = nullptr, *xg = nullptr, *h = nullptr;
-    float *eo = nullptr, *logits = nullptr, *w = nullptr, *row_weight = nullptr;
+    float *eo = nullptr, *w = nullptr, *row_weight = nullptr;
     GroupWeight *group = nullptr; // device pointers of the experts' weights: [E] gate/up, [E] down
     int *sel = nullptr, *counts = nullptr, *row_token = nullptr, *slot_row = nullptr, *rank = nullptr; // counts: [E] counts, [E] offsets, [9 E] GEMM row records
     bool owns_workspace = true; // false: the per-call buffers belong to the object this one was created beside
@@ -220,7 +281,7 @@ int xfthip_moe_create(int hidden, int intermediate, int experts, int max_tokens,
     bool ok = hipMalloc((void **)&m->router, (size_t)hidden * experts * 4) == hipSuccess
             && hipMalloc((void **)&m->xn, T * hidden * 2) == hipSuccess && hipMalloc((void **)&m->xg, 2 * T * hidden * 2) == hipSuccess
             && hipMalloc((void **)&m->h, 2 * T * intermediate * 2) == hipSuccess && hipMalloc((void **)&m->eo, 2 * T * hidden * 4) == hipSuccess
-            && hipMalloc((void **)&m->logits, T * experts * 4) == hipSuccess && hipMalloc((void **)&m->w, T * 2 * 4) == hipSuccess
+            && hipMalloc((void **)&m->w, T * 2 * 4) == hipSuccess
             && hipMalloc((void **)&m->sel, T * 2 * 4) == hipSuccess && hipMalloc((void **)&m->counts, (2 + 9) * 64) == hipSuccess && hipMalloc((void **)&m->group, 2 * 64 * sizeof(GroupWeight)) == hipSuccess
             && hipMalloc((void **)&m->row_token, 2 * T * 4) == hipSuccess && hipMalloc((void **)&m->row_weight, 2 * T * 4) == hipSuccess
             && hipMalloc((void **)&m->slot_row, 2 * T * 4) == hipSuccess && hipMalloc((void **)&m->rank, 2 * T * 4) == hipSuccess;
@@ -261,7 +322,7 @@ int xfthip_moe_create_beside(xfthip_moe_t first, const float *router_host, const
 int xfthip_moe_destroy(xfthip_moe_t m) {
     if (!m) return 0;
     void *own[] = {m->router, m->ln, m->group};
-    void *workspace[] = {m->xn, m->xg, m->h, m->eo, m->logits, m->w, m->row_weight, m->sel, m->counts, m->row_token, m->slot_row, m->rank};
+    void *workspace[] = {m->xn, m->xg, m->h, m->eo, m->w, m->row_weight, m->sel, m->counts, m->row_token, m->slot_row, m->rank};
     for (void *b : own)
         if (b) (void)hipFree(b);
     if (m->owns_workspace)
@@ -303,21 +364,11 @@ int xfthip_moe_forward(xfthip_moe_t m, const float *x_in, int in_stride, float *
     hipStream_t st = (hipStream_t)stream;
     const int T = tokens, H = m->hidden;
     // residual (mlp_mixtral.h:116-121: the output starts as a copy of the input): combine_kernel reads it from x_in
-    if (do_norm) {
-        if (int rc = xfthip_rmsnorm(m->xn, XFTHIP_BF16, x_in, XFTHIP_F32, m->ln, T, H, in_stride, H, 1e-6f, st)) return rc;
-    } else {
-        hipLaunchKernelGGL(narrow_rows_kernel2, dim3(T), dim3(256), 0, st, x_in, in_stride, m->xn, H);
-    }
-    const float *logits = logits_override;
-    if (!logits) {
-        hipLaunchKernelGGL(router_kernel<8>, dim3(T), dim3(64), 0, st, m->xn, H, m->router, m->logits, H);
-        logits = m->logits;
-    }
-    if (int rc = xfthip_moe_top2(logits, T, m->E, m->sel, m->w, st)) return rc;
+    hipLaunchKernelGGL((do_norm ? route_kernel<true, 8> : route_kernel<false, 8>), dim3(T), dim3(kRouteThreads), 0, st, x_in, in_stride, m->ln, 1e-6f, m->xn, m->router,
+            logits_override, m->sel, m->w, H);
     int *gemm_rows = m->counts + 2 * m->E;
     hipLaunchKernelGGL(build_lists_kernel, dim3(1), dim3(64 * m->E), 0, st, m->sel, m->w, T, m->E, m->counts, m->counts + m->E, m->row_token,
             m->row_weight, m->slot_row, m->rank, gemm_rows);
-    hipLaunchKernelGGL(gather_rows_kernel, dim3(2 * T), dim3(256), 0, st, m->xn, H, m->row_token, m->xg, H);
     XFT_CHECK_HIP(hipGetLastError());
     if (sel_host_out || w_host_out) {
         XFT_CHECK_HIP(hipStreamSynchronize(st));
@@ -343,12 +394,16 @@ int xfthip_moe_forward(xfthip_moe_t m, const float *x_in, int in_stride, float *
         const PackedWeight &g0 = m->gateup[0]->pw, &d0 = m->down[0]->pw;
         for (const PackedWeight *w : {&g0, &d0}) uniform = uniform && (w->kind == XFTHIP_W_BF16 || w->KT * ktile_of(w->kind) == w->K);
     }
+    const float *eo = m->eo;
+    int parts = 1;
     if (uniform && m->gateup[0]->pw.kind != XFTHIP_W_W8A8 && m->down[0]->pw.kind != XFTHIP_W_W8A8) {
-        if (int rc = gemm_grouped_rows_dev(m->gateup.data(), m->E, m->group, 2 * T, T, gemm_rows + 6, 9, m->xg, H, m->h, m->inter, XFTHIP_BF16, st))
+        if (int rc = gemm_grouped_rows_dev(m->gateup.data(), m->E, m->group, 2 * T, T, gemm_rows + 6, 9, m->xn, H, m->h, m->inter, XFTHIP_BF16, st, m->row_token))
             return rc;
-        if (int rc = gemm_grouped_rows_dev(m->down.data(), m->E, m->group + m->E, 2 * T, T, gemm_rows + 6, 9, m->h, m->inter, m->eo, H, XFTHIP_F32, st))
+        if (int rc = gemm_grouped_rows_dev(m->down.data(), m->E, m->group + m->E, 2 * T, T, gemm_rows + 6, 9, m->h, m->inter, m->eo, H, XFTHIP_F32, st, nullptr,
+                    0.0f, 0.0f, &parts, &eo))
             return rc;
     } else {
+        hipLaunchKernelGGL(gather_rows_kernel, dim3(2 * T), dim3(256), 0, st, m->xn, H, m->row_token, m->xg, H);
         const int hint = (2 * T + m->E - 1) / m->E;
         for (int e = 0; e < m->E; ++e) {
             if (int rc = gemm_rows_dev(m->gateup[e], T, hint, gemm_rows + 9 * e, m->xg, H, m->h, m->inter, XFTHIP_BF16, st)) return rc;
@@ -356,7 +411,8 @@ int xfthip_moe_forward(xfthip_moe_t m, const float *x_in, int in_stride, float *
         }
     }
     const int wide = (((size_t)x_out | ((size_t)out_stride * 4) | (size_t)x_in | ((size_t)in_stride * 4)) & 15) == 0 && H % 4 == 0;
-    hipLaunchKernelGGL(combine_kernel, dim3(T), dim3(256), 0, st, x_out, out_stride, x_in, in_stride, m->eo, m->sel, m->slot_row, m->w, H, wide);
+    hipLaunchKernelGGL(combine_kernel, dim3(T), dim3(256), 0, st, x_out, out_stride, x_in, in_stride, eo, parts,
+            (size_t)2 * T * H, m->sel, m->slot_row, m->w, H, wide);
     XFT_CHECK_HIP(hipGetLastError());
     return 0;
 }

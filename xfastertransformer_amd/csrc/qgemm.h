@@ -41,7 +41,7 @@ struct SkinnyParams {
     // (0 = M) is the row count the host expects, used where it chooses between forms.  No residual epilogues.
     const int *rows_dev;
     int m_hint;
-    // Several weights of one shape and kind behind one launch (M > 32 kernel only): weight e multiplies the rows
+    // Several weights of one shape and kind behind one launch: weight e multiplies the rows
     // that record e of rows_dev (records rows_stride ints apart) names; M bounds the sum of their rows, and their
     // rows of C must tile [0, sum of rows) without gaps.
     const GroupWeight *group;
@@ -92,7 +92,8 @@ __host__ __device__ inline int band_rows(int nblocks_m, int units) {
 
 int qgemm_skinny(const PackedWeight &pw, const SkinnyParams &p, hipStream_t stream); // M <= 32
 bool skinny_can_fuse_norm(const PackedWeight &pw, int M); // may SkinnyParams::norm_x be used
-int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p, hipStream_t stream); // any M, built for M > 32
+// any M, built for M > 32; parts / part: as in gemm_grouped_rows_dev
+int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p, hipStream_t stream, int *parts = nullptr, const float **part = nullptr);
 // the K-split workspace of qgemm_mfma launches on `stream` (allocated on the stream's first call: before a capture, say)
 int qgemm_split_reserve(hipStream_t stream, float **out = nullptr);
 // xfthip_gemm / xfthip_gemm_gateup_silu (by the weight's flag) with the row count in device memory: rows_dev =
@@ -104,10 +105,11 @@ int gemm_rows_dev(xfthip_weight_t w, int m_max, int m_hint, const int *rows_dev,
 // of rows_dev (rows_stride ints apart) the rows of weight e; rows_max bounds the sum of the rows, rows_each_max the
 // rows of one weight (up to 32 of those: the few-row kernel, one grid row a weight; more: the tiled kernel, row
 // blocks numbered across the weights); the weights' rows of C tile [0, sum of rows).  a_rows: as in SkinnyParams.
-// glu_alpha > 0: gate / up weights combine as clamped_glu instead of as SwiGLU.
+// glu_alpha > 0: gate / up weights combine as clamped_glu instead of as SwiGLU.  parts / part (fp32 results only): where K was split, the parts
+// stay as they are, *parts of [rows_max][N] one after the other from *part on, until the stream's next product; else C is written, *parts = 1.
 int gemm_grouped_rows_dev(const xfthip_weight_t *w, int n_group, const GroupWeight *table_dev, int rows_max, int rows_each_max,
         const int *rows_dev, int rows_stride, const void *A, int lda, void *C, int ldc, int c_dtype, hipStream_t stream,
-        const int *a_rows = nullptr, float glu_limit = 0.0f, float glu_alpha = 0.0f);
+        const int *a_rows = nullptr, float glu_limit = 0.0f, float glu_alpha = 0.0f, int *parts = nullptr, const float **part = nullptr);
 
 int gemm_w8a8_from_bf16(xfthip_weight_t w, int M, const void *A, int lda, void *C, int ldc, int c_dtype, int epilogue,
         const float *bias, const void *res, int ldres, int res_dtype, float gamma, hipStream_t stream);

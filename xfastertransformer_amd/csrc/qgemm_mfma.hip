@@ -204,7 +204,7 @@ int qgemm_split_reserve(hipStream_t stream, float **out) {
     return 0;
 }
 
-int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t stream) {
+int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t stream, int *parts, const float **part) {
     SkinnyParams p = p0;
     p.packed = pw.packed;
     p.scale = pw.scale;
@@ -232,6 +232,10 @@ int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t strea
     XFT_REQUIRE(kernel, "qgemm_mfma: this library was built for BF16 weights only");
     const int rc = kernel(p, stream);
     if (rc || p.ksplit <= 1) return rc;
+    if (parts) {
+        *parts = p.ksplit, *part = p.split_part;
+        return 0;
+    }
     const size_t outs = (size_t)p.M * p.N;
     if (p.N % 4 == 0) // the parts are [M][N] fp32 in a 256-byte aligned buffer: 16-byte loads need only N % 4 == 0
         hipLaunchKernelGGL(qgemm_split_finish_kernel<4>, dim3((unsigned)((outs / 4 + 255) / 256)), dim3(256), 0, stream, p);
