@@ -100,6 +100,36 @@ def test_w8a8_large_m_bit_exact(xh, orc, M, K, N):
     dw.free()
 
 
+# K in parts: 64-row blocks with parts of unequal depth, a ragged K; 128 x 256 blocks with 2 and 3 parts
+@pytest.mark.parametrize("M,K,N", [(33, 4096, 1040), (65, 1008, 240), (130, 11008, 2064), (257, 5632, 80), (1030, 8192, 2064), (700, 14336, 1040)])
+def test_w8a8_parts_of_k_bit_exact(xh, orc, M, K, N):
+    test_w8a8_large_m_bit_exact(xh, orc, M, K, N)
+
+
+def test_w8a8_captured_without_a_parts_buffer(xh, orc):
+    """A captured call on a stream that has no buffer for parts of K runs unsplit: same bits, on every replay."""
+    import ctypes as C
+    M, K, N = 64, 4096, 1024
+    rng = np.random.default_rng(9)
+    w = orc.quantize(orc.W_W8A8, (rng.standard_normal((K, N)) * 0.02).astype(np.float32))
+    dw = xh.Weight(xh.W_W8A8, K, N, w.q, w.scale, w.zero)
+    ad = xh.DeviceBuffer.from_numpy(orc.to_bf16(orc.round_bf16(rng.standard_normal((M, K)))))
+    qa, s, z, sm, ldq = xh.w8a8_quantize_rows(ad.ptr, xh.BF16, M, K, K)
+    cd, cg = xh.DeviceBuffer(M * N * 4), xh.DeviceBuffer(M * N * 4)
+    xh.gemm_w8a8(dw, M, qa, ldq, s, z, sm, cd.ptr, N, xh.F32)
+    xh.synchronize()
+    stream, graph = xh.Stream(), C.c_void_p()
+    assert xh.lib.hipStreamBeginCapture(stream.h, 1) == 0  # as another library would; 1: thread-local checks
+    xh.gemm_w8a8(dw, M, qa, ldq, s, z, sm, cg.ptr, N, xh.F32, stream=stream.h)
+    assert xh.lib.xfthip_graph_end(stream.h, C.byref(graph)) == 0
+    for _ in range(3):
+        assert xh.lib.xfthip_graph_launch(graph, stream.h) == 0
+        xh.synchronize()
+        assert np.array_equal(cg.to_numpy(np.uint32, (M, N)), cd.to_numpy(np.uint32, (M, N)))
+    xh.lib.xfthip_graph_destroy(graph)
+    dw.free()
+
+
 def test_w8a8_model_shape_rows_2048(xh, orc):
     """[2048, 4096] x [4096, 4096] at the model's size: sampled rows against the oracle (rows are
     independent in this path), every output finite."""

@@ -162,6 +162,7 @@ enum ScratchPurpose {
     kScratchPurposes
 };
 int stream_scratch(ScratchPurpose purpose, hipStream_t stream, size_t bytes, bool zero_new, void **out);
+bool stream_scratch_held(ScratchPurpose purpose, hipStream_t stream, size_t bytes); // does that buffer exist
 // While one of these lives, the calling thread's stream_scratch calls take the buffers of `key` whatever stream they
 // name: for work recorded on a capture stream of the library's own that will be launched on `key`.
 struct ScratchKeyScope {

@@ -97,12 +97,6 @@ __global__ __launch_bounds__(256) void qgemm_split_finish_kernel(SkinnyParams p)
     for (int v = 0; v < VEC; ++v) store_from_f32(p.C, p.c_dtype, ci + v, x[v]);
 }
 
-// Partial results of the K split: one buffer per stream and device (stream_scratch), allocated once at its upper
-// bound (64 KB of results a CU in 4 parts: 67 MB on 256 CUs; a split that needs more is not taken), so
-// nothing is allocated or freed on a stream once its buffer exists.  Launches on one stream are ordered; launches
-// on different streams work in different buffers.
-size_t split_bound_floats() { return (size_t)device_cu_count() * 65536; }
-
 // Which tile, how many parts of K and how many K groups a workgroup: the cheapest by a cost model of the launch.
 //   time = start + rounds of resident blocks (steps of 64 k times what a step costs with so many blocks on a CU, + pipeline fill and
 //          results) + the sum of the parts of a split K
@@ -134,7 +128,7 @@ constexpr TileCost kTiles[] = {
 
 constexpr float kSplitStart[3] = {3.0f, 4.0f, 3.0f}, kSplitMb[3] = {0.3f, 0.35f, 0.3f}; // launch and megabytes of a split K's sum
 
-void choose_tile(SkinnyParams &p, int kind, int ktile) {
+void choose_tile(SkinnyParams &p, int kind, int ktile, bool may_split = true) {
     const int cus = device_cu_count(), kt_n = (p.K + ktile - 1) / ktile, cls = kind == XFTHIP_W_BF16 ? 1 : kind == XFTHIP_W_NF4 ? 2 : 0;
     // activations straight into LDS: steps of 64 k, byte offsets of 32 bits
     const bool direct = p.K % 64 == 0 && (size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32);
@@ -164,11 +158,11 @@ void choose_tile(SkinnyParams &p, int kind, int ktile) {
             row_blocks = (p.m_hint + t.rows - 1) / t.rows;
         }
         for (int want : {1, 2, 3, 4, 6, 8}) {
-            if (want > 1 && (p.gateup || p.K / want < 512)) break;
+            if (want > 1 && (!may_split || p.gateup || p.K / want < 512)) break;
             int part = (kt_n + want - 1) / want; // packed tiles
             if (kind == XFTHIP_W_BF16) part = (part + 1) / 2 * 2; // (whole steps of 64)
             const int parts = (kt_n + part - 1) / part, span = parts > 1 ? part * ktile : p.K;
-            if (parts > 1 && (size_t)parts * p.M * p.N > split_bound_floats()) break;
+            if (parts > 1 && (size_t)parts * p.M * p.N > qgemm_split_bound()) break;
             const int band = band_rows(row_blocks, col_blocks * parts), bands = (row_blocks + band - 1) / band;
             const long blocks = ((long)bands * col_blocks * parts + 7) / 8 * 8 * band;
             float steps = (float)((span + 63) / 64);
@@ -197,9 +191,21 @@ void choose_tile(SkinnyParams &p, int kind, int ktile) {
 
 } // namespace
 
+// Partial results of the K split: one buffer per stream and device (stream_scratch), allocated once at its upper
+// bound (64 KB of results a CU in 4 parts: 67 MB on 256 CUs; a split that needs more is not taken), so
+// nothing is allocated or freed on a stream once its buffer exists.  Launches on one stream are ordered; launches
+// on different streams work in different buffers.
+size_t qgemm_split_bound() { return (size_t)device_cu_count() * 65536; }
+
+bool qgemm_split_usable(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess || status == hipStreamCaptureStatusNone) return true;
+    return stream_scratch_held(kScratchGemmSplit, stream, qgemm_split_bound() * sizeof(float));
+}
+
 int qgemm_split_reserve(hipStream_t stream, float **out) {
     void *p = nullptr;
-    if (int rc = stream_scratch(kScratchGemmSplit, stream, split_bound_floats() * sizeof(float), false, &p)) return rc;
+    if (int rc = stream_scratch(kScratchGemmSplit, stream, qgemm_split_bound() * sizeof(float), false, &p)) return rc;
     if (out) *out = (float *)p;
     return 0;
 }
@@ -216,8 +222,9 @@ int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t strea
     p.ksplit = 0, p.split_ktiles = 0, p.split_part = nullptr;
     const int ktile = ktile_of(pw.kind), kt_n = (pw.K + ktile - 1) / ktile;
     choose_tile(p, pw.kind, ktile);
+    if (p.ksplit > 1 && !qgemm_split_usable(stream)) p.ksplit = 0, choose_tile(p, pw.kind, ktile, false);
     if (p.ksplit > 1) {
-        if ((size_t)p.ksplit * p.M * p.N > split_bound_floats()) p.ksplit = 0; // cannot happen within the bound; stay correct anyway
+        if ((size_t)p.ksplit * p.M * p.N > qgemm_split_bound()) p.ksplit = 0; // cannot happen within the bound; stay correct anyway
         else if (int rc = qgemm_split_reserve(stream, &p.split_part)) return rc;
     }
     if (p.ksplit <= 1) p.ksplit = 0;

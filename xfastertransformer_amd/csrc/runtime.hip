@@ -68,6 +68,14 @@ int stream_scratch(ScratchPurpose purpose, hipStream_t stream, size_t bytes, boo
     return 0;
 }
 
+bool stream_scratch_held(ScratchPurpose purpose, hipStream_t stream, size_t bytes) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lk(g_scratch_registry_mu);
+    const auto it = g_scratch_registry.find(std::make_tuple((int)purpose, dev, g_scratch_key_set ? g_scratch_key : stream));
+    return it != g_scratch_registry.end() && it->second.bytes >= bytes;
+}
+
 } // namespace xfthip
 
 using namespace xfthip;

@@ -132,6 +132,9 @@ struct W8A8Params {
     const void *res;
     int ldres, res_dtype;
     float gamma;
+    // more than 32 rows: K in parts of split_tiles x 64 where ksplit > 1, int32 sums [part][M][N] to `part`
+    int ksplit, split_tiles;
+    int *part;
 };
 
 // NT column tiles per wave, MT 16-row activation tiles; U = 4 k tiles (256 k) per load batch;
@@ -318,7 +321,7 @@ __device__ inline float w8a8_epilogue(int epi, float x, float bias, bool has_bia
 // two instead of six weight tiles in registers the block fits two workgroups a CU; every operand read from LDS feeds
 // two MFMAs, where the 128 x 128 block (three workgroups a CU) needs one read per MFMA and is bound by the LDS port.
 template <int WN, int WM, int WR, bool DIRECT = false>
-__global__ __launch_bounds__(256 * WR, DIRECT ? 2 : 1) void w8a8_mfma_kernel(W8A8Params p, int nblocks_n, int nblocks_m) {
+__global__ __launch_bounds__(256 * WR, DIRECT ? 2 : 1) void w8a8_mfma_kernel(W8A8Params p, int nblocks_n, int nblocks_m, int height) {
     static_assert(!DIRECT || (WR == 1 && WM == 4), "direct-to-LDS form: four waves, 128 rows");
     constexpr int ROWS = 32 * WM, BROWS = ROWS * WR, ROWB = DIRECT ? 128 : 64 + 16; // rows of a wave / of the block, LDS row pitch in bytes
     constexpr int CHUNKS = BROWS * 4; // 16-byte chunks of an activation tile
@@ -330,19 +333,36 @@ __global__ __launch_bounds__(256 * WR, DIRECT ? 2 : 1) void w8a8_mfma_kernel(W8A
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_a[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = lane >> 5, nl = lane & 31;
-    // block -> (column block, row block): blocks that share a column block sit on the same XCD; row
-    // blocks are walked in bands of 8, all column blocks of a band before the next band
-    int nb, mb;
+    // block -> (row block, column block, part of K), the row blocks of a column block in a band side by side on one XCD.  height 0: an XCD has
+    // a run of column blocks, bands of 8 row blocks; else units of (band of `height` row blocks, part, column block) are dealt out to the XCDs in
+    // turn (launch_w8a8_mfma has when)
+    int nb, mb, part = 0;
     {
-        constexpr int BAND = 8;
-        const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
-        const int nb8 = (nblocks_n + 7) >> 3;
-        if (slot >= nb8 * nblocks_m) return;
-        const int band = slot / (nb8 * BAND), rem = slot - band * (nb8 * BAND);
-        const int left = nblocks_m - band * BAND, rows_in_band = left < BAND ? left : BAND;
-        nb = rem / rows_in_band + xcd * nb8;
-        mb = band * BAND + rem % rows_in_band;
-        if (nb >= nblocks_n) return;
+        const int id = blockIdx.x, xcd = id & 7, slot = id >> 3; // gridDim.x is a multiple of 8
+        if (height == 0) {
+            const int nb8 = (nblocks_n + 7) >> 3;
+            if (slot >= nb8 * nblocks_m) return;
+            const int band = slot / (nb8 * 8), rem = slot - band * (nb8 * 8);
+            const int left = nblocks_m - band * 8, rows_in_band = left < 8 ? left : 8;
+            nb = rem / rows_in_band + xcd * nb8;
+            mb = band * 8 + rem % rows_in_band;
+            if (nb >= nblocks_n) return;
+        } else {
+            const int per_band = (p.ksplit > 1 ? p.ksplit : 1) * nblocks_n, bands = (nblocks_m + height - 1) / height;
+            const int unit = (slot / height) * 8 + xcd;
+            if (unit >= bands * per_band) return;
+            const int band = unit / per_band, rem = unit - band * per_band;
+            part = rem / nblocks_n;
+            nb = rem - part * nblocks_n;
+            mb = band * height + slot % height;
+            if (mb >= nblocks_m) return;
+        }
+    }
+    if (p.ksplit > 1) { // this workgroup's range of K
+        const int kt0 = part * p.split_tiles, k_left = p.K - kt0 * 64, k_span = p.split_tiles * 64;
+        p.packed += (size_t)kt0 * 1024;
+        p.qa += (size_t)kt0 * 64;
+        p.K = k_left < k_span ? k_left : k_span;
     }
     const int wave_c = wave & 3, wave_r = wave >> 2;
     const int n32_0 = (nb * 4 + wave_c) * WN;
@@ -549,6 +569,19 @@ __global__ __launch_bounds__(256 * WR, DIRECT ? 2 : 1) void w8a8_mfma_kernel(W8A
     }
 
     // ---- epilogue: lane holds C[m0 + 32 m + 8 (j / 4) + 4 h + j % 4][32 (n32_0 + t) + nl] ----------
+    if (p.ksplit > 1) { // the sums as they are, 128 bytes a half wave
+        int *out = p.part + (size_t)part * p.M * p.N;
+#pragma unroll
+        for (int t = 0; t < WN; ++t)
+#pragma unroll
+            for (int m = 0; m < WM; ++m)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const int row = m0 + mw + 32 * m + 8 * (j >> 2) + 4 * h + (j & 3), col = 32 * (n32_0 + t) + nl;
+                    if (row < p.M && col < p.N) out[(size_t)row * p.N + col] = acc[t][m][j];
+                }
+        return;
+    }
     // Each wave drops one 32-row block of its int32 sums at a time into an LDS patch of its own (constant
     // offsets, so the accumulators stay in registers), then walks the patch in 8-column chunks, consecutive
     // lanes along a row: dequantisation, the epilogue of the call and 16-byte stores run in that short loop.
@@ -676,13 +709,59 @@ __global__ __launch_bounds__(256 * WR, DIRECT ? 2 : 1) void w8a8_mfma_kernel(W8A
     }
 }
 
+// The parts of a split K added up (int32: exact, the value of one pass), four columns a thread (N is a multiple of 16), then the dequantisation
+// and the epilogue of the call as above.
+__global__ __launch_bounds__(256) void w8a8_split_finish_kernel(W8A8Params p) {
+    const int nv = p.N / 4;
+    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= (size_t)p.M * nv) return;
+    const int m = (int)(idx / nv), n0 = (int)(idx - (size_t)m * nv) * 4;
+    i32x4 sum = {0, 0, 0, 0};
+    for (int s = 0; s < p.ksplit; ++s) sum += *(const i32x4 *)(p.part + ((size_t)s * p.M + m) * p.N + n0);
+    const bool has_res = p.epi == XFTHIP_EPI_RESMUL || p.epi == XFTHIP_EPI_RESIDENTIAL || p.epi == XFTHIP_EPI_RESEXT;
+    const float sA = p.sA[m], zA = p.zA[m], sumA = p.sumA[m];
+    float x[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int n = n0 + v;
+        const float t0 = ((float)sum[v] * sA) * p.scaleB[n];
+        const float t1 = (p.sumB[n] * p.scaleB[n]) * zA;
+        const float t2 = sumA * (p.zeroB ? p.zeroB[n] : 0.0f);
+        x[v] = w8a8_epilogue(p.epi, (t0 + t1) + t2, p.bias ? p.bias[n] : 0.0f, p.bias != nullptr,
+                has_res ? load_as_f32(p.res, p.res_dtype, (size_t)m * p.ldres + n) : 0.0f, p.gamma);
+    }
+    const size_t ci = (size_t)m * p.ldc + n0;
+    // whole 16-byte (fp32) or 8-byte (16-bit) stores where the row start allows them
+    if (p.c_dtype == XFTHIP_F32 && (((uintptr_t)p.C | ((size_t)p.ldc * 4)) & 15) == 0) {
+        *(float4 *)((float *)p.C + ci) = make_float4(x[0], x[1], x[2], x[3]);
+    } else if (p.c_dtype == XFTHIP_BF16 && (((uintptr_t)p.C | ((size_t)p.ldc * 2)) & 7) == 0) {
+        const uint32_t lo = f32_to_bf16_ref(x[0]) | ((uint32_t)f32_to_bf16_ref(x[1]) << 16);
+        const uint32_t hi = f32_to_bf16_ref(x[2]) | ((uint32_t)f32_to_bf16_ref(x[3]) << 16);
+        *(uint2 *)((uint16_t *)p.C + ci) = make_uint2(lo, hi);
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) store_from_f32(p.C, p.c_dtype, ci + v, x[v]);
+    }
+}
+
 template <int WN, int WM, int WR, bool DIRECT = false>
 static int launch_w8a8_mfma(const W8A8Params &p, hipStream_t stream) {
     const int n32 = (p.NTILES + 1) / 2;
     const int brows = 32 * WM * WR;
     const int nblocks_n = (n32 + 4 * WN - 1) / (4 * WN);
     const int nblocks_m = (p.M + brows - 1) / brows;
-    const int blocks = ((nblocks_n + 7) / 8) * 8 * nblocks_m;
+    // Units dealt out in turn where K is split or where that leaves the first XCD, which has the most, 3 % fewer blocks than runs of column
+    // blocks (1300 rows x 11008 columns in 128 x 256: 61 against 66, 97 us against 106).  With equal loads runs are faster by up to 13 % (256 rows x
+    // 11008 columns in 64 x 128 42 us against 48, 450 x 22016 76 against 84), why is not known.
+    const int per_band = nblocks_n * (p.ksplit > 1 ? p.ksplit : 1), units_8 = (nblocks_n + 7) / 8;
+    int height = band_rows(nblocks_m, per_band), load = 0;
+    const int units = (nblocks_m + height - 1) / height * per_band;
+    for (int u = 0; u < units; u += 8) {
+        const int left = nblocks_m - u / per_band * height;
+        load += left < height ? left : height;
+    }
+    if (p.ksplit <= 1 && load * 100 > units_8 * nblocks_m * 97) height = 0;
+    const int blocks = height ? (units + 7) / 8 * 8 * height : units_8 * 8 * nblocks_m;
     const size_t tiles = DIRECT ? 4 * (size_t)brows * 128 : 3 * (size_t)brows * (64 + 16), patches = 4 * WR * 32 * (size_t)(32 * WN * 4 + 32);
     // the result patches reuse the activation tiles; the per-row statistics sit behind both
     const size_t smem = (tiles > patches ? tiles : patches) + 3 * (size_t)brows * sizeof(float);
@@ -691,11 +770,62 @@ static int launch_w8a8_mfma(const W8A8Params &p, hipStream_t stream) {
                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         XFT_CHECK_HIP(attr);
     }
-    hipLaunchKernelGGL((w8a8_mfma_kernel<WN, WM, WR, DIRECT>), dim3(blocks), dim3(256 * WR), smem, stream, p, nblocks_n, nblocks_m);
+    hipLaunchKernelGGL((w8a8_mfma_kernel<WN, WM, WR, DIRECT>), dim3(blocks), dim3(256 * WR), smem, stream, p, nblocks_n, nblocks_m, height);
     XFT_CHECK_HIP(hipGetLastError());
+    if (p.ksplit > 1) {
+        hipLaunchKernelGGL(w8a8_split_finish_kernel, dim3((unsigned)(((size_t)p.M * p.N / 4 + 255) / 256)), dim3(256), 0, stream, p);
+        XFT_CHECK_HIP(hipGetLastError());
+    }
     return 0;
 }
 
+// Block tile (0: 64 x 128 through registers, 1: 128 x 256 straight into LDS) and parts of K: the cheapest by a model of the launch like that of
+// the weight-only kernels (choose_tile there): rounds of resident blocks, steps of 64 k, what streaming the weights adds, the sum of the parts.
+// Microseconds, least squares on 16 shapes of 2048 .. 28672 columns x 1024 .. 14336 deep, 33 to 4000 rows, weights that do not fit the Infinity
+// Cache.  `large`: the 128 x 256 blocks of whole K give every CU one, which is where they were taken before there were parts; the form of
+// that rule is left only for one that is 8 % cheaper.  Against it alone: 1.16 times as fast in the geometric mean, one of
+// 200 timings 9 % slower, the others within 5; with the quantisation of the rows 33 x 4096 x 14336 97 -> 32 us, 256 rows 96 -> 46, 1024 126 -> 92.
+static int choose_w8a8_tile(W8A8Params &p, bool direct, bool large, hipStream_t stream, int *tile) {
+    struct Cost {
+        int rows, cols, resident;
+        float fixed, step, more, stream;
+    };
+    constexpr Cost kCost[2] = {{64, 128, 4, 0.3f, 0.39f, 0.14f, 0.058f}, {128, 256, 2, 2.9f, 0.55f, 0.51f, 0.051f}};
+    const int cus = device_cu_count(), kt = (p.K + 63) / 64;
+    float best = 1e30f;
+    for (int t = 0; t < (direct ? 2 : 1); ++t) {
+        const Cost &c = kCost[t];
+        const int row_blocks = (p.M + c.rows - 1) / c.rows, col_blocks = (p.N + c.cols - 1) / c.cols;
+        for (int want : {1, 2, 3, 4, 6, 8, 12}) {
+            if (want > 1 && p.K / want < 256) break;
+            int part = (kt + want - 1) / want;
+            if (t) part = (part + 3) / 4 * 4; // (whole step pairs)
+            const int parts = (kt + part - 1) / part;
+            if (parts > 1 && (size_t)parts * p.M * p.N > qgemm_split_bound()) break;
+            const int band = band_rows(row_blocks, col_blocks * parts);
+            const long blocks = ((long)((row_blocks + band - 1) / band) * col_blocks * parts + 7) / 8 * 8 * band;
+            const long slots = (long)cus * c.resident, full = blocks / slots, rest = blocks - full * slots;
+            float us = (float)full * ((float)part * (c.step + c.more * (float)(c.resident - 1)) + c.fixed);
+            if (rest) {
+                const float x = (float)rest / (float)cus, fullest = (float)((rest + cus - 1) / cus);
+                us += (float)part * (x <= 1.0f ? c.step * (0.74f + 0.26f * x) : c.step + c.more * (0.55f * fullest + 0.45f * x - 1.0f)) + c.fixed;
+            }
+            us += 9.8f + c.stream * 1e-6f * (float)p.N * (float)p.K;
+            if (parts > 1) us += 3.0f + 0.43f * 4e-6f * (float)parts * (float)p.M * (float)p.N;
+            else if ((t == 1) == (direct && large)) us *= 0.92f;
+            if (us < best) best = us, *tile = t, p.ksplit = parts > 1 ? parts : 0, p.split_tiles = part;
+        }
+    }
+    if (p.ksplit == 0) return 0;
+    if (!qgemm_split_usable(stream)) { // (captured without the parts' buffer)
+        p.ksplit = 0, *tile = direct && large;
+        return 0;
+    }
+    float *parts = nullptr;
+    if (int rc = qgemm_split_reserve(stream, &parts)) return rc;
+    p.part = (int *)parts;
+    return 0;
+}
 
 } // namespace xfthip
 
@@ -737,21 +867,16 @@ int xfthip_gemm_w8a8(xfthip_weight_t w, int M, const int8_t *qa, int ldq, const 
         p.qa = qa, p.ldq = ldq, p.sA = scaleA, p.zA = zeroA, p.sumA = sumA;
         p.C = C, p.ldc = ldc, p.c_dtype = c_dtype, p.epi = epilogue, p.bias = bias;
         p.res = res, p.ldres = ldres, p.res_dtype = res_dtype, p.gamma = gamma;
-        const int n32 = (pw.NTILES + 1) / 2;
-        // Staged through registers (other K): 128 x 128 tiles once they give every CU its three resident workgroups
-        // (registers allow three), else 128 x 256 with one (eight-wave 256 x 256 blocks were no better anywhere)
-        const long t_large = (long)((n32 + 7) / 8) * ((M + 127) / 128);
-        const long t_mid = (long)((n32 + 3) / 4) * ((M + 127) / 128);
-        // 128 x 256 blocks with the activation rows straight into LDS, two workgroups a CU, wherever they give every
-        // CU a block and K is a whole number of step pairs (the kernel keeps a lane's byte offset into the rows in 32
-        // bits).  With the quantisation of the rows, 2048 / 4096 / 8192 rows on 4096x4096 / 11008x4096 / 4096x11008:
-        // 58 / 130 / 129, 94 / 251 / 226 and 184 / 488 / 483 us against 64 / 163 / 148, 112 / 309 / 317 and
-        // 231 / 583 / 604 us for the forms below.
-        if (t_large >= cus && pw.K % 256 == 0 && (size_t)M * (size_t)ldq < ((size_t)1 << 32))
-            return launch_w8a8_mfma<2, 4, 1, true>(p, (hipStream_t)stream);
-        if (t_mid >= 3 * cus) return launch_w8a8_mfma<1, 4, 1>(p, (hipStream_t)stream);
-        if (t_large >= cus) return launch_w8a8_mfma<2, 4, 1>(p, (hipStream_t)stream);
-        return launch_w8a8_mfma<1, 2, 1>(p, (hipStream_t)stream);
+        const long t_large = (long)((pw.N + 255) / 256) * ((M + 127) / 128), t_mid = (long)((pw.N + 127) / 128) * ((M + 127) / 128);
+        // The activation rows straight into LDS takes a K of whole step pairs (and a lane's byte offset into the rows in 32 bits).  Without it: 128 x
+        // 128 tiles once they give every CU its three resident workgroups (registers allow three), else 128 x 256 with one
+        // (eight-wave 256 x 256 blocks were no better anywhere)
+        const bool direct = pw.K % 256 == 0 && (size_t)M * (size_t)ldq < ((size_t)1 << 32);
+        if (!direct && t_mid >= 3 * cus) return launch_w8a8_mfma<1, 4, 1>(p, (hipStream_t)stream);
+        if (!direct && t_large >= cus) return launch_w8a8_mfma<2, 4, 1>(p, (hipStream_t)stream);
+        int tile = 0;
+        if (int rc = choose_w8a8_tile(p, direct, t_large >= cus, (hipStream_t)stream, &tile)) return rc;
+        return tile ? launch_w8a8_mfma<2, 4, 1, true>(p, (hipStream_t)stream) : launch_w8a8_mfma<1, 2, 1>(p, (hipStream_t)stream);
     }
     for (int m0 = 0; m0 < M; m0 += 32) {
         W8A8Params p = {};
