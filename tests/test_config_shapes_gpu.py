@@ -371,3 +371,16 @@ def test_argmax_ties_and_model_shape(xh, orc):
     lg2[5, 1000] = 60.0
     got2 = xh.argmax(xh.DeviceBuffer.from_numpy(lg2).ptr, 7, 1001)
     assert np.array_equal(got2, lg2.argmax(1).astype(np.int32))
+
+
+@pytest.mark.parametrize("cols", [1, 4, 260, 4096, 32764, 32768, 32772, 151936, 40963])
+def test_argmax_rounds_of_columns(xh, cols):
+    """Columns in rounds of 32768, the last one of few: ties across rounds and threads, rows without a finite value."""
+    rng = np.random.default_rng(cols)
+    lg = rng.standard_normal((5, cols)).astype(np.float32)
+    for r in range(3):
+        lg[r, rng.integers(0, cols, 4)] = 9.0
+    lg[3, cols - 1] = 20.0
+    lg[4] = -np.inf
+    got = xh.argmax(xh.DeviceBuffer.from_numpy(lg).ptr, 5, cols)
+    assert np.array_equal(got, lg.argmax(1).astype(np.int32))
