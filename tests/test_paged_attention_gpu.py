@@ -121,6 +121,81 @@ def test_paged_decode_column_groups(xh, orc, B, qH, kvH, block_size, max_ctx):
     test_paged_decode_matches_oracle(xh, orc, B, qH, kvH, block_size, max_ctx)
 
 
+def _decode64(xh, orc, rng, ctx, qH, kvH, change=None, sharp=1.0, block_size=16):
+    """A decode call and its softmax in 64 bits: the output, the reference, sum of p |v| and the largest argument of an exponential (in
+    magnitude) of every row, sequences in order.  `change(values, tokens in order, sequence)` edits a sequence's values."""
+    D, B = 128, len(ctx)
+    ctx = np.asarray(ctx, np.int32)
+    block_num = int(sum((c + block_size) // block_size for c in ctx)) + 3
+    tab, _ = _tables(rng, ctx, block_size, block_num)
+    where = [tab[b, np.arange(c + 1) // block_size] * block_size + np.arange(c + 1) % block_size for b, c in enumerate(ctx)]
+    kc, vc = _bf(orc, rng, (block_num * block_size, kvH, D)), _bf(orc, rng, (block_num * block_size, kvH, D))
+    q = orc.round_bf16(rng.standard_normal((B, qH, D)).astype(np.float32) * sharp)
+    if change:
+        for b in range(B):
+            change(vc, where[b], b)
+    slots = np.asarray([w[-1] for w in where], np.int32)
+    dev = lambda a: xh.DeviceBuffer.from_numpy(np.ascontiguousarray(a))
+    bits = lambda a: dev(orc.to_bf16(a))
+    dq, dk, dv, dkc, dvc = bits(q), bits(kc[slots]), bits(vc[slots]), bits(kc), bits(vc)
+    dt, dc, ds, out = dev(tab), dev(ctx), dev(slots), xh.DeviceBuffer(B * qH * D * 2)
+    xh.paged_attention_decode(out.ptr, dq.ptr, dk.ptr, dv.ptr, qH, kvH, D, qH * D, kvH * D, qH * D, D ** -0.5, B, dkc.ptr, dvc.ptr, block_num,
+                              block_size, dt.ptr, tab.shape[1], dc.ptr, ds.ptr, int(ctx.max()))
+    xh.synchronize()
+    ref, size, slack = (np.zeros((B, qH, D)) for _ in range(3))
+    for b in range(B):
+        k, v = kc[where[b]].astype(np.float64), vc[where[b]].astype(np.float64)
+        for h in range(qH):
+            x = k[:, h * kvH // qH] @ q[b, h].astype(np.float64) * D ** -0.5
+            p = np.exp(x - x.max())
+            p /= p.sum()
+            with np.errstate(invalid="ignore"):
+                ref[b, h], size[b, h] = p @ v[:, h * kvH // qH], p @ np.abs(v[:, h * kvH // qH])
+            # an argument is off by the score's 128 products and additions, and by its own roundings; n probabilities are added up in fp32
+            spread = (np.abs(k[:, h * kvH // qH]) @ np.abs(q[b, h].astype(np.float64))).max() * D ** -0.5
+            slack[b, h] = 2 * spread * 132 * 2.0 ** -24 + 2 * (np.abs(x).max() + 8) * 2.0 ** -22 + (len(x) + 64) * 2.0 ** -24
+    return orc.from_bf16(out.to_numpy(np.uint16, (B, qH, D))).astype(np.float64), ref, size, slack
+
+
+@pytest.mark.parametrize("qH,kvH,ctx,sharp", [(32, 8, [8200, 33], 1.0), (32, 8, [1500] * 40, 1.0), (8, 1, [4000, 500], 6.0), (4, 4, [3100], 12.0)])
+def test_paged_decode_against_64_bits(xh, orc, qH, kvH, ctx, sharp):
+    """Bound: half a step of the bf16 result (8 significant bits: 2^-8 of it at most), and what the fp32 scores, exponentials and sums are off by,
+    relative to sum p |v|: long contexts whose outputs are small beside the values, and scores of which one takes nearly everything."""
+    got, ref, size, slack = _decode64(xh, orc, np.random.default_rng(len(ctx) + qH), ctx, qH, kvH, sharp=sharp)
+    bound = np.abs(ref) * 2.0 ** -8 + size * slack
+    worst = float((np.abs(got - ref) / bound).max())
+    print(f"paged decode heads {qH}/{kvH}, {len(ctx)} x {max(ctx)}, queries x {sharp}: {worst:.3f} of the bound", flush=True)
+    assert worst <= 1.0
+
+
+def test_paged_decode_probabilities_in_32_bits(xh, orc):
+    """Values that nearly cancel: the first token's 1 against four tokens of the same lower probability e, whose values are bf16 parts of -1 / e.
+    What is left shows the probabilities' own precision.  Bound: an argument of the exponential between -8 and 0, two roundings of it and a unit
+    in the last place of the function, 2^-24 of the sums, together below 2^-20 of sum p |v|; a probability in 16 bits is off by up to 2^-17."""
+    D, H, rng = 128, 32, np.random.default_rng(2)
+    q, k, v = np.zeros((1, H, D), np.float32), np.zeros((5, H, D), np.float32), np.zeros((5, H, D), np.float32)
+    q[0, :, 0] = 1.0
+    k[1:, :, 0] = orc.round_bf16(-rng.uniform(5, 80, H).astype(np.float32))
+    e = np.exp(k[1, :, 0].astype(np.float64) * D ** -0.5)
+    v[0] = 1.0
+    left = np.repeat(-1.0 / e[:, None], D, 1)
+    for t in range(1, 5):
+        v[t] = orc.round_bf16(left.astype(np.float32))
+        left -= v[t]
+    dev = lambda a: xh.DeviceBuffer.from_numpy(np.ascontiguousarray(a))
+    bits = lambda a: dev(orc.to_bf16(a))
+    dq, dk, dv, dkc, dvc = bits(q), bits(k[4:]), bits(v[4:]), bits(k), bits(v)
+    dt, dc, ds, out = dev(np.zeros((1, 1), np.int32)), dev(np.asarray([4], np.int32)), dev(np.asarray([4], np.int32)), xh.DeviceBuffer(H * D * 2)
+    xh.paged_attention_decode(out.ptr, dq.ptr, dk.ptr, dv.ptr, H, H, D, H * D, H * D, H * D, D ** -0.5, 1, dkc.ptr, dvc.ptr, 1, 5, dt.ptr, 1, dc.ptr, ds.ptr, 4)
+    xh.synchronize()
+    got = orc.from_bf16(out.to_numpy(np.uint16, (H, D))).astype(np.float64)
+    p = np.stack([np.ones(H)] + [e] * 4)[:, :, None] / (1.0 + 4.0 * e)[None, :, None]
+    ref, size = (p * v).sum(0), (p * np.abs(v)).sum(0)
+    worst = float((np.abs(got - ref) / (np.abs(ref) * 2.0 ** -8 + size * 2.0 ** -20)).max())
+    print(f"paged decode, values that cancel: {worst:.3f} of the bound", flush=True)
+    assert worst <= 1.0
+
+
 @pytest.mark.parametrize("qH,kvH,lens,block_size", [(32, 4, [33, 500, 1, 700, 65], 16), (16, 4, [31, 32, 33, 64, 96, 97], 5), (8, 8, [40] * 70, 16),
                                                     (24, 3, [600, 200, 450, 20, 7], 16), (4, 2, [3, 90, 17], 4)])
 def test_paged_prefill_side_by_side(xh, orc, qH, kvH, lens, block_size):

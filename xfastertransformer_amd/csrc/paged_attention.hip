@@ -60,8 +60,6 @@ union BFrag {
     uint32_t u[4];
     u32x4 q;
 };
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 // grid (nsplit, kv_heads * column groups, batch), 256 threads.  head_size = 128.
 // The columns of a workgroup are up to 16 query heads of one key / value head; a wave takes every fourth 32-token block of
@@ -72,12 +70,13 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 //     (whole 256-byte rows across 16 lanes), turns its 8 x 8 values round with 32 byte permutes and so holds the operands
 //     of 8 products whose row r stands for dim 8 r + j - no LDS, no exchange.  Lane group g takes the tokens 4 g .. + 3 of
 //     both 16-token score tiles, the ones whose probabilities it holds.
-// The probabilities stay at 16 bits of mantissa and more: each goes in as the sum of two bf16 values (upper half, rounded
-// rest), one product each; sums of probabilities are those of the fp32 values.
+// The probabilities stay fp32: each goes in as the sum of three bf16 values (8 bits each, cut off one after the other), one
+// product each.  Two parts were off by up to 2^-17, more than the exponential; the third costs 0.6 % of the call below, 4 % of one
+// sequence of 64000 tokens.
 // The next block's keys are requested once this block's scores are done, its values once this block's are turned; the
 // cache rows of the block after that (a table look-up a lane) a block earlier.
 // Bound by the cache's trip from HBM.  32 sequences of 2100 .. 4100 tokens, 32 query / 8 KV heads, 408 MB:
-// 86 us, 4.7 TB/s (244 us with a workgroup a query head on the vector ALUs, every head of a group reading the cache again).  212
+// 87 us, 4.7 TB/s (244 us with a workgroup a query head on the vector ALUs, every head of a group reading the cache again).  about 215
 // registers, two workgroups a CU; held to three, 63 of them spill.
 __global__ __launch_bounds__(256, 2) void paged_decode_kernel(PagedParams p) {
     constexpr int D = 128;
@@ -167,13 +166,15 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(PagedParams p) {
             psum += e[i];
         }
         l = l * alpha + psum;
-        BFrag hi, lo;
+        BFrag pp[3];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float x = e[2 * i], y = e[2 * i + 1];
-            hi.u[i] = __builtin_amdgcn_perm(f2u(y), f2u(x), 0x07060302u);
-            const f32x2_t rest = {x - u2f(f2u(x) & 0xFFFF0000u), y - u2f(f2u(y) & 0xFFFF0000u)};
-            lo.u[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, bf16x2_t));
+            float x = e[2 * i], y = e[2 * i + 1];
+#pragma unroll
+            for (int part = 0; part < 3; ++part) {
+                pp[part].u[i] = __builtin_amdgcn_perm(f2u(y), f2u(x), 0x07060302u);
+                x -= u2f(f2u(x) & 0xFFFF0000u), y -= u2f(f2u(y) & 0xFFFF0000u);
+            }
         }
         // ---- values: 8 tokens x 8 dims turned round, then O^T ----
         BFrag vt[8];
@@ -191,8 +192,8 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(PagedParams p) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             o[j] = o[j] * alpha;
-            o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[j].v, lo.v, o[j], 0, 0, 0);
-            o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[j].v, hi.v, o[j], 0, 0, 0);
+#pragma unroll
+            for (int part = 2; part >= 0; --part) o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[j].v, pp[part].v, o[j], 0, 0, 0);
         }
     }
     // ---- merge the four waves; row 4 g + r of product j is dim 8 (4 g + r) + j ----
