@@ -196,6 +196,26 @@ def test_paged_decode_probabilities_in_32_bits(xh, orc):
     assert worst <= 1.0
 
 
+@pytest.mark.parametrize("qH,kvH,n", [(8, 2, 5), (8, 2, 32), (32, 8, 33), (20, 1, 700), (4, 4, 4000)])
+def test_paged_decode_infinite_values(xh, orc, qH, kvH, n):
+    """Infinities and NaN among the values, at the first, the last and the highest-scored tokens: every dimension of the output is what the sum of
+    fp32 products gives (infinite with one sign, NaN with both or beside a NaN, finite where all values are)."""
+    marks = {0: np.inf, 1: -np.inf, 2: np.nan}
+
+    def change(v, where, b):
+        for t, d in ((0, 3), (n - 1, 5), (n // 2, 6)):
+            v[where[t], :, 4 * d + b % 3] = marks[b % 3]
+        v[where[:], :, 70] = np.inf  # (all tokens: the highest-scored one of every head among them)
+        v[where[0], :, 71], v[where[n - 1], :, 71] = np.inf, -np.inf if n > 1 else np.inf
+
+    rng = np.random.default_rng(n)
+    got, ref, size, slack = _decode64(xh, orc, rng, [n - 1] * 3, qH, kvH, change)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+    assert np.array_equal(got[np.isinf(got)], ref[np.isinf(ref)])
+    fine = np.isfinite(ref)
+    assert (np.abs(got[fine] - ref[fine]) <= np.abs(ref[fine]) * 2.0 ** -8 + size[fine] * slack[fine]).all()
+
+
 @pytest.mark.parametrize("qH,kvH,lens,block_size", [(32, 4, [33, 500, 1, 700, 65], 16), (16, 4, [31, 32, 33, 64, 96, 97], 5), (8, 8, [40] * 70, 16),
                                                     (24, 3, [600, 200, 450, 20, 7], 16), (4, 2, [3, 90, 17], 4)])
 def test_paged_prefill_side_by_side(xh, orc, qH, kvH, lens, block_size):

@@ -200,11 +200,54 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(PagedParams p) {
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
     if (g == 0) s_m[wave][cl] = m, s_l[wave][cl] = l;
+    bool nan = false;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        float *dst = &s_o[wave][cl][8 * (4 * g + r)];
-        *(f32x4 *)dst = f32x4 {o[0][r], o[1][r], o[2][r], o[3][r]};
-        *(f32x4 *)(dst + 4) = f32x4 {o[4][r], o[5][r], o[6][r], o[7][r]};
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) nan |= o[j][r] != o[j][r];
+    if (__builtin_amdgcn_ballot_w64(nan) == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float *dst = &s_o[wave][cl][8 * (4 * g + r)];
+            *(f32x4 *)dst = f32x4 {o[0][r], o[1][r], o[2][r], o[3][r]};
+            *(f32x4 *)(dst + 4) = f32x4 {o[4][r], o[5][r], o[6][r], o[7][r]};
+        }
+    } else {
+        // A value that is not finite, times a part of a probability that is zero or times the zero of a slot past the end: the wave's blocks
+        // again, a column at a time, one product a value in fp32 and none for those slots
+        const float ref = m == -INFINITY ? 0.0f : m;
+        for (int col = 0; col < cols; ++col) {
+            float acc[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+            for (blk = b0 + wave; blk < b1; blk += 4) {
+                const int rows = row_of(blk);
+                load_keys(rows);
+                load_values(rows);
+#pragma unroll
+                for (int a = 0; a < 2; ++a) {
+                    f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[a][s].v, qf[s].v, sc, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float e = __shfl(__expf(sc[r] * p.scale - ref), 16 * g + col, 64);
+                        const bool seen = 32 * blk + 16 * a + 4 * g + r < n;
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) {
+                            const uint32_t w = vf[4 * a + r].u[j >> 1];
+                            acc[j] = seen ? fmaf(e, u2f(j & 1 ? w & 0xFFFF0000u : w << 16), acc[j]) : acc[j];
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                acc[j] += __shfl_xor(acc[j], 16, 64);
+                acc[j] += __shfl_xor(acc[j], 32, 64);
+                if (g == 0) s_o[wave][col][8 * cl + j] = acc[j];
+            }
+        }
     }
     __syncthreads();
     for (int v = threadIdx.x; v < cols * D; v += 256) {
