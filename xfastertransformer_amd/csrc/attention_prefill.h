@@ -66,8 +66,12 @@ union HFrag32 {
 // two k-steps (the queries' dims and, through a lane-half exchange, the probabilities' tokens permuted to match) -
 // 8 operand reads a block and wave instead of 16, widened by every wave in registers: correct, and 354 us against
 // 292: the 160 widening instructions a wave and block cost more than the LDS port had.
-template <int NW, int CT, bool INT8>
+// SCALED (FP16 cache): the queries carry the softmax scale and log2 e (rounded to fp16 once: 2^-12 relative, the size of
+// the rounding of the fp16 probabilities), so that a score leaves the MFMA in the log2 domain, relative to the reference point.  Without, the
+// queries are exact and the scale is applied to the fp32 scores, 16 instructions a block.
+template <int NW, int CT, bool INT8, bool SCALED = !INT8>
 __device__ inline void attn_prefill32_unit(const AttnParams &p, const int kvh, const int cgroup, const int b, unsigned char *lds) {
+    static_assert(SCALED ? !INT8 : (INT8 || CT == 1), "queries without the scale: an INT8 cache, or one column tile a wave");
     constexpr int D = 128, NT = NW * 64, WC = 32 * CT;
     // FP16 cache, one tile a wave: reference point and row sums through the MFMAs (below); with two tiles a wave the
     // 64 registers this takes are not there, and the vector ALUs have the time
@@ -198,10 +202,8 @@ __device__ inline void attn_prefill32_unit(const AttnParams &p, const int kvh, c
     };
 
     // ---- this wave's queries: B operand of the score MFMA, k-step s covers dims 16 s + 8 h .. + 8 ----
-    // FP16 cache: the queries carry the softmax scale and log2 e (rounded to fp16 once: 2^-12 relative, the size of
-    // the rounding of the fp16 probabilities), so that a score leaves the MFMA in the log2 domain.
     const float c1 = p.scale * 1.4426950408889634f;
-    const float qmul = INT8 ? 1.0f : c1;
+    const float qmul = SCALED ? c1 : 1.0f;
     HFrag32 qf[CT][8];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
@@ -217,7 +219,7 @@ __device__ inline void attn_prefill32_unit(const AttnParams &p, const int kvh, c
     float m_run[CT], l_run[CT]; // m_run == kNegBig: the column has seen no token yet
     float vref = 0.0f; // INT8: the value scales are taken relative to this (0 = not set yet)
     f32x16 o[CT][4];
-    // FP16 cache: the score MFMAs start from -m_run instead of 0, so a score arrives relative to the column's
+    // FP16 cache: the score MFMAs start from -m_run instead of 0 (SCALED), so a score arrives relative to the column's
     // reference point with no vector instruction spent on it, and the row sums of the probabilities come out of
     // two more MFMAs against a tile of ones (the matrix pipes have the slack, the vector ALUs do not).
     f32x16 negm[VIA_MFMA ? CT : 1], lacc[VIA_MFMA ? CT : 1];
@@ -243,7 +245,7 @@ __device__ inline void attn_prefill32_unit(const AttnParams &p, const int kvh, c
         f32x16 sc[CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-            if constexpr (!VIA_MFMA) {
+            if constexpr (!VIA_MFMA || !SCALED) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sc[ct][r] = 0.0f;
             } else {
@@ -334,6 +336,10 @@ __device__ inline void attn_prefill32_unit(const AttnParams &p, const int kvh, c
                         for (int r = 0; r < 16; ++r) o[ct][dt][r] *= oscale;
                 }
             } else {
+                if constexpr (!SCALED) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) x[r] = fmaf(x[r], c1, negm[ct][r]);
+                }
                 if (masked) {
                     asm volatile("" ::: "memory");
 #pragma unroll
