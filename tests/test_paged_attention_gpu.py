@@ -259,6 +259,44 @@ def test_paged_prefill_as_exact_as_alone(xh, orc, qH, kvH, lens):
         assert a <= 1.02 * b, f"{n} tokens: error among others / alone {a / b:.4f}"
 
 
+def _captured(xh, stream, call, out, shape):
+    """Three replays of `call(stream)` captured on `stream`, each into a cleared output."""
+    graph = C.c_void_p()
+    xh.check(xh.lib.xfthip_graph_begin(stream.h))
+    call(stream.h)
+    xh.check(xh.lib.xfthip_graph_end(stream.h, C.byref(graph)))
+    for _ in range(3):
+        out.upload(np.zeros(shape, np.uint16))
+        xh.check(xh.lib.xfthip_graph_launch(graph, stream.h))
+        xh.synchronize()
+        yield out.to_numpy(np.uint16, shape)
+    xh.lib.xfthip_graph_destroy(graph)
+
+
+def test_paged_decode_captured_behind_an_unsplit_call(xh, orc):
+    """A stream's first call brings all its buffers: one that splits no context, then, captured, one that does."""
+    D, qH, kvH, B, n = 128, 32, 8, 32, 300
+    rng = np.random.default_rng(1)
+    dev = lambda a: xh.DeviceBuffer.from_numpy(a)
+    bits = lambda *shape: dev(orc.to_bf16(_bf(orc, rng, shape)))
+    q, k, v, kc, vc = bits(B, qH * D), bits(B, kvH * D), bits(B, kvH * D), bits(B * n, kvH * D), bits(B * n, kvH * D)
+    table, ctx, slots = dev(np.arange(B, dtype=np.int32)), dev(np.full(B, n - 1, np.int32)), dev(np.arange(1, B + 1, dtype=np.int32) * n - 1)
+    out = xh.DeviceBuffer(B * qH * D * 2)
+
+    def call(batch, stream=None):
+        xh.paged_attention_decode(out.ptr, q.ptr, k.ptr, v.ptr, qH, kvH, D, qH * D, kvH * D, qH * D, D ** -0.5, batch, kc.ptr, vc.ptr, B, n, table.ptr, 1,
+                                  ctx.ptr, slots.ptr, n - 1, stream=stream)
+
+    call(4)
+    xh.synchronize()
+    want = out.to_numpy(np.uint16, (B, qH * D))[:4].copy()
+    stream = xh.Stream()
+    call(B, stream.h)
+    stream.synchronize()
+    for got in _captured(xh, stream, lambda st: call(4, st), out, (B, qH * D)):
+        assert np.array_equal(got[:4], want)
+
+
 def test_invoke_attention_serving_loop(orc):
     """xft::invokeAttention on host buffers: prefill of two sequences, then decode steps that append to
     the paged cache; outputs against the oracle and the caller's cache arrays kept current."""

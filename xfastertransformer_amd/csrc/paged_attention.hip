@@ -447,10 +447,10 @@ extern "C" int xfthip_paged_attention_decode(void *out, const void *q, const voi
     if (nsplit > cap) nsplit = cap;
     if (nsplit > kMaxSplits) nsplit = kMaxSplits;
     if (nsplit < 1) nsplit = 1;
-    const size_t need = (size_t)batch * q_heads * nsplit * 130;
+    // The parts of any split call: below 2 CUs workgroups of 16 columns (4.3 MB on 256 CUs).  Taken by the stream's first call, split or not, so that
+    // none behind it allocates (a captured one must not).
     void *part = nullptr;
-    if (nsplit > 1)
-        if (int rc = stream_scratch(kScratchPagedParts, st, need * sizeof(float), false, &part)) return rc;
+    if (int rc = stream_scratch(kScratchPagedParts, st, (size_t)2 * device_cu_count() * 16 * 130 * sizeof(float), false, &part)) return rc;
     PagedParams p = {};
     p.out = (uint16_t *)out, p.q = (const uint16_t *)q, p.kc = (const uint16_t *)kcache, p.vc = (const uint16_t *)vcache;
     p.tables = block_tables, p.ctx = context_lens, p.part = (float *)part;
