@@ -297,6 +297,27 @@ def test_paged_decode_captured_behind_an_unsplit_call(xh, orc):
         assert np.array_equal(got[:4], want)
 
 
+def test_paged_prefill_captured_with_other_lengths(xh, orc):
+    """A warm-up of one sequence, then, captured, the same tokens as ten sequences, each with a partly filled block."""
+    D, qH, kvH, T, rng = 128, 16, 4, 100, np.random.default_rng(3)
+    bits = lambda n: xh.DeviceBuffer.from_numpy(orc.to_bf16(_bf(orc, rng, (T, n * D))))
+    q, k, v, kc, vc = bits(qH), bits(kvH), bits(kvH), bits(kvH), bits(kvH)
+    slots, out = xh.DeviceBuffer.from_numpy(np.arange(T, dtype=np.int32)), xh.DeviceBuffer(T * qH * D * 2)
+
+    def call(lens, stream=None):
+        xh.paged_attention_prefill(out.ptr, q.ptr, k.ptr, v.ptr, qH, kvH, D, qH * D, kvH * D, qH * D, D ** -0.5, lens, kc.ptr, vc.ptr, T, 1, slots.ptr,
+                                   stream=stream)
+
+    call([10] * 10)
+    xh.synchronize()
+    want = out.to_numpy(np.uint16, (T, qH * D)).copy()
+    stream = xh.Stream()
+    call([T], stream.h)
+    stream.synchronize()
+    for got in _captured(xh, stream, lambda st: call([10] * 10, st), out, (T, qH * D)):
+        assert np.array_equal(got, want)
+
+
 def test_invoke_attention_serving_loop(orc):
     """xft::invokeAttention on host buffers: prefill of two sequences, then decode steps that append to
     the paged cache; outputs against the oracle and the caller's cache arrays kept current."""

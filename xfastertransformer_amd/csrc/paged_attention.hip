@@ -478,14 +478,13 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
     std::vector<int> order(batch), first(batch);
     for (int b = 0, at = 0; b < batch; at += token_lens_host[b], ++b) order[b] = b, first[b] = at;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return token_lens_host[x] > token_lens_host[y]; });
-    size_t most = 0; // 32-token blocks of the largest launch
-    for (int b = 0; b < batch; b += per_launch) {
-        size_t blocks = 0;
-        for (int i = b; i < batch && i < b + per_launch; ++i) blocks += (token_lens_host[order[i]] + 31) / 32;
-        most = std::max(most, blocks);
-    }
+    // Scratch for the keys and values of any lengths that add up to these tokens (a sequence of a launch fills its last 32-token block), with the bytes of
+    // the whole q | k | v rows: a later call of no more bytes allocates nothing, whatever its lengths (a captured one must not)
+    size_t total = 0;
+    for (int b = 0; b < batch; ++b) total += token_lens_host[b];
+    const size_t kv_bytes = (total + 31 * kSeqs) * kv_heads * 128 * 4;
     void *scratch = nullptr;
-    if (int rc = stream_scratch(kScratchPagedKv, st, most * 32 * kv_heads * 128 * 4, false, &scratch)) return rc;
+    if (int rc = stream_scratch(kScratchPagedKv, st, kv_bytes + total * q_heads * 128 * 2, false, &scratch)) return rc;
     const int G = q_heads / kv_heads;
     for (int b = 0; b < batch; b += per_launch) {
         SeqBatch s = {};
