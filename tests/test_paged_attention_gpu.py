@@ -259,6 +259,15 @@ def test_paged_prefill_as_exact_as_alone(xh, orc, qH, kvH, lens):
         assert a <= 1.02 * b, f"{n} tokens: error among others / alone {a / b:.4f}"
 
 
+_streams = []
+
+
+def _stream(xh):
+    """One no test before has used: scratch is kept by a stream's handle, which a destroyed one's successor may get."""
+    _streams.append(xh.Stream())
+    return _streams[-1]
+
+
 def _captured(xh, stream, call, out, shape):
     """Three replays of `call(stream)` captured on `stream`, each into a cleared output."""
     graph = C.c_void_p()
@@ -290,16 +299,18 @@ def test_paged_decode_captured_behind_an_unsplit_call(xh, orc):
     call(4)
     xh.synchronize()
     want = out.to_numpy(np.uint16, (B, qH * D))[:4].copy()
-    stream = xh.Stream()
+    stream = _stream(xh)
     call(B, stream.h)
     stream.synchronize()
     for got in _captured(xh, stream, lambda st: call(4, st), out, (B, qH * D)):
         assert np.array_equal(got[:4], want)
 
 
-def test_paged_prefill_captured_with_other_lengths(xh, orc):
-    """A warm-up of one sequence, then, captured, the same tokens as ten sequences, each with a partly filled block."""
-    D, qH, kvH, T, rng = 128, 16, 4, 100, np.random.default_rng(3)
+@pytest.mark.parametrize("qH,kvH,warm,lens", [(16, 4, [100], [10] * 10), (4, 1, [150] * 2, [200])])
+def test_paged_prefill_captured_with_other_lengths(xh, orc, qH, kvH, warm, lens):
+    """A warm-up, then, captured, no more tokens in other lengths: in ten sequences, each with a partly filled block, and in a single one, whose
+    keys are split among workgroups."""
+    D, T, rng = 128, sum(warm), np.random.default_rng(3)
     bits = lambda n: xh.DeviceBuffer.from_numpy(orc.to_bf16(_bf(orc, rng, (T, n * D))))
     q, k, v, kc, vc = bits(qH), bits(kvH), bits(kvH), bits(kvH), bits(kvH)
     slots, out = xh.DeviceBuffer.from_numpy(np.arange(T, dtype=np.int32)), xh.DeviceBuffer(T * qH * D * 2)
@@ -308,14 +319,15 @@ def test_paged_prefill_captured_with_other_lengths(xh, orc):
         xh.paged_attention_prefill(out.ptr, q.ptr, k.ptr, v.ptr, qH, kvH, D, qH * D, kvH * D, qH * D, D ** -0.5, lens, kc.ptr, vc.ptr, T, 1, slots.ptr,
                                    stream=stream)
 
-    call([10] * 10)
+    call(lens)
     xh.synchronize()
-    want = out.to_numpy(np.uint16, (T, qH * D)).copy()
-    stream = xh.Stream()
-    call([T], stream.h)
+    n = sum(lens)
+    want = out.to_numpy(np.uint16, (T, qH * D))[:n].copy()
+    stream = _stream(xh)
+    call(warm, stream.h)
     stream.synchronize()
-    for got in _captured(xh, stream, lambda st: call([10] * 10, st), out, (T, qH * D)):
-        assert np.array_equal(got, want)
+    for got in _captured(xh, stream, lambda st: call(lens, st), out, (T, qH * D)):
+        assert np.array_equal(got[:n], want)
 
 
 def test_invoke_attention_serving_loop(orc):

@@ -82,7 +82,7 @@ void attention_workspace_destroy(AttnWorkspace *w) {
 }
 
 // the workspace of plain calls on `stream`
-static int attention_stream_workspace(hipStream_t stream, AttnWorkspace *w) {
+int attention_stream_workspace(hipStream_t stream, AttnWorkspace *w) {
     void *parts = nullptr, *tickets = nullptr;
     if (int rc = stream_scratch(kScratchAttnParts, stream, (size_t)kWsSlots * kSlotFloats * sizeof(float), false, &parts)) return rc;
     if (int rc = stream_scratch(kScratchAttnTickets, stream, (size_t)kWsSlots * sizeof(unsigned int), true, &tickets)) return rc;

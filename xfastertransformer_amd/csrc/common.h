@@ -180,6 +180,7 @@ struct AttnWorkspace {
 };
 int attention_workspace_create(AttnWorkspace *w, int slots); // allocates; not for use during stream capture
 void attention_workspace_destroy(AttnWorkspace *w);
+int attention_stream_workspace(hipStream_t stream, AttnWorkspace *w); // that of attention_launch without one on this stream; its first call allocates
 // resolves the device address of the statically allocated workspace behind xfthip_attention_static
 // for the current device (idempotent, allocates nothing)
 int attention_static_scratch_init();

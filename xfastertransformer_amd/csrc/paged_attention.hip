@@ -486,6 +486,12 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
     void *scratch = nullptr;
     if (int rc = stream_scratch(kScratchPagedKv, st, kv_bytes + total * q_heads * 128 * 2, false, &scratch)) return rc;
     const int G = q_heads / kv_heads;
+    for (int b = 0; b < batch; ++b) // likewise what one of these sequences by itself splits its keys through
+        if (attention_split_count(token_lens_host[b], kv_heads * ((token_lens_host[b] * G + 15) / 16)) > 1) {
+            AttnWorkspace of_stream;
+            if (int rc = attention_stream_workspace(st, &of_stream)) return rc;
+            break;
+        }
     for (int b = 0; b < batch; b += per_launch) {
         SeqBatch s = {};
         s.n = std::min(per_launch, batch - b);
