@@ -259,6 +259,39 @@ def test_paged_prefill_as_exact_as_alone(xh, orc, qH, kvH, lens):
         assert a <= 1.02 * b, f"{n} tokens: error among others / alone {a / b:.4f}"
 
 
+# rows of q | k | v in one buffer; the results over the queries in place, at the buffer's start in a row length of their own, and one head on
+@pytest.mark.parametrize("o_stride,shift", [(None, 0), (16, 0), (24, 1), (None, 1), (None, 16)])
+@pytest.mark.parametrize("phase,B", [("decode", 3), ("decode", 70), ("prompt", 3), ("prompt", 70)])
+def test_paged_results_over_their_inputs(xh, orc, phase, B, o_stride, shift):
+    """Results that lie over the call's queries, keys or values, in their rows or others', are those of a call with a buffer of their own."""
+    D, qH, kvH, rng = 128, 16, 4, np.random.default_rng(B)
+    lens = [1] * B if phase == "decode" else [int(n) for n in rng.integers(1, 60, B)]
+    T, stride, n = sum(lens), (qH + 2 * kvH) * D, 40
+    o = stride if o_stride is None else o_stride * D
+    rows = orc.to_bf16(_bf(orc, rng, (T + 2, stride)))
+    dev = lambda a: xh.DeviceBuffer.from_numpy(a)
+    kc, vc = (dev(orc.to_bf16(_bf(orc, rng, (max(B * n, T), kvH * D)))) for _ in range(2))
+    slots = dev(np.arange(1, B + 1, dtype=np.int32) * n - 1 if phase == "decode" else np.arange(T, dtype=np.int32))
+    table, ctx = dev(np.arange(B, dtype=np.int32)), dev(np.full(B, n - 1, np.int32))
+
+    def call(buf, out, o):
+        at = lambda heads: C.c_void_p(buf.ptr.value + heads * D * 2)
+        if phase == "decode":
+            xh.paged_attention_decode(out, at(0), at(qH), at(qH + kvH), qH, kvH, D, stride, stride, o, D ** -0.5, B, kc.ptr, vc.ptr, B, n, table.ptr, 1,
+                                      ctx.ptr, slots.ptr, n - 1)
+        else:
+            xh.paged_attention_prefill(out, at(0), at(qH), at(qH + kvH), qH, kvH, D, stride, stride, o, D ** -0.5, lens, kc.ptr, vc.ptr, T, 1, slots.ptr)
+        xh.synchronize()
+
+    own, buf = xh.DeviceBuffer(T * qH * D * 2), dev(rows)
+    call(buf, own.ptr, qH * D)
+    want = own.to_numpy(np.uint16, (T, qH * D))
+    call(buf, C.c_void_p(buf.ptr.value + shift * D * 2), o)
+    flat = buf.to_numpy(np.uint16, ((T + 2) * stride,))
+    got = np.stack([flat[shift * D + t * o:shift * D + t * o + qH * D] for t in range(T)])
+    assert np.array_equal(got, want)
+
+
 _streams = []
 
 

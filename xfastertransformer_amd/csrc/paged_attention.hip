@@ -260,7 +260,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(PagedParams p) {
             ll = fmaf(s_l[w][col], f, ll);
             acc = fmaf(s_o[w][col][d], f, acc);
         }
-        if (p.nsplit == 1) {
+        if (!p.part) {
             p.out[(size_t)b * p.o_stride + hq * D + d] = f32_to_bf16_ref(acc / ll);
         } else {
             float *dst = p.part + (((size_t)b * p.q_heads + hq) * p.nsplit + split) * (D + 2);
@@ -409,6 +409,21 @@ __global__ __launch_bounds__(256, 3) void paged_prefill_few_kernel(AttnParams al
     attn_unit<false, 4, false>(p, 0, blockIdx.x % all.kv.H, cg, 0, lds, [] { __syncthreads(); });
 }
 
+// Rows of `out` and of `x` (strides and widths in elements) that lie such that writing one row of the former may change another row, or another
+// head, of the latter: a workgroup that writes its results must not do so before all others have read.
+bool in_the_way(const void *out, long o_stride, long o_width, const void *x, long x_stride, long x_width, long rows) {
+    const long d = ((const char *)out - (const char *)x) / 2;
+    if (d >= (rows - 1) * x_stride + x_width || -d >= (rows - 1) * o_stride + o_width) return false;
+    if (o_stride != x_stride) return true;
+    const long at = (d % x_stride + x_stride) % x_stride; // where a row of `out` begins beside the rows of `x`
+    return d != 0 && (at < x_width || x_stride - at < o_width);
+}
+
+// rows of 16-byte pieces -> contiguous rows
+__global__ __launch_bounds__(256) void paged_copy_rows_kernel(uint16_t *dst, const uint16_t *src, int stride, int width) {
+    for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8) *(u32x4 *)(dst + (size_t)blockIdx.x * width + i) = *(const u32x4 *)(src + (size_t)blockIdx.x * stride + i);
+}
+
 int check_common(const void *out, const void *q, const void *k, const void *v, int q_heads, int kv_heads, int head_size, int q_stride,
         int kv_stride, int o_stride, const void *kc, const void *vc, int block_size) {
     XFT_REQUIRE(out && q && k && v && kc && vc, "xfthip_paged_attention: null argument");
@@ -448,9 +463,12 @@ extern "C" int xfthip_paged_attention_decode(void *out, const void *q, const voi
     if (nsplit > kMaxSplits) nsplit = kMaxSplits;
     if (nsplit < 1) nsplit = 1;
     // The parts of any split call: below 2 CUs workgroups of 16 columns (4.3 MB on 256 CUs).  Taken by the stream's first call, split or not, so that
-    // none behind it allocates (a captured one must not).
+    // none behind it allocates (a captured one must not).  Results that may lie over queries still to be read go by way of it as well.
+    const bool apart = !in_the_way(out, o_stride, q_heads * 128, q, q_stride, q_heads * 128, batch);
+    const size_t any = (size_t)2 * device_cu_count() * 16 * 130, need = (size_t)batch * q_heads * nsplit * 130;
     void *part = nullptr;
-    if (int rc = stream_scratch(kScratchPagedParts, st, (size_t)2 * device_cu_count() * 16 * 130 * sizeof(float), false, &part)) return rc;
+    if (int rc = stream_scratch(kScratchPagedParts, st, std::max(any, apart ? 0 : need) * sizeof(float), false, &part)) return rc;
+    if (nsplit == 1 && apart) part = nullptr;
     PagedParams p = {};
     p.out = (uint16_t *)out, p.q = (const uint16_t *)q, p.kc = (const uint16_t *)kcache, p.vc = (const uint16_t *)vcache;
     p.tables = block_tables, p.ctx = context_lens, p.part = (float *)part;
@@ -459,7 +477,7 @@ extern "C" int xfthip_paged_attention_decode(void *out, const void *q, const voi
     hipLaunchKernelGGL(paged_store_kernel, dim3(batch), dim3(256), 0, st, (uint16_t *)kcache, (uint16_t *)vcache, (const uint16_t *)k,
             (const uint16_t *)v, slot_mapping, kv_stride, kv_heads * 128, block_num * block_size);
     hipLaunchKernelGGL(paged_decode_kernel, dim3(nsplit, kv_heads * colgroups, batch), dim3(256), 0, st, p);
-    if (nsplit > 1) hipLaunchKernelGGL(paged_merge_kernel, dim3(q_heads, batch), dim3(128), 0, st, p);
+    if (part) hipLaunchKernelGGL(paged_merge_kernel, dim3(q_heads, batch), dim3(128), 0, st, p);
     XFT_CHECK_HIP(hipGetLastError());
     return 0;
 }
@@ -483,8 +501,24 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
     size_t total = 0;
     for (int b = 0; b < batch; ++b) total += token_lens_host[b];
     const size_t kv_bytes = (total + 31 * kSeqs) * kv_heads * 128 * 4;
+    const size_t q_bytes = total * q_heads * 128 * 2, copied = total * kv_heads * 128 * 2;
+    // results that may lie over rows still to be read: those rows are read from a copy
+    const bool q_apart = !in_the_way(out, o_stride, q_heads * 128, q, q_stride, q_heads * 128, (long)total);
+    const bool kv_apart = batch <= per_launch || (!in_the_way(out, o_stride, q_heads * 128, k, kv_stride, kv_heads * 128, (long)total)
+                                                         && !in_the_way(out, o_stride, q_heads * 128, v, kv_stride, kv_heads * 128, (long)total));
     void *scratch = nullptr;
-    if (int rc = stream_scratch(kScratchPagedKv, st, kv_bytes + total * q_heads * 128 * 2, false, &scratch)) return rc;
+    if (int rc = stream_scratch(kScratchPagedKv, st, kv_bytes + q_bytes + (kv_apart ? 0 : 2 * copied), false, &scratch)) return rc;
+    auto copy_rows = [&](const void *&x, int &stride, int heads, size_t at) {
+        uint16_t *to = (uint16_t *)((char *)scratch + at);
+        hipLaunchKernelGGL(paged_copy_rows_kernel, dim3((unsigned)total), dim3(256), 0, st, to, (const uint16_t *)x, stride, heads * 128);
+        x = to, stride = heads * 128;
+    };
+    if (!q_apart) copy_rows(q, q_stride, q_heads, kv_bytes);
+    if (!kv_apart) {
+        int stride = kv_stride;
+        copy_rows(k, stride, kv_heads, kv_bytes + q_bytes);
+        copy_rows(v, kv_stride, kv_heads, kv_bytes + q_bytes + copied);
+    }
     const int G = q_heads / kv_heads;
     for (int b = 0; b < batch; ++b) // likewise what one of these sequences by itself splits its keys through
         if (attention_split_count(token_lens_host[b], kv_heads * ((token_lens_host[b] * G + 15) / 16)) > 1) {
