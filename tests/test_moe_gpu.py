@@ -39,6 +39,30 @@ def test_top2_selection_and_weights(xh, orc):
     assert np.abs(w.sum(1) - 1).max() < 1e-6
 
 
+@pytest.mark.parametrize("hidden", [512, 4096, 4104])
+def test_routing_by_infinite_router_weights(xh, orc, hidden):
+    """A router weight that is infinite decides for or against its expert by the sign of its column's activation, whatever the width leaves over of a
+    round of columns."""
+    inter, E, T = 128, 8, 6
+    rng = np.random.default_rng(hidden)
+    router = (rng.standard_normal((hidden, E)) * 0.05).astype(np.float32)
+    router[0, 5] = np.inf
+    x = orc.round_bf16(rng.standard_normal((T, hidden)))
+    x[:, 0] = [1.0, -1.0, 2.0, -0.5, 0.25, -3.0]
+    moe = xh.MoE(hidden, inter, E, T, router, None)
+    one = xh.Weight(xh.W_BF16, hidden, 2 * inter, np.zeros((hidden, 2 * inter), np.uint16), flags=xh.WF_GATEUP), xh.Weight(xh.W_BF16, inter, hidden, np.zeros((inter, hidden), np.uint16))
+    for e in range(E):
+        moe.set_expert(e, *one)
+    xd, od = xh.DeviceBuffer.from_numpy(x), xh.DeviceBuffer(x.nbytes)
+    sel, w = moe.forward(xd.ptr, od.ptr, T, False)
+    logits = x.astype(np.float64) @ np.where(np.isinf(router), 0.0, router)
+    logits[:, 5] = np.sign(x[:, 0]) * np.inf
+    order = np.argsort(-logits, 1, kind="stable")[:, :2]
+    assert np.array_equal(sel, order)
+    assert np.array_equal(w[x[:, 0] > 0], np.tile(np.float32([1.0, 0.0]), (3, 1)))
+    assert np.array_equal(od.to_numpy(np.float32, x.shape), x)
+
+
 def _experts(orc, rng, kind, hidden, inter, E):
     out = []
     for _ in range(E):

@@ -92,8 +92,8 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(const float *__res
             const int k = k0 + i * kRouteThreads + tid;
             const uint16_t bits = f32_to_bf16_ref(NORM ? (x[i] * rstd) * g[i] : x[i]);
             if (k < hidden) out[k] = bits;
-            if (given) continue; // (uniform)
-            const float v = k < hidden ? bf16_to_f32(bits) : 0.0f;
+            if (given || k >= hidden) continue; // (a zero in place of a column past the end would make NaN of an infinite weight)
+            const float v = bf16_to_f32(bits);
             acc[0] = fmaf(v, lo[i].x, acc[0]), acc[1] = fmaf(v, lo[i].y, acc[1]), acc[2] = fmaf(v, lo[i].z, acc[2]), acc[3] = fmaf(v, lo[i].w, acc[3]);
             acc[4] = fmaf(v, hi[i].x, acc[4]), acc[5] = fmaf(v, hi[i].y, acc[5]), acc[6] = fmaf(v, hi[i].z, acc[6]), acc[7] = fmaf(v, hi[i].w, acc[7]);
         }
