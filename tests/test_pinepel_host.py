@@ -4,6 +4,7 @@ import json
 import os
 
 import numpy as np
+import pytest
 
 import plan_util as u
 from oracle import pinepel_ref as ref
@@ -83,3 +84,15 @@ def test_directory_is_recognised_by_its_config(tmp_path):
     assert is_plan(tmp_path)
     (tmp_path / "config.ini").write_text("[llama]\n")
     assert not is_plan(tmp_path)
+
+
+@pytest.mark.parametrize("entries", [
+    [(0, [1, 2, 3], [2]), (1, (7,), [0])], [(0, np.arange(5, dtype=np.int32), []), (1, np.arange(9, 3, -2, dtype=np.int32), [])],
+    [(0, np.arange(4, dtype=np.int64), []), (1, [np.int64(5)], [])], [(0, np.arange(12, dtype=np.int32)[::3], []), (1, [3, 4], [])],
+    [(0, np.arange(3, dtype=np.int32).reshape(3, 1), []), (2, [[4], [5]], [])], [(0, [[1], [2]], [0])], []])
+def test_tokens_of_a_step_in_any_form(entries):
+    """Lists, tuples, integer arrays of any type and stride and columns of tokens reach the library as one run of int32."""
+    from xfastertransformer_amd import capi
+    want = np.asarray([t for e in entries for t in e[1]], np.int32)
+    got = capi._token_ids(entries)
+    assert got.dtype == np.int32 and got.flags.c_contiguous and got.shape == want.shape and np.array_equal(got, want)

@@ -602,6 +602,13 @@ class Plan:
             pass
 
 
+def _token_ids(entries):
+    """The tokens of a step's entries one after the other, int32.  int32 vectors as they are: token by token, 8000 of them took 0.8 ms."""
+    if len(entries) and all(isinstance(e[1], np.ndarray) and e[1].dtype == np.int32 and e[1].ndim == 1 for e in entries):
+        return np.concatenate([e[1] for e in entries])
+    return np.asarray([t for e in entries for t in e[1]], np.int32)
+
+
 class PlanModel(Model):
     """A device model over a finished Plan; act = BF16 or F32."""
 
@@ -618,9 +625,7 @@ class PlanModel(Model):
         """entries: (slot, tokens, places wanted) each; logits fp32 [wanted, vocab]"""
         rows = np.asarray([e[0] for e in entries], np.int32)
         lens = np.asarray([len(e[1]) for e in entries], np.int32)
-        # (int32 arrays as they are: token by token, 8000 of them took 0.8 ms)
-        plain = lambda t: isinstance(t, np.ndarray) and t.dtype == np.int32 and t.ndim == 1
-        ids = np.concatenate([np.empty(0, np.int32)] + [e[1] if plain(e[1]) else np.asarray([t for t in e[1]], np.int32) for e in entries])
+        ids = _token_ids(entries)
         starts = np.concatenate([[0], np.cumsum(lens)[:-1]])
         want = np.asarray([s + w for e, s in zip(entries, starts) for w in e[2]], np.int32)
         out = np.empty((len(want), self.cfg.vocab), np.float32)
