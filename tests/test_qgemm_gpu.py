@@ -282,3 +282,24 @@ def test_gemm_rejects_bad_arguments(xh, orc):
         xh.gemm(dw, a.ptr, 1, 256, c.ptr, 64, epi=xh.EPI_BIAS)  # bias missing
     with pytest.raises(xh.XftHipError):
         xh.gemm_gateup_silu(dw, a.ptr, 1, 256, c.ptr, 32)  # not a gate/up weight
+
+
+@pytest.mark.parametrize("kind", ["int8", "bf16"])
+def test_null_stream_beside_a_capture(xh, orc, kind):
+    """A product whose K is split, on the null stream, while another stream is being captured: the bits of an ordinary call."""
+    import ctypes as C
+    M, K, N = 64, 4096, 1024
+    rng = np.random.default_rng(4)
+    w, _, _ = _random_weight(xh, orc, rng, kind, K, N)
+    a = orc.to_bf16(orc.round_bf16(rng.standard_normal((M, K), dtype=np.float32)))
+    want = _run_gemm(xh, w, a, M, K, N, xh.F32)
+    a_dev, c_dev, stream, graph = xh.DeviceBuffer.from_numpy(a), xh.DeviceBuffer(M * N * 4), xh.Stream(), C.c_void_p()
+    assert xh.lib.hipStreamBeginCapture(stream.h, 1) == 0  # 1: thread-local checks
+    try:
+        xh.gemm(w, a_dev.ptr, M, K, c_dev.ptr, N, xh.F32)
+    finally:
+        assert xh.lib.hipStreamEndCapture(stream.h, C.byref(graph)) == 0
+        xh.lib.hipGraphDestroy(graph)
+    xh.synchronize()
+    assert np.array_equal(c_dev.to_numpy(np.float32, (M, N)), want)
+    w.free()

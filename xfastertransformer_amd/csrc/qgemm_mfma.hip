@@ -198,8 +198,14 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool may_split = true) {
 size_t qgemm_split_bound() { return (size_t)device_cu_count() * 65536; }
 
 bool qgemm_split_usable(hipStream_t stream) {
+    // (the null stream cannot be captured, and must not be asked: while another one is, the answer is an error, which the launch's own check would report)
+    if (stream == nullptr) return true;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &status) != hipSuccess || status == hipStreamCaptureStatusNone) return true;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    if (status == hipStreamCaptureStatusNone) return true;
     return stream_scratch_held(kScratchGemmSplit, stream, qgemm_split_bound() * sizeof(float));
 }
 
