@@ -176,7 +176,9 @@ def _random_weight(xh, orc, rng, kind, K, N, gateup=False):
 # 128 x 128 and 128 x 256 with one and two K groups and with K in parts, bands of one to eight row blocks
 @pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])
 @pytest.mark.parametrize("M,K,N", [(33, 8192, 3088), (97, 4096, 1040), (129, 1024, 12304), (200, 4096, 6160), (450, 11008, 2064), (641, 8192, 4112), (700, 4096, 4112),
-                                   (1285, 4096, 4112), (2100, 1024, 6160), (1161, 2048, 2832), (300, 4160, 2064), (770, 2048, 80)])
+                                   (1285, 4096, 4112), (2100, 1024, 6160), (1161, 2048, 2832), (300, 4160, 2064), (770, 2048, 80),
+                                   # (a depth that is no whole number of 64, whole and broken packed tiles of BF16 weights)
+                                   (2000, 1056, 4112), (1000, 1056, 4112), (300, 8224, 2064), (130, 8224, 2064), (2000, 1064, 4112), (700, 1064, 2064)])
 def test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N):
     """Bound: K + 8 additions and the epilogue's few operations in fp32, each off by 2^-24 of what has been added up so far at most; NF4 values
     go in as two bf16 parts, off by 2^-17."""

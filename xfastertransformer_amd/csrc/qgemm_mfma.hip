@@ -4,6 +4,7 @@
 // file picks the weight kind.
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "qgemm.h"
@@ -128,15 +129,47 @@ constexpr TileCost kTiles[] = {
 
 constexpr float kSplitStart[3] = {3.0f, 4.0f, 3.0f}, kSplitMb[3] = {0.3f, 0.35f, 0.3f}; // launch and megabytes of a split K's sum
 
+// The same for activations staged through registers (K no whole number of 64, or more than 4 GB of them) and more than 256 rows: thresholds, as the
+// constants above are those of other forms.  128-row tiles where they give every CU a block; below, K in parts while 64-row tiles give a CU
+// less than two, and 32-row tiles where that is not enough.  With the model alone: INT8 450 x 4096 x 11040 71 -> 94 us, BF16 700 x 4096 x 4000 44
+// -> 52.  BF16 weights, K a whole number of packed tiles: 2048 x 4096 x 11040 184 us, in the form for a ragged K 464, 1024 x 12288 x 4000
+// 147 and 341.  false: up to 256 rows, where the model is the better one (1.03 to 2.7 times), and BF16 weights with a ragged K that do not fill the
+// device with 128 x 256 (128 x 128 is 1.2 times slower than 64-row tiles there).
+bool choose_staged_tile(SkinnyParams &p, int kind, int ktile, bool may_split) {
+    const int cus = device_cu_count(), kt_n = (p.K + ktile - 1) / ktile;
+    const long cols = (p.N + 127) / 128, large = (long)((p.N + 255) / 256) * ((p.M + 127) / 128), small = cols * ((p.M + 63) / 64);
+    const bool bf16 = kind == XFTHIP_W_BF16;
+    if (p.M <= 256) return false;
+    if (large >= cus && (bf16 || p.M >= 512)) {
+        p.tile = 4;
+        return true;
+    }
+    if (bf16 && p.K % ktile != 0) return false;
+    if (bf16 && p.M >= 512 && cols * ((p.M + 127) / 128) >= cus) {
+        p.tile = 3;
+        return true;
+    }
+    long want = 1;
+    if (may_split && !p.gateup) {
+        const long few = cols * ((p.M + 31) / 32);
+        if (2 * few <= cus && kt_n >= 16) want = std::min({2L * cus / few, (long)kt_n / 8, 16L});
+        else if (p.K >= 8192 && small < 2 * cus) want = std::min((2L * cus + small - 1) / small, (long)p.K / 2048);
+        want = std::min(want, (long)(qgemm_split_bound() / ((size_t)p.M * p.N)));
+    }
+    if (want >= 2) {
+        p.split_ktiles = (kt_n + (int)want - 1) / (int)want;
+        p.ksplit = (kt_n + p.split_ktiles - 1) / p.split_ktiles;
+    }
+    p.tile = !bf16 && small * std::max(p.ksplit, 1) < 2 * cus ? 1 : 2;
+    return true;
+}
+
 void choose_tile(SkinnyParams &p, int kind, int ktile, bool may_split = true) {
     const int cus = device_cu_count(), kt_n = (p.K + ktile - 1) / ktile, cls = kind == XFTHIP_W_BF16 ? 1 : kind == XFTHIP_W_NF4 ? 2 : 0;
     // activations straight into LDS: steps of 64 k, byte offsets of 32 bits
     const bool direct = p.K % 64 == 0 && (size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32);
     p.tile = 2, p.kgroups = 1, p.direct = 0;
-    if (!direct && !p.rows_dev && (long)((p.N + 255) / 256) * ((p.M + 127) / 128) >= cus) {
-        p.tile = 4; // staged through registers: only where it fills the device
-        return;
-    }
+    if (!direct && !p.rows_dev && choose_staged_tile(p, kind, ktile, may_split)) return;
     float best = 1e30f;
     for (const TileCost &t : kTiles) {
         if (t.rows == 32 && kind == XFTHIP_W_BF16) continue; // (not built: two bytes a weight want more rows behind them)

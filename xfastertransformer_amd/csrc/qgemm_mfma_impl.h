@@ -876,15 +876,15 @@ static int launch_big(const SkinnyParams &p, hipStream_t stream) {
     if constexpr (WM == 4) {
         // 128-row tiles: the activations straight into LDS, two workgroups a CU, or (at most a block a CU) two K groups a workgroup: 2048
         // rows x 4096 columns, K = 4096 / 11008, INT8 963 / 993 against 926 / 934 TFLOP/s, UINT4 859 / 954 against 812 / 926, NF4 519 / 569
-        // against 492 / 532.  Staged through registers only for a ragged K or more than 4 GB of activations (128 x 256 alone).
+        // against 492 / 532.  Staged through registers only for a ragged K or more than 4 GB of activations.
         if (p.direct) return p.kgroups == 2 ? launch_big2<KIND, WN, WM, NEED_SUM, false, false, true, 2>(p, stream)
                                             : launch_big2<KIND, WN, WM, NEED_SUM, false, false, true>(p, stream);
-        if constexpr (WN == 2) {
-            return launch_big2<KIND, WN, WM, NEED_SUM, true>(p, stream);
-        } else {
-            set_error("qgemm_mfma: the 128 x 128 tile takes its activations straight into LDS");
-            return 2;
+        if constexpr (WN == 2 || KIND == XFTHIP_W_BF16) {
+            if (p.K % StepTraits<KIND>::KTILE == 0) return launch_big2<KIND, WN, WM, NEED_SUM, false>(p, stream);
         }
+        if constexpr (WN == 2) return launch_big2<KIND, WN, WM, NEED_SUM, true>(p, stream);
+        set_error("qgemm_mfma: no 128 x 128 tile for this K");
+        return 2;
     } else {
         if (p.K % StepTraits<KIND>::KTILE != 0) return launch_big2<KIND, WN, WM, NEED_SUM, true>(p, stream);
         return launch_big2<KIND, WN, WM, NEED_SUM, false>(p, stream);
