@@ -147,7 +147,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     int nb, mb, part;
     {
         const int parts = p.ksplit > 1 ? p.ksplit : 1;
-        const int BAND = band_rows(nblocks_m, parts * nblocks_n);
+        const int BAND = DEVROWS ? band_rows(nblocks_m, parts * nblocks_n) : p.band; // (its divisions: not in every workgroup where the host can)
         const int id = blockIdx.x, xcd = id & 7, slot = id >> 3; // gridDim.x is a multiple of 8
         const int nbands = (nblocks_m + BAND - 1) / BAND;
         const int units = nbands * parts * nblocks_n;
@@ -857,8 +857,10 @@ static int launch_big2(const SkinnyParams &p, hipStream_t stream) {
                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         XFT_CHECK_HIP(attr);
     }
+    SkinnyParams q = p;
+    q.band = band;
     hipLaunchKernelGGL((qgemm_mfma_kernel<KIND, WN, WM, NEED_SUM, KTAIL, DEVROWS, DIRECT, WSETS, KG>), dim3(blocks), dim3(256 * KG), smem, stream,
-            p, nblocks_n, nblocks_m);
+            q, nblocks_n, nblocks_m);
     XFT_CHECK_HIP(hipGetLastError());
     return 0;
 }
