@@ -116,18 +116,18 @@ __global__ __launch_bounds__(256) void qgemm_split_finish_kernel(SkinnyParams p)
 struct TileCost {
     int rows, cols, kgroups, resident;
     float fixed; // a block's pipeline fill and results
-    float step[3], more[3]; // per step of a block alone on a CU; per further resident block.  INT8 and UINT4, BF16, NF4
+    float step[4], more[4]; // per step of a block alone on a CU; per further resident block.  INT8, BF16, NF4, UINT4
 };
 constexpr TileCost kTiles[] = {
-        {32, 128, 1, 4, 0.6f, {0.26f, 0.0f, 0.39f}, {0.15f, 0.0f, 0.26f}},
-        {64, 128, 1, 4, 1.2f, {0.35f, 0.56f, 0.51f}, {0.27f, 0.34f, 0.43f}},
-        {128, 128, 1, 2, 1.7f, {0.71f, 0.64f, 0.90f}, {0.26f, 0.36f, 0.65f}},
-        {128, 128, 2, 1, 4.3f, {1.0f, 1.14f, 1.38f}, {}},
-        {128, 256, 1, 2, 3.1f, {0.92f, 0.93f, 1.59f}, {0.73f, 0.77f, 1.34f}},
-        {128, 256, 2, 1, 8.7f, {1.49f, 1.8f, 2.63f}, {}},
+        {32, 128, 1, 4, 0.6f, {0.26f, 0.0f, 0.39f, 0.247f}, {0.15f, 0.0f, 0.26f, 0.143f}},
+        {64, 128, 1, 4, 1.2f, {0.35f, 0.56f, 0.51f, 0.357f}, {0.27f, 0.34f, 0.43f, 0.275f}},
+        {128, 128, 1, 2, 1.7f, {0.71f, 0.64f, 0.90f, 0.71f}, {0.26f, 0.36f, 0.65f, 0.26f}},
+        {128, 128, 2, 1, 4.3f, {1.0f, 1.14f, 1.38f, 1.0f}, {}},
+        {128, 256, 1, 2, 3.1f, {0.92f, 0.93f, 1.59f, 0.92f}, {0.73f, 0.77f, 1.34f, 0.73f}},
+        {128, 256, 2, 1, 8.7f, {1.49f, 1.8f, 2.63f, 1.49f}, {}},
 };
 
-constexpr float kSplitStart[3] = {3.0f, 4.0f, 3.0f}, kSplitMb[3] = {0.3f, 0.35f, 0.3f}; // launch and megabytes of a split K's sum
+constexpr float kSplitStart[4] = {3.0f, 4.0f, 3.0f, 3.0f}, kSplitMb[4] = {0.3f, 0.35f, 0.3f, 0.3f}; // launch and megabytes of a split K's sum
 
 // The same for activations staged through registers (K no whole number of 64, or more than 4 GB of them) and more than 256 rows: thresholds, as the
 // constants above are those of other forms.  128-row tiles where they give every CU a block; below, K in parts while 64-row tiles give a CU
@@ -165,7 +165,7 @@ bool choose_staged_tile(SkinnyParams &p, int kind, int ktile, bool may_split) {
 }
 
 void choose_tile(SkinnyParams &p, int kind, int ktile, bool may_split = true) {
-    const int cus = device_cu_count(), kt_n = (p.K + ktile - 1) / ktile, cls = kind == XFTHIP_W_BF16 ? 1 : kind == XFTHIP_W_NF4 ? 2 : 0;
+    const int cus = device_cu_count(), kt_n = (p.K + ktile - 1) / ktile, cls = kind == XFTHIP_W_BF16 ? 1 : kind == XFTHIP_W_NF4 ? 2 : kind == XFTHIP_W_UINT4 ? 3 : 0;
     // activations straight into LDS: steps of 64 k, byte offsets of 32 bits
     const bool direct = p.K % 64 == 0 && (size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32);
     p.tile = 2, p.kgroups = 1, p.direct = 0;
