@@ -90,10 +90,24 @@ __host__ __device__ inline int band_rows(int nblocks_m, int units) {
     return best;
 }
 
+// The form of a product of up to 32 rows without prologue and RoPE, K of whole tiles: column tiles a block, k tiles a load batch, K slices (waves)
+struct SkinnyForm {
+    int nt, u, kslices;
+};
+// k tiles a load batch of a block of nt column tiles and mt 16-row tiles: what the kernels are built with and what skinny_form counts slices in
+constexpr int skinny_batch(int kind, int mt, bool group, int nt) {
+    if (kind == XFTHIP_W_UINT4 || kind == XFTHIP_W_NF4 || nt > 3) return 1;
+    const bool int8 = kind == XFTHIP_W_INT8;
+    if (nt == 3) return mt == 1 ? 1 : 2;
+    if (mt == 1) return nt == 1 ? (int8 || group ? 4 : 2) : (group && !int8 ? 4 : 2);
+    return nt == 2 && int8 && group ? 1 : 2;
+}
+SkinnyForm skinny_form(int kind, const SkinnyParams &p);
 int qgemm_skinny(const PackedWeight &pw, const SkinnyParams &p, hipStream_t stream); // M <= 32
 bool skinny_can_fuse_norm(const PackedWeight &pw, int M); // may SkinnyParams::norm_x be used
 // any M, built for M > 32; parts / part: as in gemm_grouped_rows_dev
 int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p, hipStream_t stream, int *parts = nullptr, const float **part = nullptr);
+void qgemm_mfma_form(int kind, SkinnyParams &p); // the tile, K groups and K parts it takes, into p (ksplit: 0 where K is whole)
 // the K-split workspace of qgemm_mfma launches on `stream` (allocated on the stream's first call: before a capture, say)
 int qgemm_split_reserve(hipStream_t stream, float **out = nullptr);
 size_t qgemm_split_bound(); // its floats

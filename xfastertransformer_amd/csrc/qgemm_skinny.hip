@@ -1,7 +1,7 @@
 // Dequant-fused weight-only GEMM for few activation rows (M <= 32): the decode-time shape.
 // Replaces MMHelper::compute* (reference src/utils/matmul_helper.h:565-1705) for
 // INT8 / UINT4 / NF4 / BF16 weights against bf16 activations.  The kernel lives in
-// qgemm_skinny_impl.h; this file checks the fused options and picks the weight kind.
+// qgemm_skinny_impl.h; this file checks the fused options, picks the weight kind and the form.
 #include "qgemm.h"
 
 namespace xfthip {
@@ -20,6 +20,62 @@ static inline size_t skinny_norm_lds_bytes(int M, int K) {
 bool skinny_can_fuse_norm(const PackedWeight &pw, int M) {
     return M <= 4 && pw.kind != XFTHIP_W_W8A8 && pw.KT * ktile_of(pw.kind) == pw.K && pw.K % 4 == 0
             && skinny_norm_lds_bytes(M, pw.K) <= (size_t)36 * 1024;
+}
+
+// What sets the time is the CU with the most column tiles: blocks are spread over the CUs in turn, so that it is w = ceil(blocks / CUs) blocks of nt
+// tiles.  A tile costs least in blocks of two (an activation fragment serves both; wider blocks lose some of that to registers), a block half a
+// tile more for its sums over the waves.  All blocks of a CU run side by side: 8 waves between them keep enough loads in flight (more K
+// slices only add sums), two a block at least.  BF16 at up to 16 rows: single tiles, whose stream alone is 32 KB a block.
+// Timed over 20 shapes of 512 .. 32000 columns x 1408 .. 14336 deep, six row counts, four kinds, all forms: 0.96 .. 0.99 of the best form on
+// average.  Against two tiles (3 .. 6 at 17 .. 32 rows) in 8 slices throughout, geometric mean at up to 4 / 16 / 32 rows: UINT4 1.13 / 1.16 /
+// 1.07 times as fast, NF4 1.12 / 1.14 / 1.08, INT8 1.04 / 1.08 / 1.07, BF16 1.03 / 1.03 / 1.05; UINT4 24 x 4096 x 28672 30 -> 22 us, 6 rows
+// 25 -> 15.6, 16 x 8192 x 10240 19 -> 14.
+// More than 8 tiles a CU, where the blocks come in rounds anyway: the form that was best over 55296 .. 151936 columns (UINT4 16 x 4096 x 128256
+// 101 -> 52 us, INT8 32 rows 126 -> 101, NF4 6 rows 115 -> 74, BF16 6 rows 166 -> 152).
+// Several weights behind one launch: the same over the columns of those that have rows, as many as there are rows at most.  8 weights each of
+// 28672 x 4096 and 4096 x 14336, a layer of 10 / 32 tokens: UINT4 224 / 306 -> 142 / 207 us, NF4 284 / 384 -> 200 / 280,
+// INT8 255 / 333 -> 214 / 276, BF16 400 / 501 -> 394 / 484.
+SkinnyForm skinny_form(int kind, const SkinnyParams &p) {
+    const bool four = kind == XFTHIP_W_UINT4 || kind == XFTHIP_W_NF4;
+    const int cus = device_cu_count(), mt = p.M <= 16 ? 1 : 2;
+    const int weights = !p.group ? 1 : p.m_hint < 1 ? 1 : p.m_hint < p.group_n ? p.m_hint : p.group_n;
+    auto form = [&](int nt, int kslices) { // a batch a slice at least
+        const int u = skinny_batch(kind, mt, p.group != nullptr, nt), batches = p.KT / u;
+        kslices = kslices < 8 ? kslices : 8;
+        kslices = kslices < batches ? kslices : batches;
+        return SkinnyForm {nt, u, kslices > 1 ? kslices : 1};
+    };
+    auto per_cu = [&](int nt) { return ((p.NTILES + nt - 1) / nt * weights + cus - 1) / cus; };
+    const long tiles = (long)p.NTILES * weights;
+    // (two slices against eight: 3 % faster at K = 4096, 2 % slower at 2048)
+    if (kind == XFTHIP_W_BF16 && p.group && mt == 1) return form(p.gateup ? 2 : 1, p.gateup && p.K >= 4096 ? 2 : 8);
+    if (p.group && tiles >= 8 * cus) { // K slices by the depth
+        if (four && mt == 1) return form(p.M <= 4 ? 2 : 4, p.KT < 32 ? 4 : p.KT / 8);
+        if (four) return form(4, p.KT / 16);
+        if (kind == XFTHIP_W_INT8) return mt == 1 ? form(2, p.KT / 8) : form(2, 4);
+        return form(2, 2);
+    }
+    if (tiles > 8 * cus) {
+        if (mt == 2) return form(4, four ? 2 : kind == XFTHIP_W_INT8 ? 3 : 1);
+        if (four) return form(4, 4);
+        // (BF16, 16 rows of 128256 columns: single tiles in 8 slices 199 us, 171 before, 166 in this form)
+        if (kind == XFTHIP_W_BF16 && p.M > 8) return form(2, 1);
+        return form(kind == XFTHIP_W_INT8 || p.gateup ? 2 : 1, 8);
+    }
+    int nt = p.gateup ? 2 : 1;
+    if (kind != XFTHIP_W_BF16 || mt == 2) {
+        float least = 1e30f;
+        for (int n : {1, 2, 3, 4, 6}) {
+            if ((p.gateup && n % 2) || (n >= 4 && mt == 1) || (n % 3 == 0 && p.group)) continue;
+            const int w = per_cu(n);
+            // (17 .. 32 rows, two blocks of four tiles on a CU: well for 4-bit codes, 1.2 times the time of four blocks of two for the others)
+            const float tile = n == 1 ? 1.2f : n == 2 ? 1.0f : n == 4 && w > 1 && !four ? 1.3f : 1.1f;
+            const float cost = (float)w * ((float)n * tile + 0.5f);
+            if (cost < least) least = cost, nt = n;
+        }
+    }
+    const int least = kind == XFTHIP_W_BF16 ? 1 : 2, slices = 8 / per_cu(nt);
+    return form(nt, slices > least ? slices : least);
 }
 
 int qgemm_skinny(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t stream) {

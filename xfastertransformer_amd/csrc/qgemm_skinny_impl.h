@@ -720,92 +720,23 @@ static int dispatch_tail(const SkinnyParams &p, int kslices, hipStream_t stream)
     return 2;
 }
 
-// The form of a product without prologue and RoPE, K of whole tiles: column tiles a block, k tiles a load batch, K slices (waves)
-struct SkinnyForm {
-    int nt, u, kslices;
-};
-
-// What sets the time is the CU with the most column tiles: blocks are spread over the CUs in turn, so that it is w = ceil(blocks / CUs) blocks of nt
-// tiles.  A tile costs least in blocks of two (an activation fragment serves both; wider blocks lose some of that to registers), a block half a
-// tile more for its sums over the waves.  All blocks of a CU run side by side: 8 waves between them keep enough loads in flight (more K
-// slices only add sums), two a block at least.  BF16 at up to 16 rows: single tiles, whose stream alone is 32 KB a block.
-// Timed over 20 shapes of 512 .. 32000 columns x 1408 .. 14336 deep, six row counts, four kinds, all forms: 0.96 .. 0.99 of the best form on
-// average.  Against two tiles (3 .. 6 at 17 .. 32 rows) in 8 slices throughout, geometric mean at up to 4 / 16 / 32 rows: UINT4 1.13 / 1.16 /
-// 1.07 times as fast, NF4 1.12 / 1.14 / 1.08, INT8 1.04 / 1.08 / 1.07, BF16 1.03 / 1.03 / 1.05; UINT4 24 x 4096 x 28672 30 -> 22 us, 6 rows
-// 25 -> 15.6, 16 x 8192 x 10240 19 -> 14.
-// More than 8 tiles a CU, where the blocks come in rounds anyway: the form that was best over 55296 .. 151936 columns (UINT4 16 x 4096 x 128256
-// 101 -> 52 us, INT8 32 rows 126 -> 101, NF4 6 rows 115 -> 74, BF16 6 rows 166 -> 152).
-// Several weights behind one launch: the same over the columns of those that have rows, as many as there are rows at most.  8 weights each of
-// 28672 x 4096 and 4096 x 14336, a layer of 10 / 32 tokens: UINT4 224 / 306 -> 142 / 207 us, NF4 284 / 384 -> 200 / 280,
-// INT8 255 / 333 -> 214 / 276, BF16 400 / 501 -> 394 / 484.
-template <int KIND>
-static SkinnyForm choose_form(const SkinnyParams &p) {
-    constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4;
-    const int cus = device_cu_count(), mt = p.M <= 16 ? 1 : 2;
-    const int weights = !p.group ? 1 : p.m_hint < 1 ? 1 : p.m_hint < p.group_n ? p.m_hint : p.group_n;
-    auto form = [&](int nt, int u, int kslices) { // a batch a slice at least
-        const int batches = p.KT / u;
-        kslices = kslices < 8 ? kslices : 8;
-        kslices = kslices < batches ? kslices : batches;
-        return SkinnyForm {nt, u, kslices > 1 ? kslices : 1};
-    };
-    auto per_cu = [&](int nt) { return ((p.NTILES + nt - 1) / nt * weights + cus - 1) / cus; };
-    const long tiles = (long)p.NTILES * weights;
-    // (two slices against eight: 3 % faster at K = 4096, 2 % slower at 2048)
-    if (KIND == XFTHIP_W_BF16 && p.group && mt == 1) return form(p.gateup ? 2 : 1, 4, p.gateup && p.K >= 4096 ? 2 : 8);
-    if (p.group && tiles >= 8 * cus) { // K slices by the depth
-        if (FOUR && mt == 1) return form(p.M <= 4 ? 2 : 4, 1, p.KT < 32 ? 4 : p.KT / 8);
-        if (FOUR) return form(4, 1, p.KT / 16);
-        if (KIND == XFTHIP_W_INT8) return mt == 1 ? form(2, 2, p.KT / 8) : form(2, 1, 4);
-        return form(2, 2, 2);
-    }
-    if (tiles > 8 * cus) {
-        if (mt == 2) return form(4, 1, FOUR ? 2 : KIND == XFTHIP_W_INT8 ? 3 : 1);
-        if (FOUR) return form(4, 1, 4);
-        // (BF16, 16 rows of 128256 columns: single tiles in 8 slices 199 us, 171 before, 166 in this form)
-        if (KIND == XFTHIP_W_BF16 && p.M > 8) return form(2, 2, 1);
-        return form(KIND == XFTHIP_W_INT8 || p.gateup ? 2 : 1, 2, 8);
-    }
-    int nt = p.gateup ? 2 : 1;
-    if (KIND != XFTHIP_W_BF16 || mt == 2) {
-        float least = 1e30f;
-        for (int n : {1, 2, 3, 4, 6}) {
-            if ((p.gateup && n % 2) || (n >= 4 && mt == 1) || (n % 3 == 0 && p.group)) continue;
-            const int w = per_cu(n);
-            // (17 .. 32 rows, two blocks of four tiles on a CU: well for 4-bit codes, 1.2 times the time of four blocks of two for the others)
-            const float tile = n == 1 ? 1.2f : n == 2 ? 1.0f : n == 4 && w > 1 && !FOUR ? 1.3f : 1.1f;
-            const float cost = (float)w * ((float)n * tile + 0.5f);
-            if (cost < least) least = cost, nt = n;
-        }
-    }
-    int u = 1;
-    if (FOUR) u = 1;
-    else if (mt == 2) u = nt > 3 || (KIND == XFTHIP_W_INT8 && p.group && nt == 2) ? 1 : 2;
-    else if (KIND == XFTHIP_W_INT8) u = nt == 1 ? 4 : nt == 3 ? 1 : 2;
-    else u = 2;
-    const int least = KIND == XFTHIP_W_BF16 ? 1 : 2, slices = 8 / per_cu(nt);
-    return form(nt, u, slices > least ? slices : least);
-}
-
+// (skinny_form has the rule; the load batches are its own)
 template <int KIND, int MT, bool NEED_SUM, bool STAGE, bool GROUP>
 static int launch_form(const SkinnyParams &p, hipStream_t stream) {
-    // (load batches of one and two tiles as choose_form has them)
-    constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4, INT8 = KIND == XFTHIP_W_INT8;
-    constexpr int U1 = FOUR ? 1 : MT == 1 && (INT8 || GROUP) ? 4 : 2, U2 = FOUR || (INT8 && GROUP && MT == 2) ? 1 : !INT8 && GROUP && MT == 1 ? 4 : 2;
-    const SkinnyForm f = choose_form<KIND>(p);
+    constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4;
+    const SkinnyForm f = skinny_form(KIND, p);
     switch (f.nt) {
-        case 1: return launch<KIND, 1, MT, U1, NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
-        case 2: return launch<KIND, 2, MT, U2, NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
+        case 1: return launch<KIND, 1, MT, skinny_batch(KIND, MT, GROUP, 1), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
+        case 2: return launch<KIND, 2, MT, skinny_batch(KIND, MT, GROUP, 2), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
         case 3:
-            if constexpr (GROUP) break;
-            else if constexpr (MT == 2) return launch<KIND, 3, MT, U2, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
-            else if constexpr (KIND != XFTHIP_W_BF16) return launch<KIND, 3, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            if constexpr (!GROUP && (MT == 2 || KIND != XFTHIP_W_BF16))
+                return launch<KIND, 3, MT, skinny_batch(KIND, MT, false, 3), NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
             break;
         case 4:
-            if constexpr (MT == 2 || FOUR) return launch<KIND, 4, MT, 1, NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
+            if constexpr (MT == 2 || FOUR) return launch<KIND, 4, MT, skinny_batch(KIND, MT, GROUP, 4), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
             break;
         case 6:
-            if constexpr (MT == 2 && !GROUP) return launch<KIND, 6, MT, 1, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            if constexpr (MT == 2 && !GROUP) return launch<KIND, 6, MT, skinny_batch(KIND, MT, false, 6), NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
             break;
     }
     set_error("qgemm_skinny: no form of %d column tiles", f.nt);
@@ -860,8 +791,7 @@ static int dispatch_shape(const SkinnyParams &p, hipStream_t stream) {
     }
     // 17 .. 32 rows: the kernel holds one workgroup a CU and a column block costs about the same time whether it
     // is 16 or 96 columns wide (a chain of load round trips over the wave's K slice), so the blocks are made wide
-    // enough for one round over the CUs where the registers allow it: 3 tiles for the 768 of a 7B QKV projection
-    // (384 two-tile blocks took two rounds: 23.2 us), 6 for the 1376 of its gate/up
+    // enough for one round over the CUs where the registers allow it
     const int per_cu = (p.NTILES + cus - 1) / cus;
     if (p.rope) return dispatch_sum<KIND, 4, 2>(p, kslices, stream);
     if (p.gateup) {
