@@ -132,6 +132,13 @@ int xfthip_quantize_weight(int kind, int K, int N, const float *W_host, void *q_
 
 /* ---- weight-only GEMM --------------------------------------------------------------- */
 /*
+ * Which form of the kernels a product [M, K] x [K, N] takes on the current device (or on 256 compute units where none is in
+ * use), rows without gaps, no prologue or RoPE epilogue: for tests of all of them, and for tuning.  Up to 32 rows {16-column tiles a
+ * block, k tiles a load batch, K slices, 0, 0} (zeros where K is no whole number of weight tiles), above {rows of a block, its
+ * columns, K groups a workgroup, parts of K, 1 where the activations go straight into LDS}.  No counterpart in the reference.
+ */
+int xfthip_gemm_form(int kind, int flags, int has_zero, int M, int K, int N, int form[5]);
+/*
  * C[M,N] = epilogue(A[M,K] * deq(W)[K,N]).  Replaces MMHelper::compute and its
  * compute_bias/_silu/_gelu/_resmul/_residential/_resext variants
  * (matmul_helper.h:565-1705; W8A8: onednn_amx_gemm_f32s8f32_compute, :2762-2965).

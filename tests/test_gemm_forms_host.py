@@ -1,0 +1,54 @@
+"""The shapes of the GPU tests of the products take every form of the kernels that any shape takes: which form a product takes is decided on the
+host and needs no device."""
+import os
+import random
+import sys
+
+import pytest
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+import test_qgemm_gpu as gpu  # noqa: E402
+
+PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "xfastertransformer_amd")
+pytestmark = pytest.mark.skipif(not os.path.exists(os.path.join(PKG, "libxft_hip.so")), reason="library not built (run __graft_entry__.build())")
+
+
+@pytest.fixture(scope="module")
+def xh():
+    from xfastertransformer_amd import capi
+    return capi
+
+
+def _form(xh, kind, M, K, N, gateup=False):
+    """What tells one built kernel from another, and whether K goes in parts."""
+    code, zero = {"int8": (xh.W_INT8, False), "int8z": (xh.W_INT8, True), "uint4": (xh.W_UINT4, True), "nf4": (xh.W_NF4, False),
+                  "bf16": (xh.W_BF16, False)}[kind]
+    f = xh.gemm_form(code, M, K, N, xh.WF_GATEUP if gateup else 0, zero)
+    if M <= 32:
+        return (M + 15) // 16, M > 4, f[0], f[1]
+    rows, cols, groups, parts, direct = f
+    return rows, cols, groups, direct, parts > 1, K % (32 if kind == "bf16" else 64) != 0
+
+
+@pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])
+def test_every_form_is_tested(xh, kind):
+    rng, reached = random.Random(5), {}
+    for _ in range(30000):
+        M, gateup = int(2 ** rng.uniform(0, 12.5)), rng.random() < 0.3 and kind != "int8z"
+        K = int(2 ** rng.uniform(7, 14.2))
+        K = K // 8 * 8 if M > 32 and rng.random() < 0.3 else max(128, K // 128 * 128)
+        N = max(32, int(2 ** rng.uniform(5, 17.3)) // 32 * 32)
+        reached.setdefault(_form(xh, kind, M, K, N, gateup), (M, K, N, gateup))
+    tested = {_form(xh, kind, M, K, N) for M, K, N in gpu.MANY_ROWS + gpu.FEW_ROWS}
+    if kind != "int8z":
+        tested |= {_form(xh, kind, M, K, 2 * I, True) for M, K, I in gpu.GATE_UP}
+    missing = {f: shape for f, shape in reached.items() if f not in tested}
+    assert len(reached) > 15 and not missing
+
+
+def test_staged_tiles_of_a_ragged_depth(xh):
+    """K no whole number of 64: 128-row tiles through registers wherever they fill the device, BF16 weights whole packed tiles in 128 x 128 as well."""
+    assert xh.gemm_form(xh.W_BF16, 2048, 11040, 4096) == (128, 256, 1, 1, 0)
+    assert xh.gemm_form(xh.W_BF16, 1024, 11040, 4096) == (128, 128, 1, 1, 0)
+    assert xh.gemm_form(xh.W_INT8, 2048, 11040, 4096) == (128, 256, 1, 1, 0)
+    assert xh.gemm_form(xh.W_INT8, 450, 11040, 4096) == (64, 128, 1, 2, 0)

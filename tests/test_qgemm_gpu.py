@@ -172,13 +172,18 @@ def _random_weight(xh, orc, rng, kind, K, N, gateup=False):
     return w, W, np.abs(W)
 
 
-# more shapes than the tiles of qgemm_mfma, so that every one is taken somewhere with a ragged last block: 32 and 64 rows with K in parts,
-# 128 x 128 and 128 x 256 with one and two K groups and with K in parts, bands of one to eight row blocks
+# Shapes that between them take every form that any shape takes (test_gemm_forms_host.py checks that they do), with ragged last blocks: 32 and 64
+# rows, 128 x 128 and 128 x 256 with one and two K groups, each with K whole and in parts, bands of one to eight row blocks
+MANY_ROWS = [(33, 8192, 3088), (97, 4096, 1040), (129, 1024, 12304), (200, 4096, 6160), (450, 11008, 2064), (641, 8192, 4112), (700, 4096, 4112),
+             (1285, 4096, 4112), (2100, 1024, 6160), (1161, 2048, 2832), (300, 4160, 2064), (770, 2048, 80),
+             # (a depth that is no whole number of 64, whole and broken packed tiles of BF16 weights)
+             (2000, 1056, 4112), (1000, 1056, 4112), (300, 8224, 2064), (130, 8224, 2064), (2000, 1064, 4112), (700, 1064, 2064),
+             (5526, 12368, 32), (2308, 256, 2512), (2335, 9216, 400), (2129, 12288, 400), (5008, 5248, 160), (2089, 18304, 224), (2307, 3072, 2480),
+             (2423, 9216, 784), (1158, 4480, 3296), (1841, 10368, 32)]
+
+
 @pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])
-@pytest.mark.parametrize("M,K,N", [(33, 8192, 3088), (97, 4096, 1040), (129, 1024, 12304), (200, 4096, 6160), (450, 11008, 2064), (641, 8192, 4112), (700, 4096, 4112),
-                                   (1285, 4096, 4112), (2100, 1024, 6160), (1161, 2048, 2832), (300, 4160, 2064), (770, 2048, 80),
-                                   # (a depth that is no whole number of 64, whole and broken packed tiles of BF16 weights)
-                                   (2000, 1056, 4112), (1000, 1056, 4112), (300, 8224, 2064), (130, 8224, 2064), (2000, 1064, 4112), (700, 1064, 2064)])
+@pytest.mark.parametrize("M,K,N", MANY_ROWS)
 def test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N):
     """Bound: K + 8 additions and the epilogue's few operations in fp32, each off by 2^-24 of what has been added up so far at most; NF4 values
     go in as two bf16 parts, off by 2^-17."""
@@ -194,15 +199,22 @@ def test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N):
 
 
 # on 256 CUs: 1, 2, 3, 4 (at 17 rows and more) and 6 column tiles a block, ragged last blocks, 8 to 1 K slices, and more than 8 tiles a CU
+FEW_ROWS = [(M, K, N) for K, N in [(1280, 1040), (1280, 4112), (1280, 9232), (768, 13328), (768, 18448), (768, 28672), (768, 36880), (256, 36880)]
+            for M in (3, 13, 29)]
+
+
 @pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])
-@pytest.mark.parametrize("M", [3, 13, 29])
-@pytest.mark.parametrize("K,N", [(1280, 1040), (1280, 4112), (1280, 9232), (768, 13328), (768, 18448), (768, 28672), (768, 36880), (256, 36880)])
+@pytest.mark.parametrize("M,K,N", FEW_ROWS)
 def test_few_rows_every_form_against_64_bits(xh, orc, kind, M, K, N):
     test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N)
 
 
+GATE_UP = [(3, 768, 1040), (13, 768, 14336), (29, 768, 9232), (29, 768, 18448), (100, 1024, 1040), (700, 2048, 2064), (1285, 4096, 2064), (2100, 1024, 3088),
+           (23, 128, 16), (2, 128, 17392), (12, 128, 17408), (1966, 13312, 1280)]
+
+
 @pytest.mark.parametrize("kind", ["int8", "uint4", "nf4", "bf16"])
-@pytest.mark.parametrize("M,K,I", [(3, 768, 1040), (13, 768, 14336), (29, 768, 9232), (29, 768, 18448), (100, 1024, 1040), (700, 2048, 2064), (1285, 4096, 2064), (2100, 1024, 3088)])
+@pytest.mark.parametrize("M,K,I", GATE_UP)
 def test_mfma_gateup_every_tile_against_64_bits(xh, orc, kind, M, K, I):
     """silu(g) u: off by what the bounds of g and u (test above) make of it, |silu'| <= 1.1, and 2^-20 of the value for the exponential."""
     rng = np.random.default_rng(M + I)
@@ -305,3 +317,54 @@ def test_null_stream_beside_a_capture(xh, orc, kind):
     xh.synchronize()
     assert np.array_equal(c_dev.to_numpy(np.float32, (M, N)), want)
     w.free()
+
+
+@pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])
+@pytest.mark.parametrize("M,K,N", [(33, 8192, 3088), (200, 4096, 6160), (700, 4096, 4112), (641, 8192, 4112), (2308, 256, 2512), (2335, 9216, 400), (2129, 12288, 400),
+                                   (2100, 1024, 6160), (2000, 1056, 4112), (13, 768, 13328), (29, 768, 28672), (3, 768, 36880)])
+def test_epilogues_of_the_forms_against_64_bits(xh, orc, kind, M, K, N):
+    """Bias and residual on top of the sums, and bf16 results: the bound of the product, three more roundings of 2^-24 of the terms, and half a step
+    of the bf16 result (8 significant bits: 2^-8 of it at most)."""
+    rng = np.random.default_rng(M + K + N)
+    w, W, size = _random_weight(xh, orc, rng, kind, K, N)
+    A = orc.round_bf16(rng.standard_normal((M, K), dtype=np.float32))
+    bias, res = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    y = A.astype(np.float64) @ W
+    bound = np.abs(A).astype(np.float64) @ size * ((K + 8) * 2.0 ** -24 + (2.0 ** -16 if kind == "nf4" else 0.0))
+    got = _run_gemm(xh, w, orc.to_bf16(A), M, K, N, xh.F32, xh.EPI_RESIDENTIAL, bias, res)
+    assert (np.abs(got - (y + bias + res)) <= bound + 3 * 2.0 ** -24 * (np.abs(y) + np.abs(bias) + np.abs(res))).all()
+    got = _run_gemm(xh, w, orc.to_bf16(A), M, K, N, xh.BF16)
+    assert (np.abs(got - y) <= bound * (1 + 2.0 ** -8) + np.abs(y) * 2.0 ** -8).all()
+    w.free()
+
+
+@pytest.mark.parametrize("kind", ["int8", "uint4", "bf16"])
+def test_captured_without_a_parts_buffer(xh, orc, kind):
+    """A product whose K is split, captured on a stream that has no buffer for the parts, runs unsplit: within the bound of the product, the
+    same bits on every replay (not those of the split form, whose sums have another order)."""
+    import ctypes as C
+    M, K, N = 64, 4096, 1024
+    rng = np.random.default_rng(6)
+    w, W, size = _random_weight(xh, orc, rng, kind, K, N)
+    assert xh.gemm_form({"int8": xh.W_INT8, "uint4": xh.W_UINT4, "bf16": xh.W_BF16}[kind], M, K, N, has_zero=kind == "uint4")[3] > 1
+    A = orc.round_bf16(rng.standard_normal((M, K), dtype=np.float32))
+    a, out, graph = xh.DeviceBuffer.from_numpy(orc.to_bf16(A)), xh.DeviceBuffer(M * N * 4), C.c_void_p()
+    _unused.append(xh.Stream())
+    stream = _unused[-1]
+    assert xh.lib.hipStreamBeginCapture(stream.h, 1) == 0  # as another library would; 1: thread-local checks
+    xh.gemm(w, a.ptr, M, K, out.ptr, N, xh.F32, stream=stream.h)
+    assert xh.lib.xfthip_graph_end(stream.h, C.byref(graph)) == 0
+    bound, first = np.abs(A).astype(np.float64) @ size * (K + 8) * 2.0 ** -24, None
+    for _ in range(3):
+        out.zero()
+        assert xh.lib.xfthip_graph_launch(graph, stream.h) == 0
+        xh.synchronize()
+        got = out.to_numpy(np.float32, (M, N))
+        assert (np.abs(got - A.astype(np.float64) @ W) <= bound).all()
+        first = got if first is None else first
+        assert np.array_equal(got, first)
+    xh.lib.xfthip_graph_destroy(graph)
+    w.free()
+
+
+_unused = []  # streams kept alive: scratch is kept by a stream's handle, which a destroyed one's successor may get

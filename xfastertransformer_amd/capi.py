@@ -235,6 +235,13 @@ def quantize_weight(kind, W):
     return q, scale, (None if kind == W_NF4 else zero)
 
 
+def gemm_form(kind, M, K, N, flags=0, has_zero=False):
+    """Which form of the kernels a product takes (include/xft_hip.h); needs no device."""
+    form = (C.c_int * 5)()
+    check(lib.xfthip_gemm_form(kind, flags, int(has_zero), M, K, N, form))
+    return tuple(form)
+
+
 def gemm(w, A_dev, M, lda, C_dev, ldc, c_dtype=BF16, epi=EPI_NONE, bias=None, res=None, ldres=0, res_dtype=F32,
          gamma=1.0, stream=None):
     check(lib.xfthip_gemm(w.h, M, A_dev, lda, C_dev, ldc, c_dtype, epi, bias, res, ldres, res_dtype,

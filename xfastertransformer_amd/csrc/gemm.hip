@@ -84,6 +84,27 @@ int gemm_grouped_rows_dev(const xfthip_weight_t *w, int n_group, const GroupWeig
 
 extern "C" {
 
+int xfthip_gemm_form(int kind, int flags, int has_zero, int M, int K, int N, int form[5]) {
+    XFT_REQUIRE(form && M > 0 && K > 0 && N > 0, "xfthip_gemm_form: bad argument");
+    XFT_REQUIRE(kind == XFTHIP_W_INT8 || kind == XFTHIP_W_UINT4 || kind == XFTHIP_W_NF4 || kind == XFTHIP_W_BF16, "xfthip_gemm_form: weight kind %d not supported", kind);
+    const float zero = 0.0f;
+    const int ktile = ktile_of(kind);
+    SkinnyParams p = {};
+    p.M = M, p.K = K, p.N = N, p.lda = K, p.KT = (K + ktile - 1) / ktile, p.NTILES = (N + 15) / 16;
+    p.zero = has_zero ? &zero : nullptr, p.gateup = (flags & XFTHIP_WF_GATEUP) ? 1 : 0;
+    for (int i = 0; i < 5; ++i) form[i] = 0;
+    if (M <= 32) {
+        if (K % ktile != 0) return 0;
+        const SkinnyForm f = skinny_form(kind, p);
+        form[0] = f.nt, form[1] = f.u, form[2] = f.kslices;
+        return 0;
+    }
+    qgemm_mfma_form(kind, p);
+    form[0] = p.tile == 1 ? 32 : p.tile == 2 ? 64 : 128, form[1] = p.tile == 4 ? 256 : 128;
+    form[2] = p.kgroups, form[3] = p.ksplit > 1 ? p.ksplit : 1, form[4] = p.direct;
+    return 0;
+}
+
 int xfthip_gemm(xfthip_weight_t w, int M, const void *A, int lda, void *C, int ldc, int c_dtype, int epilogue,
         const float *bias, const void *res, int ldres, int res_dtype, float gamma, xfthip_stream_t stream) {
     if (int rc = check_common("xfthip_gemm", w, M, A, lda, C, ldc)) return rc;

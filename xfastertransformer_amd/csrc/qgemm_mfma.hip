@@ -249,6 +249,10 @@ int qgemm_split_reserve(hipStream_t stream, float **out) {
     return 0;
 }
 
+void qgemm_mfma_form(int kind, SkinnyParams &p) {
+    choose_tile(p, kind, ktile_of(kind));
+}
+
 int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t stream, int *parts, const float **part) {
     SkinnyParams p = p0;
     p.packed = pw.packed;
