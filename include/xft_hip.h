@@ -327,6 +327,8 @@ int xfthip_attention_static(xfthip_kvcache_t c, const void *q, int qStride, void
  * maps, new token included: fp32 scores, softmax(scale * s), fp32 P.V, bf16 out [batch, o_stride].
  * max_context: the largest context_lens value (host copy); every table row must hold
  * max_context / block_size + 1 valid entries.  All pointers but none of the integers are device memory.
+ * out may lie over q, k and v.  A first call on a stream allocates scratch (a later one only if it is the first of its size whose out lies over
+ * rows of q that are not its own).
  * The reference reads query / key / value row 0 for every sequence and indexes the KV head with the
  * query head (attention_kernels.cpp:51-61); this entry point uses row b and head hq / (q_heads / kv_heads),
  * the same for batch 1 without grouped heads.
@@ -339,6 +341,7 @@ int xfthip_paged_attention_decode(void *out, const void *q, const void *k, const
  * Prefill: sequences lie back to back in q / k / v (token_lens_host[b] rows each, host array); causal
  * self-attention per sequence (the reference's selfAttention call, attention_kernels.cpp:141-151) and
  * every token's key / value row stored at slot_mapping[token] (device int32, one entry per token).
+ * out may lie over q, k and v.  The scratch grows with the tokens of a call.
  */
 int xfthip_paged_attention_prefill(void *out, const void *q, const void *k, const void *v, int q_heads, int kv_heads,
         int head_size, int q_stride, int kv_stride, int o_stride, float scale, int batch, const int *token_lens_host,

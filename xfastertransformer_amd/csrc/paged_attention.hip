@@ -453,9 +453,10 @@ extern "C" int xfthip_paged_attention_decode(void *out, const void *q, const voi
             max_context / block_size + 1, table_stride);
     XFT_REQUIRE(block_num > 0, "xfthip_paged_attention_decode: bad block count");
     hipStream_t st = (hipStream_t)stream;
-    // One workgroup a CU, at least one 32-token block a wave (1, 2 or 4 workgroups a CU: 1 x 1000 tokens, 8 KV heads 10.3 / 11.7 / 11.6 us,
-    // 64 x 500, 4 KV heads 15.0 / 17.5 / 19.1, 1 x 9000 16.8 / 16.8 / 16.9, 32 x 4100 86.6 / 87.2 / 85.2; 64 splits in place of 32 cost
-    // 1 x 9000 2.5 us)
+    // About one workgroup a CU, at least one 32-token block a wave (1, 2 or 4 workgroups a CU: 1 x 1000 tokens, 8 KV heads 10.3 / 11.7 / 11.6 us,
+    // 64 x 500, 4 KV heads 15.0 / 17.5 / 19.1, 1 x 9000 16.8 / 16.8 / 16.9, 32 x 4100 86.6 / 87.2 / 85.2), 32 splits at most: below 8 (sequence, KV head,
+    // column group) units part of the CUs stay idle (64 splits cost 1 x 9000 2.5 us; with 32, 1 x 32000 tokens, 8 query / 1 KV heads take 25 us, 1 x 100000 54,
+    // against 49 and 79 with a workgroup a query head and 64 splits)
     const int colgroups = (q_heads / kv_heads + 15) / 16, units = batch * kv_heads * colgroups;
     int nsplit = (device_cu_count() + units - 1) / units;
     const int cap = (max_context + 1 + 127) / 128;

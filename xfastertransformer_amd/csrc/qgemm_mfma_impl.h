@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     // XCDs carry the same load whatever the number of column blocks (43 blocks of 256 columns dealt out block by block
     // would give three XCDs 6 and five XCDs 5).
     // Row counts on the device: the row blocks that are there are numbered, so that all workgroups past them come last.
-    int group_before = 0; // (lane e of every wave, groups) row blocks of the weights before weight e of its 64
+    int group_upto = 0; // (lane e of every wave, groups) row blocks of the weights up to and including weight e of its 64
     if constexpr (DEVROWS) {
         if (p.group) {
             nblocks_m = 0;
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
                     const int up = __shfl_up(n, off, 64);
                     n += lane >= off ? up : 0;
                 }
-                group_before = n; // (inclusive; of the last 64)
+                group_upto = n; // (of the last 64)
                 nblocks_m += __builtin_amdgcn_readlane(n, 63);
             }
         } else if (p.rows_dev) {
@@ -166,9 +166,9 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
         // row, weight after weight, by their device-side row counts
         int e = 0, first = 0;
         if (p.group_n <= 64) {
-            const unsigned long long before = __builtin_amdgcn_ballot_w64(group_before <= mb);
-            e = __builtin_popcountll(before); // (group_before is ascending over the lanes)
-            first = e ? __builtin_amdgcn_readlane(group_before, e - 1) : 0;
+            const unsigned long long before = __builtin_amdgcn_ballot_w64(group_upto <= mb);
+            e = __builtin_popcountll(before); // (group_upto is ascending over the lanes)
+            first = e ? __builtin_amdgcn_readlane(group_upto, e - 1) : 0;
         } else {
             for (; e < p.group_n; ++e) {
                 const int nblk = (p.rows_dev[e * p.rows_stride] + ROWS - 1) / ROWS;
