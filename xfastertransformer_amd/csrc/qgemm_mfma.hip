@@ -164,7 +164,8 @@ bool choose_staged_tile(SkinnyParams &p, int kind, int ktile, bool may_split) {
     return true;
 }
 
-void choose_tile(SkinnyParams &p, int kind, int ktile, bool may_split = true) {
+// own_sum: the caller adds the parts in a pass that it makes anyway
+void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_split = true) {
     const int cus = device_cu_count(), kt_n = (p.K + ktile - 1) / ktile, cls = kind == XFTHIP_W_BF16 ? 1 : kind == XFTHIP_W_NF4 ? 2 : kind == XFTHIP_W_UINT4 ? 3 : 0;
     // activations straight into LDS: steps of 64 k, byte offsets of 32 bits
     const bool direct = p.K % 64 == 0 && (size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32);
@@ -211,7 +212,7 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool may_split = true) {
                 const float x = (float)rest / (float)cus, fullest = (float)((rest + cus - 1) / cus);
                 us += steps * (x <= 1.0f ? t.step[cls] * (0.77f + 0.23f * x) : t.step[cls] + t.more[cls] * (0.55f * fullest + 0.45f * x - 1.0f)) + t.fixed;
             }
-            if (parts > 1) us += kSplitStart[cls] + kSplitMb[cls] * 4e-6f * (float)parts * (float)p.M * (float)p.N;
+            if (parts > 1) us += (own_sum ? 0.0f : kSplitStart[cls]) + (own_sum ? 0.15f : kSplitMb[cls]) * 4e-6f * (float)parts * (float)p.M * (float)p.N;
             if (us < best) {
                 best = us;
                 p.tile = t.rows == 32 ? 1 : t.rows == 64 ? 2 : t.cols == 128 ? 3 : 4;
@@ -250,7 +251,7 @@ int qgemm_split_reserve(hipStream_t stream, float **out) {
 }
 
 void qgemm_mfma_form(int kind, SkinnyParams &p) {
-    choose_tile(p, kind, ktile_of(kind));
+    choose_tile(p, kind, ktile_of(kind), false);
 }
 
 int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t stream, int *parts, const float **part) {
@@ -264,8 +265,8 @@ int qgemm_mfma(const PackedWeight &pw, const SkinnyParams &p0, hipStream_t strea
     p.N = pw.N;
     p.ksplit = 0, p.split_ktiles = 0, p.split_part = nullptr;
     const int ktile = ktile_of(pw.kind), kt_n = (pw.K + ktile - 1) / ktile;
-    choose_tile(p, pw.kind, ktile);
-    if (p.ksplit > 1 && !qgemm_split_usable(stream)) p.ksplit = 0, choose_tile(p, pw.kind, ktile, false);
+    choose_tile(p, pw.kind, ktile, parts != nullptr);
+    if (p.ksplit > 1 && !qgemm_split_usable(stream)) p.ksplit = 0, choose_tile(p, pw.kind, ktile, false, false);
     if (p.ksplit > 1) {
         if ((size_t)p.ksplit * p.M * p.N > qgemm_split_bound()) p.ksplit = 0; // cannot happen within the bound; stay correct anyway
         else if (int rc = qgemm_split_reserve(stream, &p.split_part)) return rc;
