@@ -213,9 +213,10 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_sp
                 us += steps * (x <= 1.0f ? t.step[cls] * (0.77f + 0.23f * x) : t.step[cls] + t.more[cls] * (0.55f * fullest + 0.45f * x - 1.0f)) + t.fixed;
             }
             if (parts > 1) us += (own_sum ? 0.0f : kSplitStart[cls]) + (own_sum ? 0.15f : kSplitMb[cls]) * 4e-6f * (float)parts * (float)p.M * (float)p.N;
-            // (an expert's last block is half empty on average: the gate / up product of 8 INT8 experts of width 2816 at width 2048, 700 tokens, took 7 us
-            // more in 128 x 256 than in 64-row blocks, which were to take 1 more; the layer 137 -> 129)
-            if (p.group && t.rows == 128) us *= 1.05f;
+            // (an expert's last block is half empty on average.  8 INT8 experts of width 2816 at width 2048, 700 tokens: 7 us more in 128 x 256 than in 64-row
+            // blocks, which were to take 1 more; the layer 137 -> 129.  With down projections priced so as well, 256 tokens of the Mixtral shape
+            // lose 0.7 %)
+            if (p.group && p.gateup && t.rows == 128) us *= 1.05f;
             if (us < best) {
                 best = us;
                 p.tile = t.rows == 32 ? 1 : t.rows == 64 ? 2 : t.cols == 128 ? 3 : 4;
