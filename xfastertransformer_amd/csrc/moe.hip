@@ -43,7 +43,7 @@ __global__ void top2_kernel(const float *__restrict__ logits, int M, int E, int 
 // weights (GateTypeSelector: fp32 for quantised weight types, src/utils/type_selector.h:93-111) unless they are given, and its two experts.
 // One workgroup a token, bound by a chain of load round trips: everything for the first 4096 columns is requested at once, router weights before
 // the norm is known.  The tokens' workgroups all read the same router weights: their waves start at places apart, so that they do not ask
-// the same L2 channel at a time.  In place of a norm, a router of one wave a token and a selection: 256 tokens of width 4096 6 + 33 + 5 -> 13 us
+// the same L2 channel at a time.  In place of a norm, a router of one wave a token and a selection: 256 tokens of width 4096 6 + 33 + 5 -> 10 us
 // (4 waves a token, weights requested behind the norm: 24).
 constexpr int kRouteThreads = 1024, kRouteCols = 4; // columns a thread and round
 template <bool NORM, int E>
