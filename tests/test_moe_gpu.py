@@ -195,6 +195,24 @@ def test_mixtral_mlp_many_rows_an_expert(xh, orc, tokens):
     test_mixtral_mlp_bf16_experts(xh, orc, tokens, 352, 736)  # (a depth that is no whole number of steps)
 
 
+@pytest.mark.parametrize("kind,hidden,inter,tokens", [(0, 1056, 3600, 256), (1, 1056, 3600, 160), (0, 2048, 2816, 100), (2, 2048, 2816, 300)])
+def test_mixtral_mlp_down_projection_in_parts(xh, orc, kind, hidden, inter, tokens):
+    """The down projection's K in parts that the combination adds: a depth that is no whole number of weight tiles, and whole ones."""
+    E, rng = 8, np.random.default_rng(inter + tokens)
+    experts = _experts(orc, rng, kind, hidden, inter, E)
+    x, lo = orc.round_bf16(rng.standard_normal((tokens, hidden))), rng.standard_normal((tokens, E)).astype(np.float32)
+    ln, router = rng.uniform(0.8, 1.2, hidden).astype(np.float32), np.zeros((hidden, E), np.float32)
+    moe = xh.MoE(hidden, inter, E, tokens, router, ln)
+    for e, (gu, dn) in enumerate(experts):
+        moe.set_expert(e, xh.Weight(kind, gu.K, gu.N, gu.q, gu.scale, gu.zero, flags=xh.WF_GATEUP), xh.Weight(kind, dn.K, dn.N, dn.q, dn.scale, dn.zero))
+    xd, lod, od = xh.DeviceBuffer.from_numpy(x), xh.DeviceBuffer.from_numpy(lo), xh.DeviceBuffer(x.nbytes)
+    moe.forward(xd.ptr, od.ptr, tokens, True, lod.ptr)
+    xh.synchronize()
+    got = od.to_numpy(np.float32, x.shape)
+    exp, _, _ = orc.mixtral_mlp(x, ln, router, experts, lo, rounding="bf16")
+    assert np.abs(got - exp).max() < 2e-2 and _cos(got, exp) >= 0.9999
+
+
 @pytest.mark.parametrize("tokens", [12, 70])
 def test_mixtral_mlp_experts_of_different_layouts(xh, orc, tokens):
     """Experts that cannot share a launch (some INT8 weights carry a zero-point vector, some do not) go through the
