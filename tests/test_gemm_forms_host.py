@@ -52,3 +52,13 @@ def test_staged_tiles_of_a_ragged_depth(xh):
     assert xh.gemm_form(xh.W_BF16, 1024, 11040, 4096) == (128, 128, 1, 1, 0)
     assert xh.gemm_form(xh.W_INT8, 2048, 11040, 4096) == (128, 256, 1, 1, 0)
     assert xh.gemm_form(xh.W_INT8, 450, 11040, 4096) == (64, 128, 1, 2, 0)
+
+
+def test_few_rows_of_a_wide_weight(xh):
+    """Shallow and deep K over many columns, and a stretch of columns that leaves a CU four blocks of two tiles."""
+    assert xh.gemm_form(xh.W_INT8, 8, 2048, 151936)[:3] == (2, 2, 3)
+    assert xh.gemm_form(xh.W_BF16, 8, 2048, 151936)[:3] == (2, 2, 3)
+    assert xh.gemm_form(xh.W_INT8, 8, 8192, 55296)[:3] == (2, 2, 1)
+    assert xh.gemm_form(xh.W_BF16, 32, 1024, 65024)[:3] == (2, 2, 2)
+    assert xh.gemm_form(xh.W_BF16, 32, 8192, 28672)[:3] == (2, 2, 1)
+    assert xh.gemm_form(xh.W_INT8, 32, 5120, 27648)[:3] == (4, 1, 4)

@@ -56,11 +56,17 @@ SkinnyForm skinny_form(int kind, const SkinnyParams &p) {
         return form(2, 2);
     }
     if (tiles > 8 * cus) {
-        if (mt == 2) return form(4, four ? 2 : kind == XFTHIP_W_INT8 ? 3 : 1);
+        // (a shallow K goes by its own counts, for no reason that is known: in the forms for a deeper one INT8 8 rows of 1024 x 65024 17.6 us, of
+        // 2048 x 151936 55.0, here 15.3 and 49.9; BF16 32 rows of 1024 x 65024 35.6 and 29.4.  INT8 8 rows of 8192 x 55296: 83 us in 8 slices, 74 in one;
+        // 32 rows of 3584 x 100000 79 in 3, 77 in 4, of 8192 x 55296 92 and 102)
+        const bool shallow = p.K <= 2048;
+        if (mt == 2 && kind == XFTHIP_W_BF16 && shallow) return form(2, p.K < 2048 ? 2 : 1);
+        if (mt == 2) return form(4, four ? 2 : kind == XFTHIP_W_INT8 ? (p.KT > 32 && p.KT % 32 ? 4 : 3) : 1);
         if (four) return form(4, 4);
+        if (shallow && (kind == XFTHIP_W_INT8 || p.M > 8 || p.K > 1024)) return form(2, 3);
         // (BF16, 16 rows of 128256 columns: single tiles in 8 slices 199 us, 171 before, 166 in this form)
         if (kind == XFTHIP_W_BF16 && p.M > 8) return form(2, 1);
-        return form(kind == XFTHIP_W_INT8 || p.gateup ? 2 : 1, 8);
+        return form(kind == XFTHIP_W_INT8 || p.gateup ? 2 : 1, kind == XFTHIP_W_INT8 && p.K >= 8192 ? 1 : 8);
     }
     int nt = p.gateup ? 2 : 1;
     if (kind != XFTHIP_W_BF16 || mt == 2) {
@@ -68,13 +74,16 @@ SkinnyForm skinny_form(int kind, const SkinnyParams &p) {
         for (int n : {1, 2, 3, 4, 6}) {
             if ((p.gateup && n % 2) || (n >= 4 && mt == 1) || (n % 3 == 0 && p.group)) continue;
             const int w = per_cu(n);
-            // (17 .. 32 rows, two blocks of four tiles on a CU: well for 4-bit codes, 1.2 times the time of four blocks of two for the others)
-            const float tile = n == 1 ? 1.2f : n == 2 ? 1.0f : n == 4 && w > 1 && !four ? 1.3f : 1.1f;
+            // (17 .. 32 rows, two blocks of four tiles on a CU: well for 4-bit codes and a deep INT8 K (32 rows x 27648 x 5120 41.6 -> 36.1 us), 1.2
+            // times the time of four blocks of two for the others)
+            const bool dear = n == 4 && w > 1 && !four && !(kind == XFTHIP_W_INT8 && p.KT >= 80);
+            const float tile = n == 1 ? 1.2f : n == 2 ? 1.0f : dear ? 1.3f : 1.1f;
             const float cost = (float)w * ((float)n * tile + 0.5f);
             if (cost < least) least = cost, nt = n;
         }
     }
-    const int least = kind == XFTHIP_W_BF16 ? 1 : 2, slices = 8 / per_cu(nt);
+    // (BF16, four blocks of two tiles on a CU: one slice each, 32 rows x 28672 x 8192 101 -> 88 us, with SwiGLU 8 rows x 28672 x 4096 1.07 times as fast)
+    const int least = kind == XFTHIP_W_BF16 ? 1 : 2, slices = kind == XFTHIP_W_BF16 && nt == 2 && per_cu(nt) > 2 ? 1 : 8 / per_cu(nt);
     return form(nt, slices > least ? slices : least);
 }
 
