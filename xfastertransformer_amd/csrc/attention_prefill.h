@@ -436,8 +436,8 @@ __device__ inline void attn_prefill32_unit(const AttnParams &p, const int kvh, c
                 const float v0 = o[ct][dt][4 * q] * inv, v1 = o[ct][dt][4 * q + 1] * inv, v2 = o[ct][dt][4 * q + 2] * inv,
                             v3 = o[ct][dt][4 * q + 3] * inv;
                 if (p.out_dtype == XFTHIP_BF16) {
-                    const uint32_t lo = f32_to_bf16_ref(v0) | ((uint32_t)f32_to_bf16_ref(v1) << 16);
-                    const uint32_t hi = f32_to_bf16_ref(v2) | ((uint32_t)f32_to_bf16_ref(v3) << 16);
+                    const uint32_t lo = f32x2_to_bf16(v0, v1);
+                    const uint32_t hi = f32x2_to_bf16(v2, v3);
                     uint16_t *dst = (uint16_t *)p.out + idx;
                     if ((((uintptr_t)dst) & 7) == 0) {
                         *(uint2 *)dst = make_uint2(lo, hi);

@@ -80,11 +80,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(void *__restrict__ out
             if constexpr (OUT_BF16) {
                 uint32_t pk[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t lo = f32_to_bf16_ref((x[c][2 * i] * var) * w[c][2 * i]);
-                    const uint32_t hi = f32_to_bf16_ref((x[c][2 * i + 1] * var) * w[c][2 * i + 1]);
-                    pk[i] = lo | (hi << 16);
-                }
+                for (int i = 0; i < 4; ++i) pk[i] = f32x2_to_bf16((x[c][2 * i] * var) * w[c][2 * i], (x[c][2 * i + 1] * var) * w[c][2 * i + 1]);
                 *(uint4 *)((uint16_t *)out + obase + col) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
             } else {
                 float *o = (float *)out + obase + col;
@@ -353,8 +349,8 @@ __global__ __launch_bounds__(256) void rope_kv_block_kernel(RopeKvParams p, int 
             u32x4 olo, ohi;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                olo[e] = (uint32_t)f32_to_bf16_ref(lo[2 * e]) | ((uint32_t)f32_to_bf16_ref(lo[2 * e + 1]) << 16);
-                ohi[e] = (uint32_t)f32_to_bf16_ref(hi[2 * e]) | ((uint32_t)f32_to_bf16_ref(hi[2 * e + 1]) << 16);
+                olo[e] = f32x2_to_bf16(lo[2 * e], lo[2 * e + 1]);
+                ohi[e] = f32x2_to_bf16(hi[2 * e], hi[2 * e + 1]);
             }
             uint16_t *dst = (uint16_t *)p.qkv + tok * p.stride + (size_t)head * 128;
             *(u32x4 *)(dst + 8 * c) = olo;

@@ -44,7 +44,7 @@ __device__ inline float2 load2(const void *p, size_t i) {
 }
 template <bool BF16>
 __device__ inline void store2(void *p, size_t i, float2 v) {
-    if constexpr (BF16) *(uint32_t *)((uint16_t *)p + i) = f32_bits_to_bf16_sel(f2u(v.x)) | (f32_bits_to_bf16_sel(f2u(v.y)) << 16);
+    if constexpr (BF16) *(uint32_t *)((uint16_t *)p + i) = f32x2_to_bf16(v.x, v.y);
     else *(float2 *)((float *)p + i) = v;
 }
 

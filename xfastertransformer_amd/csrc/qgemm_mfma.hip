@@ -88,8 +88,8 @@ __global__ __launch_bounds__(256) void qgemm_split_finish_kernel(SkinnyParams p)
             return;
         }
         if (p.c_dtype == XFTHIP_BF16 && ((((uintptr_t)p.C) | ((size_t)p.ldc * 2)) & 7) == 0) {
-            const uint32_t lo = f32_to_bf16_ref(x[0]) | ((uint32_t)f32_to_bf16_ref(x[1]) << 16);
-            const uint32_t hi = f32_to_bf16_ref(x[2]) | ((uint32_t)f32_to_bf16_ref(x[3]) << 16);
+            const uint32_t lo = f32x2_to_bf16(x[0], x[1]);
+            const uint32_t hi = f32x2_to_bf16(x[2], x[3]);
             *(uint2 *)((uint16_t *)p.C + ci) = make_uint2(lo, hi);
             return;
         }

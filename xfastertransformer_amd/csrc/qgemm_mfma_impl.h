@@ -23,9 +23,6 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// f32_to_bf16_ref() as selects (bf16_convert.h): the same bits for every input
-__device__ inline uint32_t f32_to_bf16_sel(float f) { return f32_bits_to_bf16_sel(__float_as_uint(f)); }
-
 union MFrag {
     bf16x8 v;
     uint32_t u[4];
@@ -725,9 +722,8 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
                     u32x4 o;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const uint32_t b0 = p.c_dtype == XFTHIP_BF16 ? f32_to_bf16_sel(v[2 * e]) : f32_to_fp16_bits(v[2 * e]);
-                        const uint32_t b1 = p.c_dtype == XFTHIP_BF16 ? f32_to_bf16_sel(v[2 * e + 1]) : f32_to_fp16_bits(v[2 * e + 1]);
-                        o[e] = b0 | (b1 << 16);
+                        o[e] = p.c_dtype == XFTHIP_BF16 ? f32x2_to_bf16(v[2 * e], v[2 * e + 1])
+                                                        : (uint32_t)f32_to_fp16_bits(v[2 * e]) | ((uint32_t)f32_to_fp16_bits(v[2 * e + 1]) << 16);
                     }
                     *(u32x4 *)((uint16_t *)p.C + ci) = o;
                 }

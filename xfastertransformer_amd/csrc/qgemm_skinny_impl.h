@@ -415,8 +415,8 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
                     for (int i = 0; i < NB; ++i) {
                         const int ci = c + i * (int)blockDim.x * 4;
                         const float4 v = vv[i], w = ww[i];
-                        const uint32_t lo = f32_to_bf16_ref((v.x * var) * w.x) | ((uint32_t)f32_to_bf16_ref((v.y * var) * w.y) << 16);
-                        const uint32_t hi = f32_to_bf16_ref((v.z * var) * w.z) | ((uint32_t)f32_to_bf16_ref((v.w * var) * w.w) << 16);
+                        const uint32_t lo = f32x2_to_bf16((v.x * var) * w.x, (v.y * var) * w.y);
+                        const uint32_t hi = f32x2_to_bf16((v.z * var) * w.z, (v.w * var) * w.w);
                         if (ci < p.K) *(uint2 *)(xn + (size_t)m * pitch + ci) = make_uint2(lo, hi);
                     }
                 }

@@ -229,8 +229,8 @@ __global__ __launch_bounds__(KS > 4 ? 64 * KS : 256) void tile_gemm_kernel(TileG
                     if (p.c_dtype == XFTHIP_F32)
                         *(f32x4 *)((float *)p.C + at) = acc[t][m];
                     else
-                        *(uint2 *)((uint16_t *)p.C + at) = make_uint2(f32_to_bf16_ref(acc[t][m][0]) | ((uint32_t)f32_to_bf16_ref(acc[t][m][1]) << 16),
-                                f32_to_bf16_ref(acc[t][m][2]) | ((uint32_t)f32_to_bf16_ref(acc[t][m][3]) << 16));
+                        *(uint2 *)((uint16_t *)p.C + at) = make_uint2(f32x2_to_bf16(acc[t][m][0], acc[t][m][1]),
+                                f32x2_to_bf16(acc[t][m][2], acc[t][m][3]));
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)

@@ -681,9 +681,8 @@ __global__ __launch_bounds__(256 * WR, DIRECT ? 2 : 1) void w8a8_mfma_kernel(W8A
                         i32x4 o;
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
-                            const uint32_t b0 = p.c_dtype == XFTHIP_BF16 ? f32_bits_to_bf16_sel(f2u(v[2 * e])) : f32_to_fp16_bits(v[2 * e]);
-                            const uint32_t b1 = p.c_dtype == XFTHIP_BF16 ? f32_bits_to_bf16_sel(f2u(v[2 * e + 1])) : f32_to_fp16_bits(v[2 * e + 1]);
-                            o[e] = (int)(b0 | (b1 << 16));
+                            o[e] = (int)(p.c_dtype == XFTHIP_BF16 ? f32x2_to_bf16(v[2 * e], v[2 * e + 1])
+                                                                  : (uint32_t)f32_to_fp16_bits(v[2 * e]) | ((uint32_t)f32_to_fp16_bits(v[2 * e + 1]) << 16));
                         }
                         *(i32x4 *)((uint16_t *)p.C + ci) = o;
                     }
@@ -735,8 +734,8 @@ __global__ __launch_bounds__(256) void w8a8_split_finish_kernel(W8A8Params p) {
     if (p.c_dtype == XFTHIP_F32 && (((uintptr_t)p.C | ((size_t)p.ldc * 4)) & 15) == 0) {
         *(float4 *)((float *)p.C + ci) = make_float4(x[0], x[1], x[2], x[3]);
     } else if (p.c_dtype == XFTHIP_BF16 && (((uintptr_t)p.C | ((size_t)p.ldc * 2)) & 7) == 0) {
-        const uint32_t lo = f32_to_bf16_ref(x[0]) | ((uint32_t)f32_to_bf16_ref(x[1]) << 16);
-        const uint32_t hi = f32_to_bf16_ref(x[2]) | ((uint32_t)f32_to_bf16_ref(x[3]) << 16);
+        const uint32_t lo = f32x2_to_bf16(x[0], x[1]);
+        const uint32_t hi = f32x2_to_bf16(x[2], x[3]);
         *(uint2 *)((uint16_t *)p.C + ci) = make_uint2(lo, hi);
     } else {
 #pragma unroll
