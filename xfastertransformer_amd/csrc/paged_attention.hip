@@ -382,9 +382,8 @@ __device__ inline AttnParams seq_params(const AttnParams &all, const SeqBatch &s
 
 // attn_prefill32_kernel over sequences: (sequence, KV head) pairs go to the XCDs in turn, an XCD walks the column groups of one
 // pair, longest history first, before it starts the next
-template <bool SCALED>
 __global__ __launch_bounds__(256, 2) void paged_prefill_attn_kernel(AttnParams all, SeqBatch s) {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[3 * 16384];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kRingLds];
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     int group = 0, hi = (s.many * all.kv.H + 7) / 8 - 1;
     while (group < hi) {
@@ -397,7 +396,7 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn_kernel(AttnParams a
     const AttnParams p = seq_params(all, s, s.first + i);
     const int ncg = (p.S * p.G + 127) / 128;
     if (at >= ncg) return; // (a longer sequence shares the group)
-    attn_prefill32_unit<4, 1, false, SCALED>(p, pair % all.kv.H, ncg - 1 - at, 0, lds);
+    attn_prefill_ring_unit(p, pair % all.kv.H, ncg - 1 - at, 0, lds);
 }
 
 // attn_kernel over sequences, each walked by one workgroup a column group: grid (KV heads x the longest's column groups, sequences)
@@ -558,22 +557,16 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
         AttnParams p = {};
         p.kv = kv, p.q = (const uint16_t *)q, p.qStride = q_stride, p.out = out, p.oStride = o_stride, p.out_dtype = XFTHIP_BF16;
         p.B = 1, p.G = G, p.scale = scale, p.nsplit = 1;
-        // Those that attention_launch would take to the form for many columns, then the others: in that form too where they are enough together,
-        // but with exact queries, as the form for few columns has them, which they would take alone (12 x 200 tokens, 32 query / 8 KV heads
-        // 30 us against 52 in that one, 8 x 600, 16 / 4 heads 38 against 79)
-        auto many = [&](int at, int count, bool scaled) {
-            const int groups = (count * kv_heads + 7) / 8;
-            s.first = at, s.many = count;
-            for (int g = 0; g < groups; ++g) // (the sequences are sorted: the group's first pair belongs to its longest)
-                s.grp0[g + 1] = s.grp0[g] + (int)(((long)s.rows[at + g * 8 / kv_heads] * G + 127) / 128);
-            if (scaled) hipLaunchKernelGGL(paged_prefill_attn_kernel<true>, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
-            else hipLaunchKernelGGL(paged_prefill_attn_kernel<false>, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
-        };
-        if (n_long > 0) many(0, n_long, true);
-        s.first = n_long, s.many = s.n - n_long;
-        if (waves >= 4L * device_cu_count()) many(n_long, s.n - n_long, false);
-        else if (s.many > 0)
-            hipLaunchKernelGGL(paged_prefill_few_kernel, dim3(kv_heads * ((s.rows[n_long] * G + 15) / 16), s.many), dim3(256), 0, st, p, s);
+        // Those that attention_launch would take to the form for many columns, and the others with them where they are enough together (12 x 200
+        // tokens, 32 query / 8 KV heads 21 us against 52 in the form for few columns, 8 x 600, 16 / 4 heads 29 against 79)
+        s.first = 0, s.many = waves >= 4L * device_cu_count() ? s.n : n_long;
+        const int groups = (s.many * kv_heads + 7) / 8;
+        for (int g = 0; g < groups; ++g) // (the sequences are sorted: the group's first pair belongs to its longest)
+            s.grp0[g + 1] = s.grp0[g] + (int)(((long)s.rows[g * 8 / kv_heads] * G + 127) / 128);
+        if (s.many > 0) hipLaunchKernelGGL(paged_prefill_attn_kernel, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
+        s.first = s.many, s.many = s.n - s.many;
+        if (s.many > 0)
+            hipLaunchKernelGGL(paged_prefill_few_kernel, dim3(kv_heads * ((s.rows[s.first] * G + 15) / 16), s.many), dim3(256), 0, st, p, s);
         XFT_CHECK_HIP(hipGetLastError());
     }
     return 0;
