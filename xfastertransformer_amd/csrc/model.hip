@@ -870,7 +870,7 @@ int xfthip_model_step(xfthip_model_t m, int n, const int *rows_host, const int *
     m->cur_B = 0;
     for (int r = 0; r < c.max_batch; ++r)
         if (m->row_pos[r] >= 0) m->cur_B = r + 1;
-    if (int rc = plan_logits(m, want_host, n_want, logits_host, st)) return rc;
+    if (n_want > 0) return plan_logits(m, want_host, n_want, logits_host, st); // (which waits for everything in front of the logits)
     XFT_CHECK_HIP(hipStreamSynchronize(st));
     return 0;
 }

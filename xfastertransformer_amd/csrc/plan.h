@@ -335,7 +335,7 @@ struct PageTable {
     int pages_for(int tokens) const { return (tokens / unit + kPageTokens - 1) / kPageTokens; }
 };
 
-constexpr int kLogitPieces = 4; // of a logits copy to the host
+constexpr int kLogitPieces = 8; // of a logits copy to the host
 
 // What a model from a plan adds to xfthip_model: the page pool and the state slots, scratch, the step's description.
 struct PlanState {
@@ -358,7 +358,11 @@ struct PlanState {
     // pinned images of what else a step copies: the rows whose logits are wanted, a decode call's slots, the page table, logits
     int *want_host = nullptr, *dec_host = nullptr, *table_pinned = nullptr;
     float *logits_pinned = nullptr;
-    hipEvent_t fetched[kLogitPieces - 1] = {}; // behind all pieces of the logits but the last
+    // a logits copy: which copy each piece belongs to that has arrived (pinned, a cache line each), how many workgroups have sent their share
+    // of a piece, the copies made so far
+    uint32_t *arrived = nullptr;
+    unsigned *sent = nullptr;
+    uint32_t fetches = 0;
     int *tok_seg = nullptr, *tok_pos = nullptr, *ids = nullptr, *seg = nullptr, *dec_rows = nullptr;
     std::vector<int> seg_off_host, seg_len_host, seg_pos_host, seg_row_host; // the step's segments
     std::vector<int> dec_list; // slots of the decode call in flight

@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <map>
 
 #include "model_impl.h"
@@ -506,23 +507,62 @@ int plan_head(xfthip_model *m, const int *rows_dev, int n, int at, hipStream_t s
     return plan.cfg.logit_softcap > 0.0f ? plan_softcap(logits, (size_t)n * c.vocab, plan.cfg.logit_softcap, st) : 0;
 }
 
-// Behind the head: `floats` logits into the caller's pageable memory by way of a pinned buffer, in up to kLogitPieces pieces of 512 KB or more, so
-// that the host moves one on while the card sends the next.  The stream is idle on return.  Bound by the host's way where the caller's memory is
-// fresh (16 rows of 32000, 2 MB: 48 us for the card's way, 60 to 80 for the host's, one after the other before; a decode step of 16 sequences
-// 470 -> 445 us with it and plan_describe_kernel)
-static int plan_fetch_logits(PlanState &p, const float *logits, size_t floats, float *logits_host, hipStream_t st) {
-    const size_t pieces = std::min<size_t>(std::max<size_t>(floats / (128 * 1024), 1), kLogitPieces), each = ((floats + pieces - 1) / pieces + 63) / 64 * 64;
-    for (size_t i = 0; i < pieces; ++i) {
-        const size_t at = std::min(i * each, floats), n = std::min(each, floats - at);
-        if (n == 0) continue;
-        XFT_CHECK_HIP(hipMemcpyAsync(p.logits_pinned + at, logits + at, n * 4, hipMemcpyDeviceToHost, st));
-        if (i + 1 < pieces) XFT_CHECK_HIP(hipEventRecord(p.fetched[i], st));
+// `floats` logits into pinned host memory, piece after piece of `each`; behind the last store of a piece its flag becomes `stamp`.  Two sets of workgroups
+// take the pieces in turn, so that one is sending while the other waits for its stores to arrive.  Bound by the way to the host (2 MB: about 45 us).
+__global__ __launch_bounds__(256) void plan_fetch_kernel(const float *src, float *dst, size_t floats, size_t each, unsigned *sent, uint32_t *arrived, uint32_t stamp) {
+    const int set = blockIdx.x & 1, part = blockIdx.x >> 1, parts = gridDim.x >> 1;
+    const bool wide = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
+    for (int piece = set; piece * each < floats; piece += 2) {
+        const size_t from = piece * each, to = from + each < floats ? from + each : floats;
+        size_t done = from;
+        if (wide) {
+            const float4 *s = (const float4 *)(src + from);
+            float4 *d = (float4 *)(dst + from);
+            const size_t n = (to - from) / 4, step = (size_t)parts * 256;
+            size_t i = (size_t)part * 256 + threadIdx.x;
+            for (; i + 3 * step < n; i += 4 * step) {
+                const float4 x0 = s[i], x1 = s[i + step], x2 = s[i + 2 * step], x3 = s[i + 3 * step];
+                d[i] = x0, d[i + step] = x1, d[i + 2 * step] = x2, d[i + 3 * step] = x3;
+            }
+            for (; i < n; i += step) d[i] = s[i];
+            done += n * 4;
+        }
+        for (size_t i = done + (size_t)part * 256 + threadIdx.x; i < to; i += (size_t)parts * 256) dst[i] = src[i];
+        dev_drain(); // this wave's stores have arrived
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            __threadfence_system();
+            if (atomicAdd(sent + piece, 1u) == (unsigned)parts - 1) {
+                atomicExch(sent + piece, 0u);
+                __hip_atomic_store(arrived + 16 * piece, stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
     }
-    for (size_t i = 0; i < pieces; ++i) {
-        const size_t at = std::min(i * each, floats), n = std::min(each, floats - at);
-        if (i + 1 < pieces && n > 0) XFT_CHECK_HIP(hipEventSynchronize(p.fetched[i]));
-        if (i + 1 == pieces) XFT_CHECK_HIP(hipStreamSynchronize(st));
-        memcpy(logits_host + at, p.logits_pinned + at, n * 4);
+}
+
+// Behind the head: `floats` logits into the caller's pageable memory by way of a pinned buffer, in up to kLogitPieces pieces of 128 KB or more, so that the host
+// moves one on while the card sends the next.  Everything in front of the copy has run on return.  One launch and flags in place of a copy and an event a
+// piece, each of which the card took up 11 us after the one before (16 rows of 32000, 2 MB: 95 us and the wake-up behind them; a decode step of 16 sequences
+// over two expert layers 419 -> 375 us, of 4 over three layers of latent attention and delta rule 304 -> 284).
+static int plan_fetch_logits(PlanState &p, const float *logits, size_t floats, float *logits_host, hipStream_t st) {
+    const size_t pieces = std::min<size_t>(std::max<size_t>(floats / (32 * 1024), 1), kLogitPieces), each = ((floats + pieces - 1) / pieces + 63) / 64 * 64;
+    const uint32_t stamp = ++p.fetches;
+    hipLaunchKernelGGL(plan_fetch_kernel, dim3(2 * 16), dim3(256), 0, st, logits, p.logits_pinned, floats, each, p.sent, p.arrived, stamp);
+    XFT_CHECK_HIP(hipGetLastError());
+    // the caller's pages come into being while the card works (2 MB of fresh memory: 58 us for the host's copies with them, 38 without)
+    for (size_t at = 0; at < floats * 4; at += 4096) ((volatile char *)logits_host)[at] = 0;
+    // a decode step is waited for with an eye on the flags, a long one the ordinary way
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    bool waited = false;
+    for (size_t i = 0; i * each < floats; ++i) {
+        for (unsigned spins = 1; !waited && __atomic_load_n(p.arrived + 16 * i, __ATOMIC_ACQUIRE) != stamp; ++spins) {
+            __builtin_ia32_pause();
+            if (spins % 256 == 0 && std::chrono::steady_clock::now() > until) {
+                XFT_CHECK_HIP(hipStreamSynchronize(st));
+                waited = true;
+            }
+        }
+        memcpy(logits_host + i * each, p.logits_pinned + i * each, std::min(each, floats - i * each) * 4);
     }
     return 0;
 }
@@ -675,8 +715,6 @@ void plan_state_destroy(PlanState *p) {
     if (p->trace_buf) (void)hipFree(p->trace_buf);
     if (p->desc_host) (void)hipHostFree(p->desc_host);
     if (p->logits_pinned) (void)hipHostFree(p->logits_pinned);
-    for (hipEvent_t e : p->fetched)
-        if (e) (void)hipEventDestroy(e);
     delete p;
 }
 
@@ -1440,8 +1478,12 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
         tables_of(values, &L.cosV, &L.sinV);
     }
     ok = ok && hipHostMalloc((void **)&p->desc_host, (3 * T + 5 * (size_t)max_batch + p->logit_rows + p->table_host.size()) * 4) == hipSuccess
-            && hipHostMalloc((void **)&p->logits_pinned, (size_t)p->logit_rows * plan->cfg.vocab * 4) == hipSuccess;
-    for (hipEvent_t &e : p->fetched) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+            && hipHostMalloc((void **)&p->logits_pinned, ((size_t)p->logit_rows * plan->cfg.vocab + 31) / 32 * 128 + kLogitPieces * 64) == hipSuccess
+            && hipMalloc((void **)&p->sent, kLogitPieces * 4) == hipSuccess;
+    if (p->sent) p->owned.push_back(p->sent);
+    ok = ok && hipMemset(p->sent, 0, kLogitPieces * 4) == hipSuccess;
+    p->arrived = (uint32_t *)(p->logits_pinned + ((size_t)p->logit_rows * plan->cfg.vocab + 31) / 32 * 32);
+    if (ok) memset(p->arrived, 0, kLogitPieces * 64);
     p->dec_host = p->desc_host + 3 * T + 4 * (size_t)max_batch;
     p->want_host = p->dec_host + max_batch;
     p->table_pinned = p->want_host + p->logit_rows;
