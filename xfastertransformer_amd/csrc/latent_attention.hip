@@ -423,18 +423,25 @@ __global__ __launch_bounds__(128) void latent_merge_kernel(MfmaParams p) {
     }
 }
 
-// cache rows of positions [base, base + rows) of a slot, side by side
-__global__ __launch_bounds__(256) void latent_gather_kernel(StepView v, int slot, int base, const uint16_t *pool, int row_len, uint16_t *out) {
-    const size_t src = cache_row(v, slot, base + blockIdx.x) * row_len;
-    for (int c = threadIdx.x * 8; c < row_len; c += 2048) *(u32x4 *)(out + (size_t)blockIdx.x * row_len + c) = *(const u32x4 *)(pool + src + c);
+// cache rows of a group's contexts, side by side; a workgroup takes a row of the result
+__global__ __launch_bounds__(256) void latent_gather_kernel(StepView v, LatentGroup group, const uint16_t *pool, int row_len, uint16_t *out) {
+    int i = 0;
+    while (i + 1 < group.count && group.s[i + 1].at <= (int)blockIdx.x) ++i;
+    const LatentSegment &seg = group.s[i];
+    const int pos = seg.base + (int)blockIdx.x - seg.at;
+    const bool in = pos < seg.start + seg.n;
+    const size_t src = in ? cache_row(v, seg.slot, pos) * row_len : 0;
+    for (int c = threadIdx.x * 8; c < row_len; c += 2048)
+        *(u32x4 *)(out + (size_t)blockIdx.x * row_len + c) = in ? *(const u32x4 *)(pool + src + c) : u32x4 {0, 0, 0, 0};
 }
 
 struct ExpandedParams {
-    const uint16_t *q, *k, *vv, *rows; // queries [T][H][D + RD]; keys [ctx][H D], values [ctx][H V]; cache rows [ctx][R + RD]
+    const uint16_t *q, *k, *vv, *rows; // queries [T][H][D + RD]; keys [rows][H D], values [rows][H V]; cache rows [rows][R + RD]
     uint16_t *out; // [T][H V]
     const float *sink;
-    int off, start, n, base, H, D, RD, V, R, window;
+    int H, D, RD, V, R, window;
     float scale;
+    LatentGroup group;
 };
 
 // BF16, expanded form, for long segments: keys and values of every head made from the latents beforehand.  A workgroup takes
@@ -442,22 +449,28 @@ struct ExpandedParams {
 //   S^T = K Q^T (A = keys from LDS, B = the wave's queries in registers), O^T += V^T P^T (A = values from LDS read
 // transposed, B = probabilities straight from the score registers: half h of the wave holds tokens 8 q + 4 h + s of a block,
 // and the value operand takes its tokens in that order).
-// KSM: most 16-dim steps of a query; VTM: most 32-dim tiles of a value; EXACT: as many.  grid (heads, query blocks)
+// The segments of a step go together, since one alone is too little for the device and ends in a wave of its longest contexts.  A layer of 16 heads,
+// prompts of 940 to 1500 tokens: one by one 287 us (gather 5, products 12 and 12, attention 45 each), together 123 (6, 25, 25, 66); 24 prompts
+// of 24 to 60 tokens, prompt and 8 steps of three layers: 6.6 -> 5.2 ms.
+// KSM: most 16-dim steps of a query; VTM: most 32-dim tiles of a value; EXACT: as many.  grid (heads,
+// segments, query blocks of the longest segment)
 template <int KSM, int VTM, bool EXACT>
 __global__ __launch_bounds__(256, 2) void latent_expanded_kernel(ExpandedParams p) {
     extern __shared__ unsigned char lds[];
+    const LatentSegment seg = p.group.s[blockIdx.y];
+    const int head = blockIdx.x, q0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * 128; // the blocks with the longest contexts first
+    if (q0 >= seg.n) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, cl = lane & 31;
-    const int head = blockIdx.x, q0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * 128; // the blocks with the longest contexts first
     const int Dq = EXACT ? KSM * 16 : p.D + p.RD, ks_n = Dq / 16, V = EXACT ? VTM * 32 : p.V, vt_n = V / 32;
     const int kpitch = Dq * 2 + 16, vpitch = V * 2 + 16, bufb = 32 * (kpitch + vpitch);
     const int qi = q0 + wave * 32 + cl;
-    const int pos = p.start + (qi < p.n ? qi : p.n - 1);
-    const int wlo = p.start + q0 + wave * 32, whi_q = q0 + wave * 32 + 31;
-    const int whi = p.start + (whi_q < p.n ? whi_q : p.n - 1); // last position of the wave's queries
-    const bool wave_on = q0 + wave * 32 < p.n;
+    const int pos = seg.start + (qi < seg.n ? qi : seg.n - 1);
+    const int wlo = seg.start + q0 + wave * 32, whi_q = q0 + wave * 32 + 31;
+    const int whi = seg.start + (whi_q < seg.n ? whi_q : seg.n - 1); // last position of the wave's queries
+    const bool wave_on = q0 + wave * 32 < seg.n;
     bf16x8 qf[KSM];
     {
-        const uint16_t *row = p.q + ((size_t)(p.off + (qi < p.n ? qi : p.n - 1)) * p.H + head) * Dq + 8 * h;
+        const uint16_t *row = p.q + ((size_t)(seg.off + (qi < seg.n ? qi : seg.n - 1)) * p.H + head) * Dq + 8 * h;
 #pragma unroll
         for (int ks = 0; ks < KSM; ++ks)
             if (EXACT || ks < ks_n) qf[ks] = *(const bf16x8 *)(row + ks * 16);
@@ -469,9 +482,9 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_kernel(ExpandedParams 
         for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
     float m = kUnseen, l = 0.0f;
     const float scale2 = p.scale * kLog2e;
-    const int first = p.window > 0 && p.start + q0 + 1 > p.window ? p.start + q0 + 1 - p.window : 0;
-    const int last_q = q0 + 127 < p.n ? q0 + 127 : p.n - 1;
-    const int b0 = first >> 5, b1 = ((p.start + last_q) >> 5) + 1;
+    const int first = p.window > 0 && seg.start + q0 + 1 > p.window ? seg.start + q0 + 1 - p.window : 0;
+    const int last_q = q0 + 127 < seg.n ? q0 + 127 : seg.n - 1;
+    const int b0 = first >> 5, b1 = ((seg.start + last_q) >> 5) + 1;
     const int wfirst = p.window > 0 && wlo + 1 > p.window ? wlo + 1 - p.window : 0;
 
     constexpr int PER = (16 * KSM + 32 * VTM + 63) / 64;
@@ -498,9 +511,10 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_kernel(ExpandedParams 
         }
     }
     // (rows behind the segment's end lie inside the buffers, which hold whole blocks)
+    const int first_row = seg.base - seg.at;
     auto fetch = [&](int blk) {
 #pragma unroll
-        for (int i = 0; i < PER; ++i) stage[i] = *(const u32x4 *)(src[i] + (size_t)(uint32_t)(blk * 32 - p.base) * step[i]);
+        for (int i = 0; i < PER; ++i) stage[i] = *(const u32x4 *)(src[i] + (size_t)(uint32_t)(blk * 32 - first_row) * step[i]);
     };
     fetch(b0);
     int buf = 0;
@@ -567,7 +581,7 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_kernel(ExpandedParams 
         }
     }
     l += __shfl_xor(l, 32, 64);
-    if (qi >= p.n) return;
+    if (qi >= seg.n) return;
     float mul = 1.0f;
     if (p.sink) {
         const float s2 = p.sink[head] * kLog2e, mt = fmaxf(m, s2);
@@ -575,7 +589,7 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_kernel(ExpandedParams 
         l = l * mul + __builtin_amdgcn_exp2f(s2 - mt);
     }
     mul /= l;
-    uint16_t *out = p.out + (size_t)(p.off + qi) * p.H * p.V + (size_t)head * p.V;
+    uint16_t *out = p.out + (size_t)(seg.off + qi) * p.H * p.V + (size_t)head * p.V;
 #pragma unroll
     for (int d = 0; d < VTM; ++d)
         if (EXACT || d < vt_n) {
@@ -700,17 +714,16 @@ bool latent_expanded_takes(int act, const PlanLayer &L, int n, int ctx) {
     return (double)n * ctx * (2.0 * L.R - L.D - L.V) >= (double)(ctx - n) * L.R * (L.D + L.V);
 }
 
-int latent_gather(const StepView &v, int slot, int base, int rows, const LatentCacheView &cache, void *out, hipStream_t st) {
-    hipLaunchKernelGGL(latent_gather_kernel, dim3(rows), dim3(256), 0, st, v, slot, base, (const uint16_t *)cache.pool, cache.R + cache.RD, (uint16_t *)out);
+int latent_gather(const StepView &v, const LatentGroup &group, const LatentCacheView &cache, void *out, hipStream_t st) {
+    hipLaunchKernelGGL(latent_gather_kernel, dim3(group.rows), dim3(256), 0, st, v, group, (const uint16_t *)cache.pool, cache.R + cache.RD, (uint16_t *)out);
     XFT_CHECK_HIP(hipGetLastError());
     return 0;
 }
 
-int latent_expanded(const PlanLayer &L, int off, int start, int n, int base, const void *q, const void *k, const void *values, const void *rows, void *out,
-        hipStream_t st) {
-    const ExpandedParams p = {(const uint16_t *)q, (const uint16_t *)k, (const uint16_t *)values, (const uint16_t *)rows, (uint16_t *)out, L.sink, off, start, n,
-            base, L.s.heads, L.D, L.RD, L.V, L.R, L.s.window, L.s.scale};
-    const dim3 grid(L.s.heads, (n + 127) / 128);
+int latent_expanded(const PlanLayer &L, const LatentGroup &group, const void *q, const void *k, const void *values, const void *rows, void *out, hipStream_t st) {
+    const ExpandedParams p = {(const uint16_t *)q, (const uint16_t *)k, (const uint16_t *)values, (const uint16_t *)rows, (uint16_t *)out, L.sink, L.s.heads, L.D,
+            L.RD, L.V, L.R, L.s.window, L.s.scale, group};
+    const dim3 grid(L.s.heads, group.count, (group.longest + 127) / 128);
     const size_t smem = (size_t)2 * 32 * ((L.D + L.RD) * 2 + 16 + L.V * 2 + 16);
     const int ks = (L.D + L.RD) / 16, vt = L.V / 32;
     if (ks == 12 && vt == 4) return launch_expanded<12, 4, true>(p, grid, smem, st);

@@ -251,12 +251,20 @@ int latent_split_count(const PlanLayer &L, int B, int longest, int hint);
 size_t latent_part_floats(const PlanLayer &L);
 // expanded form: should a segment of n tokens that ends at position ctx take it
 bool latent_expanded_takes(int act, const PlanLayer &L, int n, int ctx);
-// cache rows of positions base .. base + rows - 1 of a slot -> out [rows][R + RD]
-int latent_gather(const StepView &v, int slot, int base, int rows, const LatentCacheView &cache, void *out, hipStream_t st);
-// one segment: tokens off .. off + n - 1 of the step at positions start .., q [T][heads][D + RD]; keys [ctx][heads D], values
-// [ctx][heads V] and gathered cache rows of the positions from base (a multiple of 32) on, whole blocks of 32; out [T][heads V]
-int latent_expanded(const PlanLayer &L, int off, int start, int n, int base, const void *q, const void *k, const void *values, const void *rows, void *out,
-        hipStream_t st);
+// Long segments that take the expanded form together: token off .. off + n - 1 of the step at positions start ..; the context from
+// position base (a multiple of 32) on lies in rows at .. of the gathered buffers, whole blocks of 32 side by side.
+struct LatentSegment {
+    int slot, off, start, n, base, at;
+};
+constexpr int kLatentGroup = 32; // (by value to the kernels: 24 bytes each of the 4 KB of arguments)
+struct LatentGroup {
+    int count = 0, rows = 0, longest = 0; // segments, gathered rows, tokens of the longest one
+    LatentSegment s[kLatentGroup];
+};
+// cache rows of the group's contexts -> out [rows][R + RD]; rows behind a context's end become zero
+int latent_gather(const StepView &v, const LatentGroup &group, const LatentCacheView &cache, void *out, hipStream_t st);
+// q [T][heads][D + RD]; keys [rows][heads D], values [rows][heads V] and gathered cache rows; out [T][heads V]
+int latent_expanded(const PlanLayer &L, const LatentGroup &group, const void *q, const void *k, const void *values, const void *rows, void *out, hipStream_t st);
 
 struct DeltaBuffers {
     void *in; // rows of the input product, of the activation type: q | k | v | beta | decay (rank) | gate (rank) from in_col on
@@ -376,7 +384,8 @@ struct PlanState {
     float *router_logits = nullptr, *expert_out = nullptr, *side_z = nullptr;
     void *eh = nullptr;
     RouteBuffers route {};
-    void *rows = nullptr, *kx = nullptr, *vx = nullptr; // gathered latents, keys and values of a long segment's context
+    void *rows = nullptr, *kx = nullptr, *vx = nullptr; // gathered latents, keys and values of long segments' contexts: context_rows rows
+    int context_rows = 0;
     float *part = nullptr; // split contexts
     size_t part_floats = 0;
     std::vector<void *> owned; // every device buffer above

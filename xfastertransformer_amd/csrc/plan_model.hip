@@ -157,7 +157,8 @@ int run_latent(xfthip_model *m, const PlanLayer &L, int run, const StepView &v, 
     if ((rc = latent_prepare(act, L, v, p.a, p.cq, cache, m->cfg.rms_eps, st))) return rc;
     if ((rc = plan_gemm(m, L.uq, T, p.cq, L.QR, p.q, qcols, act, st))) return rc;
     if ((rc = latent_rotate_q(act, L, v, p.q, st))) return rc;
-    // long segments one by one in the expanded form; the others, as far as they are neighbours, together in the absorbed one
+    // Long segments in the expanded form, as many together as the buffers hold; the others, as far as they are neighbours,
+    // together in the absorbed one.
     const size_t B = p.seg_len_host.size();
     const char *q = (const char *)p.q;
     int longest = 0, short_from = -1;
@@ -170,6 +171,17 @@ int run_latent(xfthip_model *m, const PlanLayer &L, int run, const StepView &v, 
                 (char *)p.ov + (size_t)from * H * L.V * p.esz, H * L.V, act, st);
     };
     std::vector<std::pair<int, int>> spans; // token ranges of the absorbed form
+    LatentGroup group;
+    auto expand_group = [&]() -> int {
+        const int rows = group.rows;
+        if (!group.count) return 0;
+        if (int rc = latent_gather(v, group, cache, p.rows, st)) return rc;
+        if (int rc = xfthip_gemm(L.uk, rows, p.rows, L.R + L.RD, p.kx, H * L.D, XFTHIP_BF16, XFTHIP_EPI_NONE, nullptr, nullptr, 0, XFTHIP_F32, 1.0f, st)) return rc;
+        if (int rc = xfthip_gemm(L.uv, rows, p.rows, L.R + L.RD, p.vx, H * L.V, XFTHIP_BF16, XFTHIP_EPI_NONE, nullptr, nullptr, 0, XFTHIP_F32, 1.0f, st)) return rc;
+        if (int rc = latent_expanded(L, group, p.q, p.kx, p.vx, p.rows, p.ov, st)) return rc;
+        group.count = group.rows = group.longest = 0;
+        return 0;
+    };
     for (size_t i = 0; i < B; ++i) {
         const int n = p.seg_len_host[i], off = p.seg_off_host[i], start = p.seg_pos_host[i];
         const int from = L.s.window > 0 && start + 1 > L.s.window ? (start + 1 - L.s.window) & ~31 : 0, rows = start + n - from;
@@ -183,11 +195,12 @@ int run_latent(xfthip_model *m, const PlanLayer &L, int run, const StepView &v, 
             short_from = -1;
         }
         if (!expand) continue;
-        if ((rc = latent_gather(v, p.seg_row_host[i], from, rows, cache, p.rows, st))) return rc;
-        if ((rc = xfthip_gemm(L.uk, rows, p.rows, L.R + L.RD, p.kx, H * L.D, XFTHIP_BF16, XFTHIP_EPI_NONE, nullptr, nullptr, 0, XFTHIP_F32, 1.0f, st))) return rc;
-        if ((rc = xfthip_gemm(L.uv, rows, p.rows, L.R + L.RD, p.vx, H * L.V, XFTHIP_BF16, XFTHIP_EPI_NONE, nullptr, nullptr, 0, XFTHIP_F32, 1.0f, st))) return rc;
-        if ((rc = latent_expanded(L, off, start, n, from, p.q, p.kx, p.vx, p.rows, p.ov, st))) return rc;
+        const int held = (int)pad32(rows);
+        if ((group.count == kLatentGroup || group.rows + held > p.context_rows) && (rc = expand_group())) return rc;
+        group.s[group.count++] = {p.seg_row_host[i], off, start, n, from, group.rows};
+        group.rows += held, group.longest = std::max(group.longest, n);
     }
+    if ((rc = expand_group())) return rc;
     if (!spans.empty()) {
         for (auto &s : spans)
             if ((rc = absorb(s.first, s.second))) return rc;
@@ -1417,14 +1430,14 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
     alloc(&p->router_logits, T * routes * 4), alloc(&p->eh, T * eh * e), alloc(&p->expert_out, T * eo * 4);
     alloc(&p->route.sel, T * top * 4), alloc(&p->route.weight, T * top * 4), alloc(&p->route.slot_row, T * top * 4), alloc(&p->route.row_token, T * top * 4);
     alloc(&p->route.group_rows, experts * 12);
-    // the expanded form's context (whole blocks of 32 tokens; cleared: rows behind the end meet zero weights)
+    // the expanded form's contexts, in whole blocks of 32 tokens: at least the longest one's, and as many as a pass of fresh prompts has
     if (act_dtype == XFTHIP_BF16 && max_tokens >= 32) {
-        const size_t ctx = pad32(max_seq) + 32;
+        const size_t ctx = std::max<size_t>(pad32(max_seq) + 32, std::min<size_t>(T + 31 * (size_t)std::min(max_batch, kLatentGroup), (size_t)max_batch * (pad32(max_seq) + 32)));
         size_t kx = 0, vx = 0, rl = 0;
         for (const PlanLayer &L : p->layers)
             if (L.s.mixer == XFTHIP_MIXER_LATENT && latent_expanded_takes(act_dtype, L, 1 << 20, 1 << 20))
                 kx = std::max(kx, (size_t)L.s.heads * L.D), vx = std::max(vx, (size_t)L.s.heads * L.V), rl = std::max(rl, (size_t)(L.R + L.RD));
-        if (kx) alloc(&p->rows, ctx * rl * e, true), alloc(&p->kx, ctx * kx * e, true), alloc(&p->vx, ctx * vx * e, true);
+        if (kx) alloc(&p->rows, ctx * rl * e, true), alloc(&p->kx, ctx * kx * e, true), alloc(&p->vx, ctx * vx * e, true), p->context_rows = (int)ctx;
     }
     for (const PlanLayer &L : p->layers) {
         if (L.s.mixer == XFTHIP_MIXER_LATENT) p->part_floats = std::max(p->part_floats, latent_part_floats(L));
