@@ -246,20 +246,24 @@ struct ScanParams {
 // rows run side by side and the read-out needs none of its own.  q, k, g of CT tokens are staged in LDS, the next CT on
 // their way through registers.  grid (segments, heads, column groups of COLS).
 // ONE: one decay a head, a scalar beside beta.
-// One prompt of 32 heads is one wave a SIMD: the time is about 75 vector instructions a token and the latency of the
-// reductions in them.  (KD = 128 as 32 lanes x 4 rows x 2 columns, half the LDS reads: 510 us for 2048 tokens against 440 as
-// 16 x 8 x 1.)
+// What bounds it is the issue of instructions and, with few waves, their latency: four multiply-adds and less than one LDS read a state value.  So whatever
+// else a token needs is kept small: the tokens of a full chunk are straight-line code whose LDS reads carry their offsets and go out a token ahead of
+// their use; the read-outs' sums over the lanes, which nothing waits for, are left in LDS and added up for CT tokens at once, where a sum across the
+// lanes was as many instructions as the one that the chain needs; the last half of the column groups walk the segments backwards, so that an XCD and a CU
+// (which take every 8th and every 256th workgroup) get long and short ones.  16 heads of 128 x 128, before and after: two prompts of 3000 tokens
+// at most 690 / 600 us, four of 940 to 1500 420 / 350, eight of 800 at most 404 / 272, 16 of 400 346 / 230, 24 of 500 600 / 520.
+// (KD = 128 as 32 lanes x 4 rows x 2 columns, half the LDS reads: 510 us for 2048 tokens against 440 as 16 x 8 x 1.)
 template <int L, int RV, int C, bool ONE>
 __global__ __launch_bounds__(256) void delta_scan_kernel(ScanParams p) {
-    constexpr int KD = 4 * L * RV, GROUPS = 256 / L, COLS = GROUPS * C, CT = KD > 128 ? 8 : 16;
+    constexpr int KD = 4 * L * RV, GROUPS = 256 / L, COLS = GROUPS * C, CT = 8;
     constexpr int CHUNK4 = CT * KD / 4; // float4 of one array and chunk
     constexpr int ARRAYS = ONE ? 2 : 3, SCALARS = ONE ? 3 : 2; // q, k(, g); beta, q . k(, g)
     constexpr int PER = (ARRAYS * CHUNK4 + 255) / 256, PERV = (CT * COLS + 255) / 256;
     __shared__ float lds[2][ARRAYS * CT * KD];
     __shared__ float vlds[2][CT * COLS];
     __shared__ float sc[2][SCALARS * CT];
-    __shared__ float olds[2][CT * COLS];
-    const int seg = blockIdx.x, head = blockIdx.y, kvh = head / (p.H / p.KH);
+    __shared__ f32x4 sums[CT * COLS * L / 4]; // the lanes' parts of the read-outs: [token][c][column group][lane]
+    const int seg = 2 * blockIdx.z < gridDim.z ? blockIdx.x : gridDim.x - 1 - blockIdx.x, head = blockIdx.y, kvh = head / (p.H / p.KH);
     const int n = p.v.seg_len[seg], off = p.v.seg_off[seg];
     const int li = threadIdx.x % L, lc = threadIdx.x / L * C;
     const int col0 = blockIdx.z * COLS, col = col0 + lc;
@@ -318,6 +322,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(ScanParams p) {
         const int m = n - c0 < CT ? n - c0 : CT;
         if (c0 + CT < n) fetch(c0 + CT);
         const float *lq = lds[buf] + 4 * li;
+        float *part = (float *)sums + threadIdx.x;
         struct Operands {
             f32x4 q[RV], k[RV], g[ONE ? 1 : RV];
             float v[C], beta, qk, fade;
@@ -338,7 +343,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(ScanParams p) {
         };
         // the operands of the next token are on their way from LDS while this one's sums go round
         auto token = [&](const Operands &x, int i) {
-            float a[C], b[C], u[C];
+            float a[C], b[C];
 #pragma unroll
             for (int c = 0; c < C; ++c) {
                 a[c] = b[c] = 0.0f;
@@ -352,34 +357,56 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(ScanParams p) {
                     }
             }
 #pragma unroll
-            for (int c = 0; c < C; ++c) a[c] = group_sum<L>(a[c]), b[c] = group_sum<L>(b[c]);
+            for (int c = 0; c < C; ++c) a[c] = group_sum<L>(a[c]);
 #pragma unroll
             for (int c = 0; c < C; ++c) {
-                u[c] = x.beta * (x.v[c] - a[c]);
+                const float u = x.beta * (x.v[c] - a[c]);
 #pragma unroll
                 for (int r = 0; r < RV; ++r)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) s[c][r][e] = fmaf(x.k[r][e], u[c], s[c][r][e]);
-            }
-            if (li == 0) {
-#pragma unroll
-                for (int c = 0; c < C; ++c) olds[buf][i * COLS + lc + c] = fmaf(x.qk, u[c], b[c]);
+                    for (int e = 0; e < 4; ++e) s[c][r][e] = fmaf(x.k[r][e], u, s[c][r][e]);
+                const float with = fmaf(x.qk, u, b[c]);
+                part[(i * C + c) * 256] = li == 0 ? with : b[c];
             }
         };
         Operands even = read(0), odd;
-        for (int i = 0; i < m; i += 2) {
-            odd = read(i + 1 < m ? i + 1 : i);
-            token(even, i);
-            if (i + 1 >= m) break;
-            even = read(i + 2 < m ? i + 2 : i + 1);
-            token(odd, i + 1);
+        if (m == CT) {
+#pragma unroll
+            for (int i = 0; i < CT; i += 2) {
+                odd = read(i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                token(even, i);
+                __builtin_amdgcn_sched_barrier(0);
+                if (i + 2 < CT) even = read(i + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                token(odd, i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            for (int i = 0; i < m; ++i) {
+                token(even, i);
+                even = read(i + 1 < m ? i + 1 : i);
+            }
         }
-        if (c0 + CT < n) stash(buf ^ 1); // (the other buffer, and the other results, were last read before or behind this barrier one chunk ago)
+        if (c0 + CT < n) stash(buf ^ 1); // (that buffer was last read in front of the barrier one chunk ago)
+        // The read-outs of a wave's own columns: written and read by the same wave, whose LDS accesses keep their order.  64 / L column groups a wave.
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        constexpr int WG = 64 / L, OUTS = CT * C * WG;
+#pragma unroll
+        for (int o0 = 0; o0 < OUTS; o0 += 64) {
+            const int o = o0 + (threadIdx.x & 63), i = o / (C * WG), at = o % (C * WG), c = at % C, gr = (threadIdx.x >> 6) * WG + at / C;
+            if (i >= m) continue;
+            const f32x4 *x = sums + ((i * C + c) * GROUPS + gr) * (L / 4);
+            f32x4 y = x[(o >> 2) % (L / 4)]; // (lanes begin at different quarters: at the same one they would share banks)
+#pragma unroll
+            for (int r = 1; r < L / 4; ++r) y += x[(r + (o >> 2)) % (L / 4)];
+            const int vc = col0 + gr * C + c;
+            if (vc < p.VD) p.b.o[((size_t)(off + c0 + i) * p.H + head) * p.VD + vc] = (y[0] + y[1]) + (y[2] + y[3]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         __syncthreads();
-        for (int e = threadIdx.x; e < m * COLS; e += 256) {
-            const int c = col0 + e % COLS;
-            if (c < p.VD) p.b.o[((size_t)(off + c0 + e / COLS) * p.H + head) * p.VD + c] = olds[buf][e];
-        }
     }
     if (own) {
 #pragma unroll
@@ -533,14 +560,18 @@ int conv_tail(int act, const StepView &v, const void *in, int ld, int channels, 
 int delta_scan(const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st) {
     ScanParams p;
     p.v = v, p.b = b, p.H = L.s.heads, p.KH = L.s.kv_heads, p.VD = L.VD;
-    const int lanes = L.KD / 8, cols = 256 / lanes;
+    const int lanes = L.KD / 8;
     const bool one = L.head_decay();
+    // Two columns a group of lanes where one would make four waves a SIMD or more: below, the columns' chains are better hidden by each other's waves.  16
+    // heads of 128 x 128, one column / two: 4 prompts of 1500 tokens 350 / 407 us, 6 of 1000 308 / 368, 8 of 800 308 / 272, 24 of 500 650 / 510.
+    const bool two = v.longest > 1 && lanes >= 8 && L.VD % (512 / lanes) == 0 && (long)v.B * p.H * L.VD * lanes >= (long)device_cu_count() * 1024;
+    const int cols = (two ? 512 : 256) / lanes;
     const dim3 grid(v.B, p.H, (L.VD + cols - 1) / cols);
     auto launch = [&](auto several, auto single) {
         if (one) hipLaunchKernelGGL(single, grid, dim3(256), 0, st, p);
         else hipLaunchKernelGGL(several, grid, dim3(256), 0, st, p);
     };
-    const int key = (v.longest == 1 ? 0 : 1000) + L.KD; // (both forms: 256 / lanes columns a workgroup)
+    const int key = (v.longest == 1 ? 0 : two ? 2000 : 1000) + L.KD;
     switch (key) {
         case 32: launch(delta_step_kernel<4, false>, delta_step_kernel<4, true>); break;
         case 64: launch(delta_step_kernel<8, false>, delta_step_kernel<8, true>); break;
@@ -550,6 +581,9 @@ int delta_scan(const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hip
         case 1064: launch(delta_scan_kernel<8, 2, 1, false>, delta_scan_kernel<8, 2, 1, true>); break;
         case 1128: launch(delta_scan_kernel<16, 2, 1, false>, delta_scan_kernel<16, 2, 1, true>); break;
         case 1256: launch(delta_scan_kernel<32, 2, 1, false>, delta_scan_kernel<32, 2, 1, true>); break;
+        case 2064: launch(delta_scan_kernel<8, 2, 2, false>, delta_scan_kernel<8, 2, 2, true>); break;
+        case 2128: launch(delta_scan_kernel<16, 2, 2, false>, delta_scan_kernel<16, 2, 2, true>); break;
+        case 2256: launch(delta_scan_kernel<32, 2, 2, false>, delta_scan_kernel<32, 2, 2, true>); break;
         default: set_error("delta_scan: key dimension %d of a head is above 256", L.s.dim); return 2;
     }
     XFT_CHECK_HIP(hipGetLastError());
