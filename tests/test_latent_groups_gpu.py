@@ -43,3 +43,13 @@ def test_more_segments_than_a_group():
     lengths = [int(n) for n in rng.integers(32, 41, 70)]
     steps(c, [rng.integers(0, cfg["vocab"], n) for n in lengths], [lengths])
     c.free()
+
+
+@pytest.mark.parametrize("tokens,heads,kv_rank,batch", [(n, 3, 512, 1) for n in (40, 200, 400, 700, 1300, 2500)] + [(n, 40, 40, 2) for n in (40, 200, 700)])
+def test_splits_of_a_context(tokens, heads, kv_rank, batch):
+    """One new token behind contexts of 2 to 64 splits: each number of thread groups that share them in the merge, one column group and two."""
+    cfg, c = case_of([u.latent(heads=heads, kv_rank=kv_rank)], batch, 2560, batch * tokens)
+    rng = np.random.default_rng(tokens)
+    lengths = [tokens - 31 * i // 2 for i in range(batch)]
+    steps(c, [rng.integers(0, cfg["vocab"], n + 1) for n in lengths], [lengths, [n + 1 for n in lengths]])
+    c.free()
