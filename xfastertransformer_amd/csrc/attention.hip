@@ -40,6 +40,14 @@ __global__ __launch_bounds__(256, 3) void attn_kernel(AttnParams p) {
     attn_unit<INT8, 4, PIPE>(p, blockIdx.x, blockIdx.y % p.kv.H, blockIdx.y / p.kv.H, blockIdx.z, lds, [] { __syncthreads(); });
 }
 
+// Short contexts: one workgroup of 8 waves, nothing split.  The hand-over between the workgroups of a split (publish, ticket, read back) is three round
+// trips to memory, which two blocks more a wave do not cost.
+template <bool INT8>
+__global__ __launch_bounds__(512) void attn_short_kernel(AttnParams p) {
+    __shared__ AttnLds<8> lds;
+    attn_unit<INT8, 8, false>(p, 0, blockIdx.x % p.kv.H, blockIdx.x / p.kv.H, blockIdx.y, lds, [] { __syncthreads(); });
+}
+
 constexpr int kTicketParts = 8, kMaxParts = 32;
 // merges the parts of a launch of attn_kernel that took no tickets: grid (columns of a group, groups), at most 128 parts
 __global__ __launch_bounds__(128) void attn_merge_kernel(AttnParams p) {
@@ -175,6 +183,18 @@ int xfthip::attention_launch(xfthip_kvcache_t c, const void *q, int qStride, voi
     const int len = past_dev ? ((len_hint > 0 && len_hint < c->maxSeq) ? len_hint : c->maxSeq) : past + S;
     const int wgs = B * c->kv.H * p.CG;
     int nsplit = attention_split_count(len, wgs);
+    // Up to 320 tokens, and 384 of a cache half as large or with several query heads a KV head, 8 waves of one workgroup are faster than the parts of a
+    // split and their merge; beyond, a CU's own path to the L2 takes longer than the merge.  FP16, one sequence, 32 KV heads, 176 / 256 / 320 / 512 tokens:
+    // split 7.4 / 7.6 / 7.7 / 8.0 us, so 6.1 / 6.8 / 7.4 / 9.2; 8 KV heads of 32: 8.5 / 8.9 / 9.0 / 9.2 and 6.5 / 7.1 / 7.8 / 9.6; INT8, 32 KV heads: 7.3
+    // / 7.5 / 7.5 / 7.8 and 6.1 / 6.3 / 7.0 / 8.7, at 384 7.5 and 7.1.
+    if (nsplit > 1 && len <= (c->kv.int8 || p.G > 1 ? 384 : 320)) {
+        p.nsplit = 1;
+        const dim3 grid(c->kv.H * p.CG, B);
+        if (c->kv.int8) hipLaunchKernelGGL(attn_short_kernel<true>, grid, dim3(512), 0, stream, p);
+        else hipLaunchKernelGGL(attn_short_kernel<false>, grid, dim3(512), 0, stream, p);
+        XFT_CHECK_HIP(hipGetLastError());
+        return 0;
+    }
     AttnWorkspace of_stream;
     if (nsplit > 1) {
         if (wsp == nullptr) {
