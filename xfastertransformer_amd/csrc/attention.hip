@@ -183,18 +183,6 @@ int xfthip::attention_launch(xfthip_kvcache_t c, const void *q, int qStride, voi
     const int len = past_dev ? ((len_hint > 0 && len_hint < c->maxSeq) ? len_hint : c->maxSeq) : past + S;
     const int wgs = B * c->kv.H * p.CG;
     int nsplit = attention_split_count(len, wgs);
-    // Up to 320 tokens, and 384 of a cache half as large or with several query heads a KV head, 8 waves of one workgroup are faster than the parts of a
-    // split and their merge; beyond, a CU's own path to the L2 takes longer than the merge.  FP16, one sequence, 32 KV heads, 176 / 256 / 320 / 512 tokens:
-    // split 7.4 / 7.6 / 7.7 / 8.0 us, so 6.1 / 6.8 / 7.4 / 9.2; 8 KV heads of 32: 8.5 / 8.9 / 9.0 / 9.2 and 6.5 / 7.1 / 7.8 / 9.6; INT8, 32 KV heads: 7.3
-    // / 7.5 / 7.5 / 7.8 and 6.1 / 6.3 / 7.0 / 8.7, at 384 7.5 and 7.1.
-    if (nsplit > 1 && len <= (c->kv.int8 || p.G > 1 ? 384 : 320)) {
-        p.nsplit = 1;
-        const dim3 grid(c->kv.H * p.CG, B);
-        if (c->kv.int8) hipLaunchKernelGGL(attn_short_kernel<true>, grid, dim3(512), 0, stream, p);
-        else hipLaunchKernelGGL(attn_short_kernel<false>, grid, dim3(512), 0, stream, p);
-        XFT_CHECK_HIP(hipGetLastError());
-        return 0;
-    }
     AttnWorkspace of_stream;
     if (nsplit > 1) {
         if (wsp == nullptr) {
@@ -208,6 +196,15 @@ int xfthip::attention_launch(xfthip_kvcache_t c, const void *q, int qStride, voi
                     wgs, nsplit, (size_t)wgs * nsplit, wsp->slots);
             while (nsplit > 1 && (size_t)wgs * nsplit > (size_t)wsp->slots) --nsplit;
         }
+    }
+    // (Behind the workspace all the same: a stream's first call takes it, so that a longer one can be captured later.)
+    if (attention_short(c->kv.int8, p.G, len, nsplit)) {
+        p.nsplit = 1;
+        const dim3 grid(c->kv.H * p.CG, B);
+        if (c->kv.int8) hipLaunchKernelGGL(attn_short_kernel<true>, grid, dim3(512), 0, stream, p);
+        else hipLaunchKernelGGL(attn_short_kernel<false>, grid, dim3(512), 0, stream, p);
+        XFT_CHECK_HIP(hipGetLastError());
+        return 0;
     }
     p.nsplit = nsplit;
     p.ws = wsp ? wsp->ws : nullptr;
@@ -231,6 +228,14 @@ int xfthip::attention_launch(xfthip_kvcache_t c, const void *q, int qStride, voi
     }
     XFT_CHECK_HIP(hipGetLastError());
     return 0;
+}
+
+bool xfthip::attention_short(bool int8, int G, int len, int nsplit) {
+    // Up to 320 tokens, and 384 of a cache half as large or with several query heads a KV head, 8 waves of one workgroup are faster than the parts of a
+    // split and their merge; beyond, a CU's own path to the L2 takes longer than the merge.  FP16, one sequence, 32 KV heads, 176 / 256 / 320 / 512 tokens:
+    // split 7.4 / 7.6 / 7.7 / 8.0 us, so 6.1 / 6.8 / 7.4 / 9.2; 8 KV heads of 32: 8.5 / 8.9 / 9.0 / 9.2 and 6.5 / 7.1 / 7.8 / 9.6; INT8, 32 KV heads: 7.3
+    // / 7.5 / 7.5 / 7.8 and 6.1 / 6.3 / 7.0 / 8.7, at 384 7.5 and 7.1.
+    return nsplit > 1 && len <= (int8 || G > 1 ? 384 : 320);
 }
 
 int xfthip::attention_split_count(int len, int units) {

@@ -201,6 +201,8 @@ int attention_launch(xfthip_kvcache_t c, const void *q, int qStride, void *out, 
         bool strict = false);
 // the split count the launch picks for `units` (batch x kv head x column group) workgroups
 int attention_split_count(int len, int units);
+// whether, instead of `nsplit` parts, one workgroup of 8 waves takes the visible sequence; G query heads a KV head
+bool attention_short(bool int8, int G, int len, int nsplit);
 
 } // namespace xfthip
 

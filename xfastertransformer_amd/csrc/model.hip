@@ -789,7 +789,9 @@ int xfthip_model_decode(xfthip_model_t m, int steps, int *ids_out_host, xfthip_s
         }
         if (int rc = plan_decode_begin(m, steps, st)) return rc;
     }
-    const int nsplit = m->plan ? plan_decode_splits(m, B, hint) : attention_split_count(hint, B * c.kv_heads);
+    int nsplit = m->plan ? plan_decode_splits(m, B, hint) : attention_split_count(hint, B * c.kv_heads);
+    // (the same count may stand for both forms: 256 and 1500 tokens of four sequences, 32 KV heads)
+    if (!m->plan && attention_short(c.kv_dtype == XFTHIP_INT8, c.q_heads / c.kv_heads, hint, nsplit)) nsplit = 0;
     if (!m->use_graph) {
         for (int i = 0; i < steps; ++i)
             if (int rc = decode_step(m, B, st)) return rc;

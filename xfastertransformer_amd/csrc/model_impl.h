@@ -66,7 +66,7 @@ struct xfthip_model {
     int *reorder_rows = nullptr; // device [2 * max_batch]: source rows, destination rows
     hipGraphExec_t graph = nullptr;
     int graph_B = 0;
-    int graph_nsplit = 0; // attention split count the captured step was built with
+    int graph_nsplit = -1; // attention split count the captured step was built with (0: the form for short contexts)
     bool graph_ragged = false; // the captured step's last node holds the `active` mask only in this mode
     int len_hint = 0; // upper bound of the sequence length during the current decode call (0 = unknown)
     hipStream_t graph_stream = nullptr;
