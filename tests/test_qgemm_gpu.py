@@ -209,6 +209,13 @@ def test_few_rows_every_form_against_64_bits(xh, orc, kind, M, K, N):
     test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N)
 
 
+@pytest.mark.parametrize("M", [1, 4, 5, 16])
+@pytest.mark.parametrize("K,N", [(128, 40), (256, 40), (384, 16), (640, 4096), (5632, 2048)])
+def test_bf16_tiles_alone_on_their_cu_against_64_bits(xh, orc, M, K, N):
+    """One to four K slices, of as many load batches and not."""
+    test_mfma_every_tile_against_64_bits(xh, orc, "bf16", M, K, N)
+
+
 GATE_UP = [(3, 768, 1040), (13, 768, 14336), (29, 768, 9232), (29, 768, 18448), (100, 1024, 1040), (700, 2048, 2064), (1285, 4096, 2064), (2100, 1024, 3088),
            (23, 128, 16), (2, 128, 17392), (12, 128, 17408), (1966, 13312, 1280)]
 

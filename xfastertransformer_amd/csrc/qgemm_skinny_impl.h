@@ -726,7 +726,10 @@ static int launch_form(const SkinnyParams &p, hipStream_t stream) {
     constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4;
     const SkinnyForm f = skinny_form(KIND, p);
     switch (f.nt) {
-        case 1: return launch<KIND, 1, MT, skinny_batch(KIND, MT, GROUP, 1), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
+        case 1:
+            if constexpr (KIND == XFTHIP_W_BF16 && MT == 1 && !GROUP)
+                if (f.u == 4) return launch<KIND, 1, MT, 4, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+            return launch<KIND, 1, MT, skinny_batch(KIND, MT, GROUP, 1), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
         case 2: return launch<KIND, 2, MT, skinny_batch(KIND, MT, GROUP, 2), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
         case 3:
             if constexpr (!GROUP && (MT == 2 || KIND != XFTHIP_W_BF16))
