@@ -1,4 +1,4 @@
-"""Prompts over the FP16 cache in the form for many columns (128 (token, head) columns a workgroup, 32 a wave): partly filled workgroups and waves, blocks that
+"""Prompts over both caches in the form for many columns (128 (token, head) columns a workgroup, 32 a wave): partly filled workgroups and waves, blocks that
 only some waves see, every way the results leave by, and scores at the ends of the range."""
 import ctypes as C
 
@@ -23,14 +23,14 @@ def orc():
     return pyoracle
 
 
-def _cache(xh, orc, k, v):
+def _cache(xh, orc, k, v, int8=0):
     """k, v: [B, tokens, H * D]"""
     B, n, w = k.shape
-    kc, vc = orc.KVCache(0, B, w // D, n, D), orc.KVCache(0, B, w // D, n, D)
+    kc, vc = orc.KVCache(int8, B, w // D, n, D), orc.KVCache(int8, B, w // D, n, D)
     for b in range(B):
         kc.store(b, 0, k[b])
         vc.store(b, 0, v[b])
-    dc = xh.KVCache(xh.FP16, B, w // D, n, D)
+    dc = xh.KVCache(xh.INT8 if int8 else xh.FP16, B, w // D, n, D)
     dc.load(0, kc.data, kc.scales)
     dc.load(1, vc.data, vc.scales)
     return kc, vc, dc
@@ -105,4 +105,34 @@ def test_scores_at_the_ends_of_the_range(xh, orc, score):
             assert np.abs(got[i] - ref).max() < 3e-3, (i, np.abs(got[i] - ref).max())
     # (a token of the same 32-token block takes part with a weight of zero: only the queries of earlier blocks are sure to be free of it)
     assert np.isfinite(got[41:576]).all() and np.isnan(got[S - 1]).any()
+    dc.free()
+
+
+@pytest.mark.parametrize("B,S,past,qh,kvh,kind,extra,skip", [
+    (1, 512, 0, 32, 8, "bf16", 0, 0),
+    (1, 521, 0, 32, 8, "bf16", 8, 8),
+    (1, 517, 31, 32, 8, "bf16", 1, 1),
+    (2, 300, 1, 32, 8, "f32", 4, 0),
+    (16, 33, 0, 32, 32, "bf16", 0, 0),  # two blocks, the second with one token
+    (33, 31, 0, 32, 32, "f32", 0, 0),  # a single block
+    (12, 65, 0, 32, 32, "bf16", 4, 4),  # three
+    (40, 2, 700, 32, 1, "bf16", 0, 0),
+    (5, 129, 64, 28, 4, "bf16", 8, 0),
+])
+@pytest.mark.parametrize("spread", [0, 1])
+def test_int8_cache(xh, orc, B, S, past, qh, kvh, kind, extra, skip, spread):
+    """spread: the values' sizes go up and down by powers of ten from token to token and block to block, so that the scale they are taken relative to moves."""
+    rng = np.random.default_rng(S * 37 + past)
+    n = past + S
+    k, v = (rng.standard_normal((B, n, kvh * D)).astype(np.float32) for _ in range(2))
+    if spread:
+        v *= (10.0 ** (-rng.integers(0, 3, n) - 2.0 * ((np.arange(n) // 48) % 3)))[None, :, None].astype(np.float32)
+        v[:, n // 2] *= 1e3
+    kc, vc, dc = _cache(xh, orc, k, v, 1)
+    q = orc.round_bf16(rng.standard_normal((B * S, qh * D)))
+    got = _attend(xh, orc, dc, q, B, S, qh, past, xh.BF16 if kind == "bf16" else xh.F32, qh * D + extra, skip)
+    ref = orc.attention_ref_f64(q, kc.as_f32(), vc.as_f32(), qh, kvh, D, [S] * B, [past] * B, SCALE)
+    # fp16 products of probabilities and scales: 2^-11 of a value each, or 2^-25 of 2^8 times the largest scale's; bf16 results 2^-9 on top
+    size = np.abs(vc.as_f32()).max()
+    assert (np.abs(got - ref) <= 6e-4 * max(size, 1.0) + 3e-3 + np.abs(ref) * (2.0 ** -8 if kind == "bf16" else 0.0)).all(), np.abs(got - ref).max()
     dc.free()

@@ -62,12 +62,11 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(AttnParams p) {
 // two pairs' keys and values in its L2 instead of all of them.
 template <bool INT8>
 __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(AttnParams p, int ncg, int npairs) {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[INT8 ? 2 * kP32BufBytes : kRingLds];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[INT8 ? kRingLdsInt8 : kRingLds];
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     const int pair = (slot / ncg) * 8 + xcd;
     if (pair >= npairs) return;
-    if constexpr (INT8) attn_prefill32_unit<4>(p, pair % p.kv.H, ncg - 1 - slot % ncg, pair / p.kv.H, lds);
-    else attn_prefill_ring_unit(p, pair % p.kv.H, ncg - 1 - slot % ncg, pair / p.kv.H, lds);
+    attn_prefill_ring_unit<INT8>(p, pair % p.kv.H, ncg - 1 - slot % ncg, pair / p.kv.H, lds);
 }
 
 // Split-KV merge workspace: `slots` partial-result slots of kSlotFloats floats and one ticket per

@@ -509,12 +509,4 @@ __device__ inline float swap32(float x) { // value of lane ^ 32
     return __uint_as_float(hi ? r[0] : r[1]);
 }
 
-
-// ---- prefill: many columns per (sequence, KV head), K / V blocks shared through LDS (attention_prefill.h) -----
-// Layout of a 32-token block in LDS: keys 32 rows of 256 B at a pitch of 272 B, values 128 dim rows of 64 B (token
-// slots as in the cache) at a pitch of 80 B, so that the lanes one 128-bit LDS read serves together touch
-// different banks.
-constexpr int kPfKPitch = 272, kPfVPitch = 80;
-constexpr int kPfBufBytes = 32 * kPfKPitch + 128 * kPfVPitch; // 18,944 B per buffer
-
 } // namespace xfthip

@@ -22,20 +22,15 @@
 // exceeds it by more than 2^8 (probabilities up to 256 are exact enough in fp16 and in the fp32 sums), so the
 // 64 accumulator registers of a lane are rescaled in few blocks only.
 //
-// Two forms, of four waves a workgroup and two workgroups a CU.  FP16 cache: attn_prefill_ring_unit.  INT8
-// cache (attn_prefill32_unit): codes are widened to fp16
-// (exact) on their way into LDS, the key scale multiplies the score row, the value scale the probability; the
-// value scales are taken relative to a running reference that is part of the same lazy rescaling (it moves when
-// a block's largest scale leaves [ref / 1024, 4 ref]), so fp16 probabilities stay in range whatever the scales.
+// Four waves a workgroup, two workgroups a CU.  INT8 cache: codes are widened to fp16 (exact) on their way into LDS, the key scale multiplies
+// the score row, the value scale the probability; the value scales are taken relative to a running reference that moves lazily, too (when a
+// block's largest scale leaves [ref / 1024, 4 ref]), so fp16 probabilities stay in range whatever the scales.
 #pragma once
 #include <type_traits>
 
 #include "attention_dev.h"
 
 namespace xfthip {
-
-constexpr int kP32ScaleBytes = 256; // 32 key scales + 32 value scales of a block (INT8 cache)
-constexpr int kP32BufBytes = kPfBufBytes + kP32ScaleBytes;
 
 union HFrag32 {
     f16x8 v;
@@ -66,220 +61,7 @@ __device__ inline void store_direct(const AttnParams &p, const size_t base, cons
         }
 }
 
-// INT8 cache, NW waves a workgroup, 32 columns a wave; two workgroups a CU.  Measured and not kept: the block kept in LDS as codes (8 KB
-// instead of 16), a lane's 128-bit read serving two k-steps (the queries' dims and, through a lane-half exchange, the
-// probabilities' tokens permuted to match) - 8 operand reads a block and wave instead of 16, widened by every wave in
-// registers: correct, and 354 us against 292 (4 x 2048 tokens, 32 query / 8 KV heads): the 160 widening instructions a wave
-// and block cost more than the reads had.
-template <int NW>
-__device__ inline void attn_prefill32_unit(const AttnParams &p, const int kvh, const int cgroup, const int b, unsigned char *lds) {
-    constexpr int D = 128, NT = NW * 64, WC = 32;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int h = lane >> 5, cl = lane & 31;
-    int past = p.past;
-    if (p.past_dev) {
-        past = p.past_dev[b];
-        past = past < 0 ? 0 : (past > p.kv.S - p.S ? p.kv.S - p.S : past);
-    }
-    past = __builtin_amdgcn_readfirstlane(past);
-    const int ncols = p.S * p.G;
-    const int c0 = (cgroup * NW + wave) * WC; // first column of this wave
-    const int c = c0 + cl;
-    const bool cvalid = c < ncols;
-    const int cs = cvalid ? c / p.G : 0, cj = cvalid ? c % p.G : 0;
-    const int limit = cvalid ? past + cs + 1 : 0; // tokens [0, limit) are visible to this column
-    const int lim_min = c0 + WC - 1 < ncols ? past + c0 / p.G + 1 : 0; // every column of the wave sees at least this many
-    int wave_last = c0 + WC - 1;
-    wave_last = wave_last < ncols ? wave_last : ncols - 1;
-    const int wave_lim = c0 < ncols ? past + wave_last / p.G + 1 : 0; // no column of the wave sees a token from here on
-    const int wave_nblk = (wave_lim + 31) >> 5;
-    int wg_last = (cgroup + 1) * NW * WC - 1;
-    wg_last = wg_last < ncols ? wg_last : ncols - 1;
-    const int nblk = (past + wg_last / p.G + 1 + 31) >> 5;
-
-    const size_t bh = (size_t)b * p.kv.H + kvh;
-    const ATTN_GLOBAL char *kbase = (const ATTN_GLOBAL char *)p.kv.k + bh * p.kv.S * D;
-    const ATTN_GLOBAL char *vbase = (const ATTN_GLOBAL char *)p.kv.v + bh * p.kv.S * D;
-    const ATTN_GLOBAL float *ksc = (const ATTN_GLOBAL float *)p.kv.kscale + bh * p.kv.S;
-    const ATTN_GLOBAL float *vsc = (const ATTN_GLOBAL float *)p.kv.vscale + bh * p.kv.S;
-
-    // ---- the block copy global -> registers -> LDS (widened on the way): 256 + 256 chunks of 16 bytes ----
-    constexpr int CHUNKS = 256, PER = (CHUNKS + NT - 1) / NT;
-    u32x4 kstage[PER], vstage[PER];
-    f32x4 sstage; // threads 0..7 carry 4 key scales each, threads 8..15 4 value scales
-    auto fetch = [&](const int blk) {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int ch = threadIdx.x + NT * i;
-            if (CHUNKS % NT == 0 || ch < CHUNKS) {
-                kstage[i] = *(const ATTN_GLOBAL u32x4 *)(kbase + (size_t)blk * (32 * D) + (size_t)ch * 16);
-                vstage[i] = *(const ATTN_GLOBAL u32x4 *)(vbase + (size_t)blk * (32 * D) + (size_t)ch * 16);
-            }
-        }
-        if (threadIdx.x < 16) sstage = *(const ATTN_GLOBAL f32x4 *)((threadIdx.x < 8 ? ksc : vsc) + (blk << 5) + 4 * (threadIdx.x & 7));
-    };
-    auto widen16 = [&](const u32x4 raw, u32x4 &lo, u32x4 &hi) {
-        HFrag x, y;
-        widen_i8x4(raw[0], x.h[0], x.h[1]);
-        widen_i8x4(raw[1], x.h[2], x.h[3]);
-        widen_i8x4(raw[2], y.h[0], y.h[1]);
-        widen_i8x4(raw[3], y.h[2], y.h[3]);
-        lo = x.q, hi = y.q;
-    };
-    auto stash = [&](const int buf) {
-        unsigned char *kb = lds + buf * kP32BufBytes, *vb = kb + 32 * kPfKPitch;
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int ch = threadIdx.x + NT * i;
-            if (CHUNKS % NT == 0 || ch < CHUNKS) {
-                u32x4 lo, hi;
-                widen16(kstage[i], lo, hi); // token ch / 8, dims 16 (ch % 8) ..
-                *(u32x4 *)(kb + (ch >> 3) * kPfKPitch + (ch & 7) * 32) = lo;
-                *(u32x4 *)(kb + (ch >> 3) * kPfKPitch + (ch & 7) * 32 + 16) = hi;
-                widen16(vstage[i], lo, hi); // dim ch / 2, token slots 16 (ch % 2) ..
-                *(u32x4 *)(vb + (ch >> 1) * kPfVPitch + (ch & 1) * 32) = lo;
-                *(u32x4 *)(vb + (ch >> 1) * kPfVPitch + (ch & 1) * 32 + 16) = hi;
-            }
-        }
-        if (threadIdx.x < 16) *(f32x4 *)(kb + kPfBufBytes + 16 * threadIdx.x) = sstage;
-    };
-
-    // ---- this wave's queries: B operand of the score MFMA, k-step s covers dims 16 s + 8 h .. + 8 ----
-    const float c1 = p.scale * 1.4426950408889634f;
-    HFrag32 qf[8];
-    {
-        const uint16_t *qrow = p.q + ((size_t)b * p.S + cs) * p.qStride + (size_t)(kvh * p.G + cj) * D;
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            u32x4 raw = {0u, 0u, 0u, 0u};
-            if (cvalid) raw = *(const u32x4 *)(qrow + 16 * s + 8 * h);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) qf[s].u[i] = pack_f16(u2f(raw[i] << 16), u2f(raw[i] & 0xFFFF0000u));
-        }
-    }
-    float m_run = kNegBig, l_run = 0.0f; // m_run == kNegBig: the column has seen no token yet
-    float vref = 0.0f; // the value scales are taken relative to this (0 = not set yet)
-    f32x16 o[4];
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
-
-    auto compute = [&](const int buf, const int blk) {
-        const int t0 = blk << 5;
-        const unsigned char *kb = lds + buf * kP32BufBytes, *vb = kb + 32 * kPfKPitch;
-        const unsigned char *krow = kb + cl * kPfKPitch + 16 * h;
-        HFrag32 kf[8];
-#pragma unroll
-        for (int s = 0; s < 8; ++s) kf[s].q = *(const u32x4 *)(krow + 32 * s);
-        f32x16 x;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[r] = 0.0f;
-#pragma unroll
-        for (int s = 0; s < 8; ++s) x = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s].v, qf[s].v, x, 0, 0, 0);
-        // the value operands are read only now: they reuse the key operands' registers and their LDS latency
-        // passes behind the softmax arithmetic
-        __builtin_amdgcn_sched_barrier(0);
-        HFrag32 vf[2][4];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt) vf[t][dt].q = *(const u32x4 *)(vb + (32 * dt + cl) * kPfVPitch + 16 * (2 * t + h));
-        const bool masked = t0 + 32 > lim_min; // wave-uniform
-        // scales of this lane's 16 tokens (8 q + 4 h ..)
-        f32x4 ks[4], vs[4];
-        float vmax = 0.0f, vmove = 1.0f;
-        const float *sl = (const float *)(kb + kPfBufBytes);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            ks[q] = *(const f32x4 *)(sl + 8 * q + 4 * h) * c1; // key scale and softmax scale in one factor
-            vs[q] = *(const f32x4 *)(sl + 32 + 8 * q + 4 * h);
-            // (tokens no column of the wave sees stay out: behind the sequence's end the cache may hold anything)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) vmax = fmaxf(vmax, t0 + 8 * q + 4 * h + r < wave_lim ? vs[q][r] : 0.0f);
-        }
-        vmax = fmaxf(vmax, swap32(vmax)); // the block's largest value scale, the same in every lane
-        // value scales relative to vref; vref follows the blocks' largest scale lazily, like the maximum
-        if (vmax > 4.0f * vref || (vmax > 0.0f && vmax * 1024.0f < vref)) { // wave-uniform
-            vmove = vref > 0.0f ? vref / vmax : 1.0f;
-            vref = vmax;
-        }
-        const float vinv = vref > 0.0f ? 1.0f / vref : 0.0f;
-        float pr[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[r] *= ks[r >> 2][r & 3];
-        if (masked) {
-            // only the blocks on the causal diagonal pay for the mask (a real branch)
-            asm volatile("" ::: "memory");
-#pragma unroll
-            for (int r = 0; r < 16; ++r) x[r] = (t0 + 8 * (r >> 2) + 4 * h + (r & 3)) < limit ? x[r] : kNegBig;
-        }
-        float bmax = fmaxf(fmaxf(x[0], x[1]), x[2]);
-#pragma unroll
-        for (int r = 3; r < 15; r += 2) bmax = fmaxf(fmaxf(bmax, x[r]), x[r + 1]);
-        bmax = fmaxf(bmax, x[15]);
-        bmax = fmaxf(bmax, swap32(bmax));
-        const float m_new = bmax > m_run + 8.0f ? bmax : m_run;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        m_run = m_new;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) pr[r] = __builtin_amdgcn_exp2f(x[r] - m_new);
-        if (masked) {
-            // a masked score is kNegBig: 2^(kNegBig - m) is already 0 unless the column has seen nothing yet
-            asm volatile("" ::: "memory");
-#pragma unroll
-            for (int r = 0; r < 16; ++r) pr[r] = x[r] > 0.5f * kNegBig ? pr[r] : 0.0f;
-        }
-        float psum = (pr[0] + pr[1]) + (pr[2] + pr[3]);
-#pragma unroll
-        for (int r = 4; r < 16; r += 4) psum += (pr[r] + pr[r + 1]) + (pr[r + 2] + pr[r + 3]);
-        l_run = l_run * alpha + psum; // (this lane's 16 rows; the two halves are added at the end)
-        const float oscale = alpha * vmove; // what the running output is multiplied by before this block is added
-#pragma unroll
-        for (int r = 0; r < 16; ++r) pr[r] *= vs[r >> 2][r & 3] * vinv;
-        if (__builtin_amdgcn_ballot_w64(oscale != 1.0f) != 0) {
-            // the running output is rescaled only when some column's reference point moved (a real branch)
-            asm volatile("" ::: "memory");
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[dt][r] *= oscale;
-        }
-        HFrag32 pf[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            pf[t].u[0] = pack_f16(pr[4 * t], pr[4 * t + 1]);
-            pf[t].u[1] = pack_f16(pr[4 * t + 2], pr[4 * t + 3]);
-            pf[t].u[2] = pack_f16(pr[4 * t + 8], pr[4 * t + 9]);
-            pf[t].u[3] = pack_f16(pr[4 * t + 10], pr[4 * t + 11]);
-        }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][dt].v, pf[t].v, o[dt], 0, 0, 0);
-    };
-
-    if (nblk > 0) {
-        fetch(0);
-        stash(0);
-    }
-    __syncthreads();
-    for (int blk = 0; blk < nblk; ++blk) {
-        const bool more = blk + 1 < nblk; // uniform over the workgroup
-        if (more) fetch(blk + 1);
-        if (blk < wave_nblk) compute(blk & 1, blk);
-        if (more) stash((blk + 1) & 1);
-        __syncthreads();
-    }
-
-    l_run += swap32(l_run);
-    if (!cvalid) return;
-    const float inv = vref / l_run;
-    const size_t base = ((size_t)b * p.S + cs) * p.oStride + (size_t)(kvh * p.G + cj) * D;
-    store_direct(p, base, h, o, inv);
-}
-
-// FP16 cache: four waves a workgroup, 128 columns, two workgroups a CU.
+// 128 columns a workgroup.  Figures are those of the FP16 cache where nothing else is said.
 //
 // A wave's time on a block of 32 tokens is the product phase - scores of block b + 1 and values of block b, 16 MFMAs (512 clocks), and behind each the
 // read of the operand that takes its place: keys of block b + 2, values of block b + 1 - and the softmax phase, the probabilities of the block's scores, about 45
@@ -303,11 +85,20 @@ __device__ inline void attn_prefill32_unit(const AttnParams &p, const int kvh, c
 // (The requests as assembly: after the compiler's builtin for this instruction every later counted wait becomes a wait for
 // everything.  M0 carries the LDS address of the wave's first lane; one wait state between writing it and the request.)
 //
-// The queries carry the power of two in the softmax scale (bf16 values stay exact in fp16, and in its range), the rest of it multiplies the
+// INT8: the blocks go through registers, a block ahead, where they are widened: 40 vector instructions more a block and wave, and 50 for the scales and
+// the sums of probabilities that are other numbers than those multiplied.  That wants no request in flight, so three blocks of ring are enough, and
+// the queries are read straight into registers, unscaled (the key scales are in fp32 anyway).  Call with the append, 32 query / 8 KV heads, against two
+// buffers whose operands were all read in front of the products: 4 x 2000 tokens 264 -> 218 us, 12 x 200 41 -> 30, 2 x 700 behind 1900 134 -> 110; with 32
+// KV heads 360 -> 300, 57 -> 46, 148 -> 130.  Measured and not kept: the block in LDS as codes, widened by every wave (354 us for 4 x 2048).
+//
+// FP16: the queries carry the power of two in the softmax scale (bf16 values stay exact in fp16, and in its range), the rest of it multiplies the
 // scores in fp32.  The row sums are those of the rounded probabilities.
 constexpr int kRing = 4, kLook = kRing - 1, kRingBlock = 16384, kRingLds = kRing * kRingBlock;
+constexpr int kScaleBytes = 256; // 32 key scales and 32 value scales of a block
+constexpr int kRingLdsInt8 = 3 * (kRingBlock + kScaleBytes);
 
-// lds: kRingLds bytes; every thread of 256 calls it
+// lds: kRingLds or kRingLdsInt8 bytes; every thread of 256 calls it
+template <bool INT8>
 __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh, const int cgroup, const int b, unsigned char *lds) {
     constexpr int D = 128, NW = 4, WC = 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -326,16 +117,18 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
     const int limit = cvalid ? past + cs + 1 : 0; // tokens [0, limit) are visible to this column
     const int lim_min = c0 + WC - 1 < ncols ? past + c0 / p.G + 1 : 0; // every column of the wave sees at least this many
     const int wave_last = c0 + WC - 1 < ncols ? c0 + WC - 1 : ncols - 1;
-    const int wave_nblk = c0 < ncols ? (past + wave_last / p.G + 1 + 31) >> 5 : 0; // no column of the wave sees a token of this block or later ones
+    const int wave_lim = c0 < ncols ? past + wave_last / p.G + 1 : 0, wave_nblk = (wave_lim + 31) >> 5; // no column of the wave sees a token from here on
     const int wg_last = (cgroup + 1) * NW * WC - 1 < ncols ? (cgroup + 1) * NW * WC - 1 : ncols - 1;
     const int nblk = (past + wg_last / p.G + 1 + 31) >> 5;
     const size_t bh = (size_t)b * p.kv.H + kvh;
+    auto slot = [](const int blk) { return INT8 ? blk % 3 : blk & (kRing - 1); };
     auto sgpr_ptr = [](const void *ptr) { // the same in every lane; said so, for a scalar register pair
         const uint64_t bits = (uint64_t)(uintptr_t)ptr;
         return (const char *)(uintptr_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(bits >> 32)) << 32) |
                 (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)bits));
     };
-    const char *k_uniform = sgpr_ptr((const char *)p.kv.k + bh * p.kv.S * D * 2), *v_uniform = sgpr_ptr((const char *)p.kv.v + bh * p.kv.S * D * 2);
+    constexpr int ESZ = INT8 ? 1 : 2, BLOCK = 32 * D * ESZ; // bytes of a cached value, of a block's keys
+    const char *k_uniform = sgpr_ptr((const char *)p.kv.k + bh * p.kv.S * D * ESZ), *v_uniform = sgpr_ptr((const char *)p.kv.v + bh * p.kv.S * D * ESZ);
 
     // ---- requests: this wave's share of a block is key segment w and dims 32 w .. of the values ----
     uint32_t rq_koff[2], rq_voff[2];
@@ -348,7 +141,7 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
     auto request = [&](const int blk_raw) {
         const int blk = __builtin_amdgcn_readfirstlane(blk_raw < nblk ? blk_raw : nblk - 1); // (past the end: the last block again, never read as itself)
-        const char *ks = k_uniform + (size_t)blk * (32 * D * 2), *vs = v_uniform + (size_t)blk * (32 * D * 2);
+        const char *ks = k_uniform + (size_t)blk * BLOCK, *vs = v_uniform + (size_t)blk * BLOCK;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const uint32_t kd = lds0 + 2048 * (uint32_t)wave + 1024 * i + (blk_raw & (kRing - 1)) * kRingBlock, vd = kd + 8192;
@@ -356,36 +149,78 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(vd), "v"(rq_voff[i]), "s"(vs) : "memory");
         }
     };
-    request(0);
-    request(1);
+    // ---- INT8: a thread's 16 codes of a block's keys and of its values, by way of registers, where they are widened (exact) ----
+    // (eight lanes write eight rows of a segment, which fall on different banks)
+    const ATTN_GLOBAL float *scales = (const ATTN_GLOBAL float *)(h ? p.kv.vscale : p.kv.kscale) + bh * p.kv.S + cl;
+    const int ck = lane >> 3, tk = 8 * wave + (lane & 7), vd = 32 * wave + cl; // 16 dims 16 ck .. of token tk; token slots 16 h .. of dim vd
+    u32x4 kstage, vstage;
+    float sstage; // wave 0: a key or value scale a lane
+    auto fetch = [&](const int blk) {
+        kstage = *(const ATTN_GLOBAL u32x4 *)(const ATTN_GLOBAL char *)(k_uniform + (size_t)blk * BLOCK + tk * D + 16 * ck);
+        vstage = *(const ATTN_GLOBAL u32x4 *)(const ATTN_GLOBAL char *)(v_uniform + (size_t)blk * BLOCK + vd * 32 + 16 * h);
+        if (wave == 0) sstage = scales[blk << 5];
+    };
+    auto stash = [&](const int blk) {
+        unsigned char *block = lds + slot(blk) * kRingBlock;
+        auto put = [](unsigned char *row, const int c, const int turn, const u32x4 raw) { // chunks c and c + 1 of a row
+            HFrag32 lo, hi;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                h2 a, b;
+                widen_i8x4(raw[i], a, b);
+                lo.u[2 * i] = __builtin_bit_cast(uint32_t, a), lo.u[2 * i + 1] = __builtin_bit_cast(uint32_t, b);
+                widen_i8x4(raw[2 + i], a, b);
+                hi.u[2 * i] = __builtin_bit_cast(uint32_t, a), hi.u[2 * i + 1] = __builtin_bit_cast(uint32_t, b);
+            }
+            *(u32x4 *)(row + ((c ^ turn) << 4)) = lo.q;
+            *(u32x4 *)(row + (((c + 1) ^ turn) << 4)) = hi.q;
+        };
+        put(block + (ck >> 1) * 2048 + tk * 64, 2 * (ck & 1), (tk >> 2) & 3, kstage);
+        put(block + 8192 + vd * 64, 2 * h, (vd >> 2) & 3, vstage);
+        if (wave == 0) *(float *)(lds + 3 * kRingBlock + slot(blk) * kScaleBytes + 4 * lane) = sstage;
+    };
+    if constexpr (INT8) {
+        fetch(0);
+    } else {
+        request(0);
+        request(1);
+    }
 
-    // ---- this wave's queries, through the ring's upper half: B operand of the score MFMA, k-step s covers dims 16 s + 8 h .. + 8 ----
+    // ---- this wave's queries: B operand of the score MFMA, k-step s covers dims 16 s + 8 h .. + 8 ----
+    float c1 = p.scale * 1.4426950408889634f, qmul = 1.0f;
+    HFrag32 qf[8];
+    auto take_query = [&](const int s, const u32x4 raw) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) qf[s].u[i] = pack_f16(u2f(raw[i] << 16) * qmul, u2f(raw[i] & 0xFFFF0000u) * qmul);
+    };
+    // FP16: through the ring's upper half
     unsigned char *qbuf = lds + (kRing / 2) * kRingBlock + wave * 8192;
     const uint64_t qrow = (uint64_t)(uintptr_t)(p.q + ((size_t)b * p.S + cs) * p.qStride + (size_t)(kvh * p.G + cj) * D);
     auto of_column = [&](uint64_t mine, int r) { // the 64 bits that column r of the wave holds
         return (uint64_t)(uint32_t)__shfl((int)(uint32_t)mine, r, 64) | ((uint64_t)(uint32_t)__shfl((int)(mine >> 32), r, 64) << 32);
     };
+    if constexpr (!INT8) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int r = 4 * i + (lane >> 4); // the 16-byte chunk c of a row sits in slot c ^ (row & 15)
-        const uint64_t src = of_column(qrow, r) + (((lane & 15) ^ (r & 15)) << 4);
-        const uint32_t dst = lds0 + (kRing / 2) * kRingBlock + 8192 * (uint32_t)wave + i * 1024;
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory");
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    float c1 = p.scale * 1.4426950408889634f, qmul = u2f(f2u(c1) & 0x7F800000u);
-    if (!(qmul > 0.0f) || qmul > 1.0f) qmul = 1.0f;
-    c1 /= qmul;
-    HFrag32 qf[8];
+        for (int i = 0; i < 8; ++i) {
+            const int r = 4 * i + (lane >> 4); // the 16-byte chunk c of a row sits in slot c ^ (row & 15)
+            const uint64_t src = of_column(qrow, r) + (((lane & 15) ^ (r & 15)) << 4);
+            const uint32_t dst = lds0 + (kRing / 2) * kRingBlock + 8192 * (uint32_t)wave + i * 1024;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory");
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        qmul = u2f(f2u(c1) & 0x7F800000u);
+        if (!(qmul > 0.0f) || qmul > 1.0f) qmul = 1.0f;
+        c1 /= qmul;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        const u32x4 raw = *(const u32x4 *)(qbuf + cl * 256 + (((2 * s + h) ^ (cl & 15)) << 4));
+        for (int s = 0; s < 8; ++s) take_query(s, *(const u32x4 *)(qbuf + cl * 256 + (((2 * s + h) ^ (cl & 15)) << 4)));
+    } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) qf[s].u[i] = pack_f16(u2f(raw[i] << 16) * qmul, u2f(raw[i] & 0xFFFF0000u) * qmul);
+        for (int s = 0; s < 8; ++s) take_query(s, *(const u32x4 *)((const uint16_t *)(uintptr_t)qrow + 16 * s + 8 * h)); // (past the last column: the first one's)
     }
 
     const h2 ones2 = {(_Float16)1.0f, (_Float16)1.0f};
     float m_run = 0.0f, l_run[2] = {0.0f, 0.0f}; // reference point, row sums of this lane's rows
+    float vref = 0.0f; // INT8: the value scales are taken relative to this (0 = not set yet)
     unsigned long long unset = ~0ull; // lanes whose column has seen nothing above minus infinity yet
     f32x16 o[4], x; // x: the scores
     HFrag32 kf[8], vf[2][4], pf[2];
@@ -398,8 +233,18 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
 
     auto softmax = [&](const int blk) {
         const int t0 = blk << 5;
+        const float *sl = (const float *)(lds + 3 * kRingBlock + slot(blk) * kScaleBytes); // INT8: key scales, value scales; this lane's 16 tokens are 8 q + 4 h ..
+        if constexpr (INT8) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) x[r] = fmaf(x[r], c1, -m_run);
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 ks = *(const f32x4 *)(sl + 8 * q + 4 * h) * c1; // key scale and softmax scale in one factor
+#pragma unroll
+                for (int r = 0; r < 4; ++r) x[4 * q + r] = fmaf(x[4 * q + r], ks[r], -m_run);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) x[r] = fmaf(x[r], c1, -m_run);
+        }
         if (t0 + 32 > lim_min) {
             // only the blocks on the causal diagonal pay for the mask (a real branch)
             asm volatile("" ::: "memory");
@@ -432,6 +277,38 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
         float pr[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) pr[r] = __builtin_amdgcn_exp2f(x[r]); // (a masked score is kNegBig: 0)
+        if constexpr (INT8) {
+            // (the sums are those of the probabilities as they are: with the scales and rounded, they are other numbers)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) l_run[r >> 2 & 1] += (pr[r] + pr[r + 1]) + (pr[r + 2] + pr[r + 3]);
+            __builtin_amdgcn_sched_barrier(0); // (the scales' registers only now)
+            f32x4 vs[4];
+            float vmax = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) vs[q] = *(const f32x4 *)(sl + 32 + 8 * q + 4 * h);
+            if (t0 + 32 > wave_lim) {
+                // tokens no column of the wave sees stay out: behind the sequence's end the cache may hold anything (a real branch)
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int r = 0; r < 16; ++r) vs[r >> 2][r & 3] = t0 + 8 * (r >> 2) + 4 * h + (r & 3) < wave_lim ? vs[r >> 2][r & 3] : 0.0f;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) vmax = fmaxf(fmaxf(vmax, vs[r >> 2][r & 3]), vs[r >> 2][(r & 3) + 1]);
+            vmax = fmaxf(vmax, swap32(vmax)); // the block's largest value scale, the same in every lane
+            // value scales relative to vref; vref follows the blocks' largest scale lazily, like the maximum
+            if (vmax > 4.0f * vref || (vmax > 0.0f && vmax * 1024.0f < vref)) { // wave-uniform
+                asm volatile("" ::: "memory");
+                const float vmove = vref > 0.0f ? vref / vmax : 1.0f;
+                vref = vmax;
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[dt][r] *= vmove;
+            }
+            const float vinv = vref > 0.0f ? 1.0f / vref : 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) pr[r] *= vs[r >> 2][r & 3] * vinv;
+        }
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             pf[t].u[0] = pack_f16(pr[4 * t], pr[4 * t + 1]);
@@ -439,13 +316,13 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
             pf[t].u[2] = pack_f16(pr[4 * t + 8], pr[4 * t + 9]);
             pf[t].u[3] = pack_f16(pr[4 * t + 10], pr[4 * t + 11]);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) l_run[i & 1] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, pf[t].u[i]), ones2, l_run[i & 1], false);
+            for (int i = 0; i < 4 && !INT8; ++i) l_run[i & 1] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, pf[t].u[i]), ones2, l_run[i & 1], false);
         }
     };
     // scores of block `next` (keys already read), values of the block in front of it; reads the keys of block next + 1, the values of block next
     auto products = [&](auto with_values, const int next) {
         constexpr bool VALUES = decltype(with_values)::value;
-        const unsigned char *kb = lds + ((next + 1) & (kRing - 1)) * kRingBlock, *vb = lds + (next & (kRing - 1)) * kRingBlock + 8192;
+        const unsigned char *kb = lds + slot(next + 1) * kRingBlock, *vb = lds + slot(next) * kRingBlock + 8192;
 #pragma unroll
         for (int r = 0; r < 16; ++r) x[r] = 0.0f;
         // (one read behind each MFMA: held up by a burst of them, the wave would issue no MFMA)
@@ -465,20 +342,36 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
         }
     };
     // every wave has read its queries, and the first two blocks are in
+    if constexpr (INT8) {
+        stash(0);
+        if (nblk > 1) {
+            fetch(1);
+            stash(1);
+        }
+        if (nblk > 2) fetch(2);
+    }
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    request(2);
+    if constexpr (!INT8) request(2);
 #pragma unroll
     for (int s = 0; s < 8; ++s) kf[s].q = *(const u32x4 *)(lds + (s & 1 ? at1 : at0) + (s >> 1) * 2048);
     __builtin_amdgcn_sched_barrier(0);
     products(std::false_type {}, 0);
     for (int blk = 0; blk < nblk; ++blk) {
         // the block asked for goes where block blk - 1 was, which every wave has read for the last time in front of the barrier behind block blk - 1's softmax
-        request(blk + kLook);
-        if (blk < wave_nblk) softmax(blk);
+        // (INT8: as much holds for block blk + 2, which is a register set ahead instead)
+        if constexpr (INT8) {
+            if (blk + 2 < nblk) stash(blk + 2);
+            if (blk + 3 < nblk) fetch(blk + 3);
+            if (blk < wave_nblk) softmax(blk);
+        } else {
+            request(blk + kLook);
+            if (blk < wave_nblk) softmax(blk);
+        }
         // block blk + 2 is in: everything but the requests just made
         __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (INT8) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(1);
         if (blk < wave_nblk) products(std::true_type {}, blk + 1);
@@ -489,7 +382,7 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
 
     float l = l_run[0] + l_run[1];
     l += swap32(l);
-    const float inv = 1.0f / l;
+    const float inv = (INT8 ? vref : 1.0f) / l;
     const size_t base = ((size_t)b * p.S + cs) * p.oStride + (size_t)(kvh * p.G + cj) * D;
     if (p.out_dtype == XFTHIP_BF16 && (((uintptr_t)p.out | ((size_t)p.oStride * 2)) & 15) == 0) {
         // whole rows through LDS, four of 256 bytes a store (from the registers: 16 stores of 32 rows' 16 bytes)

@@ -396,7 +396,7 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn_kernel(AttnParams a
     const AttnParams p = seq_params(all, s, s.first + i);
     const int ncg = (p.S * p.G + 127) / 128;
     if (at >= ncg) return; // (a longer sequence shares the group)
-    attn_prefill_ring_unit(p, pair % all.kv.H, ncg - 1 - at, 0, lds);
+    attn_prefill_ring_unit<false>(p, pair % all.kv.H, ncg - 1 - at, 0, lds);
 }
 
 // attn_kernel over sequences, each walked by one workgroup a column group: grid (KV heads x the longest's column groups, sequences)
