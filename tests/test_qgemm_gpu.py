@@ -200,7 +200,7 @@ def test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N):
 
 # on 256 CUs: 1, 2, 3, 4 (at 17 rows and more) and 6 column tiles a block, ragged last blocks, 8 to 1 K slices, and more than 8 tiles a CU
 FEW_ROWS = [(M, K, N) for K, N in [(1280, 1040), (1280, 4112), (1280, 9232), (768, 13328), (768, 18448), (768, 28672), (768, 36880), (256, 36880)]
-            for M in (3, 13, 29)]
+            for M in (3, 13, 29)] + [(13, 4096, 1040)]
 
 
 @pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])
@@ -209,10 +209,10 @@ def test_few_rows_every_form_against_64_bits(xh, orc, kind, M, K, N):
     test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N)
 
 
-@pytest.mark.parametrize("M", [1, 4, 5, 16])
-@pytest.mark.parametrize("K,N", [(128, 40), (256, 40), (384, 16), (640, 4096), (5632, 2048)])
+@pytest.mark.parametrize("M", [4, 5, 16])
+@pytest.mark.parametrize("K,N", [(3968, 40), (4096, 40), (4224, 16), (4480, 4096), (5632, 2048)])
 def test_bf16_tiles_alone_on_their_cu_against_64_bits(xh, orc, M, K, N):
-    """One to four K slices, of as many load batches and not."""
+    """The shallowest K of the form and one below it; slices of as many load batches, of one more and of an odd number (the last sum's)."""
     test_mfma_every_tile_against_64_bits(xh, orc, "bf16", M, K, N)
 
 

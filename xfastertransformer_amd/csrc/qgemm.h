@@ -95,7 +95,7 @@ struct SkinnyForm {
     int nt, u, kslices;
 };
 // k tiles a load batch of a block of nt column tiles and mt 16-row tiles: what the kernels are built with and what skinny_form counts slices in
-// (but BF16 single tiles that are a CU's only block: 4)
+// (but BF16 single tiles that are a CU's only block: skinny_form)
 constexpr int skinny_batch(int kind, int mt, bool group, int nt) {
     if (kind == XFTHIP_W_UINT4 || kind == XFTHIP_W_NF4 || nt > 3) return 1;
     const bool int8 = kind == XFTHIP_W_INT8;

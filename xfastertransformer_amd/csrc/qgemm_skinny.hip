@@ -82,10 +82,11 @@ SkinnyForm skinny_form(int kind, const SkinnyParams &p) {
             if (cost < least) least = cost, nt = n;
         }
     }
-    // A BF16 tile alone on its CU: batches of four k tiles in four slices, the bytes in flight of batches of two in eight with half the sums and half the
-    // waits. K x N at 4 | 16 rows: 5632 x 2048 7.6 | 10.2 -> 7.6 | 9.6 us, 11008 x 4096 17.4 | 20.8 -> 17.0 | 19.6, 8192 x 3072 12.2 | 14.3 -> 11.3 | 13.5,
-    // 14336 x 4096 21.8 | 26.6 -> 21.1 | 23.7.  (Two tiles a CU 10.9 | 13.7 us for 4096 x 6144, so 11.4 | 13.8.)
-    if (kind == XFTHIP_W_BF16 && mt == 1 && nt == 1 && !p.group && per_cu(1) == 1) return SkinnyForm {1, 4, p.KT / 4 < 4 ? (p.KT / 4 > 1 ? p.KT / 4 : 1) : 4};
+    // A BF16 tile alone on its CU, 5 .. 16 rows: batches of four k tiles in four slices, the bytes in flight of batches of two in eight with half the waits (and two
+    // sums a wave, so that an fp32 sum is as short).  16 rows, K x N: 5632 x 2048 10.2 -> 9.6 us, 11008 x 4096 20.8 -> 19.6, 8192 x 3072 14.3 -> 13.5, 14336 x 4096 26.6
+    // -> 23.7, 23.9 -> 22.5 where the weights lie in the Infinity Cache.  Not for a shallow K, up to 4 rows or two tiles a CU, which lose there: 16 rows of
+    // 2048 x 2048 4.6 -> 4.8, 3 of 14336 x 4096 18.7 -> 19.4; 1 of 4096 x 6144 10.5 -> 11.0.
+    if (kind == XFTHIP_W_BF16 && mt == 1 && nt == 1 && !p.group && p.M > 4 && p.K >= 4096 && per_cu(1) == 1) return SkinnyForm {1, 4, 4};
     // (BF16, four blocks of two tiles on a CU: one slice each, 32 rows x 28672 x 8192 101 -> 88 us, with SwiGLU 8 rows x 28672 x 4096 1.07 times as fast)
     const int least = kind == XFTHIP_W_BF16 ? 1 : 2, slices = kind == XFTHIP_W_BF16 && nt == 2 && per_cu(nt) > 2 ? 1 : 8 / per_cu(nt);
     return form(nt, slices > least ? slices : least);

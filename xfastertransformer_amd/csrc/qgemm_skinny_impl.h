@@ -211,12 +211,16 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
         const int nt0 = blk * NT;
         auto tile_of = [&](int t) { return tile_index(blk, t); };
 
-        f32x4 acc[NT][MT];
+        // (a BF16 tile alone on its CU has half the slices: two sums a wave in turn, so that as many are added up as short ones)
+        constexpr int SUMS = KIND == XFTHIP_W_BF16 && NT == 1 && MT == 1 && U == 4 && !GROUP ? 2 : 1;
+        f32x4 acc[SUMS][NT][MT];
         f32x4 accS[MT];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int m = 0; m < MT; ++m) acc[t][m] = f32x4 {0.f, 0.f, 0.f, 0.f};
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int i = 0; i < SUMS; ++i) acc[i][t][m] = f32x4 {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int m = 0; m < MT; ++m) accS[m] = f32x4 {0.f, 0.f, 0.f, 0.f};
 
@@ -319,14 +323,14 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
                             widen_nf4(wbuf[buf][u][t], i, lut, whi, wlo);
 #pragma unroll
                             for (int m = 0; m < MT; ++m) {
-                                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wlo, a[m].v, acc[t][m], 0, 0, 0);
-                                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(whi, a[m].v, acc[t][m], 0, 0, 0);
+                                acc[0][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wlo, a[m].v, acc[0][t][m], 0, 0, 0);
+                                acc[0][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(whi, a[m].v, acc[0][t][m], 0, 0, 0);
                             }
                         } else {
                             bf16x8 wv = widen<KIND>(wbuf[buf][u][t], i, nullptr);
 #pragma unroll
                             for (int m = 0; m < MT; ++m)
-                                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, a[m].v, acc[t][m], 0, 0, 0);
+                                acc[u % SUMS][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, a[m].v, acc[u % SUMS][t][m], 0, 0, 0);
                         }
                     }
                     if constexpr (need_sum) {
@@ -466,7 +470,7 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) mine[(m * 16 + ml) * LD + t * 16 + 4 * g + r] = acc[t][m][r];
+                for (int r = 0; r < 4; ++r) mine[(m * 16 + ml) * LD + t * 16 + 4 * g + r] = SUMS == 2 ? acc[0][t][m][r] + acc[SUMS - 1][t][m][r] : acc[0][t][m][r];
         if (g == 0) {
 #pragma unroll
             for (int m = 0; m < MT; ++m) mine[ROWS * LD + m * 16 + ml] = accS[m][0];
@@ -727,7 +731,7 @@ static int launch_form(const SkinnyParams &p, hipStream_t stream) {
     const SkinnyForm f = skinny_form(KIND, p);
     switch (f.nt) {
         case 1:
-            if constexpr (KIND == XFTHIP_W_BF16 && MT == 1 && !GROUP)
+            if constexpr (KIND == XFTHIP_W_BF16 && MT == 1 && STAGE && !GROUP)
                 if (f.u == 4) return launch<KIND, 1, MT, 4, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
             return launch<KIND, 1, MT, skinny_batch(KIND, MT, GROUP, 1), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
         case 2: return launch<KIND, 2, MT, skinny_batch(KIND, MT, GROUP, 2), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
