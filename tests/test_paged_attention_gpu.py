@@ -225,12 +225,13 @@ def test_paged_prefill_side_by_side(xh, orc, qH, kvH, lens, block_size):
 
 
 @pytest.mark.parametrize("qH,kvH,lens", [(32, 8, [200] * 8), (32, 8, [511, 150, 512, 600, 130]), (16, 4, [500, 270, 300, 20, 400]), (8, 8, [40] * 70)])
-def test_paged_prefill_as_exact_as_alone(xh, orc, qH, kvH, lens):
+@pytest.mark.parametrize("size,key,scale", [(24.0, 1.0, 128 ** -0.5), (1.5e-4, 1e4, 128 ** -0.5), (1.0, 1e4, 1.5e-5)])
+def test_paged_prefill_as_exact_as_alone(xh, orc, qH, kvH, lens, size, key, scale):
     """A sequence among others is as near to the 64-bit result as in a call of its own (2 % for another order of the sums): the same roundings of
     queries, probabilities and results, whatever else there is to do.  Large scores show a rounding of the queries: one of 2^-12 moves
-    scores of 40 by 4e-3, and with them their probabilities."""
+    scores of 40 by 4e-3, and with them their probabilities; so do small queries, or a small scale, and keys near the end of the range."""
     D, T, rng = 128, sum(lens), np.random.default_rng(len(lens))
-    q, k, v = (orc.round_bf16(rng.standard_normal((T, n, D)).astype(np.float32) * by) for n, by in ((qH, 24.0), (kvH, 1.0), (kvH, 1.0)))
+    q, k, v = (orc.round_bf16(rng.standard_normal((T, n, D)).astype(np.float32) * by) for n, by in ((qH, size), (kvH, key), (kvH, 1.0)))
     dq, dk, dv = (xh.DeviceBuffer.from_numpy(orc.to_bf16(a)) for a in (q, k, v))
     ds = xh.DeviceBuffer.from_numpy(np.arange(T, dtype=np.int32))
     dkc, dvc = xh.DeviceBuffer(T * kvH * D * 2), xh.DeviceBuffer(T * kvH * D * 2)
@@ -239,7 +240,7 @@ def test_paged_prefill_as_exact_as_alone(xh, orc, qH, kvH, lens):
     def call(to, at, n):
         p = lambda buf, width: C.c_void_p(buf.ptr.value + at * width)
         xh.paged_attention_prefill(p(to, qH * D * 2), p(dq, qH * D * 2), p(dk, kvH * D * 2), p(dv, kvH * D * 2), qH, kvH, D, qH * D, kvH * D, qH * D,
-                                   D ** -0.5, n, dkc.ptr, dvc.ptr, T, 1, p(ds, 4))
+                                   scale, n, dkc.ptr, dvc.ptr, T, 1, p(ds, 4))
 
     starts = np.concatenate([[0], np.cumsum(lens)])
     call(out, 0, lens)
@@ -250,7 +251,7 @@ def test_paged_prefill_as_exact_as_alone(xh, orc, qH, kvH, lens):
     for at, n in zip(starts, lens):
         off = []
         for h in range(qH):
-            x = q[at:at + n, h].astype(np.float64) @ k[at:at + n, h * kvH // qH].astype(np.float64).T * D ** -0.5
+            x = q[at:at + n, h].astype(np.float64) @ k[at:at + n, h * kvH // qH].astype(np.float64).T * scale
             x[np.triu_indices(n, 1)] = -np.inf
             p = np.exp(x - x.max(1, keepdims=True))
             ref = p / p.sum(1, keepdims=True) @ v[at:at + n, h * kvH // qH].astype(np.float64)

@@ -91,15 +91,15 @@ __device__ inline void store_direct(const AttnParams &p, const size_t base, cons
 // buffers whose operands were all read in front of the products: 4 x 2000 tokens 264 -> 218 us, 12 x 200 41 -> 30, 2 x 700 behind 1900 134 -> 110; with 32
 // KV heads 360 -> 300, 57 -> 46, 148 -> 130.  Measured and not kept: the block in LDS as codes, widened by every wave (354 us for 4 x 2048).
 //
-// FP16: the queries carry the power of two in the softmax scale (bf16 values stay exact in fp16, and in its range), the rest of it multiplies the
-// scores in fp32.  The row sums are those of the rounded probabilities.
+// FP16: the queries carry the power of two in the softmax scale, the rest of it multiplies the scores in fp32: a bf16 value x is exact in fp16 from 2^-17 / that
+// power up to 65504 / it.  Where `plain` is set, they carry nothing, as in the form for few columns.  The row sums are those of the rounded probabilities.
 constexpr int kRing = 4, kLook = kRing - 1, kRingBlock = 16384, kRingLds = kRing * kRingBlock;
 constexpr int kScaleBytes = 256; // 32 key scales and 32 value scales of a block
 constexpr int kRingLdsInt8 = 3 * (kRingBlock + kScaleBytes);
 
-// lds: kRingLds or kRingLdsInt8 bytes; every thread of 256 calls it
+// lds: kRingLds or kRingLdsInt8 bytes; every thread of 256 calls it.  plain (FP16): the queries as they are
 template <bool INT8>
-__device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh, const int cgroup, const int b, unsigned char *lds) {
+__device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh, const int cgroup, const int b, unsigned char *lds, const bool plain = false) {
     constexpr int D = 128, NW = 4, WC = 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, cl = lane & 31;
@@ -209,7 +209,7 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         qmul = u2f(f2u(c1) & 0x7F800000u);
-        if (!(qmul > 0.0f) || qmul > 1.0f) qmul = 1.0f;
+        if (plain || !(qmul > 0.0f) || qmul > 1.0f) qmul = 1.0f;
         c1 /= qmul;
 #pragma unroll
         for (int s = 0; s < 8; ++s) take_query(s, *(const u32x4 *)(qbuf + cl * 256 + (((2 * s + h) ^ (cl & 15)) << 4)));

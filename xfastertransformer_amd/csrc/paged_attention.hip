@@ -301,10 +301,10 @@ __global__ __launch_bounds__(128) void paged_merge_kernel(PagedParams p) {
 // ---- prefill: the sequences of a call side by side ---------------------------------------------------------------
 // Sequence i of a launch: tokens from row row0[i] on, rows[i] of them, 32-token blocks from blk0[i] on in the scratch copy (which holds blk0[n]
 // blocks a head).  An attention kernel takes the sequences first .. first + many - 1; grp0: workgroups of an XCD in front of their (sequence, KV
-// head) pairs 8 k .. 8 k + 7.  By value: no copy in front of the launch.
+// head) pairs 8 k .. 8 k + 7; scaled: how many of them take queries with the scale's power of two.  By value: no copy in front of the launch.
 constexpr int kSeqs = 64, kGroups = 256;
 struct SeqBatch {
-    int n, first, many;
+    int n, first, many, scaled;
     int row0[kSeqs], rows[kSeqs], blk0[kSeqs + 1];
     int grp0[kGroups + 1];
 };
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn_kernel(AttnParams a
     const AttnParams p = seq_params(all, s, s.first + i);
     const int ncg = (p.S * p.G + 127) / 128;
     if (at >= ncg) return; // (a longer sequence shares the group)
-    attn_prefill_ring_unit<false>(p, pair % all.kv.H, ncg - 1 - at, 0, lds);
+    attn_prefill_ring_unit<false>(p, pair % all.kv.H, ncg - 1 - at, 0, lds, i >= s.scaled);
 }
 
 // attn_kernel over sequences, each walked by one workgroup a column group: grid (KV heads x the longest's column groups, sequences)
@@ -558,8 +558,9 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
         p.kv = kv, p.q = (const uint16_t *)q, p.qStride = q_stride, p.out = out, p.oStride = o_stride, p.out_dtype = XFTHIP_BF16;
         p.B = 1, p.G = G, p.scale = scale, p.nsplit = 1;
         // Those that attention_launch would take to the form for many columns, and the others with them where they are enough together (12 x 200
-        // tokens, 32 query / 8 KV heads 21 us against 52 in the form for few columns, 8 x 600, 16 / 4 heads 29 against 79)
-        s.first = 0, s.many = waves >= 4L * device_cu_count() ? s.n : n_long;
+        // tokens, 32 query / 8 KV heads 21 us against 52 in the form for few columns, 8 x 600, 16 / 4 heads 29 against 79), with their queries as they are,
+        // as the form that each would take alone has them
+        s.first = 0, s.scaled = n_long, s.many = waves >= 4L * device_cu_count() ? s.n : n_long;
         const int groups = (s.many * kv_heads + 7) / 8;
         for (int g = 0; g < groups; ++g) // (the sequences are sorted: the group's first pair belongs to its longest)
             s.grp0[g + 1] = s.grp0[g] + (int)(((long)s.rows[g * 8 / kv_heads] * G + 127) / 128);
