@@ -36,14 +36,14 @@ def _cache(xh, orc, k, v, int8=0):
     return kc, vc, dc
 
 
-def _attend(xh, orc, dc, q, B, S, qh, past, out_dtype, pitch, skip):
+def _attend(xh, orc, dc, q, B, S, qh, past, out_dtype, pitch, skip, scale=SCALE):
     """Results at `skip` elements from a 256-byte border, rows `pitch` elements apart; what lies between the rows stays as it is."""
     rows, width, bf16 = q.shape[0], q.shape[1], out_dtype == xh.BF16
     qd = xh.DeviceBuffer.from_numpy(orc.to_bf16(q))
     mark = np.full(rows * pitch + skip, 7.0, np.float32)
     od = xh.DeviceBuffer.from_numpy(orc.to_bf16(mark) if bf16 else mark)
     at = C.c_void_p(od.ptr.value + skip * (2 if bf16 else 4))
-    xh.attention(dc, qd.ptr, width, at, pitch, out_dtype, B, S, qh, SCALE, past)
+    xh.attention(dc, qd.ptr, width, at, pitch, out_dtype, B, S, qh, scale, past)
     xh.synchronize()
     out = od.to_numpy(np.uint16, mark.shape) if bf16 else od.to_numpy(np.float32, mark.shape)
     out = (orc.from_bf16(out) if bf16 else out)
@@ -61,7 +61,7 @@ def _attend(xh, orc, dc, q, B, S, qh, past, out_dtype, pitch, skip):
     (2, 300, 1, 32, 8, "f32", 4, 0),
     (16, 33, 0, 32, 32, "bf16", 0, 0),  # one head a group: a wave's columns are 32 tokens
     (9, 257, 95, 8, 8, "f32", 0, 4),
-    (40, 2, 700, 32, 1, "bf16", 0, 0),  # a token's heads fill a wave; the first three blocks lie before all new tokens
+    (64, 2, 700, 128, 4, "bf16", 0, 0),  # a token's heads fill a wave; the first three blocks lie before all new tokens
     (5, 129, 64, 28, 4, "bf16", 8, 0),  # 7 heads a group: waves begin inside a token
 ])
 def test_columns_and_ways_out(xh, orc, B, S, past, qh, kvh, kind, extra, skip):
@@ -116,7 +116,7 @@ def test_scores_at_the_ends_of_the_range(xh, orc, score):
     (16, 33, 0, 32, 32, "bf16", 0, 0),  # two blocks, the second with one token
     (33, 31, 0, 32, 32, "f32", 0, 0),  # a single block
     (12, 65, 0, 32, 32, "bf16", 4, 4),  # three
-    (40, 2, 700, 32, 1, "bf16", 0, 0),
+    (64, 2, 700, 128, 4, "bf16", 0, 0),
     (5, 129, 64, 28, 4, "bf16", 8, 0),
 ])
 @pytest.mark.parametrize("spread", [0, 1])
@@ -132,7 +132,59 @@ def test_int8_cache(xh, orc, B, S, past, qh, kvh, kind, extra, skip, spread):
     q = orc.round_bf16(rng.standard_normal((B * S, qh * D)))
     got = _attend(xh, orc, dc, q, B, S, qh, past, xh.BF16 if kind == "bf16" else xh.F32, qh * D + extra, skip)
     ref = orc.attention_ref_f64(q, kc.as_f32(), vc.as_f32(), qh, kvh, D, [S] * B, [past] * B, SCALE)
-    # fp16 products of probabilities and scales: 2^-11 of a value each, or 2^-25 of 2^8 times the largest scale's; bf16 results 2^-9 on top
-    size = np.abs(vc.as_f32()).max()
-    assert (np.abs(got - ref) <= 6e-4 * max(size, 1.0) + 3e-3 + np.abs(ref) * (2.0 ** -8 if kind == "bf16" else 0.0)).all(), np.abs(got - ref).max()
+    # fp16 products of probabilities and scales: 2^-11 of a value each, or 2^-25 of the largest that the 32 columns of the query's wave see; bf16 results 2^-9 on top
+    vf = vc.as_f32()
+    size = orc.attention_ref_f64(q, kc.as_f32(), np.abs(vf), qh, kvh, D, [S] * B, [past] * B, SCALE)
+    largest = np.maximum.accumulate(np.abs(vf).max(3), 2)  # [B, KV heads, tokens]
+    column = np.arange(S)[:, None] * (qh // kvh) + np.arange(qh // kvh)
+    seen = past + np.minimum(column // 32 * 32 + 31, S * (qh // kvh) - 1) // (qh // kvh)
+    largest = largest[:, :, seen].transpose(0, 2, 1, 3).reshape(B * S, qh, 1).repeat(D, 2).reshape(size.shape)
+    bound = 2.0 ** -11 * size + 2.0 ** -25 * n * largest + 2.0 ** -18 * size + np.abs(ref) * (2.0 ** -8 if kind == "bf16" else 0.0)
+    assert (np.abs(got - ref) <= bound).all(), (np.abs(got - ref) / bound).max()
+    # and no query's row is noise: but for those that see a token a thousand times as large in their wave
+    near = bound.reshape(B * S, qh, D).max(2) < 0.1 * np.abs(ref).reshape(B * S, qh, D).max(2)
+    assert near.mean() > 0.8, near.mean()
+    dc.free()
+
+
+@pytest.mark.parametrize("kind", ["fp16", "int8"])
+@pytest.mark.parametrize("drop", [12.0, 15.5, 18.0, 21.0])
+def test_weights_among_the_subnormal_values(xh, orc, kind, drop):
+    """One key far above all others, whose probabilities lie at 2^-drop of its own: subnormal in fp16 from 2^-14 on.  Thousands of them are a share of the
+    result all the same, above and below the line alike."""
+    S, qh, kvh, int8 = 3000, 32, 8, int(kind == "int8")
+    rng = np.random.default_rng(int(drop))
+    k, v = np.zeros((1, S, kvh * D), np.float32), 1.0 + rng.standard_normal((1, S, kvh * D)).astype(np.float32)
+    k.reshape(S, kvh, D)[0, :, 0] = drop * np.log(2.0) / SCALE / 2.0
+    k.reshape(S, kvh, D)[1:, :, 1] = 0.05 * rng.standard_normal((S - 1, kvh))
+    v[0, 0] = 4.0  # (a share lost above or below the line moves the result by as much times the distance of 3 from the others' mean)
+    kc, vc, dc = _cache(xh, orc, k, v, int8)
+    q = orc.round_bf16(np.tile(np.eye(1, D, 0) * 2.0 + np.eye(1, D, 1), (S, qh)))
+    got = _attend(xh, orc, dc, q, 1, S, qh, 0, xh.F32, qh * D, 0).reshape(S, qh, D)
+    ref = orc.attention_ref_f64(q, kc.as_f32(), vc.as_f32(), qh, kvh, D, [S], [0], SCALE).reshape(S, qh, D)
+    # a probability in fp16 is off by 2^-11 of itself or 2^-25 at most (INT8: its product with a value scale relative to the one in use, the first key's 1.0
+    # among them), times a value's distance from the result, of up to 8; fp32 sums 2^-18 on top
+    n = np.arange(1, S + 1)[:, None, None]
+    size = 8.0 * (2.0 ** -11 * np.minimum(n * 2.0 ** -drop, 1.0) + 2.0 ** -25 * n) + (4.0 * 2.0 ** -11 if int8 else 0.0) + 8.0 * 2.0 ** -18
+    assert (np.abs(got - ref) <= size).all(), (np.abs(got - ref) / size).max()
+    dc.free()
+
+
+@pytest.mark.parametrize("scale", [-0.3, 0.0, 1e-30, 1.5e-6, 3e-4, 0.04, 0.11, 0.3, 0.99, 3.0])
+@pytest.mark.parametrize("size", [0.05, 1.0, 1e4])
+@pytest.mark.parametrize("kind", ["fp16", "int8"])
+def test_any_softmax_scale(xh, orc, scale, size, kind):
+    """Scales of any size and sign, with queries and keys such that the scores are about one (or, where they can't be, smaller): no query loses bits."""
+    B, S, qh, kvh = 20, 64, 32, 8
+    rng = np.random.default_rng(int(abs(scale) * 1e6) % 1000 + int(size))
+    key = min(0.1 / max(abs(scale) * size, 1e-12), 8e3)
+    k, v = (rng.standard_normal((B, S, kvh * D)).astype(np.float32) * by for by in (key, 1.0))
+    kc, vc, dc = _cache(xh, orc, k, v, int(kind == "int8"))
+    q = orc.round_bf16(rng.standard_normal((B * S, qh * D)) * size)
+    got = _attend(xh, orc, dc, q, B, S, qh, 0, xh.F32, qh * D, 0, scale)
+    ref = orc.attention_ref_f64(q, kc.as_f32(), vc.as_f32(), qh, kvh, D, [S] * B, [0] * B, scale)
+    # every probability (INT8: product of probability and scale) in fp16, 2^-11 of it at most and half of that in the root mean square at random; an INT8 cache's
+    # value scales beside 1.2 times that; the first tokens, of one value, have nothing to average
+    off = np.sqrt(((got - ref) ** 2).reshape(B, S, -1).mean((0, 2))) / np.sqrt((ref ** 2).reshape(B, S, -1).mean((0, 2)))
+    assert off.max() < 4e-4, off
     dc.free()

@@ -91,8 +91,8 @@ __device__ inline void store_direct(const AttnParams &p, const size_t base, cons
 // buffers whose operands were all read in front of the products: 4 x 2000 tokens 264 -> 218 us, 12 x 200 41 -> 30, 2 x 700 behind 1900 134 -> 110; with 32
 // KV heads 360 -> 300, 57 -> 46, 148 -> 130.  Measured and not kept: the block in LDS as codes, widened by every wave (354 us for 4 x 2048).
 //
-// FP16: the queries carry the power of two in the softmax scale, the rest of it multiplies the scores in fp32: a bf16 value x is exact in fp16 from 2^-17 / that
-// power up to 65504 / it.  Where `plain` is set, they carry nothing, as in the form for few columns.  The row sums are those of the rounded probabilities.
+// FP16: the queries carry the power of two in the softmax scale, the rest of it multiplies the scores in fp32: a bf16 value is exact in fp16 from 2^-17 / that
+// power up to 65504 / it.  Of a scale below 2^-4 / log2 e they carry a power of two of their own.  Where `plain` is set, they carry nothing, as in the form for few columns.  The row sums are those of the rounded probabilities.
 constexpr int kRing = 4, kLook = kRing - 1, kRingBlock = 16384, kRingLds = kRing * kRingBlock;
 constexpr int kScaleBytes = 256; // 32 key scales and 32 value scales of a block
 constexpr int kRingLdsInt8 = 3 * (kRingBlock + kScaleBytes);
@@ -209,7 +209,22 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         qmul = u2f(f2u(c1) & 0x7F800000u);
-        if (plain || !(qmul > 0.0f) || qmul > 1.0f) qmul = 1.0f;
+        if (plain || qmul > 1.0f) {
+            qmul = 1.0f;
+        } else if (qmul < 0.0625f) {
+            // A scale that small would push ordinary queries among fp16's subnormal values: the power of two that takes the column's own largest value to 2^13 or more
+            // instead (a real branch)
+            asm volatile("" ::: "memory");
+            uint32_t top = 0; // its exponent
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const u32x4 raw = *(const u32x4 *)(qbuf + cl * 256 + (((2 * s + h) ^ (cl & 15)) << 4));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) top = max(top, max(raw[i] << 1 >> 24, raw[i] << 17 >> 24));
+            }
+            top = max(top, (uint32_t)__shfl_xor((int)top, 32, 64));
+            qmul = u2f((267u - min(max(top, 14u), 254u)) << 23);
+        }
         c1 /= qmul;
 #pragma unroll
         for (int s = 0; s < 8; ++s) take_query(s, *(const u32x4 *)(qbuf + cl * 256 + (((2 * s + h) ^ (cl & 15)) << 4)));
@@ -357,6 +372,9 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
     for (int s = 0; s < 8; ++s) kf[s].q = *(const u32x4 *)(lds + (s & 1 ? at1 : at0) + (s >> 1) * 2048);
     __builtin_amdgcn_sched_barrier(0);
     products(std::false_type {}, 0);
+    // Where the loop begins in the 32 bytes that are fetched at a time is worth 6 % (512 tokens behind 8000, by the number of 4-byte steps behind a border: 156,
+    // 150, 150, 146, 148, 152, 154, 152 us; 4 x 2000 tokens 144 to 146.5, 2 x 1000 with 16 / 4 heads 23.9 to 24.9), so it is said.
+    if constexpr (!INT8) asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
     for (int blk = 0; blk < nblk; ++blk) {
         // the block asked for goes where block blk - 1 was, which every wave has read for the last time in front of the barrier behind block blk - 1's softmax
         // (INT8: as much holds for block blk + 2, which is a register set ahead instead)
