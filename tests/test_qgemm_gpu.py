@@ -375,3 +375,15 @@ def test_captured_without_a_parts_buffer(xh, orc, kind):
 
 
 _unused = []  # streams kept alive: scratch is kept by a stream's handle, which a destroyed one's successor may get
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 16])
+def test_ragged_k_in_one_sum(xh, M):
+    """BF16 weights, K no multiple of the 32-row weight tile: what cancels in the first two tiles leaves the third's as it is.  In two sums in turn, the third
+    tile's 1 is lost beside the first's 2^24."""
+    K, N = 232, 48
+    A, W = np.zeros((M, K), np.float32), np.zeros((K, N), np.float32)
+    A[:, [3, 35, 70]], W[3], W[35], W[70] = [4096.0, 4096.0, 1.0], 4096.0, -4096.0, 1.0
+    dw = xh.Weight(xh.W_BF16, K, N, xh.f32_to_bf16_bits(W))
+    assert (_run_gemm(xh, dw, xh.f32_to_bf16_bits(A), M, K, N, xh.F32) == 1.0).all()
+    dw.free()

@@ -212,7 +212,7 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
         auto tile_of = [&](int t) { return tile_index(blk, t); };
 
         // (a BF16 tile alone on its CU has half the slices: two sums a wave in turn, so that as many are added up as short ones)
-        constexpr int SUMS = KIND == XFTHIP_W_BF16 && NT == 1 && MT == 1 && U == 4 && !GROUP ? 2 : 1;
+        constexpr int SUMS = KIND == XFTHIP_W_BF16 && NT == 1 && MT == 1 && U == 4 && STAGE && !KTAIL && !NORM && !GROUP ? 2 : 1;
         f32x4 acc[SUMS][NT][MT];
         f32x4 accS[MT];
 #pragma unroll
