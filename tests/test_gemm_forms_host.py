@@ -62,3 +62,11 @@ def test_few_rows_of_a_wide_weight(xh):
     assert xh.gemm_form(xh.W_BF16, 32, 1024, 65024)[:3] == (2, 2, 2)
     assert xh.gemm_form(xh.W_BF16, 32, 8192, 28672)[:3] == (2, 2, 1)
     assert xh.gemm_form(xh.W_INT8, 32, 5120, 27648)[:3] == (4, 1, 4)
+
+
+@pytest.mark.parametrize("M,K,N,form", [(16, 4096, 2048, (1, 4, 4)), (13, 4096, 512, (1, 4, 4)), (12, 4096, 512, (1, 2, 8)), (8, 5632, 2048, (1, 2, 8)), (16, 4128, 4096, (1, 2, 8)),
+                                        (16, 3968, 4096, (1, 2, 8)), (7, 4096, 4096, (1, 4, 4)), (7, 11008, 4096, (1, 4, 4)), (7, 8192, 3072, (1, 4, 4)), (6, 11008, 4096, (1, 2, 8)),
+                                        (8, 4480, 4096, (1, 2, 8)), (8, 8192, 3056, (1, 2, 8)), (5, 32768, 64, (1, 2, 8))])
+def test_bf16_tiles_alone_on_their_cu(xh, M, K, N, form):
+    """Four slices of four k tiles where they gain (256 CUs): many rows, or most CUs at work over slices of whole pairs of batches; eight of two elsewhere."""
+    assert xh.gemm_form(xh.W_BF16, M, K, N)[:3] == form

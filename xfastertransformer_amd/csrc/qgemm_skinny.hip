@@ -82,11 +82,16 @@ SkinnyForm skinny_form(int kind, const SkinnyParams &p) {
             if (cost < least) least = cost, nt = n;
         }
     }
-    // A BF16 tile alone on its CU, 5 .. 16 rows: batches of four k tiles in four slices, the bytes in flight of batches of two in eight with half the waits (and two
-    // sums a wave, so that an fp32 sum is as short).  16 rows, K x N: 5632 x 2048 10.2 -> 9.6 us, 11008 x 4096 20.8 -> 19.6, 8192 x 3072 14.3 -> 13.5, 14336 x 4096 26.6
-    // -> 23.7, 23.9 -> 22.5 where the weights lie in the Infinity Cache.  Not for a shallow K, up to 4 rows or two tiles a CU, which lose there: 16 rows of
-    // 2048 x 2048 4.6 -> 4.8, 3 of 14336 x 4096 18.7 -> 19.4; 1 of 4096 x 6144 10.5 -> 11.0.
-    if (kind == XFTHIP_W_BF16 && mt == 1 && nt == 1 && !p.group && p.M > 4 && p.K >= 4096 && per_cu(1) == 1) return SkinnyForm {1, 4, 4};
+    // A BF16 tile alone on its CU, 13 .. 16 rows: batches of four k tiles in four slices, the bytes in flight of batches of two in eight with half the waits (and two
+    // sums a wave, so that an fp32 sum is as short).  16 rows, K x N: 5632 x 2048 10.2 -> 9.7 us, 11008 x 4096 20.8 -> 19.6, 8192 x 3072 14.3 -> 13.8, 14336 x 4096 26.2
+    // -> 24.9, 23.5 -> 22.0 where the weights lie in the Infinity Cache.  With fewer rows only where most CUs have a tile and a slice is a whole number of two
+    // batches, or many of them: 8 rows of 4096 x 4096 8.4 -> 8.1, 11008 x 4096 20.5 -> 19.9, 8192 x 3072 13.1 -> 12.3, but 4480 x 4096 8.9 -> 9.1, 4096 x 512 5.7 -> 5.9,
+    // 5 of 32768 x 64 25.4 -> 26.5 (8 of 14336 x 4096 22.5 in both, 19.4 -> 19.9 out of the Infinity Cache).  Not for a K of half a batch, a shallow one, up to 4 rows or two tiles a CU, which lose: 16 rows of 4128 x 4096 9.4 -> 9.6, of 2048 x
+    // 2048 4.6 -> 4.8, 3 of 14336 x 4096 18.7 -> 19.4; 1 of 4096 x 6144 10.5 -> 11.0.
+    if (kind == XFTHIP_W_BF16 && mt == 1 && nt == 1 && !p.group && p.K >= 4096 && p.KT % 4 == 0 && per_cu(1) == 1) {
+        const bool filled = 4 * p.NTILES >= 3 * cus && (p.KT % 32 == 0 || p.K >= 8192);
+        if (p.M > (filled ? 6 : 12)) return SkinnyForm {1, 4, 4};
+    }
     // (BF16, four blocks of two tiles on a CU: one slice each, 32 rows x 28672 x 8192 101 -> 88 us, with SwiGLU 8 rows x 28672 x 4096 1.07 times as fast)
     const int least = kind == XFTHIP_W_BF16 ? 1 : 2, slices = kind == XFTHIP_W_BF16 && nt == 2 && per_cu(nt) > 2 ? 1 : 8 / per_cu(nt);
     return form(nt, slices > least ? slices : least);
