@@ -392,6 +392,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(ScanParams p) {
         // The read-outs of a wave's own columns: written and read by the same wave, whose LDS accesses keep their order.  64 / L column groups a wave.
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         constexpr int WG = 64 / L, OUTS = CT * C * WG;
 #pragma unroll
         for (int o0 = 0; o0 < OUTS; o0 += 64) {
@@ -404,8 +405,6 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(ScanParams p) {
             const int vc = col0 + gr * C + c;
             if (vc < p.VD) p.b.o[((size_t)(off + c0 + i) * p.H + head) * p.VD + vc] = (y[0] + y[1]) + (y[2] + y[3]);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
         __syncthreads();
     }
     if (own) {
