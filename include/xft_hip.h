@@ -675,7 +675,9 @@ size_t xfthip_plan_weight_bytes(xfthip_plan_t p);
 /*
  * A device model over a finished plan, which must outlive it.  act_dtype: XFTHIP_BF16 (activations and cache in bf16, products
  * on the bf16 matrix units) or XFTHIP_F32 (everything in 32 bits).  max_batch: sequence slots; pool_tokens: tokens the page
- * pool holds over all sequences (0 = max_batch * max_seq).
+ * pool holds over all sequences (0 = max_batch * max_seq).  max_tokens: tokens of a step, which its scratch memory is sized by; latent attention in bf16
+ * also keeps heads * (dim + vdim) + kv_rank + rot_dim values for each of max_seq context tokens, and for up to max_tokens + 992 as far as an eighth of
+ * the device memory left by everything else holds them.
  */
 int xfthip_model_create_from_plan(xfthip_plan_t p, int act_dtype, int max_batch, int max_seq, int max_tokens, int pool_tokens,
         xfthip_model_t *out);

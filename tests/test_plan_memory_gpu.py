@@ -1,0 +1,44 @@
+"""A plan model on a device that has room for it with one context in the expanded form of latent attention, but not with all of a step's."""
+import numpy as np
+import pytest
+
+import plan_util as u
+from oracle import pinepel_ref as ref
+
+pytestmark = pytest.mark.gpu
+HEADS, DIM, ROT, RANK, SLOTS, SEQ, TOKENS = 64, 128, 64, 128, 256, 64, 16384
+
+
+def test_model_that_just_fits():
+    import torch
+    from xfastertransformer_amd import capi as xh
+    xh.init(0)
+    torch.cuda.init()
+    left = lambda: torch.cuda.mem_get_info()[0]
+    cfg = u.config([u.latent(heads=HEADS, dim=DIM, rot=ROT, vdim=DIM, kv_rank=RANK, q_rank=64)])
+    bits = u.weights(cfg, 17)
+    plan, w = u.build_plan(xh, cfg, bits), u.oracle_weights(bits)
+    rng = np.random.default_rng(4)
+    texts = [rng.integers(0, cfg["vocab"], int(n)) for n in rng.integers(33, SEQ + 1, 40)]
+    want = np.stack([ref.forward(cfg, w, t)[-1] for t in texts])
+
+    def step(model):
+        got = model.step([(i, t, [len(t) - 1]) for i, t in enumerate(texts)])
+        assert u.rel_rms(got, want).max() < 0.06
+
+    before = left()
+    model = xh.PlanModel(plan, xh.BF16, SLOTS, SEQ, TOKENS)
+    used = before - left()
+    step(model)  # (and the stream has its scratch memory)
+    model.free()
+    more = (TOKENS + 31 * 32 - SEQ - 32) * (2 * HEADS * DIM + RANK + ROT) * 2  # the contexts behind the first
+    assert 0.2 * used < more < 0.8 * used
+    room, ballast = used - more // 2, []
+    while left() > room + (64 << 20):
+        ballast.append(xh.DeviceBuffer(min(left() - room, 16 << 30)))
+    model = xh.PlanModel(plan, xh.BF16, SLOTS, SEQ, TOKENS)
+    step(model)
+    model.free()
+    for b in ballast:
+        b.free()
+    plan.free()

@@ -1430,15 +1430,6 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
     alloc(&p->router_logits, T * routes * 4), alloc(&p->eh, T * eh * e), alloc(&p->expert_out, T * eo * 4);
     alloc(&p->route.sel, T * top * 4), alloc(&p->route.weight, T * top * 4), alloc(&p->route.slot_row, T * top * 4), alloc(&p->route.row_token, T * top * 4);
     alloc(&p->route.group_rows, experts * 12);
-    // the expanded form's contexts, in whole blocks of 32 tokens: at least the longest one's, and as many as a pass of fresh prompts has
-    if (act_dtype == XFTHIP_BF16 && max_tokens >= 32) {
-        const size_t ctx = std::max<size_t>(pad32(max_seq) + 32, std::min<size_t>(T + 31 * (size_t)std::min(max_batch, kLatentGroup), (size_t)max_batch * (pad32(max_seq) + 32)));
-        size_t kx = 0, vx = 0, rl = 0;
-        for (const PlanLayer &L : p->layers)
-            if (L.s.mixer == XFTHIP_MIXER_LATENT && latent_expanded_takes(act_dtype, L, 1 << 20, 1 << 20))
-                kx = std::max(kx, (size_t)L.s.heads * L.D), vx = std::max(vx, (size_t)L.s.heads * L.V), rl = std::max(rl, (size_t)(L.R + L.RD));
-        if (kx) alloc(&p->rows, ctx * rl * e, true), alloc(&p->kx, ctx * kx * e, true), alloc(&p->vx, ctx * vx * e, true), p->context_rows = (int)ctx;
-    }
     for (const PlanLayer &L : p->layers) {
         if (L.s.mixer == XFTHIP_MIXER_LATENT) p->part_floats = std::max(p->part_floats, latent_part_floats(L));
         if (L.s.mixer == XFTHIP_MIXER_GROUPED) p->part_floats = std::max(p->part_floats, grouped_part_floats(L));
@@ -1509,6 +1500,19 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
             && hipMemset(m->step, 0, 64) == hipSuccess
             && hipMalloc((void **)&m->logits, (size_t)p->logit_rows * plan->cfg.vocab * 4) == hipSuccess
             && hipMalloc((void **)&m->idlog, (size_t)m->idlog_cap * max_batch * 4) == hipSuccess;
+    // Last, the expanded form's contexts, in whole blocks of 32 tokens: the longest one's, and as many as a pass of fresh prompts has as far as an eighth of the
+    // memory that is left then holds them, so that a model that fits with the former is not refused for the latter.
+    size_t kx = 0, vx = 0, rl = 0;
+    for (const PlanLayer &L : p->layers)
+        if (max_tokens >= 32 && L.s.mixer == XFTHIP_MIXER_LATENT && latent_expanded_takes(act_dtype, L, 1 << 20, 1 << 20))
+            kx = std::max(kx, (size_t)L.s.heads * L.D), vx = std::max(vx, (size_t)L.s.heads * L.V), rl = std::max(rl, (size_t)(L.R + L.RD));
+    if (kx) {
+        const size_t longest = pad32(max_seq) + 32, fresh = std::min<size_t>(T + 31 * (size_t)std::min(max_batch, kLatentGroup), (size_t)max_batch * longest);
+        const size_t row = (rl + kx + vx) * e;
+        size_t left = 0, device = 0, ctx = longest;
+        if (ok && fresh > ctx && hipMemGetInfo(&left, &device) == hipSuccess && left > ctx * row) ctx += std::min(fresh - ctx, (left - ctx * row) / 8 / row);
+        alloc(&p->rows, ctx * rl * e, true), alloc(&p->kx, ctx * kx * e, true), alloc(&p->vx, ctx * vx * e, true), p->context_rows = (int)ctx;
+    }
     if (!ok) {
         set_error("xfthip_model_create_from_plan: out of device memory");
         xfthip_model_destroy(m);
