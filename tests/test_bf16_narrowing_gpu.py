@@ -1,4 +1,7 @@
 """Narrowing to bf16 on the device: results that leave the products in bf16 have the bits of the reference's conversion."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -30,3 +33,12 @@ def test_every_class_of_value(M):
         quiet = np.where((bits & 0x7FFFFFFF) > 0x7F800000, bits | 0x400000, bits)  # (the sum quiets a signalling NaN)
         assert np.array_equal(out.to_numpy(np.uint16, (M, N)), orc.to_bf16(quiet.view(np.float32)))
     w.free()
+
+
+def test_all_patterns():
+    """The conversion that every kernel compiles, over all 2^32 bit patterns in both halves of a pair."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    sweep = os.path.join(root, "xfastertransformer_amd", "csrc", "build", "bf16_device_sweep")
+    assert os.path.exists(sweep), "tests/bf16_device_sweep.hip is not built; run `python -m xfastertransformer_amd.build`"
+    out = subprocess.run([sweep], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0 and out.stdout == "mismatches lo=0 hi=0 one=0\n", out.stdout + out.stderr

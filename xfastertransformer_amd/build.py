@@ -112,8 +112,11 @@ def build_torch(force=True):
 
 
 def build_test_drivers(force=True):
-    """C++ programs of the test suite that call the host API the way a program written against the reference's
-    headers would (built here, not inside a GPU test)."""
+    """Programs of the test suite (built here, not inside a GPU test): one that calls the host API the way a program written against the
+    reference's headers would, one that sweeps the device's narrowing to bf16."""
+    sweep, sweep_src = os.path.join(CSRC, "build", "bf16_device_sweep"), os.path.join(ROOT, "tests", "bf16_device_sweep.hip")
+    if force or _stale(sweep, [sweep_src, os.path.join(CSRC, "common.h"), os.path.join(CSRC, "bf16_convert.h")]):
+        _run([HIPCC] + HIP_FLAGS + ["-I" + CSRC, sweep_src, "-o", sweep])
     out = os.path.join(CSRC, "build", "set_input_driver")
     src = os.path.join(ROOT, "tests", "set_input_driver.cpp")
     if force or _stale(out, [src, LIB_LAYERS, os.path.join(ROOT, "include", "models.h")]):

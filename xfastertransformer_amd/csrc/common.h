@@ -94,8 +94,8 @@ __device__ inline uint32_t f2u(float f) { return __float_as_uint(f); }
 __device__ inline float u2f(uint32_t u) { return __uint_as_float(u); }
 
 // fp32 -> bf16 exactly as the reference's bfloat16_t assignment (bf16_convert.h), by the hardware's conversion of two values: nearest even,
-// infinities and quiet NaN are the definition's, only subnormal inputs are not (all 2^32 inputs compared on the device), which go in as
-// signed zeros.  Two values take 7 vector instructions; the definition's integer steps take 9 each as selects and four branches each as written.
+// infinities and quiet NaN are the definition's, only subnormal inputs are not, which go in as signed zeros (tests/bf16_device_sweep.hip compares
+// all 2^32 inputs on the device).  Two values take 7 vector instructions; the definition's integer steps take 9 each as selects and four branches each as written.
 __device__ inline float flush_subnormal(float f) { return __builtin_fabsf(f) < 0x1p-126f ? __builtin_copysignf(0.0f, f) : f; }
 __device__ inline uint32_t f32x2_to_bf16(float lo, float hi) {
     typedef float f32x2_t __attribute__((ext_vector_type(2)));

@@ -11,6 +11,7 @@
 
 #include "../../../include/dtype.h"
 #include "../../../include/xft_hip.h"
+#include "../bf16_convert.h"
 
 namespace xfthost {
 
@@ -37,11 +38,7 @@ inline void ensure_init() {
 inline uint16_t to_bf16(float f) {
     uint32_t u;
     memcpy(&u, &f, 4);
-    uint32_t a = u & 0x7FFFFFFFu;
-    if (a > 0x7F800000u) return (uint16_t)((u >> 16) | 0x40u);
-    if (a == 0x7F800000u) return (uint16_t)(u >> 16);
-    if (a < 0x00800000u) return (uint16_t)((u >> 16) & 0x8000u);
-    return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
+    return xfthip::f32_bits_to_bf16_ref(u);
 }
 inline float from_bf16(uint16_t b) {
     uint32_t u = (uint32_t)b << 16;
