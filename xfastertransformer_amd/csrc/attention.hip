@@ -233,7 +233,9 @@ bool xfthip::attention_short(bool int8, int G, int len, int nsplit) {
     // Up to 320 tokens, and 384 of a cache half as large or with several query heads a KV head, 8 waves of one workgroup are faster than the parts of a
     // split and their merge; beyond, a CU's own path to the L2 takes longer than the merge.  FP16, one sequence, 32 KV heads, 176 / 256 / 320 / 512 tokens:
     // split 7.4 / 7.6 / 7.7 / 8.0 us, so 6.1 / 6.8 / 7.4 / 9.2; 8 KV heads of 32: 8.5 / 8.9 / 9.0 / 9.2 and 6.5 / 7.1 / 7.8 / 9.6; INT8, 32 KV heads: 7.3
-    // / 7.5 / 7.5 / 7.8 and 6.1 / 6.3 / 7.0 / 8.7, at 384 7.5 and 7.1.
+    // / 7.5 / 7.5 / 7.8 and 6.1 / 6.3 / 7.0 / 8.7, at 384 7.5 and 7.1.  Batches and portions (FP16 and INT8, 1 to 31 sequences, 1 to 8 new tokens, 8 to 64 query heads, 130 to
+    // 400 tokens, 1356 shapes) took 0.43 to 1.0 times as long, 0.71 in the mean: the more column groups, the more a split's hand-over cost (16 sequences of 130 tokens, 4 new, 32 / 8
+    // heads, INT8 17.7 and 7.6 us).
     return nsplit > 1 && len <= (int8 || G > 1 ? 384 : 320);
 }
 

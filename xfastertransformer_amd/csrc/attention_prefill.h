@@ -64,11 +64,12 @@ __device__ inline void store_direct(const AttnParams &p, const size_t base, cons
 // 128 columns a workgroup.  Figures are those of the FP16 cache where nothing else is said.
 //
 // A wave's time on a block of 32 tokens is the product phase - scores of block b + 1 and values of block b, 16 MFMAs (512 clocks), and behind each the
-// read of the operand that takes its place: keys of block b + 2, values of block b + 1 - and the softmax phase, the probabilities of the block's scores, about 45
+// read of the operand that takes its place: keys of block b + 2, values of block b + 1 - and the softmax phase, the probabilities of the block's scores, about 90
 // vector instructions, 16 of them exponentials, and the request of block b + kLook.  The two waves of a SIMD, of two workgroups, share its matrix unit
 // and vector ALU; products go first (s_setprio: 5 % slower without).  Reading all operands of a block in front of its products kept the wave from issuing
 // them, and every vector instruction of one wave - a sum of probabilities, an address, a result's narrowing - is time the other does not get:
-// against that form 4 x 2000 tokens, 32 query / 8 KV heads, 179 -> 152 us (850 TFLOP/s), 12 x 200 tokens 27 -> 22.  Tried and not kept:
+// against that form 4 x 2000 tokens, 32 query / 8 KV heads, 179 -> 152 us (145 back to back, 905 TFLOP/s), 12 x 200 tokens 27 -> 22.  Matrix unit and
+// vector ALU are busy 45 and 43 % of the clocks (INT8 27 and 60), the issue of MFMAs counted with the latter.  Tried and not kept:
 // half of the exponentials between the MFMAs (an exponential holds up the other wave's MFMAs: 8 % slower), operands read in the softmax phase (6 %), scores and values
 // in turn (the same), the scale in the queries and the reference point as the score's initial value (the same, and the queries lose bits).
 // Eight waves a workgroup that share a block and take turns at the matrix unit behind barriers: 1450 clocks a block instead of

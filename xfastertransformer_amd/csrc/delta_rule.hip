@@ -251,7 +251,8 @@ struct ScanParams {
 // their use; the read-outs' sums over the lanes, which nothing waits for, are left in LDS and added up for CT tokens at once, where a sum across the
 // lanes was as many instructions as the one that the chain needs; the last half of the column groups walk the segments backwards, so that an XCD and a CU
 // (which take every 8th and every 256th workgroup) get long and short ones.  16 heads of 128 x 128, before and after: two prompts of 3000 tokens
-// at most 690 / 600 us, four of 940 to 1500 420 / 350, eight of 800 at most 404 / 272, 16 of 400 346 / 230, 24 of 500 600 / 520.
+// at most 690 / 600 us, four of 940 to 1500 420 / 350, eight of 800 at most 404 / 272, 16 of 400 346 / 230, 24 of 500 600 / 520.  One of 2000 tokens: 32 heads 430 /
+// 377, 4 heads 408 / 343, 16 heads of 64 x 64 401 / 325, of 256 x 256 716 / 637; with one decay a head, 32 heads 409 / 350; one of 8 tokens 4.1 / 4.1.
 // (KD = 128 as 32 lanes x 4 rows x 2 columns, half the LDS reads: 510 us for 2048 tokens against 440 as 16 x 8 x 1.)
 template <int L, int RV, int C, bool ONE>
 __global__ __launch_bounds__(256) void delta_scan_kernel(ScanParams p) {
