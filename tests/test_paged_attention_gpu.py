@@ -224,6 +224,14 @@ def test_paged_prefill_side_by_side(xh, orc, qH, kvH, lens, block_size):
     test_paged_prefill_matches_oracle(xh, orc, qH, kvH, lens, block_size)
 
 
+@pytest.mark.parametrize("qH,kvH,lens", [(20, 5, [700, 33, 650, 500, 1, 90, 300, 64, 700]), (32, 8, [300, 700, 40, 41, 600]), (16, 8, [200] * 9),
+                                         (12, 3, [400] * 3 + [10] * 20), (8, 8, [600, 300, 20, 130])])
+def test_paged_prefill_bands(xh, orc, qH, kvH, lens):
+    """Several groups of 8 (sequence, KV head) pairs, walked in bands by the length of the walk: a group with pairs of two sequences, lengths that are equal and
+    far apart, several bands."""
+    test_paged_prefill_matches_oracle(xh, orc, qH, kvH, lens, 16)
+
+
 @pytest.mark.parametrize("qH,kvH,lens", [(32, 8, [200] * 8), (32, 8, [511, 150, 512, 600, 130]), (16, 4, [500, 270, 300, 20, 400]), (8, 8, [40] * 70)])
 @pytest.mark.parametrize("size,key,scale", [(24.0, 1.0, 128 ** -0.5), (1.5e-4, 1e4, 128 ** -0.5), (1.0, 1e4, 1.5e-5)])
 def test_paged_prefill_as_exact_as_alone(xh, orc, qH, kvH, lens, size, key, scale):

@@ -76,6 +76,26 @@ def test_columns_and_ways_out(xh, orc, B, S, past, qh, kvh, kind, extra, skip):
     dc.free()
 
 
+@pytest.mark.parametrize("B,S,past,qh,kvh", [
+    (7, 70, 0, 36, 9),  # 63 (sequence, KV head) pairs, 8 a group: bands of 3 and 5 groups, the last group of 7 pairs
+    (11, 130, 40, 16, 8),  # 11 groups: bands of 1, 5 and 5
+    (10, 65, 3, 32, 8),  # 10: whole bands only
+    (3, 300, 0, 24, 3),  # 9 pairs in two groups
+    (13, 66, 0, 20, 5),  # 65 pairs: 9 groups, the last of one pair
+])
+@pytest.mark.parametrize("int8", [0, 1])
+def test_bands_of_pairs(xh, orc, B, S, past, qh, kvh, int8):
+    """Every pair's every column group is walked whatever the number of pairs; tolerance as above, an INT8 cache's values as it holds them."""
+    rng = np.random.default_rng(B * S)
+    k, v = (rng.standard_normal((B, past + S, kvh * D)).astype(np.float32) for _ in range(2))
+    kc, vc, dc = _cache(xh, orc, k, v, int8)
+    q = orc.round_bf16(rng.standard_normal((B * S, qh * D)))
+    got = _attend(xh, orc, dc, q, B, S, qh, past, xh.BF16, qh * D, 0)
+    ref = orc.attention_ref_f64(q, kc.as_f32(), vc.as_f32(), qh, kvh, D, [S] * B, [past] * B, SCALE)
+    assert (np.abs(got - ref) <= 3e-3 + np.abs(ref) * 2.0 ** -8).all(), np.abs(got - ref).max()
+    dc.free()
+
+
 @pytest.mark.parametrize("score", [-1e30, -3000.0, 3000.0, 1e30])
 def test_scores_at_the_ends_of_the_range(xh, orc, score):
     """The first 40 tokens score minus infinity, far below all others (the first blocks' weights vanish once others are seen), far above them (the others' do)

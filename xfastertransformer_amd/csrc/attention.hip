@@ -56,17 +56,15 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(AttnParams p) {
 }
 
 // 32 x 32 MFMA tiles, 32 columns a wave, K / V blocks shared through LDS (attention_prefill.h); two workgroups a CU
-// Workgroups are handed to the 8 XCDs in turn by their linear index, and each XCD has an L2 of its own: the
-// (sequence, KV head) pairs are dealt to the XCDs (pair = 8 k + XCD), and an XCD walks the column groups of one
-// pair, longest history first, before it starts the next, so that the workgroups resident on an XCD share one or
-// two pairs' keys and values in its L2 instead of all of them.
 template <bool INT8>
-__global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(AttnParams p, int ncg, int npairs) {
+__global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(AttnParams p, int ncg, int npairs, PrefillBands bands) {
     __shared__ __attribute__((aligned(16))) unsigned char lds[INT8 ? kRingLdsInt8 : kRingLds];
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int pair = (slot / ncg) * 8 + xcd;
+    int first, width;
+    prefill_band(bands, slot / ncg, first, width);
+    const int at = slot - first * ncg, pair = (first + at % width) * 8 + xcd;
     if (pair >= npairs) return;
-    attn_prefill_ring_unit<INT8>(p, pair % p.kv.H, ncg - 1 - slot % ncg, pair / p.kv.H, lds);
+    attn_prefill_ring_unit<INT8>(p, pair % p.kv.H, ncg - 1 - at / width, pair / p.kv.H, lds);
 }
 
 // Split-KV merge workspace: `slots` partial-result slots of kSlotFloats floats and one ticket per
@@ -170,9 +168,10 @@ int xfthip::attention_launch(xfthip_kvcache_t c, const void *q, int qStride, voi
         if (S > 1 && waves1 >= 4L * device_cu_count()) {
             p.nsplit = 1;
             const int ncg = (S * p.G + 127) / 128, npairs = B * c->kv.H;
+            const PrefillBands bands = prefill_bands((npairs + 7) / 8);
             dim3 grid(8 * ((npairs + 7) / 8) * ncg);
-            if (c->kv.int8) hipLaunchKernelGGL(attn_prefill32_kernel<true>, grid, dim3(256), 0, stream, p, ncg, npairs);
-            else hipLaunchKernelGGL(attn_prefill32_kernel<false>, grid, dim3(256), 0, stream, p, ncg, npairs);
+            if (c->kv.int8) hipLaunchKernelGGL(attn_prefill32_kernel<true>, grid, dim3(256), 0, stream, p, ncg, npairs, bands);
+            else hipLaunchKernelGGL(attn_prefill32_kernel<false>, grid, dim3(256), 0, stream, p, ncg, npairs, bands);
             XFT_CHECK_HIP(hipGetLastError());
             return 0;
         }

@@ -61,6 +61,23 @@ __device__ inline void store_direct(const AttnParams &p, const size_t base, cons
         }
 }
 
+// Workgroups are handed to the 8 XCDs in turn by their linear index, and each XCD has an L2 of its own: the (sequence, KV head) pairs are dealt to the
+// XCDs (pair = 8 group + XCD).  An XCD takes its groups in bands of five, and the column groups of a band's pairs in turn, longest history first: what
+// runs at the end is short then.  Pair after pair instead, an XCD ended on the long walks of its last pair wherever its 64 workgroups at a time were
+// no multiple of the pairs' own: 5 x 700 tokens, 32 query / 8 KV heads 47 -> 41 us, 2 x 2000, 32 / 32 heads 123 -> 102, 5 x 1500 INT8 236 -> 197, 4 x 2000, 32 / 8
+// heads 155 -> 153, INT8 213 -> 206; 31 shapes over both caches and the paged one 1.067 times as fast in the geometric mean, the slowest the same.  Bands of 4 and 6: within
+// 0.1 % of that; of 3 or of 16 1 to 2 % slower (8 x 800 tokens 57.5 -> 60.0, 8 x 3900, 32 / 32 heads, in one 1161 -> 1353: an L2 does not hold that many pairs' keys and values).
+constexpr int kBand = 5;
+struct PrefillBands { // what is left of whole bands comes first, `rest` groups; then bands of `width`
+    int rest, width;
+};
+inline PrefillBands prefill_bands(const int groups) { return {groups % kBand, kBand}; }
+// the band of a group
+__host__ __device__ inline void prefill_band(const PrefillBands b, const int group, int &first, int &width) {
+    const bool whole = group >= b.rest;
+    width = whole ? b.width : b.rest, first = whole ? b.rest + (group - b.rest) / b.width * b.width : 0;
+}
+
 // 128 columns a workgroup.  Figures are those of the FP16 cache where nothing else is said.
 //
 // A wave's time on a block of 32 tokens is the product phase - scores of block b + 1 and values of block b, 16 MFMAs (512 clocks), and behind each the

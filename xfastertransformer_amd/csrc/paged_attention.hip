@@ -300,13 +300,14 @@ __global__ __launch_bounds__(128) void paged_merge_kernel(PagedParams p) {
 
 // ---- prefill: the sequences of a call side by side ---------------------------------------------------------------
 // Sequence i of a launch: tokens from row row0[i] on, rows[i] of them, 32-token blocks from blk0[i] on in the scratch copy (which holds blk0[n]
-// blocks a head).  An attention kernel takes the sequences first .. first + many - 1; grp0: workgroups of an XCD in front of their (sequence, KV
-// head) pairs 8 k .. 8 k + 7; scaled: how many of them take queries with the scale's power of two.  By value: no copy in front of the launch.
+// blocks a head).  An attention kernel takes the sequences first .. first + many - 1; grp0: workgroups of an XCD in front of the k-th part
+// of the walk over their (sequence, KV head) pairs; scaled: how many of them take queries with the scale's power of two.  By value: no copy in front of the launch.
 constexpr int kSeqs = 64, kGroups = 256;
 struct SeqBatch {
     int n, first, many, scaled;
     int row0[kSeqs], rows[kSeqs], blk0[kSeqs + 1];
     int grp0[kGroups + 1];
+    PrefillBands bands;
 };
 
 __device__ inline int seq_of_block(const SeqBatch &s, int blk) {
@@ -380,8 +381,9 @@ __device__ inline AttnParams seq_params(const AttnParams &all, const SeqBatch &s
     return p;
 }
 
-// attn_prefill32_kernel over sequences: (sequence, KV head) pairs go to the XCDs in turn, an XCD walks the column groups of one
-// pair, longest history first, before it starts the next
+// attn_prefill32_kernel over sequences, the longest first.  Group k of 8 pairs has n(k) column groups, those of its longest sequence.  An XCD walks a band in levels,
+// from the longest walk down: levels n(k) - 1 .. n(k + 1), which groups k and those in front of it in its band reach, are part k.
+// (6 sequences of 750 .. 1500 tokens, 32 query / 8 KV heads: group after group 113 us the call, so 106; 7 of 600 .. 1200, 16 / 4 heads 58 and 52)
 __global__ __launch_bounds__(256, 2) void paged_prefill_attn_kernel(AttnParams all, SeqBatch s) {
     __shared__ __attribute__((aligned(16))) unsigned char lds[kRingLds];
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -391,12 +393,16 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn_kernel(AttnParams a
         if (s.grp0[mid] <= slot) group = mid;
         else hi = mid - 1;
     }
-    const int pair = group * 8 + xcd, i = pair / all.kv.H, at = slot - s.grp0[group];
+    int first, width;
+    prefill_band(s.bands, group, first, width);
+    const int reach = group - first + 1, at = slot - s.grp0[group];
+    const int level = (s.rows[group * 8 / all.kv.H] * all.G + 127) / 128 - 1 - at / reach;
+    const int pair = (first + at % reach) * 8 + xcd, i = pair / all.kv.H;
     if (i >= s.many) return;
     const AttnParams p = seq_params(all, s, s.first + i);
     const int ncg = (p.S * p.G + 127) / 128;
-    if (at >= ncg) return; // (a longer sequence shares the group)
-    attn_prefill_ring_unit<false>(p, pair % all.kv.H, ncg - 1 - at, 0, lds, i >= s.scaled);
+    if (level >= ncg) return; // (a longer sequence shares the group)
+    attn_prefill_ring_unit<false>(p, pair % all.kv.H, level, 0, lds, i >= s.scaled);
 }
 
 // attn_kernel over sequences, each walked by one workgroup a column group: grid (KV heads x the longest's column groups, sequences)
@@ -562,8 +568,13 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
         // as the form that each would take alone has them
         s.first = 0, s.scaled = n_long, s.many = waves >= 4L * device_cu_count() ? s.n : n_long;
         const int groups = (s.many * kv_heads + 7) / 8;
-        for (int g = 0; g < groups; ++g) // (the sequences are sorted: the group's first pair belongs to its longest)
-            s.grp0[g + 1] = s.grp0[g] + (int)(((long)s.rows[g * 8 / kv_heads] * G + 127) / 128);
+        s.bands = prefill_bands(groups);
+        auto levels = [&](int g) { return (int)(((long)s.rows[g * 8 / kv_heads] * G + 127) / 128); }; // (the sequences are sorted: the group's first pair belongs to its longest)
+        for (int g = 0; g < groups; ++g) {
+            int band, width;
+            prefill_band(s.bands, g, band, width);
+            s.grp0[g + 1] = s.grp0[g] + (levels(g) - (g + 1 < band + width ? levels(g + 1) : 0)) * (g - band + 1);
+        }
         if (s.many > 0) hipLaunchKernelGGL(paged_prefill_attn_kernel, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
         s.first = s.many, s.many = s.n - s.many;
         if (s.many > 0)
