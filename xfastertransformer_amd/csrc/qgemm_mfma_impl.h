@@ -247,12 +247,12 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
 
     // weight source of this lane: 16-column packed tile (2 per 32-column MFMA tile), chunk of
     // its column inside the tile, and which 8-byte half (INT8) / dword pair (4-bit) it uses
-    const uint8_t *wbase[WN];
+    const XFT_GLOBAL uint8_t *wbase[WN];
 #pragma unroll
     for (int t = 0; t < WN; ++t) {
         int nt = (n32_0 + t) * 2 + (nl >> 4);
         nt = nt < p.NTILES ? nt : p.NTILES - 1;
-        wbase[t] = p.packed + (size_t)nt * p.KT * 1024 + (nl & 15) * 16;
+        wbase[t] = global_bytes(p.packed) + (size_t)nt * p.KT * 1024 + (nl & 15) * 16;
     }
     constexpr int ROW_STEP = 256 / CHUNKS_PER_ROW;
     const int a_kc = threadIdx.x % CHUNKS_PER_ROW;
@@ -306,14 +306,14 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
 #pragma unroll
         for (int t = 0; t < WN; ++t) {
             if constexpr (KIND == XFTHIP_W_INT8) {
-                const u32x4 v = *(const u32x4 *)(wbase[t] + (size_t)kt * 1024 + (2 * gq + h) * 256);
+                const u32x4 v = *(const XFT_GLOBAL u32x4 *)(wbase[t] + (size_t)kt * 1024 + (2 * gq + h) * 256);
                 wreg[buf][gq][t][0] = v[0]; wreg[buf][gq][t][1] = v[1]; wreg[buf][gq][t][2] = v[2]; wreg[buf][gq][t][3] = v[3];
             } else if constexpr (KIND == XFTHIP_W_BF16) {
                 // chunk g = 2 s + h holds k = 8 g .. 8 g + 7 (DIRECT: of the step's first or second packed tile)
-                const u32x4 v = *(const u32x4 *)(wbase[t] + ((size_t)kt * (KTILE / PACKED_K) + gq / 2) * 1024 + (2 * (gq & 1) + h) * 256);
+                const u32x4 v = *(const XFT_GLOBAL u32x4 *)(wbase[t] + ((size_t)kt * (KTILE / PACKED_K) + gq / 2) * 1024 + (2 * (gq & 1) + h) * 256);
                 wreg[buf][gq][t][0] = v[0]; wreg[buf][gq][t][1] = v[1]; wreg[buf][gq][t][2] = v[2]; wreg[buf][gq][t][3] = v[3];
             } else {
-                const u32x4 v = *(const u32x4 *)(wbase[t] + (size_t)(kt / STEPS_PER_TILE) * 1024 + ((kt % STEPS_PER_TILE) * GROUPS + gq) * 256);
+                const u32x4 v = *(const XFT_GLOBAL u32x4 *)(wbase[t] + (size_t)(kt / STEPS_PER_TILE) * 1024 + ((kt % STEPS_PER_TILE) * GROUPS + gq) * 256);
                 wreg[buf][gq][t][0] = v[0]; wreg[buf][gq][t][1] = v[1]; wreg[buf][gq][t][2] = v[2]; wreg[buf][gq][t][3] = v[3];
             }
         }

@@ -196,13 +196,13 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
     };
     // Every weight load is unconditional: out-of-range column tiles are clamped to the last valid
     // one (their results are never stored).
-    const uint8_t *wbase[NT];
+    const XFT_GLOBAL uint8_t *wbase[NT];
     auto set_wbase = [&](int it) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             int nt = tile_index(it, t);
             nt = nt < p.NTILES ? nt : p.NTILES - 1;
-            wbase[t] = p.packed + (size_t)nt * p.KT * 1024 + lane * 16;
+            wbase[t] = global_bytes(p.packed) + (size_t)nt * p.KT * 1024 + lane * 16;
         }
     };
     u32x4 wbuf[2][U][NT];
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
                 const int kt = batch * U + u;
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
-                    wbuf[buf][u][t] = __builtin_nontemporal_load((const u32x4 *)(wbase[t] + (size_t)kt * 1024));
+                    wbuf[buf][u][t] = __builtin_nontemporal_load((const XFT_GLOBAL u32x4 *)(wbase[t] + (size_t)kt * 1024));
                 if constexpr (NORM) continue; // activations are read from LDS in compute()
                 if constexpr (STAGE) {
 #pragma unroll
