@@ -412,6 +412,9 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     // after a barrier kept the MFMA pipes waiting for the address path).
     constexpr int A_EVERY = MICRO / ALOADS;
     static_assert(MICRO % ALOADS == 0, "activation slices must spread evenly over the micro-steps");
+    // UINT4: mask and exponent of a pair of codes in a scalar and a vector register of their own, so that they are one instruction (v_and_or_b32 takes no literal)
+    uint32_t nib_mask = 0x000F000Fu, nib_bits = 0x43004300u;
+    if constexpr (KIND == XFTHIP_W_UINT4) asm("" : "+s"(nib_mask), "+v"(nib_bits));
     // widened MFMA operands of (weight set wb, micro-step ms, column tile t)
     auto widen = [&](int wb, int ms, int t, MFrag &whi, MFrag &wlo) {
         const int gq = ms / SUB, sb = ms % SUB;
@@ -429,10 +432,10 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
             const uint32_t x0 = wreg[wb][gq][t][2 * sb], x1 = wreg[wb][gq][t][2 * sb + 1];
             const uint32_t x = h ? x1 : x0;
             if constexpr (KIND == XFTHIP_W_UINT4) {
-                whi.u[0] = (x & 0x000F000Fu) | 0x43004300u;
-                whi.u[1] = ((x >> 4) & 0x000F000Fu) | 0x43004300u;
-                whi.u[2] = ((x >> 8) & 0x000F000Fu) | 0x43004300u;
-                whi.u[3] = ((x >> 12) & 0x000F000Fu) | 0x43004300u;
+                whi.u[0] = (x & nib_mask) | nib_bits;
+                whi.u[1] = ((x >> 4) & nib_mask) | nib_bits;
+                whi.u[2] = ((x >> 8) & nib_mask) | nib_bits;
+                whi.u[3] = ((x >> 12) & nib_mask) | nib_bits;
             } else {
                 const uint2 e0 = lut[x & 0xFF], e1 = lut[(x >> 8) & 0xFF], e2 = lut[(x >> 16) & 0xFF], e3 = lut[x >> 24];
                 whi.u[0] = e0.x; whi.u[1] = e1.x; whi.u[2] = e2.x; whi.u[3] = e3.x;
