@@ -209,6 +209,31 @@ def test_few_rows_every_form_against_64_bits(xh, orc, kind, M, K, N):
     test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N)
 
 
+@pytest.mark.parametrize("kind", ["uint4", "nf4"])
+@pytest.mark.parametrize("M,K,N", [(5, 128, 48), (16, 384, 80), (17, 128, 4112), (31, 256, 12304), (32, 1152, 2064), (17, 4352, 16), (32, 640, 20496)])
+def test_rows_straight_into_lds_against_64_bits(xh, orc, kind, M, K, N):
+    """One load batch a slice, an odd number and unequal ones; rows that fill their 16-row tiles and a single one in the second."""
+    test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N)
+
+
+@pytest.mark.parametrize("kind", ["uint4", "nf4"])
+def test_rows_four_gigabytes_apart(xh, orc, kind):
+    """The last row begins beyond the reach of 32-bit byte offsets."""
+    M, K, N, lda = 17, 256, 48, 134217728
+    rng = np.random.default_rng(3)
+    w, W, size = _random_weight(xh, orc, rng, kind, K, N)
+    A = orc.round_bf16(rng.standard_normal((M, K), dtype=np.float32))
+    a_dev, o_dev = xh.DeviceBuffer(((M - 1) * lda + K) * 2), xh.DeviceBuffer(M * N * 4)
+    for m in range(M):
+        a_dev.upload(orc.to_bf16(A[m]), m * lda * 2)
+    xh.gemm(w, a_dev.ptr, M, lda, o_dev.ptr, N, xh.F32)
+    xh.synchronize()
+    bound = np.abs(A).astype(np.float64) @ size * ((K + 8) * 2.0 ** -24 + (2.0 ** -16 if kind == "nf4" else 0.0))
+    assert float((np.abs(o_dev.to_numpy(np.float32, (M, N)) - A.astype(np.float64) @ W) / bound).max()) <= 1.0
+    a_dev.free()
+    w.free()
+
+
 @pytest.mark.parametrize("M", [4, 5, 16])
 @pytest.mark.parametrize("K,N", [(3968, 40), (4096, 40), (4224, 16), (4480, 4096), (5632, 2048)])
 def test_bf16_tiles_alone_on_their_cu_against_64_bits(xh, orc, M, K, N):

@@ -109,6 +109,13 @@ constexpr int skinny_batch(int kind, int mt, bool group, int nt) {
     if (mt == 1) return nt == 1 ? (int8 || group ? 4 : 2) : (group && !int8 ? 4 : 2);
     return nt == 2 && int8 && group ? 1 : 2;
 }
+// Products of 4-bit codes whose activation rows go straight into LDS (mt 16-row tiles): all that are staged, but UINT4 at up to 16 rows, where it gains 2 % in the mean and
+// loses up to 8 % (skinny_form has the figures)
+constexpr bool skinny_dma(int kind, int mt) { return kind == XFTHIP_W_NF4 || (kind == XFTHIP_W_UINT4 && mt == 2); }
+// rows that lie 4 GB apart, out of reach of that form's 32-bit offsets: the form for a ragged K takes them
+inline bool skinny_far(int kind, const SkinnyParams &p) {
+    return p.M > 4 && !p.group && skinny_dma(kind, p.M > 16 ? 2 : 1) && (size_t)p.M * (size_t)p.lda * 2 >= (size_t)1 << 32;
+}
 SkinnyForm skinny_form(int kind, const SkinnyParams &p);
 int qgemm_skinny(const PackedWeight &pw, const SkinnyParams &p, hipStream_t stream); // M <= 32
 bool skinny_can_fuse_norm(const PackedWeight &pw, int M); // may SkinnyParams::norm_x be used

@@ -47,6 +47,22 @@ SkinnyForm skinny_form(int kind, const SkinnyParams &p) {
     };
     auto per_cu = [&](int nt) { return ((p.NTILES + nt - 1) / nt * weights + cus - 1) / cus; };
     const long tiles = (long)p.NTILES * weights;
+    if (p.M > 4 && !p.group && skinny_dma(kind, mt)) {
+        // Rows straight into LDS, 16 KB a wave (8 at up to 16 rows): eight waves a CU have room, so that a CU's blocks share them.  The same cost, without a price on wide blocks,
+        // which hold no rows in registers.  16 shapes of 4096 .. 57344 columns x 2048 .. 14336 deep, against rows staged through registers (with v_and_or_b32 in both): UINT4 24 and 32 rows
+        // 0.915 of the time in the geometric mean (0.62 .. 0.98; 24 x 4096 x 28672 with SwiGLU 18.7 -> 17.4 us, 24 x 4096 x 4096 7.9 -> 7.0), NF4 0.87 (0.81 .. 0.95), within 0.2 to 0.5 % of
+        // the best of 12 forms in the mean; with the constants of the other forms 2 to 3 %.
+        int best = p.gateup ? 2 : 1;
+        float least = 1e30f;
+        for (int n : {1, 2, 3, 4, 6}) {
+            if (p.gateup && n % 2) continue;
+            const float tile = mt == 2 || n < 4 ? 1.0f : n == 4 ? 1.1f : 1.2f;
+            const float cost = (float)per_cu(n) * ((float)n * tile + (mt == 2 ? 0.8f : 0.3f));
+            if (cost < least) least = cost, best = n;
+        }
+        const int w = per_cu(best), slices = w > 2 || (w == 2 && best == 6) ? 2 : w == 2 || best == 6 ? 4 : 8;
+        return SkinnyForm {best, 1, slices < p.KT ? slices : p.KT};
+    }
     // (two slices against eight: 3 % faster at K = 4096, 2 % slower at 2048)
     if (kind == XFTHIP_W_BF16 && p.group && mt == 1) return form(p.gateup ? 2 : 1, p.gateup && p.K >= 4096 ? 2 : 8);
     if (p.group && tiles >= 8 * cus) { // K slices by the depth

@@ -56,8 +56,9 @@ __device__ inline uint32_t pack_hi16(float lo, float hi) {
 }
 
 // Widen the codes of MFMA step `i` of a lane's 16-byte chunk to 8 bf16 values.
+// nib: {0x000F000F, 0x43004300} in a scalar and a vector register of their own, so that mask and exponent are one instruction (v_and_or_b32 takes no literal)
 template <int KIND>
-__device__ inline bf16x8 widen(const u32x4 &w, int i, const uint32_t *lut) {
+__device__ inline bf16x8 widen(const u32x4 &w, int i, const uint32_t (&nib)[2]) {
     Frag f;
     Frag src;
     src.q = w;
@@ -71,12 +72,12 @@ __device__ inline bf16x8 widen(const u32x4 &w, int i, const uint32_t *lut) {
     } else if constexpr (KIND == XFTHIP_W_UINT4) {
         // 0x4300 | u is the bf16 value 128 + u; the 128 is removed in the epilogue
         uint32_t a = wd[i];
-        f.u[0] = (a & 0x000F000Fu) | 0x43004300u;
-        f.u[1] = ((a >> 4) & 0x000F000Fu) | 0x43004300u;
-        f.u[2] = ((a >> 8) & 0x000F000Fu) | 0x43004300u;
-        f.u[3] = ((a >> 12) & 0x000F000Fu) | 0x43004300u;
+        f.u[0] = (a & nib[0]) | nib[1];
+        f.u[1] = ((a >> 4) & nib[0]) | nib[1];
+        f.u[2] = ((a >> 8) & nib[0]) | nib[1];
+        f.u[3] = ((a >> 12) & nib[0]) | nib[1];
     } else if constexpr (KIND == XFTHIP_W_NF4) {
-        (void)lut; // NF4 goes through widen_nf4
+        // NF4 goes through widen_nf4
     } else {
         f.q = w;
     }
@@ -119,9 +120,11 @@ __constant__ float c_nf4_gemm[16] = XFTHIP_NF4_CODE_VALUES;
 // 125 GB/s a CU from L2, measured): with more than a few rows those loads, not the weights, set the time.
 // GROUP: several weights of one shape behind one launch (SkinnyParams::group, one grid row a weight); a form of its
 // own: with the weight pointers possibly read from memory the plain kernels lost 6 % of the decode step.
-template <int KIND, int NT, int MT, int U, bool NEED_SUM, bool KTAIL, bool NORM, bool ROPE, bool STAGE = false, bool GROUP = false>
-__global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qgemm_skinny_kernel(SkinnyParams p) {
-    // (the one-tile staged form is held to 128 registers, two workgroups a CU like its unstaged twin)
+// DMA: the activation rows go straight into the patches (global_load_lds_dwordx4), a batch ahead like the weights: no registers hold them on their way, so that
+// a block can be as wide as its CU's share of the columns.
+template <int KIND, int NT, int MT, int U, bool NEED_SUM, bool KTAIL, bool NORM, bool ROPE, bool STAGE, bool GROUP, bool DMA>
+__device__ __forceinline__ void qgemm_skinny_body(SkinnyParams &p) {
+    static_assert(!DMA || (STAGE && U == 1 && !KTAIL && !GROUP && KindTraits<KIND>::KTILE == 128), "direct-to-LDS rows: a batch is one k tile of 256-byte rows");
     static_assert(!NORM || (MT == 1 && !KTAIL), "the norm prologue covers M <= 4 without a K tail");
     static_assert(!ROPE || (NT % 2 == 0 && !KTAIL), "the RoPE epilogue works on tile pairs");
     static_assert(!STAGE || (!NORM && !ROPE), "staged activation loads belong to the plain kernels");
@@ -151,6 +154,8 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
         p.C = (char *)p.C + (size_t)rec[2] * p.ldc * (p.c_dtype == XFTHIP_F32 ? 4 : 2);
     }
 
+    uint32_t nib[2] = {0x000F000Fu, 0x43004300u};
+    if constexpr (KIND == XFTHIP_W_UINT4) asm("" : "+s"(nib[0]), "+v"(nib[1]));
     uint2 *lut = nullptr;
     if constexpr (KIND == XFTHIP_W_NF4) {
         // 256-entry table: byte -> {bf16 hi parts of (low, high) nibble, bf16 lo parts}
@@ -169,7 +174,9 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
     // other's banks); it shares its LDS with the reduction area, which is used only after the K loop
     constexpr int LPR = KTILE / 8, RPI = 64 / LPR; // lanes along a row, rows a wave-load
     constexpr int SPITCH = KTILE * 2 + 16, STILE = 16 * MT * SPITCH;
-    unsigned char *stage = (unsigned char *)red + (size_t)wave * (U * STILE);
+    // DMA: two of [16 MT rows][256 bytes], the 16-byte chunk c of row r in slot c ^ (r & 15), which keeps the fragment reads on different banks
+    constexpr int PATCH = DMA ? 2 * 16 * MT * KTILE * 2 : U * STILE;
+    unsigned char *stage = (unsigned char *)red + (size_t)wave * PATCH;
     const int s_row = lane / LPR, s_kc = lane % LPR;
 
     // K slice of this wave: balanced split of the KT / U load batches
@@ -247,19 +254,31 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
             row = row < p.M ? row : p.M - 1;
             if constexpr (GROUP) row = p.a_rows ? p.a_rows[row] : row;
             s_off[j] = (uint32_t)row * (uint32_t)p.lda;
+            if constexpr (DMA) s_off[j] = s_off[j] * 2 + ((s_kc ^ ((j * RPI + s_row) & 15)) << 4); // in bytes, with this lane's chunk
         }
+        const uint32_t dma_to = DMA ? (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)stage : 0;
 
         const u32x4 zero4 = {0u, 0u, 0u, 0u};
         u32x4 abuf[2][U][MT][MPT];
 
         auto issue = [&](int buf, int batch) {
+            if constexpr (DMA) {
+                // (As assembly: after the compiler's builtin for this instruction its later counted waits become waits for everything.  M0 carries the LDS address of the wave's first lane; one wait state behind it.)
+                const uint64_t from = (uint64_t)(uintptr_t)(p.A + (size_t)batch * KTILE);
+                const uint64_t src = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(from >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)from);
+#pragma unroll
+                for (int j = 0; j < MT * MPT; ++j) {
+                    const uint32_t to = __builtin_amdgcn_readfirstlane(dma_to + buf * (PATCH / 2) + j * 1024);
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(s_off[j]), "s"(src) : "memory");
+                }
+            }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int kt = batch * U + u;
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
                     wbuf[buf][u][t] = __builtin_nontemporal_load((const XFT_GLOBAL u32x4 *)(wbase[t] + (size_t)kt * 1024));
-                if constexpr (NORM) continue; // activations are read from LDS in compute()
+                if constexpr (NORM || DMA) continue; // activations are read from LDS in compute()
                 if constexpr (STAGE) {
 #pragma unroll
                     for (int j = 0; j < MT * MPT; ++j) {
@@ -292,9 +311,18 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
                 }
             }
         };
+        // DMA: the batch in buffer buf is in, and the compiler has waited for its weights, before the next one is requested: behind that its own waits, which count
+        // without the rows' requests, would be waits for the next batch's rows
+        auto arrived = [&](int buf) {
+            if constexpr (DMA) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+                for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(wbuf[buf][0][t]));
+            }
+        };
         auto compute = [&](int buf, int batch) {
             (void)batch;
-            if constexpr (STAGE) {
+            if constexpr (STAGE && !DMA) {
                 // rows as loaded into the patch; the fragments are read back below (same wave, in order)
 #pragma unroll
                 for (int u = 0; u < U; ++u)
@@ -311,6 +339,8 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
                     for (int m = 0; m < MT; ++m) {
                         if constexpr (NORM)
                             a[m].q = *(const u32x4 *)(xn + xn_row + (batch * U + u) * KTILE + g * KL + 8 * i);
+                        else if constexpr (DMA)
+                            a[m].q = *(const u32x4 *)(stage + buf * (PATCH / 2) + (m * 16 + ml) * (KTILE * 2) + (((g * (KL / 8) + i) ^ ml) << 4));
                         else if constexpr (STAGE)
                             a[m].q = *(const u32x4 *)(stage + u * STILE + (m * 16 + ml) * SPITCH + (g * KL + 8 * i) * 2);
                         else
@@ -327,7 +357,7 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
                                 acc[0][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(whi, a[m].v, acc[0][t][m], 0, 0, 0);
                             }
                         } else {
-                            bf16x8 wv = widen<KIND>(wbuf[buf][u][t], i, nullptr);
+                            bf16x8 wv = widen<KIND>(wbuf[buf][u][t], i, nib);
 #pragma unroll
                             for (int m = 0; m < MT; ++m)
                                 acc[u % SUMS][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, a[m].v, acc[u % SUMS][t][m], 0, 0, 0);
@@ -430,20 +460,24 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
         if (nb > 0) {
             int b = 1; // next batch to issue; buffer 0 holds batch b - 1
             for (; b + 1 < nb; b += 2) {
+                arrived(0);
                 issue(1, b_begin + b);
                 XFT_FENCE();
                 compute(0, b_begin + b - 1);
                 XFT_FENCE();
+                arrived(1);
                 issue(0, b_begin + b + 1);
                 XFT_FENCE();
                 compute(1, b_begin + b);
                 XFT_FENCE();
             }
+            arrived(0);
             if (b < nb) {
                 issue(1, b_begin + b);
                 XFT_FENCE();
                 compute(0, b_begin + b - 1);
                 XFT_FENCE();
+                arrived(1);
                 compute(1, b_begin + b);
             } else {
                 compute(0, b_begin + b - 1);
@@ -478,16 +512,23 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
         __syncthreads();
 
         const int stride = ROWS * LD + ROWS;
-        auto total = [&](int m, int c) {
+        // (a thread of a wide block has many sums to make: four reads under way at a time, in the order of the waves.  24 x 4096 x 28672 UINT4 3 % faster, and blocks of few
+        // tiles, whose one sum is behind the others' loads anyway, 2 to 10 % slower)
+        auto add_up = [&](const float *at) {
             float s = 0.0f;
-            for (int w = 0; w < nwaves; ++w) s += red[(size_t)w * stride + m * LD + c];
+            int w = 0;
+            if constexpr (DMA && NT >= 4) {
+                for (; w + 4 <= nwaves; w += 4) {
+                    const float a0 = at[w * stride], a1 = at[(w + 1) * stride], a2 = at[(w + 2) * stride], a3 = at[(w + 3) * stride];
+                    s = ((s + a0) + a1) + a2;
+                    s += a3;
+                }
+            }
+            for (; w < nwaves; ++w) s += at[w * stride];
             return s;
         };
-        auto total_sum = [&](int m) {
-            float s = 0.0f;
-            for (int w = 0; w < nwaves; ++w) s += red[(size_t)w * stride + ROWS * LD + m];
-            return s;
-        };
+        auto total = [&](int m, int c) { return add_up(red + m * LD + c); };
+        auto total_sum = [&](int m) { return add_up(red + ROWS * LD + m); };
         // (c & 15 equals threadIdx.x & 15 for every caller, so the scales fetched at the start of
         // the block are the ones this thread needs)
         auto column_value = [&](int m, int c, float sumA) {
@@ -627,6 +668,17 @@ __global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qg
     }
 }
 
+template <int KIND, int NT, int MT, int U, bool NEED_SUM, bool KTAIL, bool NORM, bool ROPE, bool STAGE = false, bool GROUP = false>
+__global__ __launch_bounds__(512, (STAGE && MT == 1 && NT == 1) ? 4 : 1) void qgemm_skinny_kernel(SkinnyParams p) {
+    // (the one-tile staged form is held to 128 registers, two workgroups a CU like its unstaged twin)
+    qgemm_skinny_body<KIND, NT, MT, U, NEED_SUM, KTAIL, NORM, ROPE, STAGE, GROUP, false>(p);
+}
+
+template <int KIND, int NT, int MT, bool NEED_SUM>
+__global__ __launch_bounds__(512, 1) void qgemm_skinny_dma_kernel(SkinnyParams p) {
+    qgemm_skinny_body<KIND, NT, MT, 1, NEED_SUM, false, false, false, true, false, true>(p);
+}
+
 // k tiles per load batch, sized so that two batches of weight + activation fragments stay in
 // registers (256 VGPRs per lane at 8 waves per block)
 template <int KIND, int MT, int NT = 1>
@@ -675,9 +727,25 @@ static int launch(const SkinnyParams &p, int kslices, hipStream_t stream) {
 }
 
 template <int KIND, int NT, int MT, bool NEED_SUM>
+static int launch_dma(const SkinnyParams &p, int kslices, hipStream_t stream) {
+    constexpr int ROWS = 16 * MT, COLS = 16 * NT;
+    const size_t sums = (size_t)kslices * (ROWS * (COLS + 1) + ROWS) * sizeof(float), patches = (size_t)kslices * 2 * ROWS * KindTraits<KIND>::KTILE * 2;
+    const size_t smem = (sums > patches ? sums : patches) + (KIND == XFTHIP_W_NF4 ? 2048 : 0);
+    SkinnyParams q = p;
+    q.nblocks = (p.NTILES + NT - 1) / NT;
+    if (smem > 64 * 1024) { // more dynamic LDS than the default limit: raise it once per instantiation
+        static const hipError_t attr = hipFuncSetAttribute((const void *)qgemm_skinny_dma_kernel<KIND, NT, MT, NEED_SUM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        XFT_CHECK_HIP(attr);
+    }
+    hipLaunchKernelGGL((qgemm_skinny_dma_kernel<KIND, NT, MT, NEED_SUM>), dim3(q.nblocks), dim3(64 * kslices), smem, stream, q);
+    XFT_CHECK_HIP(hipGetLastError());
+    return 0;
+}
+
+template <int KIND, int NT, int MT, bool NEED_SUM>
 static int dispatch_tail(const SkinnyParams &p, int kslices, hipStream_t stream) {
     constexpr int U = batch_tiles<KIND, MT, NT>();
-    if (p.KT * KindTraits<KIND>::KTILE != p.K) {
+    if (p.KT * KindTraits<KIND>::KTILE != p.K || (!p.norm_x && !p.rope && skinny_far(KIND, p))) {
         if (p.norm_x || p.rope) {
             set_error("qgemm_skinny: the fused prologue / epilogue needs K to be a whole number of weight tiles");
             return 2;
@@ -729,22 +797,32 @@ template <int KIND, int MT, bool NEED_SUM, bool STAGE, bool GROUP>
 static int launch_form(const SkinnyParams &p, hipStream_t stream) {
     constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4;
     const SkinnyForm f = skinny_form(KIND, p);
-    switch (f.nt) {
-        case 1:
-            if constexpr (KIND == XFTHIP_W_BF16 && MT == 1 && STAGE && !GROUP)
-                if (f.u == 4) return launch<KIND, 1, MT, 4, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
-            return launch<KIND, 1, MT, skinny_batch(KIND, MT, GROUP, 1), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
-        case 2: return launch<KIND, 2, MT, skinny_batch(KIND, MT, GROUP, 2), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
-        case 3:
-            if constexpr (!GROUP && (MT == 2 || KIND != XFTHIP_W_BF16))
-                return launch<KIND, 3, MT, skinny_batch(KIND, MT, false, 3), NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
-            break;
-        case 4:
-            if constexpr (MT == 2 || FOUR) return launch<KIND, 4, MT, skinny_batch(KIND, MT, GROUP, 4), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
-            break;
-        case 6:
-            if constexpr (MT == 2 && !GROUP) return launch<KIND, 6, MT, skinny_batch(KIND, MT, false, 6), NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
-            break;
+    if constexpr (STAGE && !GROUP && skinny_dma(KIND, MT)) {
+        switch (f.nt) {
+            case 1: return launch_dma<KIND, 1, MT, NEED_SUM>(p, f.kslices, stream);
+            case 2: return launch_dma<KIND, 2, MT, NEED_SUM>(p, f.kslices, stream);
+            case 3: return launch_dma<KIND, 3, MT, NEED_SUM>(p, f.kslices, stream);
+            case 4: return launch_dma<KIND, 4, MT, NEED_SUM>(p, f.kslices, stream);
+            case 6: return launch_dma<KIND, 6, MT, NEED_SUM>(p, f.kslices, stream);
+        }
+    } else {
+        switch (f.nt) {
+            case 1:
+                if constexpr (KIND == XFTHIP_W_BF16 && MT == 1 && STAGE && !GROUP)
+                    if (f.u == 4) return launch<KIND, 1, MT, 4, NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+                return launch<KIND, 1, MT, skinny_batch(KIND, MT, GROUP, 1), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
+            case 2: return launch<KIND, 2, MT, skinny_batch(KIND, MT, GROUP, 2), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
+            case 3:
+                if constexpr (!GROUP && (MT == 2 || KIND != XFTHIP_W_BF16))
+                    return launch<KIND, 3, MT, skinny_batch(KIND, MT, false, 3), NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+                break;
+            case 4:
+                if constexpr (MT == 2 || FOUR) return launch<KIND, 4, MT, skinny_batch(KIND, MT, GROUP, 4), NEED_SUM, false, false, false, STAGE, GROUP>(p, f.kslices, stream);
+                break;
+            case 6:
+                if constexpr (MT == 2 && !GROUP) return launch<KIND, 6, MT, skinny_batch(KIND, MT, false, 6), NEED_SUM, false, false, false, STAGE>(p, f.kslices, stream);
+                break;
+        }
     }
     set_error("qgemm_skinny: no form of %d column tiles", f.nt);
     return 2;
@@ -772,7 +850,7 @@ static int dispatch_sum(const SkinnyParams &p, int kslices, hipStream_t stream) 
 
 template <int KIND>
 static int dispatch_shape(const SkinnyParams &p, hipStream_t stream) {
-    if (!p.norm_x && !p.rope && p.KT * KindTraits<KIND>::KTILE == p.K) {
+    if (!p.norm_x && !p.rope && p.KT * KindTraits<KIND>::KTILE == p.K && !skinny_far(KIND, p)) {
         if constexpr (KIND == XFTHIP_W_INT8) {
             if (!p.zero) return p.group ? dispatch_form<KIND, false, true>(p, stream) : dispatch_form<KIND, false, false>(p, stream);
         }
