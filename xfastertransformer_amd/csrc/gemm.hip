@@ -100,7 +100,7 @@ int xfthip_gemm_form(int kind, int flags, int has_zero, int M, int K, int N, int
         return 0;
     }
     qgemm_mfma_form(kind, p);
-    form[0] = p.tile == 1 ? 32 : p.tile == 2 ? 64 : 128, form[1] = p.tile == 4 ? 256 : 128;
+    form[0] = p.tile == 1 ? 32 : p.tile == 2 ? 64 : p.tile == 5 ? 96 : 128, form[1] = p.tile >= 4 ? 256 : 128;
     form[2] = p.kgroups, form[3] = p.ksplit > 1 ? p.ksplit : 1, form[4] = p.direct;
     return 0;
 }

@@ -39,8 +39,8 @@ struct SkinnyParams {
     // fp32 [M][N] into split_part + y * M * N; a second kernel adds the parts in order and applies the epilogue
     int ksplit, split_ktiles;
     float *split_part;
-    // M > 32 kernel, host-side row count: the block tile (1: 32 rows x 128 columns, 2: 64 x 128, 3: 128 x 128, 4: 128 x 256), its K groups
-    // a workgroup, whether the activations go straight into LDS (tiles 3 and 4); chosen by qgemm_mfma.  band: row blocks a band of the launch
+    // M > 32 kernel, host-side row count: the block tile (1: 32 rows x 128 columns, 2: 64 x 128, 3: 128 x 128, 4: 128 x 256, 5: 96 x 256), its K groups
+    // a workgroup, whether the activations go straight into LDS (tiles 3, 4 and 5); chosen by qgemm_mfma.  band: row blocks a band of the launch
     int tile, kgroups, direct, band;
     // Row count known on the device only (the experts of a sparse MLP): when rows_dev is set the kernels read
     // {rows, first row of A, first row of C} from it, M is only the upper bound that sizes the grid, and m_hint

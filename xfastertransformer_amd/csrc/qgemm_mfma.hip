@@ -113,6 +113,10 @@ __global__ __launch_bounds__(256) void qgemm_split_finish_kernel(SkinnyParams p)
 // Several weights behind one launch (the experts of a sparse MLP): the same, without K groups, over the row blocks to be expected.  Against
 // 64-row tiles with K in up to 4 parts throughout: a Mixtral-8x7B layer, INT8, 400 tokens 549 -> 490 us, 1000 tokens 1060 -> 940; 8 experts
 // of width 2816 at width 2048, BF16, 6132 tokens, two layers and all else 3.28 -> 2.98 ms.
+// 96 x 256, for 65 .. 96 rows, experts with some more than 64 and counts that are one or a few more than a multiple of 128: its constants are those of 128 x 256 by the ratios of two
+// fits to 100 timings each.  300 shapes a kind of 1024 .. 28672 columns x 1024 .. 14336 deep, 33 .. 4096 rows, against the same without it: INT8 0.985 of the time in the geometric mean
+// (384 x 28672 x 4096 with SwiGLU 100 -> 87 us, 900 x 11008 x 4096 94 -> 82; 0.79 .. 1.05), BF16 0.99, NF4 0.99, UINT4 0.98; a Mixtral-8x7B layer, INT8, of 256 / 290 / 580 / 1024 tokens
+// 381 / 425 / 640 / 873 -> 369 / 377 / 597 / 872 us, UINT4, 256 tokens 363 -> 336.
 struct TileCost {
     int rows, cols, kgroups, resident;
     float fixed; // a block's pipeline fill and results
@@ -123,6 +127,7 @@ constexpr TileCost kTiles[] = {
         {64, 128, 1, 4, 1.2f, {0.35f, 0.56f, 0.51f, 0.357f}, {0.27f, 0.34f, 0.43f, 0.275f}},
         {128, 128, 1, 2, 1.7f, {0.71f, 0.64f, 0.90f, 0.71f}, {0.26f, 0.36f, 0.65f, 0.26f}},
         {128, 128, 2, 1, 4.3f, {1.0f, 1.14f, 1.38f, 1.0f}, {}},
+        {96, 256, 1, 2, 2.3f, {0.80f, 0.85f, 1.25f, 0.75f}, {0.525f, 0.54f, 1.025f, 0.575f}},
         {128, 256, 1, 2, 3.1f, {0.92f, 0.93f, 1.59f, 0.92f}, {0.73f, 0.77f, 1.34f, 0.73f}},
         {128, 256, 2, 1, 8.7f, {1.49f, 1.8f, 2.63f, 1.49f}, {}},
 };
@@ -174,7 +179,7 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_sp
     float best = 1e30f;
     for (const TileCost &t : kTiles) {
         if (t.rows == 32 && kind == XFTHIP_W_BF16) continue; // (not built: two bytes a weight want more rows behind them)
-        if (t.rows == 128 && !direct) continue;
+        if (t.rows >= 96 && !direct) continue;
         if (t.kgroups == 2 && p.rows_dev) continue; // (not built)
         // (8 weights of 28672 x 4096 and 4096 x 14336 INT8 with 37 rows each: 386 us a layer in 32-row blocks, which read every weight tile twice,
         // 353 in 64-row ones)
@@ -206,6 +211,9 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_sp
                 if (blocks > cus || p.K % unit || span % unit || steps < 48) continue;
                 steps *= 0.5f;
             }
+            // (with few blocks a 96-row tile's share of BF16 weights is too many bytes: 150 x 4096 x 11008 33 -> 45 us in 4 parts, 384 x 4096 x 22016 102 -> 118 whole)
+            // (and 8 parts of K are dearer than the model has them: 384 x 14336 x 4096 INT8 57.6 us in 4, 64 in 8)
+            if (t.rows == 96 && (parts > 4 || (kind == XFTHIP_W_BF16 && (parts > 1 || 2 * blocks < 3L * cus)))) continue;
             const long slots = (long)cus * t.resident, full = blocks / slots, rest = blocks - full * slots;
             float us = 7.0f + (float)full * (steps * (t.step[cls] + t.more[cls] * (float)(t.resident - 1)) + t.fixed);
             if (rest) {
@@ -219,8 +227,8 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_sp
             if (p.group && p.gateup && t.rows == 128) us *= 1.05f;
             if (us < best) {
                 best = us;
-                p.tile = t.rows == 32 ? 1 : t.rows == 64 ? 2 : t.cols == 128 ? 3 : 4;
-                p.kgroups = t.kgroups, p.direct = t.rows == 128;
+                p.tile = t.rows == 32 ? 1 : t.rows == 64 ? 2 : t.rows == 96 ? 5 : t.cols == 128 ? 3 : 4;
+                p.kgroups = t.kgroups, p.direct = t.rows >= 96;
                 p.ksplit = parts > 1 ? parts : 0, p.split_ktiles = part;
             }
         }

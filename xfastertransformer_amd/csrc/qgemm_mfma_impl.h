@@ -77,7 +77,7 @@ struct StepTraits<XFTHIP_W_BF16, DIRECT> {
 //
 // DIRECT: the activation tiles go from global memory straight into LDS (global_load_lds_dwordx4: a wave instruction
 // fills 1 KiB of consecutive LDS, lane after lane, from 64 addresses of its choice) instead of through registers and
-// ds_write.  Rows are 128 bytes with no padding; the 16-byte chunk c of row r sits in slot c ^ ((r >> 1) & 7) of its
+// ds_write (tiles of 96 and 128 rows).  Rows are 128 bytes with no padding; the 16-byte chunk c of row r sits in slot c ^ ((r >> 1) & 7) of its
 // row, which a lane gets by choosing the global chunk it fetches, and which keeps the operand reads (32 rows, one
 // chunk index) free of bank conflicts.  Four LDS tiles: step k requests tile k + 3, and the barrier that ends a step
 // first waits until the wave's requests of the step before are in (vmcnt counts them in order with the weight
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     // the zero-point term (below) is always the first one it reads - no branch on the wave number inside the k loop
     constexpr bool ROTATE = DIRECT && NEED_SUM;
     const int wave_first = ROTATE ? __builtin_amdgcn_readfirstlane(wave) : 0;
-    auto row_tile = [&](int m) { return ROTATE ? (m + wave_first) % WM : m; };
+    auto row_tile = [&](int m) { return ROTATE ? (m + wave_first) % WM : m; }; // (WM == 3: the fourth wave sums what the first does)
     MFrag afr[2][WM];
     auto read_frags = [&](int slot, int ab, int ms) {
         const unsigned char *src = abuf_base + ab * (ROWS * ROWB) + nl * ROWB +
@@ -410,8 +410,8 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     // a_stage: one slice of each per micro-step, so that no wave ever queues a burst of memory
     // instructions in front of its MFMAs (a wave issues in order; 4 waves sending 12 loads each right
     // after a barrier kept the MFMA pipes waiting for the address path).
-    constexpr int A_EVERY = MICRO / ALOADS;
-    static_assert(MICRO % ALOADS == 0, "activation slices must spread evenly over the micro-steps");
+    constexpr int A_EVERY = MICRO % ALOADS == 0 ? MICRO / ALOADS : 1;
+    static_assert(ALOADS <= MICRO, "at most an activation slice a micro-step");
     // UINT4: mask and exponent of a pair of codes in a scalar and a vector register of their own, so that they are one instruction (v_and_or_b32 takes no literal)
     uint32_t nib_mask = 0x000F000Fu, nib_bits = 0x43004300u;
     if constexpr (KIND == XFTHIP_W_UINT4) asm("" : "+s"(nib_mask), "+v"(nib_bits));
@@ -462,7 +462,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
         for (int ms = 0; ms < MICRO; ++ms) {
             const int gq = ms / SUB, sb = ms % SUB;
             if (sb == 0 && !RELOAD) load_w_part(w_load, kt_cur + WD, gq);
-            if (ms % A_EVERY == 0) {
+            if (ms % A_EVERY == 0 && ms / A_EVERY < ALOADS) {
                 if constexpr (DIRECT) {
                     direct_a_part(lds_req, kt_cur + 3, ms / A_EVERY);
                 } else {
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
                 read_frags((ms + 1) & 1, lds_next, 0);
             const MFrag *a = afr[ms & 1];
             if constexpr (DIRECT && NEED_SUM) {
-                static_assert(!(DIRECT && NEED_SUM) || WM == 4, "one row tile a wave");
+                static_assert(!(DIRECT && NEED_SUM) || WM <= 4, "a row tile a wave");
                 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
                 const bf16x2_t ones2 = __builtin_bit_cast(bf16x2_t, 0x3F803F80u);
 #pragma unroll
@@ -647,7 +647,7 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
         if constexpr (DIRECT) {
             // lane halves hold the two halves of a row's k range
             const float v = rs_direct + __shfl_xor(rs_direct, 32, 64);
-            if (h == 0 && kgroup == 0) rowsum[32 * wave + nl] = v;
+            if (h == 0 && kgroup == 0 && wave < WM) rowsum[32 * wave + nl] = v;
         } else {
 #pragma unroll
         for (int i = 0; i < ALOADS; ++i) {
@@ -867,14 +867,16 @@ static int launch_big2(const SkinnyParams &p, hipStream_t stream) {
 template <int KIND, int WN, int WM, bool NEED_SUM>
 static int launch_big(const SkinnyParams &p, hipStream_t stream) {
     if (p.rows_dev) {
-        if constexpr (WM == 4) {
+        if constexpr (WM >= 3) {
             return launch_big2<KIND, WN, WM, NEED_SUM, false, true, true>(p, stream); // (taken for whole k steps only)
         } else {
             if (p.K % StepTraits<KIND>::KTILE != 0) return launch_big2<KIND, WN, WM, NEED_SUM, true, true>(p, stream);
             return launch_big2<KIND, WN, WM, NEED_SUM, false, true>(p, stream);
         }
     }
-    if constexpr (WM == 4) {
+    if constexpr (WM == 3) {
+        return launch_big2<KIND, WN, WM, NEED_SUM, false, false, true>(p, stream);
+    } else if constexpr (WM == 4) {
         // 128-row tiles: the activations straight into LDS, two workgroups a CU, or (at most a block a CU) two K groups a workgroup: 2048
         // rows x 4096 columns, K = 4096 / 11008, INT8 963 / 993 against 926 / 934 TFLOP/s, UINT4 859 / 954 against 812 / 926, NF4 519 / 569
         // against 492 / 532.  Staged through registers only for a ragged K or more than 4 GB of activations.
@@ -894,12 +896,13 @@ static int launch_big(const SkinnyParams &p, hipStream_t stream) {
 
 template <int KIND, bool NEED_SUM>
 static int dispatch_big_tile(const SkinnyParams &p, hipStream_t stream) {
-    switch (p.tile) { // (choose_tile)
+    switch (p.tile) { // (choose_tile; 5 with activations straight into LDS only)
         case 1:
             if constexpr (KIND != XFTHIP_W_BF16) return launch_big<KIND, 1, 1, NEED_SUM>(p, stream);
             break;
         case 3: return launch_big<KIND, 1, 4, NEED_SUM>(p, stream);
         case 4: return launch_big<KIND, 2, 4, NEED_SUM>(p, stream);
+        case 5: return launch_big<KIND, 2, 3, NEED_SUM>(p, stream);
         default: break;
     }
     return launch_big<KIND, 1, 2, NEED_SUM>(p, stream);
