@@ -402,56 +402,79 @@ __device__ __forceinline__ void qgemm_skinny_body(SkinnyParams &p) {
             // RMSNorm of the M rows into LDS while the first weight tiles are on their way; same
             // arithmetic as rmsnorm_vec_kernel: y = bf16((x * rstd) * w)
             float *part = red + (size_t)nwaves * (16 * MT * (16 * NT + 1) + 16 * MT);
-            xn = (uint16_t *)(part + 16);
+            xn = (uint16_t *)(part + 32);
             const int pitch = p.K + 8;
             xn_row = (ml < p.M ? ml : p.M - 1) * pitch;
-            // The norm weights are first needed behind the first row's reduction, where a miss to memory would be
-            // fully exposed: one value of each of their 128-byte lines is requested now, with the first row (4-bit
-            // kinds, whose short weight stream leaves the prologue in the open: UINT4 decode 561 -> 574 tok/s; the
-            // INT8 kernels, at their 128 registers, lose 0.7 % to the extra one)
-            constexpr bool TOUCH = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4;
-            constexpr int NB = TOUCH ? 4 : 2;
-            float w_touch = 0.0f;
-            if (TOUCH && (int)threadIdx.x * 32 < p.K) w_touch = p.norm_w[threadIdx.x * 32];
-            for (int m = 0; m < p.M; ++m) {
-                const float *row = p.norm_x + (size_t)m * p.ldx;
-                float sq = 0.0f;
-                // NB loads in flight a thread (the 4-wave workgroups of the 4-bit kinds walk a 4096-wide row in four
-                // steps: one round trip instead of four); the sums keep the order of the plain loop
-                for (int c = threadIdx.x * 4; c < p.K; c += blockDim.x * 4 * NB) {
-                    float4 v[NB];
-#pragma unroll
-                    for (int i = 0; i < NB; ++i) {
-                        const int ci = c + i * (int)blockDim.x * 4;
-                        v[i] = ci < p.K ? *(const float4 *)(row + ci) : make_float4(0.f, 0.f, 0.f, 0.f);
-                    }
-#pragma unroll
-                    for (int i = 0; i < NB; ++i) sq = fmaf(v[i].x, v[i].x, fmaf(v[i].y, v[i].y, fmaf(v[i].z, v[i].z, fmaf(v[i].w, v[i].w, sq))));
-                }
+            // NB loads in flight a thread (the 4-wave workgroups of the 4-bit kinds walk a 4096-wide row in four
+            // steps: one round trip instead of four); the sums keep the order of the plain loop
+            constexpr int NB = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4 ? 4 : 2;
+            const int stride = (int)blockDim.x * 4;
+            auto square = [](float sq, const float4 v) { return fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, sq)))); };
+            auto put = [&](int m, int c, const float4 v, const float4 w, float var) {
+                const uint32_t lo = f32x2_to_bf16((v.x * var) * w.x, (v.y * var) * w.y);
+                const uint32_t hi = f32x2_to_bf16((v.z * var) * w.z, (v.w * var) * w.w);
+                *(uint2 *)(xn + (size_t)m * pitch + c) = make_uint2(lo, hi);
+            };
+            auto sum_up = [&](int m, float sq) { // (the row's partial sums, one a wave)
 #pragma unroll
                 for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);
-                if (lane == 0) part[(m & 1) * 8 + wave] = sq;
-                __syncthreads();
-                if constexpr (TOUCH) asm volatile("" ::"v"(w_touch)); // keeps the request above alive; the value is not used
+                if (lane == 0) part[m * 8 + wave] = sq;
+            };
+            auto rstd = [&](int m) {
                 float tot = 0.0f;
-                for (int w = 0; w < nwaves; ++w) tot += part[(m & 1) * 8 + w];
-                const float var = 1.0f / sqrtf(tot / (float)p.K + p.norm_eps);
-                for (int c = threadIdx.x * 4; c < p.K; c += blockDim.x * 4 * NB) {
-                    float4 vv[NB], ww[NB];
+                for (int w = 0; w < nwaves; ++w) tot += part[m * 8 + w];
+                return 1.0f / sqrtf(tot / (float)p.K + p.norm_eps);
+            };
+            int c0 = threadIdx.x * 4;
+            asm volatile("" : "+v"(c0)); // (what follows from it would be kept in registers across the column blocks)
+            if (p.K <= stride * NB) {
+                // The workgroup holds a whole row: it and the norm weights stay in registers until the sum is known, one trip to memory in place of two.  K = 4096, 1 / 2 / 4
+                // rows: INT8, 22016 columns with SwiGLU 18.8 / 20.2 / 23.0 -> 17.8 / 19.4 / 21.6 us, 12288 with RoPE 13.1 / 14.7 / 17.9 -> 12.6 / 14.0 / 16.8; UINT4 0.91 of the time in
+                // the mean, NF4 0.96, BF16 0.97.  (Two rows at a time: INT8 1 % faster with several rows and as much slower with one; requested ahead of the
+                // weights: the same to 3 % slower; four rows: a workgroup a CU less.)
+                for (int m = 0; m < p.M; ++m) {
+                    float4 v[NB], w[NB];
 #pragma unroll
                     for (int i = 0; i < NB; ++i) {
-                        const int ci = c + i * (int)blockDim.x * 4;
-                        const int cl = ci < p.K ? ci : c; // past the row: a second read of this step's first chunk, not stored
-                        vv[i] = *(const float4 *)(row + cl);
-                        ww[i] = *(const float4 *)(p.norm_w + cl);
+                        const int c = c0 + i * stride, cl = c < p.K ? c : 0; // past the row: a read of its begin, not used
+                        w[i] = *(const float4 *)(p.norm_w + cl);
+                        v[i] = *(const float4 *)(p.norm_x + (size_t)m * p.ldx + cl);
                     }
+                    float sq = 0.0f;
 #pragma unroll
-                    for (int i = 0; i < NB; ++i) {
-                        const int ci = c + i * (int)blockDim.x * 4;
-                        const float4 v = vv[i], w = ww[i];
-                        const uint32_t lo = f32x2_to_bf16((v.x * var) * w.x, (v.y * var) * w.y);
-                        const uint32_t hi = f32x2_to_bf16((v.z * var) * w.z, (v.w * var) * w.w);
-                        if (ci < p.K) *(uint2 *)(xn + (size_t)m * pitch + ci) = make_uint2(lo, hi);
+                    for (int i = 0; i < NB; ++i) sq = square(sq, c0 + i * stride < p.K ? v[i] : make_float4(0.f, 0.f, 0.f, 0.f));
+                    sum_up(m, sq);
+                    __syncthreads();
+                    const float var = rstd(m);
+#pragma unroll
+                    for (int i = 0; i < NB; ++i)
+                        if (c0 + i * stride < p.K) put(m, c0 + i * stride, v[i], w[i], var);
+                }
+            } else {
+                for (int m = 0; m < p.M; ++m) {
+                    const float *row = p.norm_x + (size_t)m * p.ldx;
+                    float sq = 0.0f;
+                    for (int c = c0; c < p.K; c += stride * NB) {
+                        float4 v[NB];
+#pragma unroll
+                        for (int i = 0; i < NB; ++i) v[i] = c + i * stride < p.K ? *(const float4 *)(row + c + i * stride) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                        for (int i = 0; i < NB; ++i) sq = square(sq, v[i]);
+                    }
+                    sum_up(m, sq);
+                    __syncthreads();
+                    const float var = rstd(m);
+                    for (int c = c0; c < p.K; c += stride * NB) {
+                        float4 vv[NB], ww[NB];
+#pragma unroll
+                        for (int i = 0; i < NB; ++i) {
+                            const int cl = c + i * stride < p.K ? c + i * stride : c; // past the row: a second read of this step's first chunk, not stored
+                            vv[i] = *(const float4 *)(row + cl);
+                            ww[i] = *(const float4 *)(p.norm_w + cl);
+                        }
+#pragma unroll
+                        for (int i = 0; i < NB; ++i)
+                            if (c + i * stride < p.K) put(m, c + i * stride, vv[i], ww[i], var);
                     }
                 }
             }
@@ -480,6 +503,13 @@ __device__ __forceinline__ void qgemm_skinny_body(SkinnyParams &p) {
                 arrived(1);
                 compute(1, b_begin + b);
             } else {
+                if constexpr (NORM) {
+                    // (or the compiler widens the codes of both branches' products ahead of the branch and takes twice the registers)
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(wbuf[0][u][t]));
+                }
                 compute(0, b_begin + b - 1);
             }
         }
@@ -698,7 +728,7 @@ static int launch(const SkinnyParams &p, int kslices, hipStream_t stream) {
         smem = smem > patches ? smem : patches;
     }
     smem += (KIND == XFTHIP_W_NF4 ? 2048 : 0);
-    if (NORM) smem += 64 + skinny_norm_lds_bytes(p.M, p.K);
+    if (NORM) smem += 128 + skinny_norm_lds_bytes(p.M, p.K);
     int blocks = (p.NTILES + NT - 1) / NT;
     if (ROPE) blocks = (p.qH + 2 * p.kvH) * 4 / (NT / 2); // rotation pairs of the query and key heads, then value tile pairs
     SkinnyParams q = p;
