@@ -357,6 +357,23 @@ def test_many_sequences_decode_together(xh, act):
     c.free()
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65])
+def test_one_token_each(xh, n):
+    """steps of one token a sequence, described by a kernel's arguments up to 64 of them: slots out of order, a first token and later ones (the pair embedding
+    reads the token before), the logits of all in order, of all in another order, of some"""
+    cfg = whole_config()
+    c = Case(xh, cfg, 19, "f32", slots=n + 1, max_seq=64, max_tokens=n + 1)
+    slots = np.random.default_rng(n).permutation(n + 1)[:n]
+    seqs = [tokens_of(cfg, 4, 300 + i) for i in range(n)]
+    want = np.stack([c.want(s) for s in seqs])
+    for t in range(4):
+        order = np.arange(n) if t != 1 else np.arange(n)[::-1]
+        rows = [[0] if t != 2 or i % 2 == 0 else [] for i in order]
+        got = c.model.step([(int(slots[i]), seqs[i][t:t + 1], r) for i, r in zip(order, rows)])
+        c.check(got, want[[i for i, r in zip(order, rows) if r], t], f"token {t}")
+    c.free()
+
+
 def test_slots_that_sit_out(xh):
     cfg = whole_config()
     c = Case(xh, cfg, 14, "f32", slots=3, max_seq=256)

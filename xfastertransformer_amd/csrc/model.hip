@@ -867,7 +867,9 @@ int xfthip_model_step(xfthip_model_t m, int n, const int *rows_host, const int *
         total += lens_host[i];
     }
     for (int i = 0; i < n_want; ++i) XFT_REQUIRE(want_host[i] >= 0 && want_host[i] < total, "xfthip_model_step: logits of token %d of %ld asked for", want_host[i], total);
-    if (int rc = plan_run(m, n, rows_host, lens_host, ids_host, st)) return rc;
+    bool all = n_want == total && n_want <= m->plan->logit_rows; // the logits of every token, in order
+    for (int i = 0; i < n_want && all; ++i) all = want_host[i] == i;
+    if (int rc = plan_run(m, n, rows_host, lens_host, ids_host, st, all)) return rc;
     m->prompt_rows = (int)total;
     m->cur_B = 0;
     for (int r = 0; r < c.max_batch; ++r)

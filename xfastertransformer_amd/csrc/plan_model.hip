@@ -67,6 +67,25 @@ __global__ void plan_advance_kernel(const int *seg, int seg_cap, int n, const in
     last_token[seg[b]] = ids[seg[seg_cap + b] + seg[2 * seg_cap + b] - 1];
 }
 
+// A step of one token a sequence: its description (by value: no trip to the host's memory), the embeddings, and where the sequences stand behind it, in one
+// launch in place of three (plan_describe, plan_embed, plan_advance).  Up to kBeginTokens of them: 768 bytes of arguments.
+// Bound by the launch (about 4 us with the trip of the description over the bus, as much for each of the other two): a prompt and its decode steps 8.82 ->
+// 8.67 ms over two expert layers, and with the final norm inside the last pass over the residual 6.95 -> 6.89 over three of latent attention and delta rule.
+constexpr int kBeginTokens = 64;
+struct BeginTokens {
+    int row[kBeginTokens], at[kBeginTokens], id[kBeginTokens];
+};
+__global__ void plan_step_begin_kernel(EmbedTables e, BeginTokens s, float *x, int *last_token, int *tok_seg, int *tok_pos, int *tok_ids, int *seg, int seg_cap, int *pos) {
+    const int b = blockIdx.x, row = s.row[b], at = s.at[b], id = s.id[b], prev = last_token[row];
+    __syncthreads(); // (all have read the token before)
+    if (threadIdx.x == 0) {
+        tok_seg[b] = b, tok_pos[b] = at, tok_ids[b] = id;
+        seg[b] = row, seg[seg_cap + b] = b, seg[2 * seg_cap + b] = 1, seg[3 * seg_cap + b] = at;
+        last_token[row] = id, pos[row] = at + 1;
+    }
+    embed_token(e, id, at == 0, prev, x + (size_t)b * e.hidden);
+}
+
 // ahead of a step: its description from pinned host memory (tok_seg | tok_pos | ids, `stride` apart, T of each; 4 seg_cap segment entries behind
 // them) into the device's copy, which is laid out alike.  One launch of 4 us for four copies of 5 us each, which the first kernel waited for
 __global__ void plan_describe_kernel(const int *host, int stride, int T, int seg_ints, int *desc) {
@@ -356,8 +375,9 @@ int run_side(xfthip_model *m, const PlanLayer &L, int layer, int T, const void *
     return plan_gemm(m, L.side_proj, T, p.side, pad, p.y, hidden, XFTHIP_F32, st);
 }
 
-// all layer runs over the step's tokens, whose embeddings are in m->x
-int plan_layers(xfthip_model *m, const StepView &v, hipStream_t st) {
+// all layer runs over the step's tokens, whose embeddings are in m->x.  head_follows: the logits of all of them, in order, are wanted next, so the final norm joins
+// the last layer's own pass over the residual where there is one (p.final_normed)
+int plan_layers(xfthip_model *m, const StepView &v, hipStream_t st, bool head_follows) {
     PlanState &p = *m->plan;
     const xfthip_plan &plan = *p.plan;
     const int T = v.T, hidden = m->cfg.hidden;
@@ -373,8 +393,11 @@ int plan_layers(xfthip_model *m, const StepView &v, hipStream_t st) {
         return plan_norm(p.act, a, T, st);
     };
     const PlanNorm none;
-    auto enter = [&](const float *y, const float *post, bool again, const PlanLayer *next) {
-        return norm(y, post, again, next ? next->pre1 : none, next && parallel ? next->pre2 : none, nullptr);
+    const PlanNorm &behind = head_follows && !p.trace ? plan.final_norm : none; // of the last layer
+    p.final_normed = false;
+    auto enter = [&](const float *y, const float *post, bool again, const PlanLayer *next, bool last = false) {
+        p.final_normed = last && head_follows && !p.trace;
+        return norm(y, post, again, next ? next->pre1 : last ? behind : none, next && parallel ? next->pre2 : none, nullptr);
     };
     if ((rc = enter(nullptr, nullptr, plan.runs[0].add_embedding, &p.layers[plan.runs[0].layer]))) return rc;
     for (int r = 0; r < nruns; ++r) {
@@ -391,12 +414,13 @@ int plan_layers(xfthip_model *m, const StepView &v, hipStream_t st) {
             if ((ff || narrow_out) && (rc = run_feed_forward(m, L, T, p.xn2, narrow_out, st))) return rc;
             if (side && (rc = run_side(m, L, plan.runs[r].layer, T, narrow, st))) return rc;
             if (!last || side)
-                if ((rc = enter(side ? p.y : nullptr, L.side_post, join, then))) return rc;
+                if ((rc = enter(side ? p.y : nullptr, L.side_post, join, then, last))) return rc;
         } else {
-            if ((rc = norm(p.y, L.post1, !ff && join, ff ? L.pre2 : then ? then->pre1 : none, none, &L))) return rc;
+            p.final_normed = last && !ff && head_follows && !p.trace;
+            if ((rc = norm(p.y, L.post1, !ff && join, ff ? L.pre2 : then ? then->pre1 : last ? behind : none, none, &L))) return rc;
             if (ff) {
                 if ((rc = run_feed_forward(m, L, T, p.xn, nullptr, st))) return rc;
-                if ((rc = enter(p.y, L.post2, join, then))) return rc;
+                if ((rc = enter(p.y, L.post2, join, then, last))) return rc;
             }
         }
         if (p.trace) {
@@ -453,7 +477,7 @@ void plan_release(xfthip_model *m, int row) {
     }
 }
 
-int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int *ids, hipStream_t st) {
+int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int *ids, hipStream_t st, bool head_follows) {
     PlanState &p = *m->plan;
     const xfthip_model_config &c = m->cfg;
     XFT_REQUIRE(n > 0 && n <= p.slots, "a step of %d entries; the model has %d slots", n, p.slots);
@@ -484,10 +508,6 @@ int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int
         hg[i] = rows[i], hg[cap + i] = t, hg[2 * cap + i] = lens[i], hg[3 * cap + i] = at;
         for (int k = 0; k < lens[i]; ++k, ++t) hs[t] = i, hp[t] = at + k, hi[t] = ids[t];
     }
-    hipLaunchKernelGGL(plan_describe_kernel, dim3((std::max((int)T, 4 * cap) + 255) / 256), dim3(256), 0, st, p.desc_host, mt, (int)T, 4 * cap, p.desc);
-    XFT_CHECK_HIP(hipGetLastError());
-    const StepView view = view_of(m, n, (int)T, longest);
-    if (int rc = plan_embed(embed_tables(m), view, p.ids, p.last_token, m->x, st)) return rc;
     m->len_hint = deepest;
     if (p.trace) {
         const size_t need = p.plan->runs.size() * (size_t)T * c.hidden;
@@ -500,9 +520,23 @@ int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int
         }
         p.trace_tokens = (int)T;
     }
-    if (int rc = plan_layers(m, view, st)) return rc;
-    hipLaunchKernelGGL(plan_advance_kernel, dim3((n + 63) / 64), dim3(64), 0, st, p.seg, cap, n, p.ids, m->pos, p.last_token);
-    XFT_CHECK_HIP(hipGetLastError());
+    const StepView view = view_of(m, n, (int)T, longest);
+    const bool at_once = longest == 1 && n <= kBeginTokens;
+    if (at_once) {
+        BeginTokens s;
+        for (int i = 0; i < n; ++i) s.row[i] = rows[i], s.at[i] = hp[i], s.id[i] = ids[i];
+        hipLaunchKernelGGL(plan_step_begin_kernel, dim3(n), dim3(256), 0, st, embed_tables(m), s, m->x, p.last_token, p.tok_seg, p.tok_pos, p.ids, p.seg, cap, m->pos);
+        XFT_CHECK_HIP(hipGetLastError());
+    } else {
+        hipLaunchKernelGGL(plan_describe_kernel, dim3((std::max((int)T, 4 * cap) + 255) / 256), dim3(256), 0, st, p.desc_host, mt, (int)T, 4 * cap, p.desc);
+        XFT_CHECK_HIP(hipGetLastError());
+        if (int rc = plan_embed(embed_tables(m), view, p.ids, p.last_token, m->x, st)) return rc;
+    }
+    if (int rc = plan_layers(m, view, st, head_follows)) return rc;
+    if (!at_once) {
+        hipLaunchKernelGGL(plan_advance_kernel, dim3((n + 63) / 64), dim3(64), 0, st, p.seg, cap, n, p.ids, m->pos, p.last_token);
+        XFT_CHECK_HIP(hipGetLastError());
+    }
     for (int i = 0; i < n; ++i) m->row_pos[rows[i]] = std::max(m->row_pos[rows[i]], 0) + lens[i];
     return 0;
 }
@@ -514,7 +548,9 @@ int plan_head(xfthip_model *m, const int *rows_dev, int n, int at, hipStream_t s
     const xfthip_model_config &c = m->cfg;
     const PlanNormArgs a = {m->x, nullptr, nullptr, nullptr, nullptr, c.vocab, plan.final_norm, {}, p.xn, nullptr, rows_dev, c.hidden, plan.cfg.hidden, c.rms_eps, 0.0f,
             plan.cfg.norm_groups};
-    if (int rc = plan_norm(p.act, a, n, st)) return rc;
+    if (!p.final_normed)
+        if (int rc = plan_norm(p.act, a, n, st)) return rc;
+    p.final_normed = false; // (of this step's tokens only, and once)
     float *logits = m->logits + (size_t)at * c.vocab;
     if (int rc = plan_gemm(m, plan.head, n, p.xn, c.hidden, logits, c.vocab, XFTHIP_F32, st)) return rc;
     return plan.cfg.logit_softcap > 0.0f ? plan_softcap(logits, (size_t)n * c.vocab, plan.cfg.logit_softcap, st) : 0;
@@ -632,7 +668,7 @@ int plan_decode_step(xfthip_model *m, int B, hipStream_t st) {
     // (lengths and offsets only: where the segments stand is known on the device)
     p.seg_off_host.resize(B), p.seg_len_host.assign(B, 1), p.seg_pos_host.assign(B, 0), p.seg_row_host.assign(B, 0);
     for (int b = 0; b < B; ++b) p.seg_off_host[b] = b;
-    int rc = plan_layers(m, view_of(m, B, B, 1), st);
+    int rc = plan_layers(m, view_of(m, B, B, 1), st, true);
     p.trace = trace;
     if (rc) return rc;
     if ((rc = plan_head(m, nullptr, B, 0, st))) return rc;
