@@ -119,6 +119,21 @@ def test_many_experts(xh, act, routes):
     c.free()
 
 
+@pytest.mark.parametrize("act", ["f32", "bf16"])
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,conv", [(2, 2, 128, 128, 4), (4, 2, 250, 64, 2), (2, 2, 128, 130, 3), (2, 1, 64, 256, 3), (3, 3, 20, 250, 4), (3, 1, 32, 96, 4)], ids=str)
+def test_delta_tokens_one_by_one(xh, heads, kv_heads, dim, vdim, conv, act):
+    """one decay a head and the gate in the rows: states that fit a workgroup's registers whole, and others, two sequences, one of them behind a portion"""
+    cfg = u.config([(u.windowed_delta(r_heads=heads, r_kv_heads=kv_heads, r_dim=dim, r_vdim=vdim, conv=conv, left=0.0), None)])
+    c = Case(xh, cfg, 23, act)
+    a, b = tokens_of(cfg, 14, 1), tokens_of(cfg, 22, 2)
+    wa, wb = c.want(a), c.want(b)
+    c.run(3, b[:8], [8], "portion", wb[:8])
+    for i in range(14):
+        got = c.model.step([(1, a[i:i + 1], [0]), (3, b[8 + i:9 + i], [0])])
+        c.check(got, np.stack([wa[i], wb[8 + i]]), f"token {i}")
+    c.free()
+
+
 def whole_config(**kw):
     return u.config([(u.windowed_delta(), u.dense()), (u.chunked(heads=4, kv_heads=4, dim=16, vdim=16), u.moe()), (u.keyed_unit(), u.moe(experts=9, top=2, groups=3, keep=2)),
                      (u.chunked(heads=4, kv_heads=4, dim=16, vdim=16, kv_from=1, chunk=53), None), (u.windowed_delta(window=65, conv=4), u.moe(top=1)),

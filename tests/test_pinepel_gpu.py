@@ -71,6 +71,23 @@ def test_mechanism_alone(xh, name, act, mlp):
     c.free()
 
 
+@pytest.mark.parametrize("act", ["f32", "bf16"])
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,conv", [(2, 2, 128, 128, 4), (2, 2, 128, 129, 4), (4, 2, 256, 64, 2), (2, 1, 250, 65, 3), (3, 3, 64, 256, 3), (2, 1, 40, 250, 4),
+                                                          (3, 1, 32, 96, 4), (2, 2, 32, 264, 2), (4, 4, 20, 12, 3), (2, 2, 128, 100, 5)], ids=str)
+def test_delta_tokens_one_by_one(xh, heads, kv_heads, dim, vdim, conv, act):
+    """states that fit a workgroup's registers whole, up to the last column, and the first that do not; one and two heads a key head, and three; all filters;
+    from the first token, and behind a portion, while another sequence is longer"""
+    cfg = u.config([u.delta(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, conv=conv)])
+    c = Case(xh, cfg, 23, act)
+    a, b = tokens_of(cfg, 14, 1), tokens_of(cfg, 22, 2)
+    wa, wb = c.want(a), c.want(b)
+    c.run(3, b[:8], [8], "portion", wb[:8])
+    for i in range(14):
+        got = c.model.step([(1, a[i:i + 1], [0]), (3, b[8 + i:9 + i], [0])])
+        c.check(got, np.stack([wa[i], wb[8 + i]]), f"token {i}")
+    c.free()
+
+
 def whole_config(**kw):
     return u.config([u.latent(window=37), u.latent(), u.delta(), u.latent(window=70, heads=2, kv_rank=64), u.delta(heads=2, kv_heads=2, dim=32, vdim=24, conv=2)],
                     loop=dict(start=1, stop=4, times=3), **kw)

@@ -493,6 +493,112 @@ __global__ __launch_bounds__(256) void delta_output_kernel(OutParams p) {
     }
 }
 
+// A step of one token a sequence, from the input product's rows to the output product's: convolutions, norms, decays, the state's step and the gated norm of a
+// key head's heads in one workgroup, where the state of a head fits its registers (16 floats a thread).  The channels of a token are spread over the threads
+// (q | k | v | decays, 256 each) and meet in LDS; the state is requested in front of that work, so that it arrives behind it.  A key head's workgroup alone
+// touches its convolution inputs, which it shifts in place.
+// Bound by latency (a chain of two loads, two barriers, a store): a step of 16 heads of 128 x 128 in three launches / in one,
+// six layers of it, BF16: 1 sequence 148 / 119 us, 4 179 / 139, 16 223 / 175, 64 465 / 404; 64 x 64 142 / 108 .. 248 / 247, 64 x 256 171 / 129 .. 488 / 421.
+template <bool BF16, int L, bool ONE>
+__global__ __launch_bounds__(1024) void delta_decode_kernel(PrepParams p, OutParams out) {
+    constexpr int DT = BF16 ? XFTHIP_BF16 : XFTHIP_F32, KD = 8 * L, COLS = 1024 / L;
+    __shared__ __align__(16) float qs[KD], ks[KD], gs[KD], vs[256], os[256], part[8];
+    const int seg = blockIdx.x, kvh = blockIdx.y, each = p.H / p.KH, tid = threadIdx.x, lane = tid & 63;
+    const int t = p.v.seg_off[seg], row = p.v.seg_row[seg], start = p.v.seg_pos[seg];
+    const int li = tid % L, col0 = tid / L, role = tid >> 8, c = tid & 255, taps = p.taps;
+    const size_t hist = (size_t)row * (taps - 1) * p.channels, in_row = (size_t)t * p.ld;
+    f32x4 q0, q1, k0, k1;
+    float qk = 0.0f;
+    for (int r = 0; r < each; ++r) {
+        const int head = kvh * each + r;
+        const int ch = (role == 2 ? 2 * p.KH : role * p.KH + kvh) * KD + (role == 2 ? head * p.VD : 0) + c;
+        const bool conv = role == 2 ? c < p.VD : role < 2 && r == 0 && c < KD, gate = role == 3 && !ONE && c < KD;
+        float x[3] = {0.0f, 0.0f, 0.0f}, w[4] = {0.0f, 0.0f, 0.0f, 0.0f}, in = 0.0f, dt = 0.0f;
+        if (conv) { // (x, w: the last three of at most four taps)
+            in = ldb<BF16>(p.b.in, in_row + ch);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (j >= 4 - taps) w[j] = p.conv[(size_t)ch * taps + j - (4 - taps)];
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (j >= 4 - taps && start - 3 + j >= 0) x[j] = ldb<BF16>(p.b.conv_state, hist + (size_t)(j - (4 - taps)) * p.channels + ch);
+        }
+        if (gate) in = p.b.gates[(size_t)t * 2 * p.gcols + head * KD + c], dt = p.dt_bias[head * KD + c];
+        if (ONE && role == 3) in = ldb<BF16>(p.b.in, in_row + p.decay_col + head), dt = p.dt_bias[head];
+        const float decay = p.decay[head], beta = sigmoid_of<BF16>(ldb<BF16>(p.b.in, in_row + p.beta_col + head));
+        float z = 0.0f, ow = 0.0f;
+        if (tid < p.VD) {
+            z = out.row_gate ? ldb<BF16>(out.row_gate, (size_t)t * out.ld + head * p.VD + tid) : out.gates[(size_t)t * 2 * out.gcols + out.gcols + head * p.VD + tid];
+            ow = out.norm[tid];
+        }
+        float *state = p.b.state + ((size_t)row * p.H + head) * p.VD * KD + 4 * li;
+        f32x4 s[2][2];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const int col = col0 + n * COLS;
+            s[n][0] = s[n][1] = f32x4 {0.f, 0.f, 0.f, 0.f};
+            if (col < p.VD && start > 0) s[n][0] = *(const f32x4 *)(state + (size_t)col * KD), s[n][1] = *(const f32x4 *)(state + (size_t)col * KD + 4 * L);
+        }
+        if (conv) {
+            float a = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 3; ++j) a = fmaf(w[j], x[j], a);
+            a = silu_of<BF16>(fmaf(w[3], in, a));
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (j >= 4 - taps) store_from_f32(p.b.conv_state, DT, hist + (size_t)(j - (4 - taps)) * p.channels + ch, j < 2 ? x[j + 1] : in);
+            (role == 0 ? qs : role == 1 ? ks : vs)[c] = a;
+            dt = a * a;
+        }
+        if (role < 2 && r == 0) { // (whole waves)
+            const float sum = wave_total(conv ? dt : 0.0f);
+            if (lane == 0) part[tid >> 6] = sum;
+        }
+        if (gate || (ONE && role == 3 && c == 0)) gs[c] = exp_of<BF16>(-decay * softplus_of<BF16>(in + dt));
+        __syncthreads();
+        if (r == 0) {
+            const float sq = 1.0f / sqrtf((part[0] + part[1]) + (part[2] + part[3]) + 1e-6f) * p.qscale, sk = 1.0f / sqrtf((part[4] + part[5]) + (part[6] + part[7]) + 1e-6f);
+            q0 = *(const f32x4 *)(qs + 4 * li), q1 = *(const f32x4 *)(qs + 4 * (L + li)), k0 = *(const f32x4 *)(ks + 4 * li), k1 = *(const f32x4 *)(ks + 4 * (L + li));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                q0[i] *= sq, q1[i] *= sq, k0[i] *= sk, k1[i] *= sk;
+                qk = fmaf(q0[i], k0[i], fmaf(q1[i], k1[i], qk));
+            }
+            qk = group_sum<L>(qk);
+        }
+        f32x4 g0, g1;
+        if constexpr (ONE) {
+            const float fade = gs[0];
+            g0 = g1 = f32x4 {fade, fade, fade, fade};
+        } else g0 = *(const f32x4 *)(gs + 4 * li), g1 = *(const f32x4 *)(gs + 4 * (L + li));
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const int col = col0 + n * COLS;
+            if (col >= p.VD) continue; // (whole groups of L lanes)
+            f32x4 s0 = s[n][0] * g0, s1 = s[n][1] * g1;
+            float a = 0.0f, b = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a = fmaf(k0[i], s0[i], a), b = fmaf(q0[i], s0[i], b);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a = fmaf(k1[i], s1[i], a), b = fmaf(q1[i], s1[i], b);
+            a = group_sum<L>(a), b = group_sum<L>(b);
+            const float u = beta * (vs[col] - a);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s0[i] = fmaf(k0[i], u, s0[i]), s1[i] = fmaf(k1[i], u, s1[i]);
+            *(f32x4 *)(state + (size_t)col * KD) = s0, *(f32x4 *)(state + (size_t)col * KD + 4 * L) = s1;
+            if (li == 0) os[col] = fmaf(qk, u, b);
+        }
+        __syncthreads();
+        if (tid < (p.VD + 63) / 64 * 64) { // (whole waves; each adds up all of the head by itself)
+            float sq = 0.0f;
+            for (int i = lane; i < p.VD; i += 64) sq = fmaf(os[i], os[i], sq);
+            const float f = 1.0f / sqrtf(wave_total(sq) / (float)out.vdim + out.eps) * out.mul;
+            z = out.row_gate ? silu_of<BF16>(z) : sigmoid_of<BF16>(z);
+            if (tid < p.VD) store_from_f32(out.out, DT, (size_t)t * out.out_ld + head * p.VD + tid, os[tid] * f * ow * z);
+        }
+    }
+}
+
 PrepParams prep_params(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b) {
     PrepParams p;
     p.v = v, p.b = b;
@@ -504,9 +610,15 @@ PrepParams prep_params(int act, const PlanLayer &L, const StepView &v, const Del
     return p;
 }
 
-int launch_output(int act, const PlanLayer &L, int T, OutParams p, float eps, hipStream_t st) {
-    p.out = (char *)p.out + (size_t)L.out_col * (act == XFTHIP_BF16 ? 2 : 4), p.out_ld = L.out_ld;
+// row_in: the input product's rows, if the gate is in them
+OutParams out_params(int act, const PlanLayer &L, int T, const float *o, const float *gates, const void *row_in, void *out, float eps) {
+    const int esz = act == XFTHIP_BF16 ? 2 : 4;
+    OutParams p = {o, gates, L.out_norm, row_in ? (const char *)row_in + (size_t)L.out_gate_col() * esz : nullptr, L.in_ld, (char *)out + (size_t)L.out_col * esz, L.out_ld};
     p.H = L.s.heads, p.VD = L.VD, p.vdim = L.s.vdim, p.gcols = L.gcols, p.T = T, p.eps = eps, p.mul = L.mix_scale;
+    return p;
+}
+
+int launch_output(int act, const OutParams &p, int T, hipStream_t st) {
     const unsigned blocks = (unsigned)(((size_t)T * p.H + 3) / 4);
     if (act == XFTHIP_BF16) hipLaunchKernelGGL(delta_output_kernel<true>, dim3(blocks), dim3(256), 0, st, p);
     else hipLaunchKernelGGL(delta_output_kernel<false>, dim3(blocks), dim3(256), 0, st, p);
@@ -592,11 +704,41 @@ int delta_scan(const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hip
 
 int delta_output(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, float eps, hipStream_t st) {
     if (L.silu_gate()) return gated_head_norm(act, L, v.T, b.o, b.in, b.out, eps, st);
-    return launch_output(act, L, v.T, {b.o, b.gates, L.out_norm, nullptr, L.in_ld, b.out}, eps, st);
+    return launch_output(act, out_params(act, L, v.T, b.o, b.gates, nullptr, b.out, eps), v.T, st);
+}
+
+// The state of a head in the registers of one workgroup.  A second head of a key head follows the first in its workgroup: of the 29 and 40 us that six layers
+// of 16 x 128 x 128 save at 1 and 4 sequences 14 and 16 are left with 8 key heads (38 of 49 at 16, 72 of 60 at 64); a third would take what is left.
+bool delta_decodes_at_once(const PlanLayer &L, const StepView &v) {
+    return v.longest == 1 && L.s.taps >= 2 && L.s.taps <= 4 && L.KD <= 256 && L.VD <= 256 && L.KD * L.VD <= 16 * 1024 && L.s.heads <= 2 * L.s.kv_heads;
+}
+
+int delta_decode(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, float eps, hipStream_t st) {
+    const PrepParams p = prep_params(act, L, v, b);
+    const OutParams out = out_params(act, L, v.T, nullptr, b.gates, L.silu_gate() ? b.in : nullptr, b.out, eps);
+    const dim3 grid(v.B, p.KH);
+    const bool one = L.head_decay();
+    auto launch = [&](auto several, auto single) {
+        if (one) hipLaunchKernelGGL(single, grid, dim3(1024), 0, st, p, out);
+        else hipLaunchKernelGGL(several, grid, dim3(1024), 0, st, p, out);
+    };
+    switch ((act == XFTHIP_BF16 ? 0 : 1000) + L.KD) {
+        case 32: launch(delta_decode_kernel<true, 4, false>, delta_decode_kernel<true, 4, true>); break;
+        case 64: launch(delta_decode_kernel<true, 8, false>, delta_decode_kernel<true, 8, true>); break;
+        case 128: launch(delta_decode_kernel<true, 16, false>, delta_decode_kernel<true, 16, true>); break;
+        case 256: launch(delta_decode_kernel<true, 32, false>, delta_decode_kernel<true, 32, true>); break;
+        case 1032: launch(delta_decode_kernel<false, 4, false>, delta_decode_kernel<false, 4, true>); break;
+        case 1064: launch(delta_decode_kernel<false, 8, false>, delta_decode_kernel<false, 8, true>); break;
+        case 1128: launch(delta_decode_kernel<false, 16, false>, delta_decode_kernel<false, 16, true>); break;
+        case 1256: launch(delta_decode_kernel<false, 32, false>, delta_decode_kernel<false, 32, true>); break;
+        default: set_error("delta_decode: key dimension %d of a head is above 256", L.s.dim); return 2;
+    }
+    XFT_CHECK_HIP(hipGetLastError());
+    return 0;
 }
 
 int gated_head_norm(int act, const PlanLayer &L, int T, const float *o, const void *in, void *out, float eps, hipStream_t st) {
-    return launch_output(act, L, T, {o, nullptr, L.out_norm, (const char *)in + (size_t)L.out_gate_col() * (act == XFTHIP_BF16 ? 2 : 4), L.in_ld, out}, eps, st);
+    return launch_output(act, out_params(act, L, T, o, nullptr, in, out, eps), T, st);
 }
 
 } // namespace xfthip

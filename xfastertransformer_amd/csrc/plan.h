@@ -278,6 +278,9 @@ struct DeltaBuffers {
 };
 // the last taps - 1 inputs of segments of several tokens: in [T] rows of pitch ld -> conv_state
 int conv_tail(int act, const StepView &v, const void *in, int ld, int channels, int taps, void *conv_state, hipStream_t st);
+// steps of one token a sequence: all three of the following in one launch, where it takes the layer
+bool delta_decodes_at_once(const PlanLayer &L, const StepView &v);
+int delta_decode(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, float eps, hipStream_t st);
 int delta_prepare(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st);
 int delta_scan(const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st);
 int delta_output(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, float eps, hipStream_t st);

@@ -240,6 +240,7 @@ int mix_delta(xfthip_model *m, const PlanLayer &L, int store, const StepView &v,
         if ((rc = plan_gemm_heads(act, L.gates, v.T, (const char *)p.a + (size_t)first * p.esz, L.in_ld, L.gcols, L.rank, p.gates, 2 * L.gcols, XFTHIP_F32, st)))
             return rc;
     }
+    if (delta_decodes_at_once(L, v)) return delta_decode(act, L, v, b, m->cfg.rms_eps, st);
     if ((rc = delta_prepare(act, L, v, b, st))) return rc;
     if ((rc = delta_scan(L, v, b, st))) return rc;
     return delta_output(act, L, v, b, m->cfg.rms_eps, st);
