@@ -216,3 +216,38 @@ def test_lockstep_and_per_sequence_decode_alternate_at_one_batch(xh, orc):
     fresh.seq_prefill(0, pa)
     solo = [int(fresh.seq_decode([0])[0]) for _ in range(3)]
     assert a_next == solo[2], (a_next, solo)
+
+
+@pytest.mark.parametrize("rows", [1, 32, 33, 2048, 2049])
+def test_rows_taking_part(xh, orc, rows):
+    """up to 2048 cache rows the ones that step travel as bits of the first launch's arguments: rows at the borders of the words, the last row, some sitting out;
+    a released row handed to another sequence"""
+    from test_layer_model_gpu import make_layer_weights, to_device_weights
+    hidden, inter, qh, kvh, D, vocab, steps = 256, 512, 2, 1, 128, 500, 4
+    rng = np.random.default_rng(17)
+    model = xh.Model(1, hidden, inter, qh, kvh, D, vocab=vocab, max_batch=rows, max_seq=32, max_tokens=max(rows, 32), kv_dtype=xh.FP16)
+    ones = np.ones(hidden, np.float32)
+    model.set_layer(0, *to_device_weights(xh, make_layer_weights(orc, rng, 0, hidden, inter, qh, kvh, D), 0), ones, ones)
+    lm = orc.round_bf16(rng.standard_normal((hidden, vocab)) * 0.05)
+    model.set_head(orc.to_fp16(rng.standard_normal((vocab, hidden)) * 0.5), ones, xh.Weight(xh.W_BF16, hidden, vocab, orc.to_bf16(lm)))
+    at = sorted({r for r in (0, 31, 32, rows - 1) if r < rows})
+    prompts = {r: rng.integers(0, vocab, 3 + i).tolist() for i, r in enumerate(at)}
+    alone = {r: _alone(model, p, steps) for r, p in prompts.items()}
+    got = {}
+    for r in at:
+        logits = model.seq_prefill(r, prompts[r], want_logits=True)
+        got[r] = [int(model.last_ids(rows)[r])]
+        np.testing.assert_allclose(logits, alone[r][1][0], atol=2e-2, rtol=0)
+    turns = [[r for i, r in enumerate(at) if (i + t) % 3] or at for t in range(2 * steps)]
+    for rr in turns:
+        rr = [r for r in rr if len(got[r]) <= steps]
+        if not rr:
+            continue
+        for r, token in zip(rr[::-1], model.seq_decode(rr[::-1])):
+            got[r].append(int(token))  # (a row that sits out keeps its token, not its logits)
+            np.testing.assert_allclose(model.seq_logits(r), alone[r][1][len(got[r]) - 1], atol=2e-2, rtol=0)
+    for r in at:
+        assert got[r] == alone[r][0][:len(got[r])] and len(got[r]) >= 2, f"row {r}"
+    model.seq_release(at[-1])
+    np.testing.assert_allclose(model.seq_prefill(at[-1], prompts[at[0]], want_logits=True), alone[at[0]][1][0], atol=2e-2, rtol=0)
+    assert int(model.seq_decode([at[-1]])[0]) == alone[at[0]][0][1]

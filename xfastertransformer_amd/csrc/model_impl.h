@@ -59,7 +59,8 @@ struct xfthip_model {
     int row0 = 0; // cache row of the first sequence of the forward call in flight
     bool ragged = false; // rows may differ in position or sit out a step (set by the xfthip_model_seq_* calls)
     int *active = nullptr; // device [max_batch]: rows taking part in the next decode call
-    int *prompt_ids = nullptr; // device [max_tokens]: prompt of a single-sequence prefill
+    float *seq_pinned = nullptr; // pinned, of a serving loop: logits of a row [vocab] | ids of a step [max_batch] | prompt [max_tokens]
+    int *seq_ids() const { return (int *)(seq_pinned + cfg.vocab); }
     std::vector<int> row_pos; // host copy of every row's position (-1 = free row)
     unsigned char *kv_stage = nullptr; // staging buffer of xfthip_model_seq_reorder (grown on demand)
     size_t kv_stage_bytes = 0;
