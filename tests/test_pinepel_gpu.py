@@ -71,6 +71,18 @@ def test_mechanism_alone(xh, name, act, mlp):
     c.free()
 
 
+@pytest.mark.parametrize("rot,heads,kv_rank", [(2, 3, 40), (4, 3, 64), (8, 3, 64), (16, 5, 128), (24, 3, 40), (32, 16, 256), (40, 3, 500), (48, 1, 256), (64, 16, 512)], ids=str)
+@pytest.mark.parametrize("window", [None, 50], ids=["halves", "neighbours"])
+def test_queries_rotated_where_they_are_loaded(xh, rot, heads, kv_rank, window):
+    """short segments' queries are rotated by the attention itself where vectors of pairs are whole, longer ones' and all others in front of it"""
+    cfg = u.config([u.latent(heads=heads, rot=rot, kv_rank=kv_rank, window=window)])
+    c = Case(xh, cfg, 29, "bf16")
+    t = tokens_of(cfg, 150, 5)
+    c.run(0, t, [40, 1, 31, 32, 2, 33, 1, 3], "portions")
+    c.run(1, t[:12], [1], "one by one")
+    c.free()
+
+
 @pytest.mark.parametrize("act", ["f32", "bf16"])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,conv", [(2, 2, 128, 128, 4), (2, 2, 128, 129, 4), (4, 2, 256, 64, 2), (2, 1, 250, 65, 3), (3, 3, 64, 256, 3), (2, 1, 40, 250, 4),
                                                           (3, 1, 32, 96, 4), (2, 2, 32, 264, 2), (4, 4, 20, 12, 3), (2, 2, 128, 100, 5)], ids=str)

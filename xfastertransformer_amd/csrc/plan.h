@@ -240,7 +240,7 @@ struct LatentCacheView {
 };
 // the query latent's norm -> cq; the key latent's norm and the shared key part's rotation -> cache
 int latent_prepare(int act, const PlanLayer &L, const StepView &v, const void *a, void *cq, const LatentCacheView &cache, float eps, hipStream_t st);
-// rotates the rotated parts of q [T][heads][D + RD] in place
+// rotates the rotated parts of q [T][heads][D + RD] in place (nothing where latent_attention does it)
 int latent_rotate_q(int act, const PlanLayer &L, const StepView &v, void *q, hipStream_t st);
 // absorbed form: qa [T][heads][R] queries in the latent space, q their rotated parts; out [T][heads][R] weighted latents;
 // segments of up to `longest` tokens.  part: workspace of part_floats floats (split contexts).  hint: upper bound of the
