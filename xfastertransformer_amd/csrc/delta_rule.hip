@@ -496,13 +496,14 @@ __global__ __launch_bounds__(256) void delta_output_kernel(OutParams p) {
 // A step of one token a sequence, from the input product's rows to the output product's: convolutions, norms, decays, the state's step and the gated norm of a
 // key head's heads in one workgroup, where the state of a head fits its registers (16 floats a thread).  The channels of a token are spread over the threads
 // (q | k | v | decays, 256 each) and meet in LDS; the state is requested in front of that work, so that it arrives behind it.  A key head's workgroup alone
-// touches its convolution inputs, which it shifts in place.
+// touches its convolution inputs, which it shifts in place.  Every wave adds up the norms and q . k of the head by itself, over the same lanes as the
+// separate launches do, so that the results are theirs bit for bit (by way of LDS, where 16 waves at once queue for it, 1 to 8 % of a step more).
 // Bound by latency (a chain of two loads, two barriers, a store): a step of 16 heads of 128 x 128 in three launches / in one,
-// six layers of it, BF16: 1 sequence 148 / 119 us, 4 179 / 139, 16 223 / 175, 64 465 / 404; 64 x 64 142 / 108 .. 248 / 247, 64 x 256 171 / 129 .. 488 / 421.
+// six layers of it, BF16: 1 sequence 146 / 118 us, 4 174 / 138, 16 221 / 173, 64 458 / 403; 64 x 64 140 / 108 .. 243 / 247, 64 x 256 166 / 129 .. 483 / 420.
 template <bool BF16, int L, bool ONE>
 __global__ __launch_bounds__(1024) void delta_decode_kernel(PrepParams p, OutParams out) {
     constexpr int DT = BF16 ? XFTHIP_BF16 : XFTHIP_F32, KD = 8 * L, COLS = 1024 / L;
-    __shared__ __align__(16) float qs[KD], ks[KD], gs[KD], vs[256], os[256], part[8];
+    __shared__ __align__(16) float qs[KD], ks[KD], gs[KD], vs[256], os[256];
     const int seg = blockIdx.x, kvh = blockIdx.y, each = p.H / p.KH, tid = threadIdx.x, lane = tid & 63;
     const int t = p.v.seg_off[seg], row = p.v.seg_row[seg], start = p.v.seg_pos[seg];
     const int li = tid % L, col0 = tid / L, role = tid >> 8, c = tid & 255, taps = p.taps;
@@ -548,23 +549,21 @@ __global__ __launch_bounds__(1024) void delta_decode_kernel(PrepParams p, OutPar
             for (int j = 0; j < 3; ++j)
                 if (j >= 4 - taps) store_from_f32(p.b.conv_state, DT, hist + (size_t)(j - (4 - taps)) * p.channels + ch, j < 2 ? x[j + 1] : in);
             (role == 0 ? qs : role == 1 ? ks : vs)[c] = a;
-            dt = a * a;
-        }
-        if (role < 2 && r == 0) { // (whole waves)
-            const float sum = wave_total(conv ? dt : 0.0f);
-            if (lane == 0) part[tid >> 6] = sum;
         }
         if (gate || (ONE && role == 3 && c == 0)) gs[c] = exp_of<BF16>(-decay * softplus_of<BF16>(in + dt));
         __syncthreads();
         if (r == 0) {
-            const float sq = 1.0f / sqrtf((part[0] + part[1]) + (part[2] + part[3]) + 1e-6f) * p.qscale, sk = 1.0f / sqrtf((part[4] + part[5]) + (part[6] + part[7]) + 1e-6f);
+            float sq = 0.0f, sk = 0.0f;
+#pragma unroll
+            for (int i = 2 * lane; i < KD; i += 128) {
+                const float2 x = *(const float2 *)(qs + i), y = *(const float2 *)(ks + i);
+                sq = fmaf(x.x, x.x, fmaf(x.y, x.y, sq)), sk = fmaf(y.x, y.x, fmaf(y.y, y.y, sk)), qk = fmaf(x.x, y.x, fmaf(x.y, y.y, qk));
+            }
+            sq = 1.0f / sqrtf(wave_total_dpp(sq) + 1e-6f) * p.qscale, sk = 1.0f / sqrtf(wave_total_dpp(sk) + 1e-6f);
+            qk = wave_total_dpp(qk) * sq * sk;
             q0 = *(const f32x4 *)(qs + 4 * li), q1 = *(const f32x4 *)(qs + 4 * (L + li)), k0 = *(const f32x4 *)(ks + 4 * li), k1 = *(const f32x4 *)(ks + 4 * (L + li));
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                q0[i] *= sq, q1[i] *= sq, k0[i] *= sk, k1[i] *= sk;
-                qk = fmaf(q0[i], k0[i], fmaf(q1[i], k1[i], qk));
-            }
-            qk = group_sum<L>(qk);
+            for (int i = 0; i < 4; ++i) q0[i] *= sq, q1[i] *= sq, k0[i] *= sk, k1[i] *= sk;
         }
         f32x4 g0, g1;
         if constexpr (ONE) {
@@ -591,8 +590,11 @@ __global__ __launch_bounds__(1024) void delta_decode_kernel(PrepParams p, OutPar
         __syncthreads();
         if (tid < (p.VD + 63) / 64 * 64) { // (whole waves; each adds up all of the head by itself)
             float sq = 0.0f;
-            for (int i = lane; i < p.VD; i += 64) sq = fmaf(os[i], os[i], sq);
-            const float f = 1.0f / sqrtf(wave_total(sq) / (float)out.vdim + out.eps) * out.mul;
+            for (int i = 2 * lane; i < p.VD; i += 128) {
+                const float2 x = *(const float2 *)(os + i);
+                sq = fmaf(x.x, x.x, fmaf(x.y, x.y, sq));
+            }
+            const float f = 1.0f / sqrtf(wave_total_dpp(sq) / (float)out.vdim + out.eps) * out.mul;
             z = out.row_gate ? silu_of<BF16>(z) : sigmoid_of<BF16>(z);
             if (tid < p.VD) store_from_f32(out.out, DT, (size_t)t * out.out_ld + head * p.VD + tid, os[tid] * f * ow * z);
         }

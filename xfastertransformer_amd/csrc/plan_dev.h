@@ -129,6 +129,18 @@ __device__ inline float group_sum(float v) {
     return v;
 }
 
+// wave_total's sum, added up in its order, between registers instead of by way of LDS: for kernels all of whose waves need it at once
+__device__ inline float wave_total_dpp(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(f2u(v), f2u(v), false, false);
+    v = u2f(a[0]) + u2f(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(f2u(v), f2u(v), false, false);
+    v = u2f(b[0]) + u2f(b[1]);
+    v = dpp_add<0x128>(v); // row_ror:8
+    v = dpp_add<0x124>(v); // row_ror:4 (the values repeat every 8 lanes by now)
+    v = dpp_add<0x4E>(v); // quad_perm 2 3 0 1
+    return dpp_add<0xB1>(v); // quad_perm 1 0 3 2
+}
+
 // The value is in its register from here on.  What is loaded in front of a loop and changed in it would otherwise be waited for inside, and
 // with it the loads that the loop has just sent ahead.
 template <class V>
