@@ -100,6 +100,21 @@ def test_delta_tokens_one_by_one(xh, heads, kv_heads, dim, vdim, conv, act):
     c.free()
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,fewer,more", [(8, 8, 32, 32, 64, 65), (8, 8, 40, 30, 64, 65), (16, 8, 64, 40, 64, 65), (16, 16, 64, 128, 64, 65)], ids=str)
+def test_delta_many_sequences(xh, heads, kv_heads, dim, vdim, fewer, more):
+    """the last number of sequences whose step a layer takes in one launch, and the first that it does not: bit for bit the same"""
+    cfg = u.config([u.delta(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim)])
+    tokens = np.random.default_rng(dim).integers(0, cfg["vocab"], (more, 5))
+    got = []
+    for n in (fewer, more):
+        c = Case(xh, cfg, 31, "f32", slots=more, max_seq=32, max_tokens=more)
+        got.append(np.stack([c.model.step([(i, tokens[i, t:t + 1], [0]) for i in range(n)]) for t in range(5)], 1))
+        for i in (0, n - 1):
+            c.check(got[-1][i], c.want(tokens[i]), f"sequence {i} of {n}")
+        c.free()
+    assert np.array_equal(got[0], got[1][:fewer])
+
+
 def whole_config(**kw):
     return u.config([u.latent(window=37), u.latent(), u.delta(), u.latent(window=70, heads=2, kv_rank=64), u.delta(heads=2, kv_heads=2, dim=32, vdim=24, conv=2)],
                     loop=dict(start=1, stop=4, times=3), **kw)

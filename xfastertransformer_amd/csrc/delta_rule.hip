@@ -711,8 +711,14 @@ int delta_output(int act, const PlanLayer &L, const StepView &v, const DeltaBuff
 
 // The state of a head in the registers of one workgroup.  A second head of a key head follows the first in its workgroup: of the 29 and 40 us that six layers
 // of 16 x 128 x 128 save at 1 and 4 sequences 14 and 16 are left with 8 key heads (38 of 49 at 16, 72 of 60 at 64); a third would take what is left.
+// Smaller states only as long as a CU, which holds two workgroups, gets few after each other: a workgroup of 1024 threads takes as long for a small state as for a
+// large one.  Three launches / one, six layers of 16 heads, 32 / 64 / 128 / 256 sequences: 32 x 32 184 / 168 us, 203 / 218, 224 / 308, 255 / 474; 64 x 64 220 / 190, 243 /
+// 248, 280 / 336, 431 / 620; 64 x 128 242 / 211, 306 / 286, 437 / 482, 621 / 755; 128 x 96 254 / 220, 369 / 350, 510 / 505, 783 / 795; 128 x 128 272 / 245, 457 / 405, 594 / 559,
+// 935 / 900.  (8192 values in three rounds 1 to 7 % slower, 4096 in two 2 %.)
 bool delta_decodes_at_once(const PlanLayer &L, const StepView &v) {
-    return v.longest == 1 && L.s.taps >= 2 && L.s.taps <= 4 && L.KD <= 256 && L.VD <= 256 && L.KD * L.VD <= 16 * 1024 && L.s.heads <= 2 * L.s.kv_heads;
+    const int size = L.KD * L.VD, most = 2 * device_cu_count(), rounds = (v.B * L.s.kv_heads + most - 1) / most;
+    return v.longest == 1 && L.s.taps >= 2 && L.s.taps <= 4 && L.KD <= 256 && L.VD <= 256 && size <= 16 * 1024 && L.s.heads <= 2 * L.s.kv_heads
+            && (size == 16 * 1024 || rounds <= (size >= 12 * 1024 ? 4 : size >= 8 * 1024 ? 2 : 1));
 }
 
 int delta_decode(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, float eps, hipStream_t st) {
