@@ -1,4 +1,4 @@
-"""A plan model on a device that has room for it with one context in the expanded form of latent attention, but not with all of a step's."""
+"""A device that is short of memory: a plan model that has room for one context in the expanded form of latent attention, but not for all of a step's."""
 import ctypes as C
 
 import numpy as np
@@ -11,15 +11,28 @@ pytestmark = pytest.mark.gpu
 HEADS, DIM, ROT, RANK, SLOTS, SEQ, TOKENS = 64, 128, 64, 128, 256, 64, 16384
 
 
+def left():
+    from xfastertransformer_amd import capi as xh
+    free, device = C.c_size_t(), C.c_size_t()
+    assert xh.lib.hipMemGetInfo(C.byref(free), C.byref(device)) == 0  # (of the runtime that the library is linked with)
+    return free.value
+
+
+def test_refused_allocation_is_told_once():
+    """the call behind one that found no memory runs"""
+    from xfastertransformer_amd import capi as xh
+    xh.init(0)
+    x, w, out = xh.DeviceBuffer.from_numpy(np.arange(256, dtype=np.float32)), xh.DeviceBuffer.from_numpy(np.ones(256, np.float32)), xh.DeviceBuffer(1024)
+    with pytest.raises(xh.XftHipError, match="memory"):
+        xh.DeviceBuffer(1 << 50)
+    xh.rmsnorm(out.ptr, xh.F32, x.ptr, xh.F32, w.ptr, 1, 256)
+    y = np.arange(256.0)
+    np.testing.assert_allclose(out.to_numpy(np.float32, 256), y / np.sqrt((y * y).mean() + 1e-6), rtol=1e-6)
+
+
 def test_model_that_just_fits():
     from xfastertransformer_amd import capi as xh
     xh.init(0)
-
-    def left():
-        free, device = C.c_size_t(), C.c_size_t()
-        assert xh.lib.hipMemGetInfo(C.byref(free), C.byref(device)) == 0  # (of the runtime that the library is linked with)
-        return free.value
-
     cfg = u.config([u.latent(heads=HEADS, dim=DIM, rot=ROT, vdim=DIM, kv_rank=RANK, q_rank=64)])
     bits = u.weights(cfg, 17)
     plan, w = u.build_plan(xh, cfg, bits), u.oracle_weights(bits)

@@ -21,6 +21,7 @@ void set_error(const char *fmt, ...) {
     va_start(ap, fmt);
     vsnprintf(g_err, sizeof(g_err), fmt, ap);
     va_end(ap);
+    (void)hipGetLastError(); // told here: the runtime keeps a call's error, and the check behind the next launch would report it again
 }
 
 int device_cu_count() {
