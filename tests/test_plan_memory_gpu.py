@@ -1,9 +1,11 @@
-"""A device that is short of memory: a plan model that has room for one context in the expanded form of latent attention, but not for all of a step's."""
+"""A device that is short of memory: a plan model that has room for one context in the expanded form of latent attention, but not for all of a step's; a step
+without a buffer for the parts of a product whose K is split."""
 import ctypes as C
 
 import numpy as np
 import pytest
 
+import duvadra_util
 import plan_util as u
 from oracle import pinepel_ref as ref
 
@@ -59,4 +61,45 @@ def test_model_that_just_fits():
     model.free()
     for b in ballast:
         b.free()
+    plan.free()
+
+
+def test_step_that_finds_no_memory():
+    """A step of one token a sequence that fails half way, for want of a buffer for a product's parts on a stream of its own, leaves the sequences where they
+    stood: the same step, repeated, finds their positions and the tokens before (the pair embedding reads them) as they were."""
+    from xfastertransformer_amd import capi as xh
+    xh.init(0)
+    n, parts = 40, 64 << 20  # (a product of 40 rows, 4096 deep, takes its K in parts)
+    cfg = duvadra_util.config([(duvadra_util.chunked(), duvadra_util.dense(ff=4096))])
+    plan = duvadra_util.build_plan(xh, cfg, duvadra_util.weights(cfg, 8))
+    model, twin = (xh.PlanModel(plan, xh.BF16, n, 64, n) for _ in range(2))
+    rng, streams = np.random.default_rng(2), [xh.Stream() for _ in range(4)]
+    draw = lambda: rng.integers(0, cfg["vocab"], n).astype(np.int32)
+    entries = lambda tokens: [(i, tokens[i:i + 1], [0]) for i in range(len(tokens))]
+    tokens = draw()
+    assert np.array_equal(model.step(entries(tokens)), twin.step(entries(tokens)))
+    for s in streams:  # (one token: no parts; what a stream needs otherwise it has then)
+        few = draw()[:1]
+        assert np.array_equal(model.step(entries(few), s.h), twin.step(entries(few)))
+    ballast = []
+    while left() > parts - (8 << 20):
+        ballast.append(xh.DeviceBuffer(min(left() - (parts - (32 << 20)), 16 << 30)))
+    failed = 0
+    for s in streams:  # (a stream may have the handle, and the buffer, of one that is gone)
+        tokens = draw()
+        want = twin.step(entries(tokens))
+        try:
+            got = model.step(entries(tokens), s.h)
+        except xh.XftHipError:
+            failed += 1
+            break
+        assert np.array_equal(got, want)
+    for b in ballast:
+        b.free()
+    assert failed
+    assert np.array_equal(model.step(entries(tokens), s.h), want)
+    tokens = draw()
+    assert np.array_equal(model.step(entries(tokens), s.h), twin.step(entries(tokens)))
+    model.free()
+    twin.free()
     plan.free()

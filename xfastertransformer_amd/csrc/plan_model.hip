@@ -80,10 +80,17 @@ __global__ void plan_step_begin_kernel(EmbedTables e, BeginTokens s, float *x, i
     __syncthreads(); // (all have read the token before)
     if (threadIdx.x == 0) {
         tok_seg[b] = b, tok_pos[b] = at, tok_ids[b] = id;
-        seg[b] = row, seg[seg_cap + b] = b, seg[2 * seg_cap + b] = 1, seg[3 * seg_cap + b] = at;
+        seg[b] = row, seg[seg_cap + b] = b, seg[2 * seg_cap + b] = 1, seg[3 * seg_cap + b] = at, seg[4 * seg_cap + b] = prev;
         last_token[row] = id, pos[row] = at + 1;
     }
     embed_token(e, id, at == 0, prev, x + (size_t)b * e.hidden);
+}
+
+// a step begun so whose layers could not all be launched: its sequences stand where they stood (behind the layers, as plan_advance writes, they would not have moved)
+__global__ void plan_step_undo_kernel(const int *seg, int seg_cap, int n, int *pos, int *last_token) {
+    const int b = threadIdx.x;
+    if (b >= n) return;
+    pos[seg[b]] = seg[3 * seg_cap + b], last_token[seg[b]] = seg[4 * seg_cap + b];
 }
 
 // ahead of a step: its description from pinned host memory (tok_seg | tok_pos | ids, `stride` apart, T of each; 4 seg_cap segment entries behind
@@ -533,7 +540,10 @@ int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int
         XFT_CHECK_HIP(hipGetLastError());
         if (int rc = plan_embed(embed_tables(m), view, p.ids, p.last_token, m->x, st)) return rc;
     }
-    if (int rc = plan_layers(m, view, st, head_follows)) return rc;
+    if (int rc = plan_layers(m, view, st, head_follows)) {
+        if (at_once) hipLaunchKernelGGL(plan_step_undo_kernel, dim3(1), dim3(kBeginTokens), 0, st, p.seg, cap, n, m->pos, p.last_token);
+        return rc;
+    }
     if (!at_once) {
         hipLaunchKernelGGL(plan_advance_kernel, dim3((n + 63) / 64), dim3(64), 0, st, p.seg, cap, n, p.ids, m->pos, p.last_token);
         XFT_CHECK_HIP(hipGetLastError());
@@ -1494,7 +1504,7 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
         p->reads.push_back(from), p->cache.push_back(pool), p->state.push_back(state), p->conv_state.push_back(conv), p->means.push_back(means);
     }
     alloc(&p->table, p->table_host.size() * 4, true);
-    alloc(&p->desc, (3 * T + 4 * (size_t)max_batch) * 4, true);
+    alloc(&p->desc, (3 * T + 5 * (size_t)max_batch) * 4, true);
     alloc(&p->dec_rows, (size_t)max_batch * 4, true);
     std::map<std::vector<double>, std::pair<float *, float *>> rot; // layers of the same rotation share its tables
     auto tables_of = [&](const xfthip_plan_layer &s, float **cosT, float **sinT) {
