@@ -907,12 +907,13 @@ int xfthip_model_step(xfthip_model_t m, int n, const int *rows_host, const int *
     for (int i = 0; i < n_want; ++i) XFT_REQUIRE(want_host[i] >= 0 && want_host[i] < total, "xfthip_model_step: logits of token %d of %ld asked for", want_host[i], total);
     bool all = n_want == total && n_want <= m->plan->logit_rows; // the logits of every token, in order
     for (int i = 0; i < n_want && all; ++i) all = want_host[i] == i;
-    if (int rc = plan_run(m, n, rows_host, lens_host, ids_host, st, all)) return rc;
+    bool normed = false;
+    if (int rc = plan_run(m, n, rows_host, lens_host, ids_host, st, all ? &normed : nullptr)) return rc;
     m->prompt_rows = (int)total;
     m->cur_B = 0;
     for (int r = 0; r < c.max_batch; ++r)
         if (m->row_pos[r] >= 0) m->cur_B = r + 1;
-    if (n_want > 0) return plan_logits(m, want_host, n_want, logits_host, st); // (which waits for everything in front of the logits)
+    if (n_want > 0) return plan_logits(m, want_host, n_want, logits_host, st, normed); // (which waits for everything in front of the logits)
     XFT_CHECK_HIP(hipStreamSynchronize(st));
     return 0;
 }

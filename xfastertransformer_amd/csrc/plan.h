@@ -392,7 +392,6 @@ struct PlanState {
     float *part = nullptr; // split contexts
     size_t part_floats = 0;
     std::vector<void *> owned; // every device buffer above
-    bool final_normed = false; // xn holds the final norm of the step's residual rows already (for the plan_head that follows)
     bool trace = false;
     float *trace_buf = nullptr;
     size_t trace_floats = 0;
@@ -403,12 +402,13 @@ struct PlanState {
 int plan_reserve(xfthip_model *m, int row, int tokens);
 void plan_release(xfthip_model *m, int row);
 // residual rows of a step: entry i = the next lens[i] tokens of slot rows[i] (m->row_pos says where they stand; it moves on)
-// head_follows: plan_head of all its tokens, in order, comes next
-int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int *ids, hipStream_t st, bool head_follows = false);
-// final norm and head of the residual rows rows_dev[0 .. n) (null: rows 0 .. n - 1) into m->logits + at * vocab
-int plan_head(xfthip_model *m, const int *rows_dev, int n, int at, hipStream_t st);
+// normed (or null): plan_head of all its tokens, in order, comes next; whether xn holds their final norm already
+int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int *ids, hipStream_t st, bool *normed = nullptr);
+// final norm and head of the residual rows rows_dev[0 .. n) (null: rows 0 .. n - 1) into m->logits + at * vocab (normed: xn holds the norm)
+int plan_head(xfthip_model *m, const int *rows_dev, int n, int at, hipStream_t st, bool normed = false);
 // final norm and head of the residual rows list[0 .. n) (host), logits to host memory, as many rows at a time as fit
-int plan_logits(xfthip_model *m, const int *list, int n, float *logits_host, hipStream_t st);
+// (normed: all of a step's rows in order, whose norm xn holds)
+int plan_logits(xfthip_model *m, const int *list, int n, float *logits_host, hipStream_t st, bool normed = false);
 // upload of what a decode call of the slots in dec_list needs, for `steps` steps
 int plan_decode_begin(xfthip_model *m, int steps, hipStream_t st);
 // one decode step of the slots in dec_rows (recordable): positions and input ids from m->pos / m->ids

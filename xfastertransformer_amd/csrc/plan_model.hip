@@ -383,9 +383,9 @@ int run_side(xfthip_model *m, const PlanLayer &L, int layer, int T, const void *
     return plan_gemm(m, L.side_proj, T, p.side, pad, p.y, hidden, XFTHIP_F32, st);
 }
 
-// all layer runs over the step's tokens, whose embeddings are in m->x.  head_follows: the logits of all of them, in order, are wanted next, so the final norm joins
-// the last layer's own pass over the residual where there is one (p.final_normed)
-int plan_layers(xfthip_model *m, const StepView &v, hipStream_t st, bool head_follows) {
+// all layer runs over the step's tokens, whose embeddings are in m->x.  normed (or null): the logits of all of them, in order, are wanted next, so the final norm
+// joins the last layer's own pass over the residual where there is one; whether it did
+int plan_layers(xfthip_model *m, const StepView &v, hipStream_t st, bool *normed) {
     PlanState &p = *m->plan;
     const xfthip_plan &plan = *p.plan;
     const int T = v.T, hidden = m->cfg.hidden;
@@ -401,10 +401,11 @@ int plan_layers(xfthip_model *m, const StepView &v, hipStream_t st, bool head_fo
         return plan_norm(p.act, a, T, st);
     };
     const PlanNorm none;
-    const PlanNorm &behind = head_follows && !p.trace ? plan.final_norm : none; // of the last layer
-    p.final_normed = false;
+    const bool head_follows = normed && !p.trace;
+    const PlanNorm &behind = head_follows ? plan.final_norm : none; // of the last layer
+    if (normed) *normed = false;
     auto enter = [&](const float *y, const float *post, bool again, const PlanLayer *next, bool last = false) {
-        p.final_normed = last && head_follows && !p.trace;
+        if (last && head_follows) *normed = true;
         return norm(y, post, again, next ? next->pre1 : last ? behind : none, next && parallel ? next->pre2 : none, nullptr);
     };
     if ((rc = enter(nullptr, nullptr, plan.runs[0].add_embedding, &p.layers[plan.runs[0].layer]))) return rc;
@@ -424,7 +425,7 @@ int plan_layers(xfthip_model *m, const StepView &v, hipStream_t st, bool head_fo
             if (!last || side)
                 if ((rc = enter(side ? p.y : nullptr, L.side_post, join, then, last))) return rc;
         } else {
-            p.final_normed = last && !ff && head_follows && !p.trace;
+            if (last && !ff && head_follows) *normed = true;
             if ((rc = norm(p.y, L.post1, !ff && join, ff ? L.pre2 : then ? then->pre1 : last ? behind : none, none, &L))) return rc;
             if (ff) {
                 if ((rc = run_feed_forward(m, L, T, p.xn, nullptr, st))) return rc;
@@ -485,7 +486,7 @@ void plan_release(xfthip_model *m, int row) {
     }
 }
 
-int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int *ids, hipStream_t st, bool head_follows) {
+int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int *ids, hipStream_t st, bool *normed) {
     PlanState &p = *m->plan;
     const xfthip_model_config &c = m->cfg;
     XFT_REQUIRE(n > 0 && n <= p.slots, "a step of %d entries; the model has %d slots", n, p.slots);
@@ -540,7 +541,7 @@ int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int
         XFT_CHECK_HIP(hipGetLastError());
         if (int rc = plan_embed(embed_tables(m), view, p.ids, p.last_token, m->x, st)) return rc;
     }
-    if (int rc = plan_layers(m, view, st, head_follows)) {
+    if (int rc = plan_layers(m, view, st, normed)) {
         if (at_once) hipLaunchKernelGGL(plan_step_undo_kernel, dim3(1), dim3(kBeginTokens), 0, st, p.seg, cap, n, m->pos, p.last_token);
         return rc;
     }
@@ -553,15 +554,14 @@ int plan_run(xfthip_model *m, int n, const int *rows, const int *lens, const int
 }
 
 // rows_dev: of the step's tokens, read by the card (device or pinned host memory; the stream is waited for before a pinned list changes), or null for all
-int plan_head(xfthip_model *m, const int *rows_dev, int n, int at, hipStream_t st) {
+int plan_head(xfthip_model *m, const int *rows_dev, int n, int at, hipStream_t st, bool normed) {
     PlanState &p = *m->plan;
     const xfthip_plan &plan = *p.plan;
     const xfthip_model_config &c = m->cfg;
     const PlanNormArgs a = {m->x, nullptr, nullptr, nullptr, nullptr, c.vocab, plan.final_norm, {}, p.xn, nullptr, rows_dev, c.hidden, plan.cfg.hidden, c.rms_eps, 0.0f,
             plan.cfg.norm_groups};
-    if (!p.final_normed)
+    if (!normed)
         if (int rc = plan_norm(p.act, a, n, st)) return rc;
-    p.final_normed = false; // (of this step's tokens only, and once)
     float *logits = m->logits + (size_t)at * c.vocab;
     if (int rc = plan_gemm(m, plan.head, n, p.xn, c.hidden, logits, c.vocab, XFTHIP_F32, st)) return rc;
     return plan.cfg.logit_softcap > 0.0f ? plan_softcap(logits, (size_t)n * c.vocab, plan.cfg.logit_softcap, st) : 0;
@@ -627,13 +627,13 @@ static int plan_fetch_logits(PlanState &p, const float *logits, size_t floats, f
     return 0;
 }
 
-int plan_logits(xfthip_model *m, const int *list, int n, float *logits_host, hipStream_t st) {
+int plan_logits(xfthip_model *m, const int *list, int n, float *logits_host, hipStream_t st, bool normed) {
     PlanState &p = *m->plan;
     const size_t vocab = m->cfg.vocab;
     for (int i = 0; i < n; i += p.logit_rows) {
         const int k = std::min(n - i, p.logit_rows);
         memcpy(p.want_host, list + i, (size_t)k * 4);
-        if (int rc = plan_head(m, p.want_host, k, 0, st)) return rc;
+        if (int rc = plan_head(m, p.want_host, k, 0, st, normed)) return rc;
         if (int rc = plan_fetch_logits(p, m->logits, (size_t)k * vocab, logits_host + (size_t)i * vocab, st)) return rc;
     }
     return 0;
@@ -679,10 +679,11 @@ int plan_decode_step(xfthip_model *m, int B, hipStream_t st) {
     // (lengths and offsets only: where the segments stand is known on the device)
     p.seg_off_host.resize(B), p.seg_len_host.assign(B, 1), p.seg_pos_host.assign(B, 0), p.seg_row_host.assign(B, 0);
     for (int b = 0; b < B; ++b) p.seg_off_host[b] = b;
-    int rc = plan_layers(m, view_of(m, B, B, 1), st, true);
+    bool normed = false;
+    int rc = plan_layers(m, view_of(m, B, B, 1), st, &normed);
     p.trace = trace;
     if (rc) return rc;
-    if ((rc = plan_head(m, nullptr, B, 0, st))) return rc;
+    if ((rc = plan_head(m, nullptr, B, 0, st, normed))) return rc;
     return argmax_rows(m->logits, B, c.vocab, m->ids, p.dec_rows, m->pos, m->step, st);
 }
 
