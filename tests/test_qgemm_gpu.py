@@ -236,6 +236,41 @@ def test_rows_four_gigabytes_apart(xh, orc, kind):
     w.free()
 
 
+@pytest.mark.parametrize("kind", ["int8", "uint4", "nf4", "bf16"])
+@pytest.mark.parametrize("M,lda,gateup", [
+    (17, 120000000, 0),  # the last rows behind 2 GB, within reach of unsigned byte offsets
+    (40, 50000000, 0),
+    (17, 1 << 28, 0),  # a row 2^32 elements behind the first
+    (33, 1 << 27, 1),
+    (70, 1 << 26, 0),  # (and a product of six rows for the rest)
+])
+def test_rows_gigabytes_apart(xh, orc, kind, M, lda, gateup):
+    """Few and many rows whose places 32-bit offsets hold, of bytes or of elements, and those that they do not; with the residual, which has rows of its own."""
+    K, N = 256, 64
+    rng = np.random.default_rng(M)
+    w, W, size = _random_weight(xh, orc, rng, kind, K, N, gateup=bool(gateup))
+    A, R = orc.round_bf16(rng.standard_normal((M, K), dtype=np.float32)), rng.standard_normal((M, N), dtype=np.float32)
+    a_dev, r_dev, o_dev = xh.DeviceBuffer(((M - 1) * lda + K) * 2), xh.DeviceBuffer.from_numpy(R), xh.DeviceBuffer(M * N * 4)
+    for m in range(M):
+        a_dev.upload(orc.to_bf16(A[m]), m * lda * 2)
+    if gateup:
+        xh.gemm_gateup_silu(w, a_dev.ptr, M, lda, o_dev.ptr, N // 2, xh.F32)
+    else:
+        xh.gemm(w, a_dev.ptr, M, lda, o_dev.ptr, N, xh.F32, xh.EPI_RESIDENTIAL, res=r_dev.ptr, ldres=N)
+    xh.synchronize()
+    got = o_dev.to_numpy(np.float32, (M, N // 2 if gateup else N))
+    y, b = A.astype(np.float64) @ W, np.abs(A).astype(np.float64) @ size * ((K + 8) * 2.0 ** -24 + (2.0 ** -16 if kind == "nf4" else 0.0))
+    if gateup:  # (the bound of test_mfma_gateup_every_tile_against_64_bits)
+        g, u = y[:, :N // 2], y[:, N // 2:]
+        silu = g / (1.0 + np.exp(-g))
+        want, bound = silu * u, 1.1 * b[:, :N // 2] * np.abs(u) + b[:, N // 2:] * (np.abs(silu) + 1.1 * b[:, :N // 2]) + np.abs(silu * u) * 2.0 ** -20
+    else:
+        want, bound = y + R, b + np.abs(y + R) * 2.0 ** -23
+    assert float((np.abs(got - want) / bound).max()) <= 1.0
+    a_dev.free()
+    w.free()
+
+
 @pytest.mark.parametrize("M", [4, 5, 16])
 @pytest.mark.parametrize("K,N", [(3968, 40), (4096, 40), (4224, 16), (4480, 4096), (5632, 2048)])
 def test_bf16_tiles_alone_on_their_cu_against_64_bits(xh, orc, M, K, N):

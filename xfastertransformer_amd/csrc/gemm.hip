@@ -13,6 +13,18 @@ static int check_common(const char *fn, xfthip_weight_t w, int M, const void *A,
     return 0;
 }
 
+// Rows out of reach of the kernels' 32-bit element offsets (8 GB from the first) come in products of their own, of as many rows as are within reach.
+static int gemm_rows(const PackedWeight &pw, SkinnyParams p, hipStream_t stream) {
+    const size_t reach = ((size_t)1 << 32) - 4096, within = reach / (size_t)p.lda + 1; // (a lane adds its place in the row)
+    for (int left = p.M; left > 0; left -= p.M) {
+        p.M = (size_t)left < within ? left : (int)within;
+        if (int rc = p.M <= 32 ? qgemm_skinny(pw, p, stream) : qgemm_mfma(pw, p, stream)) return rc;
+        p.A += (size_t)p.M * p.lda, p.C = (char *)p.C + (size_t)p.M * p.ldc * (p.c_dtype == XFTHIP_F32 ? 4 : 2);
+        if (p.res) p.res = (const char *)p.res + (size_t)p.M * p.ldres * (p.res_dtype == XFTHIP_F32 ? 4 : 2);
+    }
+    return 0;
+}
+
 namespace xfthip {
 
 int gemm_rows_dev(xfthip_weight_t w, int m_max, int m_hint, const int *rows_dev, const void *A, int lda, void *C, int ldc, int c_dtype,
@@ -134,8 +146,7 @@ int xfthip_gemm(xfthip_weight_t w, int M, const void *A, int lda, void *C, int l
     p.res_dtype = res_dtype;
     p.gamma = gamma;
     p.gateup = 0;
-    if (M <= 32) return qgemm_skinny(pw, p, (hipStream_t)stream);
-    return qgemm_mfma(pw, p, (hipStream_t)stream);
+    return gemm_rows(pw, p, (hipStream_t)stream);
 }
 
 int xfthip_gemm_gateup_silu(xfthip_weight_t w, int M, const void *A, int lda, void *out, int ldo, int out_dtype,
@@ -160,8 +171,7 @@ int xfthip_gemm_gateup_silu_bias(xfthip_weight_t w, int M, const void *A, int ld
     p.c_dtype = out_dtype;
     p.gateup = 1;
     p.bias = bias;
-    if (M <= 32) return qgemm_skinny(pw, p, (hipStream_t)stream);
-    return qgemm_mfma(pw, p, (hipStream_t)stream);
+    return gemm_rows(pw, p, (hipStream_t)stream);
 }
 
 int xfthip_gemm_gateup_clamped(xfthip_weight_t w, int M, const void *A, int lda, void *out, int ldo, int out_dtype, float limit, float alpha,
@@ -181,8 +191,7 @@ int xfthip_gemm_gateup_clamped(xfthip_weight_t w, int M, const void *A, int lda,
     p.c_dtype = out_dtype;
     p.gateup = 2;
     p.glu_limit = limit, p.glu_alpha = alpha;
-    if (M <= 32) return qgemm_skinny(pw, p, (hipStream_t)stream);
-    return qgemm_mfma(pw, p, (hipStream_t)stream);
+    return gemm_rows(pw, p, (hipStream_t)stream);
 }
 
 int xfthip_gemm_gateup_silu_rmsnorm(xfthip_weight_t w, int M, const float *x, int ldx, const float *norm_weight, float eps,

@@ -112,7 +112,7 @@ constexpr int skinny_batch(int kind, int mt, bool group, int nt) {
 // Products of 4-bit codes whose activation rows go straight into LDS (mt 16-row tiles): all that are staged, but UINT4 at up to 16 rows, where it gains 2 % in the mean and
 // loses up to 8 % (skinny_form has the figures)
 constexpr bool skinny_dma(int kind, int mt) { return kind == XFTHIP_W_NF4 || (kind == XFTHIP_W_UINT4 && mt == 2); }
-// rows that lie 4 GB apart, out of reach of that form's 32-bit offsets: the form for a ragged K takes them
+// rows that lie 4 GB apart, out of reach of that form's 32-bit offsets in bytes: the form for a ragged K takes them, which counts in elements (gemm_rows: 8 GB)
 inline bool skinny_far(int kind, const SkinnyParams &p) {
     return p.M > 4 && !p.group && skinny_dma(kind, p.M > 16 ? 2 : 1) && (size_t)p.M * (size_t)p.lda * 2 >= (size_t)1 << 32;
 }
