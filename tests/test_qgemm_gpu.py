@@ -202,7 +202,7 @@ def test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N):
 
 # on 256 CUs: 1, 2, 3, 4 (at 17 rows and more) and 6 column tiles a block, ragged last blocks, 8 to 1 K slices, and more than 8 tiles a CU
 FEW_ROWS = [(M, K, N) for K, N in [(1280, 1040), (1280, 4112), (1280, 9232), (768, 13328), (768, 18448), (768, 28672), (768, 36880), (256, 36880)]
-            for M in (3, 13, 29)] + [(13, 4096, 1040)]
+            for M in (3, 13, 29)] + [(13, 4096, 1040), (13, 256, 49200)]
 
 
 @pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])
@@ -212,7 +212,8 @@ def test_few_rows_every_form_against_64_bits(xh, orc, kind, M, K, N):
 
 
 @pytest.mark.parametrize("kind", ["uint4", "nf4"])
-@pytest.mark.parametrize("M,K,N", [(5, 128, 48), (16, 384, 80), (17, 128, 4112), (31, 256, 12304), (32, 1152, 2064), (17, 4352, 16), (32, 640, 20496)])
+@pytest.mark.parametrize("M,K,N", [(5, 128, 48), (16, 384, 80), (17, 128, 4112), (31, 256, 12304), (32, 1152, 2064), (17, 4352, 16), (32, 640, 20496), (16, 128, 49168), (16, 384, 49152),
+                                   (24, 640, 37904), (32, 1152, 18944)])
 def test_rows_straight_into_lds_against_64_bits(xh, orc, kind, M, K, N):
     """One load batch a slice, an odd number and unequal ones; rows that fill their 16-row tiles and a single one in the second."""
     test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N)

@@ -48,19 +48,22 @@ SkinnyForm skinny_form(int kind, const SkinnyParams &p) {
     auto per_cu = [&](int nt) { return ((p.NTILES + nt - 1) / nt * weights + cus - 1) / cus; };
     const long tiles = (long)p.NTILES * weights;
     if (p.M > 4 && !p.group && skinny_dma(kind, mt)) {
-        // Rows straight into LDS, 16 KB a wave (8 at up to 16 rows): eight waves a CU have room, so that a CU's blocks share them.  The same cost, without a price on wide blocks,
-        // which hold no rows in registers.  16 shapes of 4096 .. 57344 columns x 2048 .. 14336 deep, against rows staged through registers (with v_and_or_b32 in both): UINT4 24 and 32 rows
-        // 0.915 of the time in the geometric mean (0.62 .. 0.98; 24 x 4096 x 28672 with SwiGLU 18.7 -> 17.4 us, 24 x 4096 x 4096 7.9 -> 7.0), NF4 0.87 (0.81 .. 0.95), within 0.2 to 0.5 % of
-        // the best of 12 forms in the mean; with the constants of the other forms 2 to 3 %.
+        // Rows straight into LDS, 16 KB a wave (8 at up to 16 rows): eight waves a CU have room, and it needs them all, so that a CU's blocks share them; wide blocks hold no
+        // rows in registers.  Against rows staged through registers (with v_and_or_b32 in both), 101 shapes of 1024 .. 151936 columns x 256 .. 28672 deep: UINT4 24 and 32 rows 0.92 of the time
+        // in the geometric mean (0.77 .. 1.02; 24 x 4096 x 28672 with SwiGLU 21.4 -> 18.7 us), NF4 0.90 (0.75 .. 1.02), at up to 16 rows 0.92 (0.78 .. 1.03); within 0.5 to 1.3 % of the
+        // best of 20 forms in the mean.  With half the waves in blocks of six tiles, and 0.8 of a tile a block, which this rule had first, up to 1.23: NF4 24 x 3584 x
+        // 37888 with SwiGLU 33.5 -> 40.4, now 28.5, UINT4 32 x 7168 x 52192 58.5 -> 68.9, now 56.0.
+        // NF4 at up to 16 rows, more than 12 tiles a CU: 16 x 4096 x 128256 77 us in three tiles, 73 staged, 68.7 in four.
+        if (mt == 1 && tiles > 12L * cus) return SkinnyForm {4, 1, p.KT > 1 ? 2 : 1};
         int best = p.gateup ? 2 : 1;
         float least = 1e30f;
         for (int n : {1, 2, 3, 4, 6}) {
             if (p.gateup && n % 2) continue;
             const float tile = mt == 2 || n < 4 ? 1.0f : n == 4 ? 1.1f : 1.2f;
-            const float cost = (float)per_cu(n) * ((float)n * tile + (mt == 2 ? 0.8f : 0.3f));
+            const float cost = (float)per_cu(n) * ((float)n * tile + (mt == 2 ? 1.2f : 0.4f));
             if (cost < least) least = cost, best = n;
         }
-        const int w = per_cu(best), slices = w > 2 || (w == 2 && best == 6) ? 2 : w == 2 || best == 6 ? 4 : 8;
+        const int w = per_cu(best), slices = w == 1 ? 8 : w == 2 ? 4 : 2;
         return SkinnyForm {best, 1, slices < p.KT ? slices : p.KT};
     }
     // (two slices against eight: 3 % faster at K = 4096, 2 % slower at 2048)
