@@ -181,7 +181,7 @@ MANY_ROWS = [(33, 8192, 3088), (97, 4096, 1040), (129, 1024, 12304), (200, 4096,
              (5526, 12368, 32), (2308, 256, 2512), (2335, 9216, 400), (2129, 12288, 400), (5008, 5248, 160), (2089, 18304, 224), (2307, 3072, 2480),
              (2423, 9216, 784), (1158, 4480, 3296), (1841, 10368, 32),
              # (96 x 256: K in parts, whole, whole for BF16 weights too)
-             (66, 4096, 12944), (652, 512, 11040), (579, 512, 12912)]
+             (66, 4096, 12944), (652, 512, 11040), (579, 512, 12912), (1155, 512, 6720)]
 
 
 @pytest.mark.parametrize("kind", ["int8", "int8z", "uint4", "nf4", "bf16"])

@@ -114,8 +114,8 @@ __global__ __launch_bounds__(256) void qgemm_split_finish_kernel(SkinnyParams p)
 // 64-row tiles with K in up to 4 parts throughout: a Mixtral-8x7B layer, INT8, 400 tokens 549 -> 490 us, 1000 tokens 1060 -> 940; 8 experts
 // of width 2816 at width 2048, BF16, 6132 tokens, two layers and all else 3.28 -> 2.98 ms.
 // 96 x 256, for 65 .. 96 rows, experts with some more than 64 and counts that are one or a few more than a multiple of 128: its constants are those of 128 x 256 by the ratios of two
-// fits to 100 timings each.  300 shapes a kind of 1024 .. 28672 columns x 1024 .. 14336 deep, 33 .. 4096 rows, against the same without it: INT8 0.985 of the time in the geometric mean
-// (384 x 28672 x 4096 with SwiGLU 100 -> 87 us, 900 x 11008 x 4096 94 -> 82; 0.79 .. 1.05), BF16 0.99, NF4 0.99, UINT4 0.98; a Mixtral-8x7B layer, INT8, of 256 / 290 / 580 / 1024 tokens
+// fits to 100 timings each.  Products that take it, 1024 .. 57344 columns x 1024 .. 28672 deep, 33 .. 2800 rows, against the same without it: INT8 and BF16 0.89 of the time in the
+// geometric mean (384 x 28672 x 4096 INT8 with SwiGLU 100 -> 87 us, 900 x 11008 x 4096 94 -> 82, 407 x 2560 x 22016 BF16 81 -> 56), UINT4 0.91, NF4 0.94; a Mixtral-8x7B layer, INT8, of 256 / 290 / 580 / 1024 tokens
 // 381 / 425 / 640 / 873 -> 369 / 377 / 597 / 872 us, UINT4, 256 tokens 363 -> 336.
 struct TileCost {
     int rows, cols, kgroups, resident;
@@ -131,6 +131,11 @@ constexpr TileCost kTiles[] = {
         {128, 256, 1, 2, 3.1f, {0.92f, 0.93f, 1.59f, 0.92f}, {0.73f, 0.77f, 1.34f, 0.73f}},
         {128, 256, 2, 1, 8.7f, {1.49f, 1.8f, 2.63f, 1.49f}, {}},
 };
+
+// What 96 x 256 has to gain by the model before a product takes it (not experts, whose rows are an estimate): 700 products that the model alone gives to it, against what they take
+// without it, lost more than 2 % in 12 % of cases (NF4 19) and up to 1.2 times (800 x 14336 x 28672 BF16 665 -> 755 us, 696 x 2560 x 11008 NF4 79 -> 91), mostly where the model saw
+// little to gain.  With these prices 4 %, and 0.931 of the time in the geometric mean (0.928 without).  Left: 4 row blocks of BF16 over 32000 columns, 1.1 to 1.2 times.
+constexpr float kPrice96[4] = {1.03f, 1.07f, 1.05f, 1.03f}; // INT8, BF16, NF4, UINT4
 
 constexpr float kSplitStart[4] = {3.0f, 4.0f, 3.0f, 3.0f}, kSplitMb[4] = {0.3f, 0.35f, 0.3f, 0.3f}; // launch and megabytes of a split K's sum
 
@@ -225,6 +230,7 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_sp
             // blocks, which were to take 1 more; the layer 137 -> 129.  With down projections priced so as well, 256 tokens of the Mixtral shape
             // lose 0.7 %)
             if (p.group && p.gateup && t.rows == 128) us *= 1.05f;
+            if (t.rows == 96 && !p.rows_dev) us *= kPrice96[cls];
             if (us < best) {
                 best = us;
                 p.tile = t.rows == 32 ? 1 : t.rows == 64 ? 2 : t.rows == 96 ? 5 : t.cols == 128 ? 3 : 4;
