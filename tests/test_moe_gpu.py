@@ -188,11 +188,51 @@ def test_mixtral_mlp_few_rows_an_expert(xh, orc, tokens):
 
 @pytest.mark.parametrize("tokens", [400, 1030])
 def test_mixtral_mlp_many_rows_an_expert(xh, orc, tokens):
-    """100 and 257 rows an expert on average: 128-row blocks, some experts' last ones of few rows, several blocks an expert."""
+    """100 and 257 rows an expert on average: blocks of 64 to 128 rows, some experts' last ones of few rows, several blocks an expert."""
     test_mixtral_mlp_vs_oracle(xh, orc, tokens, False)
     test_mixtral_mlp_four_bit_experts(xh, orc, 1, tokens)
     test_mixtral_mlp_bf16_experts(xh, orc, tokens, 512, 1024)
     test_mixtral_mlp_bf16_experts(xh, orc, tokens, 352, 736)  # (a depth that is no whole number of steps)
+
+
+@pytest.mark.parametrize("kind,hidden,inter,tokens", [(0, 1536, 2944, 300), (1, 1536, 2432, 300), (2, 1536, 2432, 300), (4, 512, 4096, 340)])
+def test_mixtral_mlp_96_rows_a_block(xh, orc, kind, hidden, inter, tokens):
+    """75 and 85 rows an expert on average, for which blocks of 96 rows are taken (the down projection's K in parts, but of BF16 weights in other blocks): experts
+    that fill one, with a row more, with two and one row, with fewer than 64, with one row and with none."""
+    E, rng = 8, np.random.default_rng(hidden + kind)
+    counts = [96, 97, 65, 1, 0, 193, 63]
+    of = np.repeat(np.arange(E), counts + [2 * tokens - sum(counts)])
+    pairs = np.stack([of[:tokens], of[tokens:]], 1)[rng.permutation(tokens)]  # (no expert has as many rows as there are tokens: two different ones each)
+    lo = rng.uniform(-9.0, -8.0, (tokens, E)).astype(np.float32)
+    np.put_along_axis(lo, pairs, rng.uniform(-1.0, 1.0, pairs.shape).astype(np.float32), 1)
+    x, ln = orc.round_bf16(rng.standard_normal((tokens, hidden))), rng.uniform(0.8, 1.2, hidden).astype(np.float32)
+    router = np.zeros((hidden, E), np.float32)
+    moe = xh.MoE(hidden, inter, E, tokens, router, ln)
+    if kind == xh.W_BF16:
+        experts = [(orc.round_bf16(rng.standard_normal((hidden, 2 * inter)) * 0.02), orc.round_bf16(rng.standard_normal((inter, hidden)) * 0.02)) for _ in range(E)]
+        for e, (gu, dn) in enumerate(experts):
+            moe.set_expert(e, xh.Weight(xh.W_BF16, hidden, 2 * inter, orc.to_bf16(gu), flags=xh.WF_GATEUP), xh.Weight(xh.W_BF16, inter, hidden, orc.to_bf16(dn)))
+    else:
+        experts = _experts(orc, rng, kind, hidden, inter, E)
+        for e, (gu, dn) in enumerate(experts):
+            moe.set_expert(e, xh.Weight(kind, gu.K, gu.N, gu.q, gu.scale, gu.zero, flags=xh.WF_GATEUP), xh.Weight(kind, dn.K, dn.N, dn.q, dn.scale, dn.zero))
+    xd, lod, od = xh.DeviceBuffer.from_numpy(x), xh.DeviceBuffer.from_numpy(lo), xh.DeviceBuffer(x.nbytes)
+    sel, w = moe.forward(xd.ptr, od.ptr, tokens, True, lod.ptr)
+    xh.synchronize()
+    got = od.to_numpy(np.float32, x.shape)
+    esel, ew = orc.moe_top2(lo)
+    assert np.array_equal(sel, esel) and np.abs(w - ew).max() < 1e-6
+    assert list(np.bincount(sel.ravel(), minlength=E)[:len(counts)]) == counts
+    if kind == xh.W_BF16:
+        xn, exp = orc.round_bf16(orc.rmsnorm(x, ln)).astype(np.float64), x.astype(np.float64).copy()
+        for e, (gu, dn) in enumerate(experts):
+            t, s_ = np.nonzero(sel == e)
+            y = xn[t] @ gu.astype(np.float64)
+            h = orc.round_bf16((y[:, :inter] / (1.0 + np.exp(-y[:, :inter])) * y[:, inter:]).astype(np.float32)).astype(np.float64)
+            exp[t] += w[t, s_, None].astype(np.float64) * (h @ dn.astype(np.float64))
+    else:
+        exp, _, _ = orc.mixtral_mlp(x, ln, router, experts, lo, rounding="bf16")
+    assert np.abs(got - exp).max() < 2e-2 and _cos(got, exp) >= 0.9999
 
 
 @pytest.mark.parametrize("kind,hidden,inter,tokens", [(0, 1056, 3600, 256), (1, 1056, 3600, 160), (0, 2048, 2816, 100), (2, 2048, 2816, 300)])
