@@ -65,8 +65,9 @@ __device__ inline void store_direct(const AttnParams &p, const size_t base, cons
 // XCDs (pair = 8 group + XCD).  An XCD takes its groups in bands of five, and the column groups of a band's pairs in turn, longest history first: what
 // runs at the end is short then.  Pair after pair instead, an XCD ended on the long walks of its last pair wherever its 64 workgroups at a time were
 // no multiple of the pairs' own: 5 x 700 tokens, 32 query / 8 KV heads 47 -> 41 us, 2 x 2000, 32 / 32 heads 123 -> 102, 5 x 1500 INT8 236 -> 197, 4 x 2000, 32 / 8
-// heads 155 -> 153, INT8 213 -> 206; 31 shapes over both caches and the paged one 1.067 times as fast in the geometric mean, the slowest the same.  Bands of 4 and 6: within
-// 0.1 % of that; of 3 or of 16 1 to 2 % slower (8 x 800 tokens 57.5 -> 60.0, 8 x 3900, 32 / 32 heads, in one 1161 -> 1353: an L2 does not hold that many pairs' keys and values).
+// heads INT8 213 -> 206, FP16 153 in either order (63 column groups fill the 64 places).  96 FP16 shapes of 1 to 12 sequences, 16 .. 64 / 4 .. 32 heads: 0.97 of the time in the geometric
+// mean, with one query head a KV head 0.90, four 0.94, six 0.99, eight and sixteen, whose pairs have many column groups, the same (0.95 .. 1.055, as the runs differ); 70 INT8 0.93, 36
+// paged 0.98.  Bands of 4 and 6: within 0.1 % of that in 31 shapes; of 3 or of 16 1 to 2 % slower (8 x 800 tokens 57.5 -> 60.0, 8 x 3900, 32 / 32 heads, in one 1161 -> 1353: an L2 does not hold that many pairs' keys and values).
 constexpr int kBand = 5;
 struct PrefillBands { // what is left of whole bands comes first, `rest` groups; then bands of `width`
     int rest, width;

@@ -77,7 +77,7 @@ struct StepTraits<XFTHIP_W_BF16, DIRECT> {
 //
 // DIRECT: the activation tiles go from global memory straight into LDS (global_load_lds_dwordx4: a wave instruction
 // fills 1 KiB of consecutive LDS, lane after lane, from 64 addresses of its choice) instead of through registers and
-// ds_write (tiles of 96 and 128 rows).  Rows are 128 bytes with no padding; the 16-byte chunk c of row r sits in slot c ^ ((r >> 1) & 7) of its
+// ds_write (the tiles of 96 and 128 rows).  Rows are 128 bytes with no padding; the 16-byte chunk c of row r sits in slot c ^ ((r >> 1) & 7) of its
 // row, which a lane gets by choosing the global chunk it fetches, and which keeps the operand reads (32 rows, one
 // chunk index) free of bank conflicts.  Four LDS tiles: step k requests tile k + 3, and the barrier that ends a step
 // first waits until the wave's requests of the step before are in (vmcnt counts them in order with the weight
@@ -217,8 +217,8 @@ __global__ __launch_bounds__(256 * KG, (DIRECT && KG == 1) ? 2 : 1) void qgemm_m
     uint2 *lut = nullptr;
     unsigned char *abuf_base = lds;
     if constexpr (KIND == XFTHIP_W_NF4) {
-        // DIRECT: the table sits behind the tiles, which then start at LDS offset 0 of the workgroup and end below 64 KiB
-        // (the requests carry their LDS address in M0)
+        // DIRECT: the table sits behind the tiles, which then start at LDS offset 0 of the workgroup.  (The requests carry their LDS address in M0, all of it: the tiles of two K
+        // groups end at 128 KiB.)
         lut = (uint2 *)(DIRECT ? lds + KG * 4 * ROWS * ROWB + (KG == 2 ? 1024 : 0) : lds);
         abuf_base = DIRECT ? lds : lds + 2048;
         if (threadIdx.x < 256) {

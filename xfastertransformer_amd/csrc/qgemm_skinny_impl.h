@@ -432,6 +432,8 @@ __device__ __forceinline__ void qgemm_skinny_body(SkinnyParams &p) {
                 // rows: INT8, 22016 columns with SwiGLU 18.8 / 20.2 / 23.0 -> 17.8 / 19.4 / 21.6 us, 12288 with RoPE 13.1 / 14.7 / 17.9 -> 12.6 / 14.0 / 16.8; UINT4 0.91 of the time in
                 // the mean, NF4 0.96, BF16 0.97.  (Two rows at a time: INT8 1 % faster with several rows and as much slower with one; requested ahead of the
                 // weights: the same to 3 % slower; four rows: a workgroup a CU less.)
+                // Wider rows (K above 4096, 4-bit weights 8192) take two trips, the norm weights with the second: 8704 .. 18176 deep, UINT4 and NF4, 0.97 .. 1.01 of the time of the form
+                // that requested one value of each of their lines with the first.
                 for (int m = 0; m < p.M; ++m) {
                     float4 v[NB], w[NB];
 #pragma unroll
@@ -756,6 +758,7 @@ static int launch(const SkinnyParams &p, int kslices, hipStream_t stream) {
     return 0;
 }
 
+// (the patches of eight slices of 17 .. 32 rows end at 128 KiB of LDS, at 130 behind NF4's table: M0, which holds a request's place there, counts beyond 16 bits)
 template <int KIND, int NT, int MT, bool NEED_SUM>
 static int launch_dma(const SkinnyParams &p, int kslices, hipStream_t stream) {
     constexpr int ROWS = 16 * MT, COLS = 16 * NT;
