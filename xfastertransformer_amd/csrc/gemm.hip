@@ -14,8 +14,10 @@ static int check_common(const char *fn, xfthip_weight_t w, int M, const void *A,
 }
 
 // Rows out of reach of the kernels' 32-bit element offsets (8 GB from the first) come in products of their own, of as many rows as are within reach.
-static int gemm_rows(const PackedWeight &pw, SkinnyParams p, hipStream_t stream) {
-    const size_t reach = ((size_t)1 << 32) - 4096, within = reach / (size_t)p.lda + 1; // (a lane adds its place in the row)
+static int gemm_rows(const PackedWeight &pw, SkinnyParams &p, hipStream_t stream) {
+    const size_t reach = ((size_t)1 << 32) - 4096; // (a lane adds its place in the row)
+    if ((size_t)p.M * p.lda <= reach) return p.M <= 32 ? qgemm_skinny(pw, p, stream) : qgemm_mfma(pw, p, stream);
+    const size_t within = reach / p.lda + 1;
     for (int left = p.M; left > 0; left -= p.M) {
         p.M = (size_t)left < within ? left : (int)within;
         if (int rc = p.M <= 32 ? qgemm_skinny(pw, p, stream) : qgemm_mfma(pw, p, stream)) return rc;
