@@ -195,7 +195,7 @@ def test_mixtral_mlp_many_rows_an_expert(xh, orc, tokens):
     test_mixtral_mlp_bf16_experts(xh, orc, tokens, 352, 736)  # (a depth that is no whole number of steps)
 
 
-@pytest.mark.parametrize("kind,hidden,inter,tokens", [(0, 1536, 2944, 300), (1, 1536, 2432, 300), (2, 1536, 2432, 300), (4, 512, 4096, 340)])
+@pytest.mark.parametrize("kind,hidden,inter,tokens", [(0, 2560, 3328, 300), (1, 2560, 2432, 300), (2, 1536, 5760, 300), (4, 512, 4224, 340)])
 def test_mixtral_mlp_96_rows_a_block(xh, orc, kind, hidden, inter, tokens):
     """75 and 85 rows an expert on average, for which blocks of 96 rows are taken (the down projection's K in parts, but of BF16 weights in other blocks): experts
     that fill one, with a row more, with two and one row, with fewer than 64, with one row and with none."""

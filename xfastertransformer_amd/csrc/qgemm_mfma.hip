@@ -132,9 +132,12 @@ constexpr TileCost kTiles[] = {
         {128, 256, 2, 1, 8.7f, {1.49f, 1.8f, 2.63f, 1.49f}, {}},
 };
 
-// What 96 x 256 has to gain by the model before a product takes it (not experts, whose rows are an estimate): 700 products that the model alone gives to it, against what they take
+// What 96 x 256 has to gain by the model before a product takes it: 700 products that the model alone gives to it, against what they take
 // without it, lost more than 2 % in 12 % of cases (NF4 19) and up to 1.2 times (800 x 14336 x 28672 BF16 665 -> 755 us, 696 x 2560 x 11008 NF4 79 -> 91), mostly where the model saw
 // little to gain.  With these prices 4 %, and 0.931 of the time in the geometric mean (0.928 without).  Left: 4 row blocks of BF16 over 32000 columns, 1.1 to 1.2 times.
+// Experts, whose rows are an estimate: 1.02 for gate and up (208 tokens UINT4 286 -> 292 us without), and 1.08 where their blocks of 96 hold no fewer rows than those of 128 would
+// (117 rows each, say): a Mixtral-8x7B layer of 130 to 1024 tokens 0.92 of the time in the geometric mean (0.79 .. 1.01); without the prices 468 tokens INT8 486 -> 548, UINT4 453 ->
+// 513, with them 505 -> 477 and 458 -> 423.
 constexpr float kPrice96[4] = {1.03f, 1.07f, 1.05f, 1.03f}; // INT8, BF16, NF4, UINT4
 
 constexpr float kSplitStart[4] = {3.0f, 4.0f, 3.0f, 3.0f}, kSplitMb[4] = {0.3f, 0.35f, 0.3f, 0.3f}; // launch and megabytes of a split K's sum
@@ -181,6 +184,17 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_sp
     const bool direct = p.K % 64 == 0 && (size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32);
     p.tile = 2, p.kgroups = 1, p.direct = 0;
     if (!direct && !p.rows_dev && choose_staged_tile(p, kind, ktile, may_split)) return;
+    auto blocks_of = [&](const int rows) { // row blocks
+        if (p.group) {
+            // expected blocks of a weight whose rows scatter normally about their share: 1 + the chances that there are more than `rows`,
+            // 2 `rows`, .. of them
+            const float each = (float)p.M / (float)p.group_n, spread = sqrtf(each) + 0.1f * each;
+            float blocks = 1.0f;
+            for (int j = rows; (float)j < each + 4.0f * spread; j += rows) blocks += 0.5f * erfcf(((float)j - each) / (1.41421356f * spread));
+            return (int)(blocks * (float)p.group_n + 0.999f);
+        }
+        return ((p.rows_dev && p.m_hint > 0 ? p.m_hint : p.M) + rows - 1) / rows;
+    };
     float best = 1e30f;
     for (const TileCost &t : kTiles) {
         if (t.rows == 32 && kind == XFTHIP_W_BF16) continue; // (not built: two bytes a weight want more rows behind them)
@@ -189,18 +203,7 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_sp
         // (8 weights of 28672 x 4096 and 4096 x 14336 INT8 with 37 rows each: 386 us a layer in 32-row blocks, which read every weight tile twice,
         // 353 in 64-row ones)
         if (t.rows == 32 && p.group && p.M > 32 * p.group_n) continue;
-        int row_blocks = (p.M + t.rows - 1) / t.rows;
-        const int col_blocks = (p.N + t.cols - 1) / t.cols;
-        if (p.group) {
-            // expected blocks of a weight whose rows scatter normally about their share: 1 + the chances that there are more than t.rows,
-            // 2 t.rows, .. of them
-            const float each = (float)p.M / (float)p.group_n, spread = sqrtf(each) + 0.1f * each;
-            float blocks = 1.0f;
-            for (int j = t.rows; (float)j < each + 4.0f * spread; j += t.rows) blocks += 0.5f * erfcf(((float)j - each) / (1.41421356f * spread));
-            row_blocks = (int)(blocks * (float)p.group_n + 0.999f);
-        } else if (p.rows_dev && p.m_hint > 0) {
-            row_blocks = (p.m_hint + t.rows - 1) / t.rows;
-        }
+        const int row_blocks = blocks_of(t.rows), col_blocks = (p.N + t.cols - 1) / t.cols;
         for (int want : {1, 2, 3, 4, 6, 8}) {
             if (want > 1 && (!may_split || p.gateup || p.K / want < 512)) break;
             int part = (kt_n + want - 1) / want; // packed tiles
@@ -230,7 +233,7 @@ void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_sp
             // blocks, which were to take 1 more; the layer 137 -> 129.  With down projections priced so as well, 256 tokens of the Mixtral shape
             // lose 0.7 %)
             if (p.group && p.gateup && t.rows == 128) us *= 1.05f;
-            if (t.rows == 96 && !p.rows_dev) us *= kPrice96[cls];
+            if (t.rows == 96) us *= !p.group ? kPrice96[cls] : 96 * row_blocks >= 128 * blocks_of(128) ? 1.08f : p.gateup ? 1.02f : 1.0f;
             if (us < best) {
                 best = us;
                 p.tile = t.rows == 32 ? 1 : t.rows == 64 ? 2 : t.rows == 96 ? 5 : t.cols == 128 ? 3 : 4;
