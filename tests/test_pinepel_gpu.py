@@ -83,6 +83,20 @@ def test_queries_rotated_where_they_are_loaded(xh, rot, heads, kv_rank, window):
     c.free()
 
 
+@pytest.mark.parametrize("window", [None, 50], ids=["halves", "neighbours"])
+def test_queries_of_many_short_segments(xh, window):
+    """8 workgroups a CU, the most whose queries the attention rotates, and one sequence more (256 CUs)"""
+    cfg = u.config([u.latent(heads=64, rot=16, kv_rank=64, dim=16, vdim=16, window=window)])
+    for n in (33, 34):
+        c = Case(xh, cfg, 7, "bf16", slots=n, max_seq=64, max_tokens=n * 31)
+        texts = [tokens_of(cfg, 33, i) for i in range(n)]
+        c.model.step([(i, t[:2], []) for i, t in enumerate(texts)])
+        got = c.model.step([(i, t[2:], [30]) for i, t in enumerate(texts)])
+        for i in (0, n // 2, n - 1):
+            c.check(got[i:i + 1], c.want(texts[i])[32:], f"sequence {i} of {n}")
+        c.free()
+
+
 @pytest.mark.parametrize("act", ["f32", "bf16"])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,conv", [(2, 2, 128, 128, 4), (2, 2, 128, 129, 4), (4, 2, 256, 64, 2), (2, 1, 250, 65, 3), (3, 3, 64, 256, 3), (2, 1, 40, 250, 4),
                                                           (3, 1, 32, 96, 4), (2, 2, 32, 264, 2), (4, 4, 20, 12, 3), (2, 2, 128, 100, 5)], ids=str)

@@ -691,10 +691,11 @@ int latent_prepare(int act, const PlanLayer &L, const StepView &v, const void *a
 
 // Steps whose segments all take the absorbed form on the matrix units (below latent_expanded_takes' 32 tokens): each workgroup rotates the queries it loads,
 // where it finds whole vectors of pairs.  Bound by the launch that goes with it (2.2 us, 2 workgroups at 4 sequences):
-// a prompt and 16 steps of 4 sequences over two such layers and one of the delta rule 6.70 -> 6.50 ms.
+// a prompt and 16 steps of 4 sequences over two such layers and one of the delta rule 6.70 -> 6.50 ms.  Up to 8 workgroups a CU: beyond, the turns in each of them are what the
+// launch took and more (six layers of 128 heads, 96 sequences of 31 tokens 7.25 ms with the launch, 7.44 without, 64 of 16 2.42 and 2.46; 32 heads, 16 of 16 450 and 435 us).
 static bool rotates_inside(int act, const PlanLayer &L, const StepView &v) {
     const int half = L.s.rot_dim / 2;
-    return act == XFTHIP_BF16 && v.longest < 32 && mfma_takes(L) && half > 0 && half % (L.s.rot_interleaved ? 4 : 8) == 0;
+    return act == XFTHIP_BF16 && v.longest < 32 && (long)v.B * ((v.longest * L.s.heads + 31) / 32) <= 8L * device_cu_count() && mfma_takes(L) && half > 0 && half % (L.s.rot_interleaved ? 4 : 8) == 0;
 }
 
 int latent_rotate_q(int act, const PlanLayer &L, const StepView &v, void *q, hipStream_t st) {
