@@ -450,3 +450,11 @@ def test_ragged_k_in_one_sum(xh, M):
     dw = xh.Weight(xh.W_BF16, K, N, xh.f32_to_bf16_bits(W))
     assert (_run_gemm(xh, dw, xh.f32_to_bf16_bits(A), M, K, N, xh.F32) == 1.0).all()
     dw.free()
+
+
+@pytest.mark.parametrize("kind", ["uint4", "nf4"])
+@pytest.mark.parametrize("M,K,N,direct", [(2100, 192, 6160, 1), (2308, 320, 2512, 1), (2000, 1088, 4112, 1), (2129, 12352, 400, 1), (2100, 64, 6160, 0)])
+def test_four_bit_steps_of_half_a_tile_against_64_bits(xh, orc, kind, M, K, N, direct):
+    """4-bit weights, K an odd number of 64: the last step of the tiles with activations straight into LDS is half a packed tile (a single half is not theirs)."""
+    assert xh.gemm_form({"uint4": xh.W_UINT4, "nf4": xh.W_NF4}[kind], M, K, N, 0, kind == "uint4")[4] == direct
+    test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N)
