@@ -18,18 +18,20 @@
 namespace xfthip {
 namespace {
 
-// KSTEP: k a step; MICRO: MFMA steps of 32 k in it; NBUF: activation tiles in LDS; WSETS: weight tiles in registers
-template <int KIND>
+// KSTEP: k a step; NBUF: activation tiles in LDS; SETS: weight tiles in registers, three (BF16, 32 registers each: two, reloaded behind the products that read them) but
+// for 128 x 128 blocks of four waves, which have room for twice as many and wait for them: 100 x 4096 x 14336, blocks alone on their CUs, INT8 98 -> 89 us, BF16 133 -> 117
+// (with two K groups, 96 x 256 and the 4-bit kinds the same or 1 to 3 % slower).
+template <int KIND, int CT, int KG>
 struct DirectTraits { // 4-bit kinds: a lane holds 32 neighbouring codes, one MFMA takes 8 of each lane group's, so that a step is a whole packed tile of 128 k
-    static constexpr int KSTEP = 128, NBUF = 2, WSETS = 2;
+    static constexpr int KSTEP = 128, NBUF = 2, SETS = 2;
 };
-template <>
-struct DirectTraits<XFTHIP_W_INT8> {
-    static constexpr int KSTEP = 64, NBUF = 4, WSETS = 3;
+template <int CT, int KG>
+struct DirectTraits<XFTHIP_W_INT8, CT, KG> {
+    static constexpr int KSTEP = 64, NBUF = 4, SETS = CT == 2 && KG == 1 ? 6 : 3;
 };
-template <>
-struct DirectTraits<XFTHIP_W_BF16> {
-    static constexpr int KSTEP = 64, NBUF = 4, WSETS = 2; // (a tile is 32 registers: reloaded behind the products that read them)
+template <int CT, int KG>
+struct DirectTraits<XFTHIP_W_BF16, CT, KG> {
+    static constexpr int KSTEP = 64, NBUF = 4, SETS = CT == 2 && KG == 1 ? 4 : 2;
 };
 
 // Slot of 16-byte chunk c of LDS row r is c ^ direct_swizzle(r).  A row is 128 or 256 bytes; an operand read is rows 0 .. 15 of a tile, 16 lanes a chunk index,
@@ -53,8 +55,8 @@ __device__ inline uint64_t uniform_address(const void *q) {
 // (a SIMD has two waves to issue from, as with two blocks a CU); the second hands its sums to the first through LDS.
 template <int KIND, int CT, int RT, bool NEED_SUM, bool DEVROWS, int KG>
 __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel(SkinnyParams p, int nblocks_n, int nblocks_m) {
-    using T = DirectTraits<KIND>;
-    constexpr int KSTEP = T::KSTEP, NBUF = T::NBUF, WSETS = T::WSETS, MICRO = KSTEP / 32;
+    using T = DirectTraits<KIND, CT, KG>;
+    constexpr int KSTEP = T::KSTEP, NBUF = T::NBUF, WSETS = T::SETS, MICRO = KSTEP / 32;
     constexpr int ROWS = 16 * RT, ROWB = KSTEP * 2, TILEB = ROWS * ROWB, CPR = KSTEP / 8; // bytes of an LDS row and tile, chunks a row
     constexpr int ALOADS = TILEB / 4096;                                                  // requests of 1 KiB a wave and tile
     constexpr bool FOUR = KIND == XFTHIP_W_UINT4 || KIND == XFTHIP_W_NF4, BF16 = KIND == XFTHIP_W_BF16, NF4 = KIND == XFTHIP_W_NF4;
@@ -182,10 +184,13 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
     };
 #define XFT_FENCE() __builtin_amdgcn_sched_barrier(0)
     // One step: the products of k tile kt, a group of RT MFMAs for each (32 k, column tile).  With them go the requests of activation tile kt + NBUF - 1, the loads of
-    // weight tile kt + WSETS - 1 (BF16: kt + 2, each behind the products that read its registers), the widening of the next group's weights and, behind the last
+    // weight tile kt + WD into the registers of the one that this step takes (4-bit: into the other set), the widening of the next group's weights and, behind the last
     // products that read it, the next activation operand.
-    constexpr int QN = MICRO * CT, AHEAD = NBUF - 1, WD = BF16 ? 2 : WSETS - 1;
-    constexpr int APG = FOUR ? 2 : (ALOADS + QN / 2 - 1) / (QN / 2); // requests a group that has some
+    // The requests come in front of the loads: the compiler's wait for a tile's weights counts only the loads behind them, so that it is also one for as many of the
+    // youngest requests.  With three tiles under way that leaves this step's out; in turn with them, and with two, each step waited for half of its own.  INT8, blocks alone
+    // on their CUs, 500 x 4096 x 14336: 128 x 128 136 -> 106 us, with two K groups 91 -> 85, 128 x 256 156 -> 152; 600 x 4096 x 4096 33 -> 30.
+    constexpr int WD = FOUR ? 1 : WSETS, AHEAD = NBUF - 1;
+    constexpr int APG = FOUR ? 2 : (ALOADS + CT - 1) / CT; // requests a group that has some
     MFrag wcur_hi, wcur_lo;
     float rs[2] = {0.0f, 0.0f};
     auto step = [&](int w_cur, int w_next, int w_load, int kt) {
@@ -195,18 +200,15 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
 #pragma unroll
             for (int t = 0; t < CT; ++t) {
                 const int q = ms * CT + t;
-                // requests first where the step's own end waits for them (two tiles), else in turn with the weights
-                const int ai = FOUR ? q : q / 2, wi = FOUR ? q - ALOADS / 2 : q / 2;
-                if ((FOUR || q % 2 == (BF16 ? 0 : 1))) {
 #pragma unroll
-                    for (int i = ai * APG; i < (ai + 1) * APG; ++i)
-                        if (i < ALOADS) request_a(kt + AHEAD, i);
-                }
-                if (!BF16 && (FOUR || q % 2 == 0) && wi >= 0 && wi < CT) load_w(w_load, kt + WD, 0, wi);
+                for (int i = q * APG; i < (q + 1) * APG; ++i)
+                    if (i < ALOADS) request_a(kt + AHEAD, i);
+                if (FOUR && q >= ALOADS / 2 && q < ALOADS / 2 + CT) load_w(w_load, kt + WD, 0, q - ALOADS / 2);
+                if (KIND == XFTHIP_W_INT8 && ms == 1) load_w(w_load, kt + WD, 0, t); // (its codes have been widened a group ago)
                 MFrag nhi, nlo;
                 if (t + 1 < CT) widen(w_cur, ms, t + 1, nhi, nlo);
                 else if (ms + 1 < MICRO) widen(w_cur, ms + 1, 0, nhi, nlo);
-                else widen(w_next, 0, 0, nhi, nlo); // the next tile's set: loaded in an earlier step (4-bit: in this one)
+                else widen(w_next, 0, 0, nhi, nlo);
                 if constexpr (NEED_SUM) {
                     if (t == 0) {
                         typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -266,16 +268,17 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
         else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WREQS) : "memory");
         ++kt;
     };
-#define XFT_STEP(s)                                                        \
-    {                                                                      \
-        step((s) % WSETS, ((s) + 1) % WSETS, ((s) + WD) % WSETS, kt);      \
-        end_step();                                                        \
+#define XFT_STEP(s)                                              \
+    {                                                            \
+        step((s) % WSETS, ((s) + 1) % WSETS, (s) % WSETS, kt);   \
+        end_step();                                              \
     }
     if constexpr (FOUR) {
         auto one = [&]() { // (the next tile's registers are copied: 16 of them a step of 128 products)
 #pragma unroll
             for (int m = 0; m < RT; ++m) read_a((kt & 1) * TILEB, 0, m);
-            XFT_STEP(0)
+            step(0, 1, 1, kt);
+            end_step();
 #pragma unroll
             for (int t = 0; t < CT; ++t) wreg[0][0][t] = wreg[1][0][t];
         };
@@ -292,17 +295,19 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
             __syncthreads();
             one();
         }
-    } else if constexpr (WSETS == 3) {
-        while (kt + 3 <= kt_n) {
-            XFT_STEP(0) XFT_STEP(1) XFT_STEP(2)
-        }
-        if (kt < kt_n) XFT_STEP(0)
-        if (kt < kt_n) XFT_STEP(1)
     } else {
-        while (kt + 2 <= kt_n) {
+        while (kt + WSETS <= kt_n) {
             XFT_STEP(0) XFT_STEP(1)
+            if constexpr (WSETS > 2) XFT_STEP(2)
+            if constexpr (WSETS > 3) XFT_STEP(3)
+            if constexpr (WSETS > 4) XFT_STEP(4)
+            if constexpr (WSETS > 5) XFT_STEP(5)
         }
         if (kt < kt_n) XFT_STEP(0)
+        if (WSETS > 2 && kt < kt_n) XFT_STEP(1)
+        if (WSETS > 3 && kt < kt_n) XFT_STEP(2)
+        if (WSETS > 4 && kt < kt_n) XFT_STEP(3)
+        if (WSETS > 5 && kt < kt_n) XFT_STEP(4)
     }
 #undef XFT_STEP
 #undef XFT_FENCE
@@ -439,7 +444,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
 
 template <int KIND, int CT, int RT, bool NEED_SUM, bool DEVROWS, int KG>
 static int launch_direct(const SkinnyParams &p, hipStream_t stream) {
-    using T = DirectTraits<KIND>;
+    using T = DirectTraits<KIND, CT, KG>;
     BlockGrid g;
     if (int rc = block_grid<DEVROWS>(p, 16 * RT, 4 * CT, g)) return rc;
     // the activation tiles, the second K group's row sums and NF4's table; reused after the k loop by the four waves' output patches and the row sums
