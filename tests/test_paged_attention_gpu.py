@@ -232,6 +232,12 @@ def test_paged_prefill_bands(xh, orc, qH, kvH, lens):
     test_paged_prefill_matches_oracle(xh, orc, qH, kvH, lens, 16)
 
 
+@pytest.mark.parametrize("qH,kvH,lens", [(32, 8, [1700, 1103, 33, 701]), (24, 24, [2101, 1500])])
+def test_paged_prefill_that_fills_the_device(xh, orc, qH, kvH, lens):
+    """Enough long walks for the form in 16 x 16 MFMAs, a short sequence beside them."""
+    test_paged_prefill_matches_oracle(xh, orc, qH, kvH, lens, 16)
+
+
 @pytest.mark.parametrize("qH,kvH,lens", [(32, 8, [200] * 8), (32, 8, [511, 150, 512, 600, 130]), (16, 4, [500, 270, 300, 20, 400]), (8, 8, [40] * 70)])
 @pytest.mark.parametrize("size,key,scale", [(24.0, 1.0, 128 ** -0.5), (1.5e-4, 1e4, 128 ** -0.5), (1.0, 1e4, 1.5e-5)])
 def test_paged_prefill_as_exact_as_alone(xh, orc, qH, kvH, lens, size, key, scale):

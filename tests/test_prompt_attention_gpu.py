@@ -208,3 +208,30 @@ def test_any_softmax_scale(xh, orc, scale, size, kind):
     off = np.sqrt(((got - ref) ** 2).reshape(B, S, -1).mean((0, 2))) / np.sqrt((ref ** 2).reshape(B, S, -1).mean((0, 2)))
     assert off.max() < 4e-4, off
     dc.free()
+
+
+@pytest.mark.parametrize("B,S,past,qh,kvh,kind,extra,skip", [
+    (3, 1025, 500, 32, 8, "bf16", 0, 0),  # 33 workgroups a pair, the last of 4 columns
+    (5, 515, 1101, 28, 4, "bf16", 8, 8),  # 7 heads a group: a wave's tiles of 16 columns begin inside a token; 21 columns in the last workgroup
+    (2, 301, 2003, 128, 2, "f32", 4, 0),  # 64 heads a group: both tiles of a wave belong to one token
+    (8, 1025, 800, 8, 8, "bf16", 1, 1),  # one head a group: every column another token; rows on 2-byte borders
+    (8, 129, 1233, 64, 8, "bf16", 4, 4),
+])
+@pytest.mark.parametrize("score,scale", [(None, SCALE), (-1e30, SCALE), (3000.0, SCALE), (None, 1e-4)])
+def test_launches_that_fill_the_device(xh, orc, B, S, past, qh, kvh, kind, extra, skip, score, scale):
+    """512 and more workgroups, 20480 and more (workgroup, 32-token block) pairs: the form in 16 x 16 MFMAs.  The first 40 tokens score as the others,
+    minus infinity, or so high that the others' weights vanish."""
+    rng = np.random.default_rng(S * 31 + past)
+    assert -(-S * (qh // kvh) // 128) * B * kvh >= 512 and -(-S * (qh // kvh) // 128) * B * kvh * ((past + S // 2) // 32) >= 20480
+    k, v = (rng.standard_normal((B, past + S, kvh * D)).astype(np.float32) for _ in range(2))
+    q = orc.round_bf16(rng.standard_normal((B * S, qh * D)))
+    if score is not None:
+        k.reshape(B, past + S, kvh, D)[:, :40, :, 0] = score
+        k.reshape(B, past + S, kvh, D)[:, 40:, :, 0] = 0.0
+        q.reshape(B * S, qh, D)[:, :, 0] = 1.0
+    kc, vc, dc = _cache(xh, orc, k, v)
+    got = _attend(xh, orc, dc, q, B, S, qh, past, xh.BF16 if kind == "bf16" else xh.F32, qh * D + extra, skip, scale)
+    ref = orc.attention_ref_f64(q, kc.as_f32(), vc.as_f32(), qh, kvh, D, [S] * B, [past] * B, scale)
+    # fp16 probabilities: 2^-11 of a value each; bf16 results 2^-9 on top
+    assert (np.abs(got - ref) <= 3e-3 + np.abs(ref) * (2.0 ** -8 if kind == "bf16" else 0.0)).all(), np.abs(got - ref).max()
+    dc.free()

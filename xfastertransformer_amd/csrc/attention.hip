@@ -55,8 +55,8 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(AttnParams p) {
     attn_merge_unit(p, blockIdx.y, blockIdx.x, s_pm, s_f);
 }
 
-// 32 x 32 MFMA tiles, 32 columns a wave, K / V blocks shared through LDS (attention_prefill.h); two workgroups a CU
-template <bool INT8>
+// 32 columns a wave, K / V blocks shared through LDS (attention_prefill.h); two workgroups a CU
+template <bool INT8, bool FINE>
 __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(AttnParams p, int ncg, int npairs, PrefillBands bands) {
     __shared__ __attribute__((aligned(16))) unsigned char lds[INT8 ? kRingLdsInt8 : kRingLds];
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(AttnParams p, in
     prefill_band(bands, slot / ncg, first, width);
     const int at = slot - first * ncg, pair = (first + at % width) * 8 + xcd;
     if (pair >= npairs) return;
-    attn_prefill_ring_unit<INT8>(p, pair % p.kv.H, ncg - 1 - at / width, pair / p.kv.H, lds);
+    attn_prefill_ring_unit<INT8, FINE>(p, pair % p.kv.H, ncg - 1 - at / width, pair / p.kv.H, lds);
 }
 
 // Split-KV merge workspace: `slots` partial-result slots of kSlotFloats floats and one ticket per
@@ -170,8 +170,11 @@ int xfthip::attention_launch(xfthip_kvcache_t c, const void *q, int qStride, voi
             const int ncg = (S * p.G + 127) / 128, npairs = B * c->kv.H;
             const PrefillBands bands = prefill_bands((npairs + 7) / 8);
             dim3 grid(8 * ((npairs + 7) / 8) * ncg);
-            if (c->kv.int8) hipLaunchKernelGGL(attn_prefill32_kernel<true>, grid, dim3(256), 0, stream, p, ncg, npairs, bands);
-            else hipLaunchKernelGGL(attn_prefill32_kernel<false>, grid, dim3(256), 0, stream, p, ncg, npairs, bands);
+            const bool fine = prefill_fine(c->kv.int8, (long)ncg * npairs, past + S / 2);
+            if (c->kv.int8 && fine) hipLaunchKernelGGL((attn_prefill32_kernel<true, true>), grid, dim3(256), 0, stream, p, ncg, npairs, bands);
+            else if (c->kv.int8) hipLaunchKernelGGL((attn_prefill32_kernel<true, false>), grid, dim3(256), 0, stream, p, ncg, npairs, bands);
+            else if (fine) hipLaunchKernelGGL((attn_prefill32_kernel<false, true>), grid, dim3(256), 0, stream, p, ncg, npairs, bands);
+            else hipLaunchKernelGGL((attn_prefill32_kernel<false, false>), grid, dim3(256), 0, stream, p, ncg, npairs, bands);
             XFT_CHECK_HIP(hipGetLastError());
             return 0;
         }

@@ -1,22 +1,22 @@
-// Prefill attention on 32 x 32 MFMA tiles: many (query token, query head) columns per (sequence, KV head).
+// Prefill attention: many (query token, query head) columns per (sequence, KV head).
 //
 // Replaces the reference's flash-style prefill (xft::selfScaledDpAttention, src/kernels/attention_kernels.h:1283-1408;
 // DecoderUtil::incrementalTileAttention / softmaxTile / updateOutTile, src/utils/decoder_util.h:606-889) and its
 // chunked prefill over a cache (xft::crossAttnByHead, attention_kernels.h:988-1123) when a launch has enough
 // columns to fill the device.
 //
-// A workgroup shares each 32-token block of keys and values through LDS; a wave owns 32 columns.  A 32 x 32 x 16 MFMA
-// (32 cycles) takes one 1 KiB operand from there, twice the work of a 16 x 16 x 32 one on the same bytes.
+// A workgroup shares each 32-token block of keys and values through LDS; a wave owns 32 columns.
 //
-//   S^T = K . Q^T   tile: 32 tokens (rows) x 32 columns; A = keys from LDS, B = the wave's queries, held in
-//                   registers for the whole walk (8 k-steps of 16 dims)
-//   O^T += V^T . P^T  4 tiles of 32 dims x 32 columns; A = values from LDS (token index innermost, as the cache
+//   S^T = K . Q^T   32 tokens (rows) x 32 columns; A = keys from LDS, B = the wave's queries, held in registers for the whole walk
+//   O^T += V^T . P^T  128 dims x 32 columns; A = values from LDS (token index innermost, as the cache
 //                   stores them), B = probabilities straight from the score registers
-// In the 32 x 32 accumulator a lane owns one column and 16 of the 32 rows (rows 8 q + 4 h + s; h = lane / 32,
-// q = 0..3, s = 0..3), the other 16 sit in the lane 32 away.  The cache stores a value block with its tokens
-// permuted (kvcache.h: 16-byte chunk c of a dim row = tokens 4 c .. 4 c + 3 and 16 + 4 c .. 16 + 4 c + 3); with the
-// score rows in natural token order, chunk c = 2 t + h is exactly what lane half h holds in registers q = t and
-// q = t + 2, so the probabilities of k-step t need no exchange between lanes.
+//
+// Two forms.  In 32 x 32 x 16 MFMAs one operand read from LDS is one MFMA; a lane owns one column and 16 of a block's tokens (8 q + 4 h + s; h = lane / 32, q = 0..3,
+// s = 0..3).  FINE, in 16 x 16 x 32 ones: two column tiles, an operand read is two MFMAs; a lane owns two columns and 8 tokens (16 tt + 4 g + r; g = lane / 16).
+// The same products take less of the card's power as 16 x 16 x 32, and more instructions.
+// The cache stores a value block with its tokens permuted (kvcache.h: 16-byte chunk c of a dim row = tokens 4 c .. 4 c + 3 and 16 + 4 c .. 16 + 4 c + 3): chunk
+// c = 2 t + h is what lane half h holds in registers q = t and q = t + 2, chunk g what lane group g holds of its two score tiles, so that the probabilities are the B
+// operand of the values without an exchange between lanes.
 //
 // Online softmax per column in the log2 domain, fp32; the reference point moves only when a block's maximum
 // exceeds it by more than 2^8 (probabilities up to 256 are exact enough in fp16 and in the fp32 sums), so the
@@ -38,13 +38,17 @@ union HFrag32 {
     u32x4 q;
 };
 
-// a lane's column: dims 32 dt + 8 q + 4 h ..
-__device__ inline void store_direct(const AttnParams &p, const size_t base, const int h, const f32x16 (&o)[4], const float inv) {
+__device__ inline f32x16 prefill_mfma(const f16x8 a, const f16x8 b, const f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+__device__ inline f32x4 prefill_mfma(const f16x8 a, const f16x8 b, const f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+
+// a lane's column: dims 32 dt + 8 q + 4 h .. (FINE: 16 dt + 4 g ..)
+template <typename Acc, int DT>
+__device__ inline void store_direct(const AttnParams &p, const size_t base, const int part, const Acc (&o)[DT], const float inv) {
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const size_t idx = base + 32 * dt + 8 * q + 4 * h;
+        for (int q = 0; q < (DT == 8 ? 1 : 4); ++q) {
+            const size_t idx = base + 128 / DT * dt + 8 * q + 4 * part;
             const float v0 = o[dt][4 * q] * inv, v1 = o[dt][4 * q + 1] * inv, v2 = o[dt][4 * q + 2] * inv, v3 = o[dt][4 * q + 3] * inv;
             if (p.out_dtype == XFTHIP_BF16) {
                 const uint32_t lo = f32x2_to_bf16(v0, v1), hi = f32x2_to_bf16(v2, v3);
@@ -59,6 +63,14 @@ __device__ inline void store_direct(const AttnParams &p, const size_t base, cons
                 dst[0] = v0, dst[1] = v1, dst[2] = v2, dst[3] = v3;
             }
         }
+}
+
+// LDS rows are 64 bytes; the 16-byte chunk c of row r lies in slot c ^ row_turn(r).  A FINE operand read is rows 0 .. 15, chunk g of lane group g; its lanes are served 16 at a
+// time, not always neighbours: 0 .. 3 and 12 .. 15 of one group go with 4 .. 11 of the next, whose chunk differs in bit 0.  So rows of the two kinds differ in bit 1.
+template <bool FINE>
+__device__ inline int row_turn(int r) {
+    if constexpr (!FINE) return (r >> 2) & 3;
+    return (((r >> 2) ^ (r >> 3)) & 1) << 1 | ((r >> 3) & 1);
 }
 
 // Workgroups are handed to the 8 XCDs in turn by their linear index, and each XCD has an L2 of its own: the (sequence, KV head) pairs are dealt to the
@@ -81,7 +93,7 @@ __host__ __device__ inline void prefill_band(const PrefillBands b, const int gro
 
 // 128 columns a workgroup.  Figures are those of the FP16 cache where nothing else is said.
 //
-// A wave's time on a block of 32 tokens is the product phase - scores of block b + 1 and values of block b, 16 MFMAs (512 clocks), and behind each the
+// A wave's time on a block of 32 tokens is the product phase - scores of block b + 1 and values of block b, 16 MFMAs of 32 x 32 (512 clocks; FINE 32 of 16 x 16), and behind each the
 // read of the operand that takes its place: keys of block b + 2, values of block b + 1 - and the softmax phase, the probabilities of the block's scores, about 90
 // vector instructions, 16 of them exponentials, and the request of block b + kLook.  The two waves of a SIMD, of two workgroups, share its matrix unit
 // and vector ALU; products go first (s_setprio: 5 % slower without).  Reading all operands of a block in front of its products kept the wave from issuing
@@ -112,16 +124,32 @@ __host__ __device__ inline void prefill_band(const PrefillBands b, const int gro
 //
 // FP16: the queries carry the power of two in the softmax scale, the rest of it multiplies the scores in fp32: a bf16 value is exact in fp16 from 2^-17 / that
 // power up to 65504 / it.  Of a scale below 2^-4 / log2 e they carry a power of two of their own.  Where `plain` is set, they carry nothing, as in the form for few columns.  The row sums are those of the rounded probabilities.
+//
+// Which form.  FINE where the launch runs for so long that the card's power bounds it (4 x 2000 tokens: 168 us in 32 x 32 MFMAs, 125 where all operands are zeros); else its instructions, twice as many MFMAs and exchanges, cost more than its power saves.
+// FP16, mean workgroups x blocks of 32 tokens a CU in brackets, us of the call: 4 x 2000 tokens, 32 / 8 heads (250) 168 -> 160, 1 x 4000 (240) 136 -> 127, 2 x 2000, 32 / 32
+// (125) 104 -> 99, 8 x 1000 (125) 97 -> 94, paged 6 x 1500 (120) 112 -> 111, 2 x 2800, 32 / 32 (190) 165 -> 158; but 3 x 1200, 32 / 32 (70) 73 -> 72, 2 x 700 behind 1900
+// (97, 1.4 workgroups a CU) 73 -> 73, 4 x 800 (40) 40 -> 42, 8 x 500 (30) 37 -> 40, 512 behind 8000, half a workgroup a CU, 153 -> 154.
+// INT8, mean tokens walked in brackets: 4 x 2000 (1000) 226 -> 217, 5 x 1500 (750) 157 -> 148, 2 x 3500, 32 / 32 (1750) 344 -> 322, 512 behind 8000 (8250) 295 -> 282,
+// 900 (450) 40.2 -> 39.4; but 8 x 400 (200) 37.0 -> 37.7, 12 x 200 (100) 28.7 -> 28.8.
+// walk: the tokens that a column sees on average
+inline bool prefill_fine(bool int8, long workgroups, long walk) {
+    const long cus = device_cu_count();
+    return int8 ? walk >= 256 : workgroups >= 2 * cus && workgroups * (walk / 32) >= 80 * cus;
+}
+
 constexpr int kRing = 4, kLook = kRing - 1, kRingBlock = 16384, kRingLds = kRing * kRingBlock;
 constexpr int kScaleBytes = 256; // 32 key scales and 32 value scales of a block
 constexpr int kRingLdsInt8 = 3 * (kRingBlock + kScaleBytes);
 
 // lds: kRingLds or kRingLdsInt8 bytes; every thread of 256 calls it.  plain (FP16): the queries as they are
-template <bool INT8>
+template <bool INT8, bool FINE>
 __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh, const int cgroup, const int b, unsigned char *lds, const bool plain = false) {
     constexpr int D = 128, NW = 4, WC = 32;
+    // column tiles a wave, their columns, score and value accumulators a column tile, k-steps of the scores; a lane's scores of a column and accumulators' registers
+    constexpr int CT = FINE ? 2 : 1, TW = 32 / CT, XT = FINE ? 2 : 1, DT = FINE ? 8 : 4, QS = FINE ? 4 : 8, V = 16 / CT, AL = V / XT;
+    using Acc = std::conditional_t<FINE, f32x4, f32x16>;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int h = lane >> 5, cl = lane & 31;
+    const int h = lane >> 5, cl = lane & 31, part = lane / TW, tl = lane % TW;
     int past = p.past;
     if (p.past_dev) {
         past = p.past_dev[b];
@@ -133,7 +161,11 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
     const int c = c0 + cl;
     const bool cvalid = c < ncols;
     const int cs = cvalid ? c / p.G : 0, cj = cvalid ? c % p.G : 0;
-    const int limit = cvalid ? past + cs + 1 : 0; // tokens [0, limit) are visible to this column
+    // (c: the column whose rows of queries and results this lane finds; its products are of columns c0 + TW ct + tl)
+    int limit[CT]; // tokens [0, limit) are visible to that column, if there is one
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) limit[ct] = FINE ? __shfl(cvalid ? past + cs + 1 : 0, TW * ct + tl, 64) : cvalid ? past + cs + 1 : 0;
+    auto token = [&](int r) { return (FINE ? 16 : 8) * (r >> 2) + 4 * part + (r & 3); }; // of score r of a column, in its block
     const int lim_min = c0 + WC - 1 < ncols ? past + c0 / p.G + 1 : 0; // every column of the wave sees at least this many
     const int wave_last = c0 + WC - 1 < ncols ? c0 + WC - 1 : ncols - 1;
     const int wave_lim = c0 < ncols ? past + wave_last / p.G + 1 : 0, wave_nblk = (wave_lim + 31) >> 5; // no column of the wave sees a token from here on
@@ -154,8 +186,8 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int kr = 16 * i + (lane >> 2), vr = 32 * wave + 16 * i + (lane >> 2);
-        rq_koff[i] = kr * 256 + wave * 64 + (((lane & 3) ^ ((kr >> 2) & 3)) << 4);
-        rq_voff[i] = vr * 64 + (((lane & 3) ^ ((vr >> 2) & 3)) << 4);
+        rq_koff[i] = kr * 256 + wave * 64 + (((lane & 3) ^ row_turn<FINE>(kr)) << 4);
+        rq_voff[i] = vr * 64 + (((lane & 3) ^ row_turn<FINE>(vr)) << 4);
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
     auto request = [&](const int blk_raw) {
@@ -194,8 +226,8 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
             *(u32x4 *)(row + ((c ^ turn) << 4)) = lo.q;
             *(u32x4 *)(row + (((c + 1) ^ turn) << 4)) = hi.q;
         };
-        put(block + (ck >> 1) * 2048 + tk * 64, 2 * (ck & 1), (tk >> 2) & 3, kstage);
-        put(block + 8192 + vd * 64, 2 * h, (vd >> 2) & 3, vstage);
+        put(block + (ck >> 1) * 2048 + tk * 64, 2 * (ck & 1), row_turn<FINE>(tk), kstage);
+        put(block + 8192 + vd * 64, 2 * h, row_turn<FINE>(vd), vstage);
         if (wave == 0) *(float *)(lds + 3 * kRingBlock + slot(blk) * kScaleBytes + 4 * lane) = sstage;
     };
     if constexpr (INT8) {
@@ -205,12 +237,14 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
         request(1);
     }
 
-    // ---- this wave's queries: B operand of the score MFMA, k-step s covers dims 16 s + 8 h .. + 8 ----
-    float c1 = p.scale * 1.4426950408889634f, qmul = 1.0f;
-    HFrag32 qf[8];
-    auto take_query = [&](const int s, const u32x4 raw) {
+    // ---- this wave's queries: B operand of the score MFMA, k-step s covers dims 128 / QS s + 8 part .. + 8 of column TW ct + tl ----
+    float c1[CT], qmul[CT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) qf[s].u[i] = pack_f16(u2f(raw[i] << 16) * qmul, u2f(raw[i] & 0xFFFF0000u) * qmul);
+    for (int ct = 0; ct < CT; ++ct) c1[ct] = p.scale * 1.4426950408889634f, qmul[ct] = 1.0f;
+    HFrag32 qf[CT][QS];
+    auto take_query = [&](const int ct, const int s, const u32x4 raw) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) qf[ct][s].u[i] = pack_f16(u2f(raw[i] << 16) * qmul[ct], u2f(raw[i] & 0xFFFF0000u) * qmul[ct]);
     };
     // FP16: through the ring's upper half
     unsigned char *qbuf = lds + (kRing / 2) * kRingBlock + wave * 8192;
@@ -227,130 +261,184 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory");
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        qmul = u2f(f2u(c1) & 0x7F800000u);
-        if (plain || qmul > 1.0f) {
-            qmul = 1.0f;
-        } else if (qmul < 0.0625f) {
-            // A scale that small would push ordinary queries among fp16's subnormal values: the power of two that takes the column's own largest value to 2^13 or more
-            // instead (a real branch)
-            asm volatile("" ::: "memory");
-            uint32_t top = 0; // its exponent
+        auto query = [&](const int ct, const int s) { return *(const u32x4 *)(qbuf + (TW * ct + tl) * 256 + (((16 / QS * s + part) ^ (tl & 15)) << 4)); };
+        const float two = u2f(f2u(c1[0]) & 0x7F800000u);
+        if (!plain && two <= 1.0f) {
 #pragma unroll
-            for (int s = 0; s < 8; ++s) {
-                const u32x4 raw = *(const u32x4 *)(qbuf + cl * 256 + (((2 * s + h) ^ (cl & 15)) << 4));
+            for (int ct = 0; ct < CT; ++ct) qmul[ct] = two;
+            if (two < 0.0625f) {
+                // A scale that small would push ordinary queries among fp16's subnormal values: the power of two that takes the column's own largest value to 2^13 or more
+                // instead (a real branch)
+                asm volatile("" ::: "memory");
 #pragma unroll
-                for (int i = 0; i < 4; ++i) top = max(top, max(raw[i] << 1 >> 24, raw[i] << 17 >> 24));
+                for (int ct = 0; ct < CT; ++ct) {
+                    uint32_t top = 0; // its exponent
+#pragma unroll
+                    for (int s = 0; s < QS; ++s) {
+                        const u32x4 raw = query(ct, s);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) top = max(top, max(raw[i] << 1 >> 24, raw[i] << 17 >> 24));
+                    }
+                    if constexpr (FINE) top = max(top, (uint32_t)__shfl_xor((int)top, 16, 64));
+                    top = max(top, (uint32_t)__shfl_xor((int)top, 32, 64));
+                    qmul[ct] = u2f((267u - min(max(top, 14u), 254u)) << 23);
+                }
             }
-            top = max(top, (uint32_t)__shfl_xor((int)top, 32, 64));
-            qmul = u2f((267u - min(max(top, 14u), 254u)) << 23);
         }
-        c1 /= qmul;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) take_query(s, *(const u32x4 *)(qbuf + cl * 256 + (((2 * s + h) ^ (cl & 15)) << 4)));
+        for (int ct = 0; ct < CT; ++ct) {
+            c1[ct] /= qmul[ct];
+#pragma unroll
+            for (int s = 0; s < QS; ++s) take_query(ct, s, query(ct, s));
+        }
     } else {
 #pragma unroll
-        for (int s = 0; s < 8; ++s) take_query(s, *(const u32x4 *)((const uint16_t *)(uintptr_t)qrow + 16 * s + 8 * h)); // (past the last column: the first one's)
+        for (int ct = 0; ct < CT; ++ct) {
+            const uint64_t row = FINE ? of_column(qrow, TW * ct + tl) : qrow; // (past the last column: the first one's)
+#pragma unroll
+            for (int s = 0; s < QS; ++s) take_query(ct, s, *(const u32x4 *)((const uint16_t *)(uintptr_t)row + 128 / QS * s + 8 * part));
+        }
     }
 
     const h2 ones2 = {(_Float16)1.0f, (_Float16)1.0f};
-    float m_run = 0.0f, l_run[2] = {0.0f, 0.0f}; // reference point, row sums of this lane's rows
+    float m_run[CT], l_run[2] = {0.0f, 0.0f}; // a column's reference point; sums of this lane's rows, of the two columns or, in turn, of the one
     float vref = 0.0f; // INT8: the value scales are taken relative to this (0 = not set yet)
-    unsigned long long unset = ~0ull; // lanes whose column has seen nothing above minus infinity yet
-    f32x16 o[4], x; // x: the scores
-    HFrag32 kf[8], vf[2][4], pf[2];
+    unsigned long long unset[CT]; // lanes whose column has seen nothing above minus infinity yet
+    Acc o[CT][DT], x[CT][XT]; // x: the scores
+    HFrag32 kf[8], vf[8], pf[2];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int ct = 0; ct < CT; ++ct) {
+        m_run[ct] = 0.0f, unset[ct] = ~0ull;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
-    // operand addresses: one of two (which half of a 64-byte row), the rest constants
-    const uint32_t at0 = cl * 64 + ((h ^ ((cl >> 2) & 3)) << 4), at1 = cl * 64 + (((2 + h) ^ ((cl >> 2) & 3)) << 4);
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < AL; ++r) o[ct][dt][r] = 0.0f;
+    }
+    // operand addresses: one of two (which half of a 64-byte row; FINE: the same), the rest constants
+    const uint32_t at0 = tl * 64 + ((part ^ row_turn<FINE>(tl)) << 4), at1 = FINE ? at0 : tl * 64 + (((2 + part) ^ row_turn<FINE>(tl)) << 4);
+    // operand i of a block's keys (k-step i; FINE: k-step i / 2, token tile i % 2), of its values (k-step i / 4, dim tile i % 4; FINE: dim tile i)
+    auto key_at = [&](const int i) { return FINE ? at0 + (i >> 1) * 2048 + (i & 1) * 1024 : (i & 1 ? at1 : at0) + (i >> 1) * 2048; };
+    auto value_at = [&](const int i) { return FINE ? at0 + i * 1024 : (i >> 2 ? at1 : at0) + (i & 3) * 2048; };
+    auto across = [](float v) { // the largest of the lanes that share a column
+        if constexpr (FINE) v = fmaxf(v, swap16(v));
+        return fmaxf(v, swap32(v));
+    };
+    auto scale_all = [&](const int ct, const float by) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < AL; ++r) o[ct][dt][r] *= by;
+    };
 
     auto softmax = [&](const int blk) {
         const int t0 = blk << 5;
-        const float *sl = (const float *)(lds + 3 * kRingBlock + slot(blk) * kScaleBytes); // INT8: key scales, value scales; this lane's 16 tokens are 8 q + 4 h ..
+        const float *sl = (const float *)(lds + 3 * kRingBlock + slot(blk) * kScaleBytes); // INT8: key scales, value scales
+        auto score = [&](const int ct, const int r) -> float { return x[ct][r / AL][r % AL]; };
+        auto set_score = [&](const int ct, const int r, const float v) { x[ct][r / AL][r % AL] = v; };
         if constexpr (INT8) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const f32x4 ks = *(const f32x4 *)(sl + 8 * q + 4 * h) * c1; // key scale and softmax scale in one factor
+            for (int q = 0; q < V / 4; ++q) {
+                const f32x4 ks = *(const f32x4 *)(sl + token(4 * q)) * c1[0]; // key scale and softmax scale in one factor (of every column)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) x[4 * q + r] = fmaf(x[4 * q + r], ks[r], -m_run);
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) set_score(ct, 4 * q + r, fmaf(score(ct, 4 * q + r), ks[r], -m_run[ct]));
             }
         } else {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) x[r] = fmaf(x[r], c1, -m_run);
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int r = 0; r < V; ++r) set_score(ct, r, fmaf(score(ct, r), c1[ct], -m_run[ct]));
         }
         if (t0 + 32 > lim_min) {
             // only the blocks on the causal diagonal pay for the mask (a real branch)
             asm volatile("" ::: "memory");
 #pragma unroll
-            for (int r = 0; r < 16; ++r) x[r] = (t0 + 8 * (r >> 2) + 4 * h + (r & 3)) < limit ? x[r] : kNegBig;
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int r = 0; r < V; ++r) set_score(ct, r, t0 + token(r) < limit[ct] ? score(ct, r) : kNegBig);
         }
         // x = log2-domain score minus the column's reference point (0 while the column has seen nothing)
-        float bmax = fmaxf(fmaxf(x[0], x[1]), x[2]);
+        float bmax[CT];
 #pragma unroll
-        for (int r = 3; r < 15; r += 2) bmax = fmaxf(fmaxf(bmax, x[r]), x[r + 1]);
-        bmax = fmaxf(bmax, x[15]);
+        for (int ct = 0; ct < CT; ++ct) {
+            bmax[ct] = fmaxf(fmaxf(score(ct, 0), score(ct, 1)), score(ct, 2));
+#pragma unroll
+            for (int r = 3; r < V - 1; r += 2) bmax[ct] = fmaxf(fmaxf(bmax[ct], score(ct, r)), score(ct, r + 1));
+            bmax[ct] = fmaxf(bmax[ct], score(ct, V - 1));
+        }
         // the reference point moves when the block's maximum exceeds it by more than 2^8, and is set by the
         // first block a column sees anything of
-        if ((__builtin_amdgcn_ballot_w64(bmax > 8.0f) | unset) != 0) {
+        if ((__builtin_amdgcn_ballot_w64(fmaxf(bmax[0], bmax[CT - 1]) > 8.0f) | unset[0] | unset[CT - 1]) != 0) {
             // a real branch: in most blocks no column of the wave moves
             asm volatile("" ::: "memory");
-            bmax = fmaxf(bmax, swap32(bmax));
-            const bool fresh = (unset >> lane) & 1, set = fresh && bmax > 0.5f * kNegBig, move = set || bmax > 8.0f;
-            const float delta = move ? bmax : 0.0f, alpha = set ? 1.0f : __builtin_amdgcn_exp2f(-delta); // (a column that sees its first tokens holds zeros)
-            unset = __builtin_amdgcn_ballot_w64(fresh && !set && cvalid);
-            m_run += delta;
-            l_run[0] *= alpha, l_run[1] *= alpha;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) x[r] -= delta;
+            for (int ct = 0; ct < CT; ++ct) {
+                const float top = across(bmax[ct]);
+                const bool fresh = (unset[ct] >> lane) & 1, set = fresh && top > 0.5f * kNegBig, move = set || top > 8.0f;
+                const float delta = move ? top : 0.0f, alpha = set ? 1.0f : __builtin_amdgcn_exp2f(-delta); // (a column that sees its first tokens holds zeros)
+                unset[ct] = __builtin_amdgcn_ballot_w64(fresh && !set && limit[ct] > 0);
+                m_run[ct] += delta;
+                l_run[ct] *= alpha;
+                if constexpr (!FINE) l_run[1] *= alpha;
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+                for (int r = 0; r < V; ++r) set_score(ct, r, score(ct, r) - delta);
+                scale_all(ct, alpha);
+            }
         }
-        float pr[16];
+        float pr[CT][V];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) pr[r] = __builtin_amdgcn_exp2f(x[r]); // (a masked score is kNegBig: 0)
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int r = 0; r < V; ++r) pr[ct][r] = __builtin_amdgcn_exp2f(score(ct, r)); // (a masked score is kNegBig: 0)
         if constexpr (INT8) {
             // (the sums are those of the probabilities as they are: with the scales and rounded, they are other numbers)
 #pragma unroll
-            for (int r = 0; r < 16; r += 4) l_run[r >> 2 & 1] += (pr[r] + pr[r + 1]) + (pr[r + 2] + pr[r + 3]);
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int r = 0; r < V; r += 4) l_run[FINE ? ct : r >> 2 & 1] += (pr[ct][r] + pr[ct][r + 1]) + (pr[ct][r + 2] + pr[ct][r + 3]);
             __builtin_amdgcn_sched_barrier(0); // (the scales' registers only now)
-            f32x4 vs[4];
+            f32x4 vs[V / 4];
             float vmax = 0.0f;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) vs[q] = *(const f32x4 *)(sl + 32 + 8 * q + 4 * h);
+            for (int q = 0; q < V / 4; ++q) vs[q] = *(const f32x4 *)(sl + 32 + token(4 * q));
             if (t0 + 32 > wave_lim) {
                 // tokens no column of the wave sees stay out: behind the sequence's end the cache may hold anything (a real branch)
                 asm volatile("" ::: "memory");
 #pragma unroll
-                for (int r = 0; r < 16; ++r) vs[r >> 2][r & 3] = t0 + 8 * (r >> 2) + 4 * h + (r & 3) < wave_lim ? vs[r >> 2][r & 3] : 0.0f;
+                for (int r = 0; r < V; ++r) vs[r >> 2][r & 3] = t0 + token(r) < wave_lim ? vs[r >> 2][r & 3] : 0.0f;
             }
 #pragma unroll
-            for (int r = 0; r < 16; r += 2) vmax = fmaxf(fmaxf(vmax, vs[r >> 2][r & 3]), vs[r >> 2][(r & 3) + 1]);
-            vmax = fmaxf(vmax, swap32(vmax)); // the block's largest value scale, the same in every lane
+            for (int r = 0; r < V; r += 2) vmax = fmaxf(fmaxf(vmax, vs[r >> 2][r & 3]), vs[r >> 2][(r & 3) + 1]);
+            vmax = across(vmax); // the block's largest value scale, the same in every lane
             // value scales relative to vref; vref follows the blocks' largest scale lazily, like the maximum
             if (vmax > 4.0f * vref || (vmax > 0.0f && vmax * 1024.0f < vref)) { // wave-uniform
                 asm volatile("" ::: "memory");
                 const float vmove = vref > 0.0f ? vref / vmax : 1.0f;
                 vref = vmax;
 #pragma unroll
-                for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) o[dt][r] *= vmove;
+                for (int ct = 0; ct < CT; ++ct) scale_all(ct, vmove);
             }
             const float vinv = vref > 0.0f ? 1.0f / vref : 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) pr[r] *= vs[r >> 2][r & 3] * vinv;
+            for (int r = 0; r < V; ++r) {
+                const float by = vs[r >> 2][r & 3] * vinv;
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) pr[ct][r] *= by;
+            }
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            pf[t].u[0] = pack_f16(pr[4 * t], pr[4 * t + 1]);
-            pf[t].u[1] = pack_f16(pr[4 * t + 2], pr[4 * t + 3]);
-            pf[t].u[2] = pack_f16(pr[4 * t + 8], pr[4 * t + 9]);
-            pf[t].u[3] = pack_f16(pr[4 * t + 10], pr[4 * t + 11]);
+        for (int t = 0; t < 2; ++t) // k-step or column t of the values' products
 #pragma unroll
-            for (int i = 0; i < 4 && !INT8; ++i) l_run[i & 1] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, pf[t].u[i]), ones2, l_run[i & 1], false);
+            for (int i = 0; i < 4; ++i) {
+                const int ct = FINE ? t : 0, r = FINE ? 2 * i : 4 * t + 2 * (i & 1) + 8 * (i >> 1);
+                pf[t].u[i] = pack_f16(pr[ct][r], pr[ct][r + 1]);
+            }
+        if constexpr (!INT8) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) l_run[FINE ? t : i & 1] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, pf[t].u[i]), ones2, l_run[FINE ? t : i & 1], false);
         }
     };
     // scores of block `next` (keys already read), values of the block in front of it; reads the keys of block next + 1, the values of block next
@@ -358,20 +446,25 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
         constexpr bool VALUES = decltype(with_values)::value;
         const unsigned char *kb = lds + slot(next + 1) * kRingBlock, *vb = lds + slot(next) * kRingBlock + 8192;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) x[r] = 0.0f;
-        // (one read behind each MFMA: held up by a burst of them, the wave would issue no MFMA)
+        for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            x = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s].v, qf[s].v, x, 0, 0, 0);
-            kf[s].q = *(const u32x4 *)(kb + (s & 1 ? at1 : at0) + (s >> 1) * 2048);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            for (int r = 0; r < V; ++r) x[ct][r / AL][r % AL] = 0.0f;
+        // (one read behind the MFMAs that it serves: held up by a burst of them, the wave would issue no MFMA)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) x[ct][FINE ? i & 1 : 0] = prefill_mfma(kf[i].v, qf[ct][FINE ? i >> 1 : i].v, x[ct][FINE ? i & 1 : 0]);
+            kf[i].q = *(const u32x4 *)(kb + key_at(i));
+            __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            if constexpr (VALUES) o[s & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[s >> 2][s & 3].v, pf[s >> 2].v, o[s & 3], 0, 0, 0);
-            vf[s >> 2][s & 3].q = *(const u32x4 *)(vb + (s >> 2 ? at1 : at0) + (s & 3) * 2048);
-            if constexpr (VALUES) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        for (int i = 0; i < 8; ++i) {
+            if constexpr (VALUES)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) o[ct][FINE ? i : i & 3] = prefill_mfma(vf[i].v, pf[FINE ? ct : i >> 2].v, o[ct][FINE ? i : i & 3]);
+            vf[i].q = *(const u32x4 *)(vb + value_at(i));
+            if constexpr (VALUES) __builtin_amdgcn_sched_group_barrier(0x008, CT, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
     };
@@ -388,12 +481,15 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if constexpr (!INT8) request(2);
 #pragma unroll
-    for (int s = 0; s < 8; ++s) kf[s].q = *(const u32x4 *)(lds + (s & 1 ? at1 : at0) + (s >> 1) * 2048);
+    for (int i = 0; i < 8; ++i) kf[i].q = *(const u32x4 *)(lds + key_at(i));
     __builtin_amdgcn_sched_barrier(0);
     products(std::false_type {}, 0);
     // Where the loop begins in the 32 bytes that are fetched at a time is worth 6 % (512 tokens behind 8000, by the number of 4-byte steps behind a border: 156,
-    // 150, 150, 146, 148, 152, 154, 152 us; 4 x 2000 tokens 144 to 146.5, 2 x 1000 with 16 / 4 heads 23.9 to 24.9), so it is said.
-    if constexpr (!INT8) asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
+    // 150, 150, 146, 148, 152, 154, 152 us; 4 x 2000 tokens 144 to 146.5, 2 x 1000 with 16 / 4 heads 23.9 to 24.9; FINE 154, 161, 172, 163, 160, 172, 154, 155, INT8 at 0, 2, 4, 6
+    // steps 293, 306, 305, 294), so it is said.
+    if constexpr (INT8 && FINE) asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
+    else if constexpr (!INT8 && FINE) asm volatile(".p2align 5");
+    else if constexpr (!INT8) asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
     for (int blk = 0; blk < nblk; ++blk) {
         // the block asked for goes where block blk - 1 was, which every wave has read for the last time in front of the barrier behind block blk - 1's softmax
         // (INT8: as much holds for block blk + 2, which is a register set ahead instead)
@@ -417,9 +513,13 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); // the requests past the end have landed
 
-    float l = l_run[0] + l_run[1];
-    l += swap32(l);
-    const float inv = (INT8 ? vref : 1.0f) / l;
+    float inv[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        float l = FINE ? l_run[ct] + swap16(l_run[ct]) : l_run[0] + l_run[1];
+        l += swap32(l);
+        inv[ct] = (INT8 ? vref : 1.0f) / l;
+    }
     const size_t base = ((size_t)b * p.S + cs) * p.oStride + (size_t)(kvh * p.G + cj) * D;
     if (p.out_dtype == XFTHIP_BF16 && (((uintptr_t)p.out | ((size_t)p.oStride * 2)) & 15) == 0) {
         // whole rows through LDS, four of 256 bytes a store (from the registers: 16 stores of 32 rows' 16 bytes)
@@ -427,11 +527,13 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
         constexpr int PITCH = 272;
         unsigned char *patch = lds + wave * (32 * PITCH);
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+        for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *(uint2 *)(patch + cl * PITCH + 64 * dt + 16 * q + 8 * h) = make_uint2(f32x2_to_bf16(o[dt][4 * q] * inv, o[dt][4 * q + 1] * inv),
-                        f32x2_to_bf16(o[dt][4 * q + 2] * inv, o[dt][4 * q + 3] * inv));
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int q = 0; q < AL / 4; ++q)
+                    *(uint2 *)(patch + (TW * ct + tl) * PITCH + 256 / DT * dt + 16 * q + 8 * part) =
+                            make_uint2(f32x2_to_bf16(o[ct][dt][4 * q] * inv[ct], o[ct][dt][4 * q + 1] * inv[ct]), f32x2_to_bf16(o[ct][dt][4 * q + 2] * inv[ct], o[ct][dt][4 * q + 3] * inv[ct]));
         const uint64_t orow = (uint64_t)(uintptr_t)((uint16_t *)p.out + base);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -442,7 +544,11 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
         }
         return;
     }
-    if (cvalid) store_direct(p, base, h, o, inv);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const size_t at_column = FINE ? of_column(base, TW * ct + tl) : base;
+        if (limit[ct] > 0) store_direct<Acc, DT>(p, at_column, part, o[ct], inv[ct]);
+    }
 }
 
 } // namespace xfthip

@@ -384,6 +384,7 @@ __device__ inline AttnParams seq_params(const AttnParams &all, const SeqBatch &s
 // attn_prefill32_kernel over sequences, the longest first.  Group k of 8 pairs has n(k) column groups, those of its longest sequence.  An XCD walks a band in levels,
 // from the longest walk down: levels n(k) - 1 .. n(k + 1), which groups k and those in front of it in its band reach, are part k.
 // (6 sequences of 750 .. 1500 tokens, 32 query / 8 KV heads: group after group 113 us the call, so 106; 7 of 600 .. 1200, 16 / 4 heads 58 and 52)
+template <bool FINE>
 __global__ __launch_bounds__(256, 2) void paged_prefill_attn_kernel(AttnParams all, SeqBatch s) {
     __shared__ __attribute__((aligned(16))) unsigned char lds[kRingLds];
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn_kernel(AttnParams a
     const AttnParams p = seq_params(all, s, s.first + i);
     const int ncg = (p.S * p.G + 127) / 128;
     if (level >= ncg) return; // (a longer sequence shares the group)
-    attn_prefill_ring_unit<false>(p, pair % all.kv.H, level, 0, lds, i >= s.scaled);
+    attn_prefill_ring_unit<false, FINE>(p, pair % all.kv.H, level, 0, lds, i >= s.scaled);
 }
 
 // attn_kernel over sequences, each walked by one workgroup a column group: grid (KV heads x the longest's column groups, sequences)
@@ -575,7 +576,9 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
             prefill_band(s.bands, g, band, width);
             s.grp0[g + 1] = s.grp0[g] + (levels(g) - (g + 1 < band + width ? levels(g + 1) : 0)) * (g - band + 1);
         }
-        if (s.many > 0) hipLaunchKernelGGL(paged_prefill_attn_kernel, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
+        const bool fine = prefill_fine(false, 8L * s.grp0[groups], s.rows[0] / 2);
+        if (s.many > 0 && fine) hipLaunchKernelGGL(paged_prefill_attn_kernel<true>, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
+        else if (s.many > 0) hipLaunchKernelGGL(paged_prefill_attn_kernel<false>, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
         s.first = s.many, s.many = s.n - s.many;
         if (s.many > 0)
             hipLaunchKernelGGL(paged_prefill_few_kernel, dim3(kv_heads * ((s.rows[s.first] * G + 15) / 16), s.many), dim3(256), 0, st, p, s);
