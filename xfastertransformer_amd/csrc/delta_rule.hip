@@ -1,6 +1,9 @@
 // The gated delta-rule recurrence of layer plans: short convolutions, unit norms, decays and step sizes (delta_prepare), the
 // walk over the tokens with the state in registers (delta_scan), the gated per-head norm behind it (delta_output).
 // Everything between the projections' outputs and the output projection's input is fp32.
+#include <algorithm>
+#include <type_traits>
+
 #include "plan_dev.h"
 
 namespace xfthip {
@@ -218,13 +221,14 @@ struct TailParams {
     const void *in;
     int ld, channels, taps;
     void *conv_state;
+    int least;
 };
-// the last taps - 1 inputs of a segment of several tokens; one thread a channel
+// the last taps - 1 inputs of a segment of `least` tokens or more; one thread a channel
 template <bool BF16>
 __global__ __launch_bounds__(256) void conv_tail_kernel(TailParams p) {
     constexpr int DT = BF16 ? XFTHIP_BF16 : XFTHIP_F32;
     const int seg = blockIdx.y, n = p.v.seg_len[seg], ch = blockIdx.x * 256 + threadIdx.x;
-    if (n <= 1 || ch >= p.channels) return;
+    if (n < p.least || ch >= p.channels) return;
     const size_t hist = (size_t)p.v.seg_row[seg] * (p.taps - 1) * p.channels;
     const int off = p.v.seg_off[seg];
     for (int s = 0; s < p.taps - 1; ++s) { // ascending: slot s is read (as a later source) only by slots below it
@@ -414,6 +418,392 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(ScanParams p) {
 #pragma unroll
             for (int r = 0; r < RV; ++r) *(f32x4 *)(state + c * KD + r * 4 * L) = s[c][r];
     }
+}
+
+// ---- segments of many tokens, kChunk at a time ----------------------------------------------------
+// Within a chunk, with G_t the product of the decays up to token t and G_t / G_s that of those behind s (always multiplied out, never divided):
+//   a_t = (G_t k_t)^T S_0 + sum_{s < t} A_ts u_s,   A_ts = k_t^T (G_t / G_s) k_s,   u_t = beta_t (v_t - a_t)
+//   o_t = (G_t q_t)^T S_0 + sum_{s <= t} B_ts u_s,  B_ts = q_t^T (G_t / G_s) k_s
+//   S   = G_16 S_0 + sum_s (G_16 / G_s) k_s u_s^T
+// so u = U (v - W S_0) with W = G k and U = (1 + beta A)^-1 beta, a triangular matrix whose entries are bounded by one (products of contractions): what a chunk does to
+// the state's columns are products of matrices that no column has a part in.
+// Record of a (chunk, head) for the scan: W [16][KD] | G q [16][KD] | (G_16 / G_s) k_s as [KD][16] | G_16 [KD] | U [16][16] | B [16][16]
+constexpr int kChunk = 16;
+__host__ __device__ constexpr size_t chunk_floats(int KD) { return (size_t)(3 * kChunk + 1) * KD + 2 * kChunk * kChunk; }
+// records in front of a segment's: ceil(n / 16) of every segment fit in floor((off + n) / 16) - floor(off / 16) + 1
+__device__ inline size_t chunk_of(int off, int seg) { return (size_t)(off / kChunk + seg); }
+
+// In place of delta_prepare for such segments: convolutions, norms and decays of a (chunk, head) by a workgroup of its own, two neighbouring channels of q, k, v or the decays a
+// thread, and what the scan needs of them.  Tokens past the segment's end have no keys, queries and step sizes.  A and B: thread (s, 1/16 of the key dims) carries k_s on from token to token,
+// 16 lanes add up.  Bound by the round trips of a workgroup, of which six share a CU (4 prompts of 1000 to 1500 tokens, 16 heads of 128 x 128: 110 us for 270 MB; delta_prepare, which
+// leaves the products to the scan, 85).
+template <int KD, bool ONE, bool BF16>
+__global__ __launch_bounds__(256) void delta_chunk_kernel(PrepParams p) {
+    constexpr int J = KD / 64, N = kChunk * KD / 4 / 256, P = KD + 4, SIZE = kChunk * P; // (rows of P: lanes that read a column of rows are on banks of their own)
+    __shared__ __align__(16) float q[SIZE], k[SIZE], g[SIZE], A[kChunk * kChunk], B[kChunk * kChunk], beta[kChunk], one[kChunk];
+    const int tid = threadIdx.x, head = blockIdx.y, seg = blockIdx.z, H = p.H, kvh = head / (H / p.KH), c0 = blockIdx.x * kChunk;
+    const int n = p.v.seg_len[seg], off = p.v.seg_off[seg], start = p.v.seg_pos[seg], taps = p.taps;
+    if (c0 >= n) return;
+    const size_t hist = (size_t)p.v.seg_row[seg] * (taps - 1) * p.channels;
+    const int cnt = n - c0 < kChunk ? n - c0 : kChunk;
+    const float decay = p.decay[head];
+    constexpr int W = KD / 2;
+    for (int w = tid; w < (ONE ? 2 : 3) * W + p.VD / 2; w += 256) {
+        if (!ONE && w >= 2 * W + p.VD / 2) {
+            const int d = 2 * (w - 2 * W - p.VD / 2);
+            const float2 dt = *(const float2 *)(p.dt_bias + head * KD + d);
+            float2 x[kChunk];
+#pragma unroll
+            for (int i = 0; i < kChunk; ++i) x[i] = *(const float2 *)(p.b.gates + (size_t)(off + c0 + (i < cnt ? i : 0)) * 2 * p.gcols + head * KD + d);
+#pragma unroll
+            for (int i = 0; i < kChunk; ++i)
+                *(float2 *)(g + i * P + d) = i < cnt ? make_float2(exp_of<BF16>(-decay * softplus_of<BF16>(x[i].x + dt.x)), exp_of<BF16>(-decay * softplus_of<BF16>(x[i].y + dt.y)))
+                                                     : make_float2(1.0f, 1.0f);
+            continue;
+        }
+        const int c = w < W ? kvh * KD + 2 * w : w < 2 * W ? (p.KH + kvh) * KD + 2 * (w - W) : 2 * p.KH * KD + head * p.VD + 2 * (w - 2 * W);
+        float2 f[4], x[kChunk + 3]; // the last of four taps; inputs from three in front of the chunk on: of earlier steps what they left, before the sequence's start zero
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            f[j] = j >= 4 - taps ? make_float2(p.conv[(size_t)c * taps + j - (4 - taps)], p.conv[(size_t)(c + 1) * taps + j - (4 - taps)]) : make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int j = 0; j < kChunk + 3; ++j) {
+            const int i = c0 + j - 3;
+            x[j] = make_float2(0.0f, 0.0f);
+            if (j >= 3) x[j] = load2<BF16>(p.b.in, (size_t)(off + (j - 3 < cnt ? i : c0)) * p.ld + c);
+            else if (j >= 4 - taps && start + i >= 0)
+                x[j] = i >= 0 ? load2<BF16>(p.b.in, (size_t)(off + i) * p.ld + c) : load2<BF16>(p.b.conv_state, hist + (size_t)(taps - 1 + i) * p.channels + c);
+        }
+#pragma unroll
+        for (int i = 0; i < kChunk; ++i) {
+            float2 a = make_float2(0.0f, 0.0f);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (j >= 4 - taps) a.x = fmaf(f[j].x, x[i + j].x, a.x), a.y = fmaf(f[j].y, x[i + j].y, a.y);
+            a = i < cnt ? make_float2(silu_of<BF16>(a.x), silu_of<BF16>(a.y)) : make_float2(0.0f, 0.0f);
+            if (w < 2 * W) *(float2 *)((w < W ? q + 2 * w : k + 2 * (w - W)) + i * P) = a;
+            else if (i < cnt) *(float2 *)(p.b.v + ((size_t)(off + c0 + i) * H + head) * p.VD + 2 * (w - 2 * W)) = a;
+        }
+    }
+    if (tid < kChunk) {
+        const size_t t = (size_t)(off + c0 + (tid < cnt ? tid : 0)) * p.ld;
+        beta[tid] = tid < cnt ? sigmoid_of<BF16>(ldb<BF16>(p.b.in, t + p.beta_col + head)) : 0.0f;
+        if constexpr (ONE) one[tid] = tid < cnt ? exp_of<BF16>(-decay * softplus_of<BF16>(ldb<BF16>(p.b.in, t + p.decay_col + head) + p.dt_bias[head])) : 1.0f;
+    }
+    __syncthreads();
+    {
+        f32x4 x[J], y[J];
+        float *qt = q + (tid >> 4) * P + 4 * (tid & 15), *kt = k + (tid >> 4) * P + 4 * (tid & 15), sq = 0.0f, sk = 0.0f;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            x[j] = *(const f32x4 *)(qt + 64 * j), y[j] = *(const f32x4 *)(kt + 64 * j);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sq = fmaf(x[j][e], x[j][e], sq), sk = fmaf(y[j][e], y[j][e], sk);
+        }
+        sq = 1.0f / sqrtf(group_sum<16>(sq) + 1e-6f) * p.qscale, sk = 1.0f / sqrtf(group_sum<16>(sk) + 1e-6f);
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[j][e] *= sq, y[j][e] *= sk;
+            *(f32x4 *)(qt + 64 * j) = x[j], *(f32x4 *)(kt + 64 * j) = y[j];
+        }
+    }
+    A[tid] = B[tid] = 0.0f;
+    __syncthreads();
+    float *rec = p.b.chunks + ((chunk_of(off, seg) + blockIdx.x) * H + head) * chunk_floats(KD);
+    {
+        const int s = tid >> 4, part = 4 * (tid & 15);
+        f32x4 r[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) r[j] = f32x4 {0.f, 0.f, 0.f, 0.f};
+        for (int t0 = s & ~3; t0 < kChunk; t0 += 4) { // (from the wave's first key on)
+            float x[4], y[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = t0 + i;
+                x[i] = y[i] = 0.0f;
+#pragma unroll
+                for (int j = 0; j < J; ++j) {
+                    const int at = t * P + part + 64 * j;
+                    const f32x4 kt = *(const f32x4 *)(k + at), qt = *(const f32x4 *)(q + at);
+                    f32x4 gt;
+                    if constexpr (ONE) gt = f32x4 {one[t], one[t], one[t], one[t]};
+                    else gt = *(const f32x4 *)(g + at);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        r[j][e] = t == s ? kt[e] : t > s ? r[j][e] * gt[e] : 0.0f;
+                        x[i] = fmaf(kt[e], r[j][e], x[i]), y[i] = fmaf(qt[e], r[j][e], y[i]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = group_sum<16>(x[i]), y[i] = group_sum<16>(y[i]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (part == 0 && t0 + i > s) A[(t0 + i) * kChunk + s] = x[i];
+                if (part == 0 && t0 + i >= s) B[(t0 + i) * kChunk + s] = y[i];
+            }
+        }
+    }
+    // a thread's channel of the keys or of the queries, in place: times the decays' products from the front, and from the back where the decays lie
+    constexpr int M = KD > 128 ? 2 : 1;
+    float x[M][kChunk], y[M][kChunk];
+    auto channel = [&](int m) { return KD > 128 ? tid : tid % KD; };
+    auto keys = [&](int m) { return KD > 128 ? m == 0 : tid < KD; };
+    const bool mine = tid < 2 * KD;
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int t = 0; t < kChunk && mine; ++t) x[m][t] = (keys(m) ? k : q)[t * P + channel(m)], y[m][t] = ONE ? one[t] : g[t * P + channel(m)];
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < M && mine; ++m) {
+        const int d = channel(m);
+        float G = 1.0f;
+        if (keys(m)) {
+#pragma unroll
+            for (int t = kChunk - 1; t >= 0; --t) g[t * P + d] = G * x[m][t], G *= y[m][t];
+            rec[3 * kChunk * KD + d] = G, G = 1.0f;
+#pragma unroll
+            for (int t = 0; t < kChunk; ++t) G *= y[m][t], k[t * P + d] = G * x[m][t];
+        } else {
+#pragma unroll
+            for (int t = 0; t < kChunk; ++t) G *= y[m][t], q[t * P + d] = G * x[m][t];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int e = i * 256 + tid, at = (e & 15) * P + (e >> 6 << 4 | (e >> 2 & 12)); // token, four key rows
+        *(f32x4 *)(rec + 4 * e) = *(const f32x4 *)(k + at), *(f32x4 *)(rec + kChunk * KD + 4 * e) = *(const f32x4 *)(q + at);
+        const float *from = g + 4 * (e & 3) * P + (e >> 2); // four tokens, key row
+        *(f32x4 *)(rec + 2 * kChunk * KD + 4 * e) = f32x4 {from[0], from[P], from[2 * P], from[3 * P]};
+    }
+    rec += (3 * kChunk + 1) * KD;
+    rec[kChunk * kChunk + tid] = B[tid];
+    if (tid >= 256 - kChunk) { // column s of -U, row by row: what token t leaves is taken from all behind it at once
+        const int s = tid - (256 - kChunk);
+        float u[kChunk];
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t) u[t] = t == s ? -1.0f : 0.0f;
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t) {
+            u[t] = t < s ? 0.0f : beta[t] * u[t];
+#pragma unroll
+            for (int r = t + 1; r < kChunk; ++r) u[r] = fmaf(-A[r * kChunk + t], u[t], u[r]);
+        }
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t) rec[t * kChunk + s] = u[t];
+    }
+}
+
+// A wave holds 16 columns of a head's state as accumulators of 16 x 16 x 4 fp32 MFMAs, key row 16 i + 4 g + r in register r of tile i (g = lane / 16): with key rows dealt to the MFMAs'
+// k slots alike they are the operand of W S_0 and (G q) S_0 as they lie, as are the results, rows of tokens, of the products with U, B and the keys: nothing moves between lanes.
+// NW waves share the key rows and add up their parts of W S_0 and (G q) S_0 through LDS; one more makes the outputs, off the chain from state to state.  Wave 0 takes v from its part, the
+// records hold -U.  C tiles of 16 columns a wave.  Every operand is requested two chunks ahead, behind its last use.
+// Bound by the chain: products, barrier, sums, the product with U and the check of it, the state's products, about 2000 clocks a chunk of which the MFMAs fill 930, and by the MFMAs where a SIMD
+// has several waves of it; the scan above takes 600 clocks a token.  prepare and scan, before and after, us: 16 heads of 128 x 128, one prompt of 1500
+// tokens 296 / 124, two of 3000 646 / 300, 4 of 1000 to 1500 429 / 264, 8 of 800 416 / 308, 16 of 400 399 / 314, one of 32 31 / 22; 16 of 64 x 64, 8 of 800 224 / 142; 8 of 256 x 256, 2 of
+// 3000 1038 / 431, 16 of 400 816 / 441; with one decay a head, 32 of 128 x 128, 2 of 3000 784 / 468, 16 of 400 603 / 526.
+// A wave for all key rows: 213 us for the prompt of 1500, two 103, four 82 (85 with two sums of every product, for as small an error as the walk token by token has).  With the stores of a last, ragged chunk in the loop every wait was one for the stores before, too: 100.
+template <int KD, int NW, int C>
+__global__ __launch_bounds__(64 * NW + 64, KD / NW == 32 && C == 1 ? 4 : 2) void delta_chunk_scan_kernel(ScanParams p) {
+    constexpr int I = KD / 16 / NW, SETS = 2;
+    __shared__ f32x4 parts[2][NW][2][C][64];
+    // (segments of one place are handed to one XCD in turn, whose share should be long and short ones)
+    const int seg = (blockIdx.x + blockIdx.y + (blockIdx.y >> 1) + (blockIdx.y >> 2)) % gridDim.x, head = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, c = lane & 15, row0 = wave * 16 * I;
+    const int n = p.v.seg_len[seg], off = p.v.seg_off[seg], last = (n - 1) / kChunk;
+    // addresses: scalar ones that move with the chunks, and these of a lane (in bytes), which do not
+    const char *records = (const char *)(p.b.chunks + (chunk_of(off, seg) * p.H + head) * chunk_floats(KD));
+    const size_t next = (size_t)p.H * chunk_floats(KD) * 4, first = ((size_t)off * p.H + head) * p.VD + blockIdx.z * 16 * C;
+    const uint32_t row = (uint32_t)p.H * p.VD * 4, at_u = (c * kChunk + 4 * g) * 4;
+    uint32_t token[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) token[r] = (4 * g + r) * row;
+    auto load = [](const char *base, uint32_t at) { return *(const f32x4 *)(base + at); };
+    auto times = [&](const f32x4 m, const f32x4 y, f32x4 d) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_mfma_f32_16x16x4f32(m[e], y[e], d, 0, 0, 0);
+        return d;
+    };
+    auto finite = [&](const f32x4 (&y)[C]) {
+        float z = 0.0f;
+#pragma unroll
+        for (int t = 0; t < C; ++t) z += (y[t][0] * 0.0f + y[t][1] * 0.0f) + (y[t][2] * 0.0f + y[t][3] * 0.0f);
+        return __builtin_amdgcn_ballot_w64(!(z == 0.0f)) == 0;
+    };
+    // what a token must not see of later ones, though their factors are zero: row t with the values up to it alone
+    auto times_row_by_row = [&](const f32x4 m, const f32x4 y, const f32x4 d) {
+        f32x4 out = d;
+#pragma unroll 1
+        for (int t = 0; t < kChunk; ++t) {
+            f32x4 z;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[e] = 4 * g + e <= t ? y[e] : 0.0f;
+            z = times(m, z, d);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (4 * g + e == t) out[e] = z[e];
+        }
+        return out;
+    };
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    auto record = [&](int chunk) { return records + (chunk < last ? chunk : last) * next; }; // (behind the last: the last again)
+    // every wave's u from the parts of W S_0 - v; sound: nothing infinite in it, nor in what it was made of
+    auto solve = [&](const f32x4 m, int chunk, int buf, f32x4 (&u)[C]) {
+        f32x4 r[C];
+#pragma unroll
+        for (int t = 0; t < C; ++t) {
+            r[t] = parts[buf][0][0][t][lane], u[t] = zero;
+#pragma unroll
+            for (int w = 1; w < NW; ++w) r[t] += parts[buf][w][0][t][lane];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int t = 0; t < C; ++t) u[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[e], r[t][e], u[t], 0, 0, 0);
+        const bool sound = finite(u);
+        if (!sound) {
+#pragma unroll
+            for (int t = 0; t < C; ++t) {
+                u[t] = times_row_by_row(m, r[t], zero);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) u[t][e] = 4 * g + e < n - chunk * kChunk ? u[t][e] : 0.0f;
+            }
+        }
+        return sound;
+    };
+    // (a buffer's readers of two chunks ago have passed the barrier of one chunk ago)
+    auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    int chunk = 0;
+    if (wave == NW) {
+        // the read-outs
+        struct Outs {
+            f32x4 u, b;
+        };
+        Outs set[SETS];
+        auto fetch = [&](Outs &o, int chunk) {
+            const char *rec = record(chunk) + (3 * kChunk + 1) * KD * 4;
+            o.u = load(rec, at_u), o.b = load(rec + kChunk * kChunk * 4, at_u);
+        };
+        // (the last chunk's stores, of which some may be left out, have a place of their own: the count of a wait in the loop would have to do without them and be that of a wait
+        // for the stores before, too)
+        auto step = [&](Outs &o, int chunk, int buf, auto whole) {
+            f32x4 u[C];
+            meet();
+            const bool sound = solve(o.u, chunk, buf, u);
+            char *out = (char *)(p.b.o + first) + (size_t)chunk * kChunk * row;
+#pragma unroll
+            for (int t = 0; t < C; ++t) {
+                f32x4 b = parts[buf][0][1][t][lane];
+#pragma unroll
+                for (int w = 1; w < NW; ++w) b += parts[buf][w][1][t][lane];
+                b = sound ? times(o.b, u[t], b) : times_row_by_row(o.b, u[t], b);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (whole() || 4 * g + e < n - chunk * kChunk) *(float *)(out + 64 * t + (token[e] + 4 * c)) = b[e];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(o, chunk + SETS);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int i = 0; i < SETS; ++i) fetch(set[i], i);
+        for (; chunk + SETS <= last; chunk += SETS)
+#pragma unroll
+            for (int i = 0; i < SETS; ++i) step(set[i], chunk + i, (chunk + i) & 1, std::true_type());
+#pragma unroll
+        for (int i = 0; i < SETS; ++i) {
+            if (chunk + i == last) step(set[i], last, last & 1, std::false_type());
+            else if (chunk + i < last) step(set[i], chunk + i, (chunk + i) & 1, std::true_type());
+        }
+        return;
+    }
+    const uint32_t at_w = row0 * 64 + lane * 16, at_x = ((row0 + c) * kChunk + 4 * g) * 4, at_fade = (row0 + 4 * g) * 4;
+    float *state = p.b.state + (((size_t)p.v.seg_row[seg] * p.H + head) * p.VD + blockIdx.z * 16 * C + c) * KD + row0 + 4 * g;
+    f32x4 s[C][I];
+#pragma unroll
+    for (int t = 0; t < C; ++t)
+#pragma unroll
+        for (int i = 0; i < I; ++i) s[t][i] = p.v.seg_pos[seg] > 0 ? *(const f32x4 *)(state + t * 16 * KD + 16 * i) : zero;
+    struct Operands {
+        f32x4 w[I], q[I], x[I], fade[I], u, v[C];
+    };
+    Operands set[SETS];
+#pragma unroll
+    for (int i = 0; i < SETS; ++i)
+#pragma unroll
+        for (int t = 0; t < C; ++t) set[i].v[t] = zero; // (one wave takes the values from its part)
+    auto fetch_w = [&](Operands &o, int chunk) {
+        const char *rec = record(chunk);
+#pragma unroll
+        for (int i = 0; i < I; ++i) o.w[i] = load(rec + 1024 * i, at_w), o.q[i] = load(rec + kChunk * KD * 4 + 1024 * i, at_w);
+        if (wave != 0) return;
+        const int here = chunk < last ? chunk : last, most = n - 1 - here * kChunk;
+        const char *v = (const char *)(p.b.v + first) + (size_t)here * kChunk * row;
+        const uint32_t end = (most < kChunk - 1 ? most : kChunk - 1) * row; // (tokens behind it: the last one's, which count for nothing)
+#pragma unroll
+        for (int t = 0; t < C; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o.v[t][r] = *(const float *)(v + 64 * t + ((token[r] < end ? token[r] : end) + 4 * c));
+    };
+    auto fetch_x = [&](Operands &o, int chunk) {
+        const char *rec = record(chunk) + 2 * kChunk * KD * 4;
+        o.u = load(rec + (kChunk + 1) * KD * 4, at_u);
+#pragma unroll
+        for (int i = 0; i < I; ++i) o.fade[i] = load(rec + kChunk * KD * 4 + 64 * i, at_fade);
+#pragma unroll
+        for (int i = 0; i < I; ++i) o.x[i] = load(rec + kChunk * 64 * i, at_x);
+    };
+#pragma unroll
+    for (int t = 0; t < C; ++t)
+#pragma unroll
+        for (int i = 0; i < I; ++i) arrived(s[t][i]);
+    auto step = [&](Operands &o, int chunk, int buf) {
+        f32x4 a[C][2], b[C][2], u[C];
+#pragma unroll
+        for (int t = 0; t < C; ++t) a[t][0] = a[t][1] = b[t][0] = b[t][1] = zero;
+#pragma unroll
+        for (int i = 0; i < I; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int t = 0; t < C; ++t)
+                    a[t][i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[i][e], s[t][i][e], a[t][i & 1], 0, 0, 0),
+                    b[t][i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[i][e], s[t][i][e], b[t][i & 1], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < C; ++t) parts[buf][wave][0][t][lane] = (a[t][0] + a[t][1]) - o.v[t], parts[buf][wave][1][t][lane] = b[t][0] + b[t][1];
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_w(o, chunk + SETS);
+        meet();
+        solve(o.u, chunk, buf, u);
+#pragma unroll
+        for (int t = 0; t < C; ++t)
+#pragma unroll
+            for (int i = 0; i < I; ++i) s[t][i] = s[t][i] * o.fade[i];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < I; ++i)
+#pragma unroll
+                for (int t = 0; t < C; ++t) s[t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.x[i][e], u[t][e], s[t][i], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_x(o, chunk + SETS);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int i = 0; i < SETS; ++i) fetch_w(set[i], i), fetch_x(set[i], i);
+    for (; chunk + SETS - 1 <= last; chunk += SETS)
+#pragma unroll
+        for (int i = 0; i < SETS; ++i) step(set[i], chunk + i, (chunk + i) & 1);
+#pragma unroll
+    for (int i = 0; i + 1 < SETS; ++i)
+        if (chunk + i <= last) step(set[i], chunk + i, (chunk + i) & 1);
+#pragma unroll
+    for (int t = 0; t < C; ++t)
+#pragma unroll
+        for (int i = 0; i < I; ++i) *(f32x4 *)(state + t * 16 * KD + 16 * i) = s[t][i];
 }
 
 // The same step for segments of one token: nothing to stage, the kernel is a read and a write of the state.
@@ -612,6 +1002,17 @@ PrepParams prep_params(int act, const PlanLayer &L, const StepView &v, const Del
     return p;
 }
 
+// Tiles of 16 columns of all states of a step: four waves each and more
+long chunk_tiles(const PlanLayer &L, const StepView &v) { return (long)v.B * L.s.heads * (L.VD / 16); }
+
+// Segments kChunk tokens at a time?  From a whole chunk on, where the walk token by token leaves most of the device idle (16 heads of 128 x 128, one prompt of 16 / 32 tokens 26 / 31 us, so 21 / 22); where
+// it does not, from two chunks on (16 prompts of 16 / 24 / 32 tokens 39 / 46 / 51 and 37 / 46 / 46), with one decay a head, which saves that walk a third of its reads, from eight (32 heads, 16
+// prompts of 32 / 64 / 400 tokens 65 / 104 / 603 and 66 / 107 / 526).
+bool chunked(const PlanLayer &L, const StepView &v, const DeltaBuffers &b) {
+    const int from = chunk_tiles(L, v) < 4L * device_cu_count() ? kChunk : L.head_decay() ? 8 * kChunk : 2 * kChunk;
+    return b.chunks && v.longest >= from && L.KD >= 64 && L.KD <= 256 && L.s.taps >= 2 && L.s.taps <= 4;
+}
+
 // row_in: the input product's rows, if the gate is in them
 OutParams out_params(int act, const PlanLayer &L, int T, const float *o, const float *gates, const void *row_in, void *out, float eps) {
     const int esz = act == XFTHIP_BF16 ? 2 : 4;
@@ -635,6 +1036,23 @@ int delta_prepare(int act, const PlanLayer &L, const StepView &v, const DeltaBuf
     const dim3 grid(v.T, (p.H + 3) / 4);
     const int width = p.KD > p.VD ? p.KD : p.VD;
     const bool tiled = p.taps >= 2 && p.taps <= 4 && width <= 256;
+    if (chunked(L, v, b)) {
+        const dim3 chunks((v.longest + kChunk - 1) / kChunk, p.H, v.B);
+        auto launch = [&](auto bf16, auto f32) {
+            if (act == XFTHIP_BF16) hipLaunchKernelGGL(bf16, chunks, dim3(256), 0, st, p);
+            else hipLaunchKernelGGL(f32, chunks, dim3(256), 0, st, p);
+        };
+        switch (L.KD + (L.head_decay() ? 1 : 0)) {
+            case 64: launch(delta_chunk_kernel<64, false, true>, delta_chunk_kernel<64, false, false>); break;
+            case 65: launch(delta_chunk_kernel<64, true, true>, delta_chunk_kernel<64, true, false>); break;
+            case 128: launch(delta_chunk_kernel<128, false, true>, delta_chunk_kernel<128, false, false>); break;
+            case 129: launch(delta_chunk_kernel<128, true, true>, delta_chunk_kernel<128, true, false>); break;
+            case 256: launch(delta_chunk_kernel<256, false, true>, delta_chunk_kernel<256, false, false>); break;
+            default: launch(delta_chunk_kernel<256, true, true>, delta_chunk_kernel<256, true, false>); break;
+        }
+        XFT_CHECK_HIP(hipGetLastError());
+        return conv_tail(act, v, p.b.in, p.ld, p.channels, p.taps, b.conv_state, st, 1); // (several workgroups read the inputs of a key head: nobody shifts those of a single token in place)
+    }
     if (tiled) {
         const dim3 tiles((v.longest + kPrepTokens - 1) / kPrepTokens, (p.H + 3) / 4, v.B);
         const int key = (act == XFTHIP_BF16 ? 0 : 10) + p.taps + (width > 128 ? 100 : 0);
@@ -661,9 +1079,9 @@ int delta_prepare(int act, const PlanLayer &L, const StepView &v, const DeltaBuf
     return conv_tail(act, v, p.b.in, p.ld, p.channels, p.taps, b.conv_state, st);
 }
 
-int conv_tail(int act, const StepView &v, const void *in, int ld, int channels, int taps, void *conv_state, hipStream_t st) {
+int conv_tail(int act, const StepView &v, const void *in, int ld, int channels, int taps, void *conv_state, hipStream_t st, int least) {
     if (v.longest <= 1 || taps <= 1) return 0;
-    const TailParams p = {v, in, ld, channels, taps, conv_state};
+    const TailParams p = {v, in, ld, channels, taps, conv_state, least};
     const dim3 grid((channels + 255) / 256, v.B);
     if (act == XFTHIP_BF16) hipLaunchKernelGGL(conv_tail_kernel<true>, grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL(conv_tail_kernel<false>, grid, dim3(256), 0, st, p);
@@ -671,11 +1089,31 @@ int conv_tail(int act, const StepView &v, const void *in, int ld, int channels, 
     return 0;
 }
 
+size_t delta_chunk_floats(const PlanLayer &L, int tokens, int segments) {
+    if (L.KD < 64 || L.KD > 256 || tokens < kChunk) return 0;
+    return (size_t)(tokens / kChunk + std::min(segments, tokens)) * L.s.heads * chunk_floats(L.KD);
+}
+
 int delta_scan(const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st) {
     ScanParams p;
     p.v = v, p.b = b, p.H = L.s.heads, p.KH = L.s.kv_heads, p.VD = L.VD;
     const int lanes = L.KD / 8;
     const bool one = L.head_decay();
+    if (chunked(L, v, b)) {
+        // Two tiles a wave where a CU has several workgroups of one in turn: 16 heads of 128 x 128, one / two, 4 prompts of 1000 to 1500 tokens 255 / 262 us, 6 of 200 to 1000 239 / 270, 8 of
+        // 800 342 / 308, 16 of 400 351 / 314; 64 x 64, whose workgroups are of half the waves, 16 of 400 134 / 140; 8 of 256 x 256, 8 of 800 484 / 439
+        const bool two = L.VD % 32 == 0 && chunk_tiles(L, v) >= (L.KD == 64 ? 8L : 4L) * device_cu_count();
+        auto scan = [&](auto one_tile, auto two_tiles, int waves) {
+            hipLaunchKernelGGL(two ? two_tiles : one_tile, dim3(v.B, p.H, L.VD / 16 / (two ? 2 : 1)), dim3(64 * waves + 64), 0, st, p);
+        };
+        switch (L.KD) {
+            case 64: scan(delta_chunk_scan_kernel<64, 2, 1>, delta_chunk_scan_kernel<64, 2, 2>, 2); break;
+            case 128: scan(delta_chunk_scan_kernel<128, 4, 1>, delta_chunk_scan_kernel<128, 4, 2>, 4); break;
+            default: scan(delta_chunk_scan_kernel<256, 4, 1>, delta_chunk_scan_kernel<256, 4, 2>, 4); break;
+        }
+        XFT_CHECK_HIP(hipGetLastError());
+        return 0;
+    }
     // Two columns a group of lanes where one would make four waves a SIMD or more: below, the columns' chains are better hidden by each other's waves.  16
     // heads of 128 x 128, one column / two: 4 prompts of 1500 tokens 350 / 407 us, 6 of 1000 308 / 368, 8 of 800 308 / 272, 24 of 500 650 / 510.
     const bool two = v.longest > 1 && lanes >= 8 && L.VD % (512 / lanes) == 0 && (long)v.B * p.H * L.VD * lanes >= (long)device_cu_count() * 1024;

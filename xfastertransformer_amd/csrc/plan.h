@@ -275,14 +275,16 @@ struct DeltaBuffers {
     void *out; // rows of the output product's input, of the activation type
     float *state; // [slots][heads][VD][KD]
     void *conv_state; // [slots][taps - 1][channels] of the activation type
+    float *chunks; // delta_chunk_floats, or null: without the form for long segments
 };
-// the last taps - 1 inputs of segments of several tokens: in [T] rows of pitch ld -> conv_state
-int conv_tail(int act, const StepView &v, const void *in, int ld, int channels, int taps, void *conv_state, hipStream_t st);
+// the last taps - 1 inputs of segments of `least` tokens or more: in [T] rows of pitch ld -> conv_state
+int conv_tail(int act, const StepView &v, const void *in, int ld, int channels, int taps, void *conv_state, hipStream_t st, int least = 2);
 // steps of one token a sequence: all three of the following in one launch, where it takes the layer
 bool delta_decodes_at_once(const PlanLayer &L, const StepView &v);
 int delta_decode(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, float eps, hipStream_t st);
 int delta_prepare(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st);
 int delta_scan(const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st);
+size_t delta_chunk_floats(const PlanLayer &L, int tokens, int segments);
 int delta_output(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, float eps, hipStream_t st);
 
 // ---- gated linear attention: S = diag(alpha) S + k v^T, o = S^T q
@@ -381,7 +383,7 @@ struct PlanState {
     int logit_rows = 0;
     // scratch (activation type unless float)
     void *xn = nullptr, *a = nullptr, *cq = nullptr, *q = nullptr, *qa = nullptr, *oc = nullptr, *ov = nullptr, *h = nullptr, *u = nullptr;
-    float *y = nullptr, *y2 = nullptr, *gates = nullptr, *dq = nullptr, *dk = nullptr, *dqk = nullptr, *dg = nullptr, *dv = nullptr, *dbeta = nullptr, *do_ = nullptr, *carry = nullptr;
+    float *y = nullptr, *y2 = nullptr, *gates = nullptr, *dq = nullptr, *dk = nullptr, *dqk = nullptr, *dg = nullptr, *dv = nullptr, *dbeta = nullptr, *do_ = nullptr, *chunks = nullptr, *carry = nullptr;
     int *last_token = nullptr; // [slots]
     void *xn2 = nullptr, *first_values = nullptr, *side = nullptr, *narrow = nullptr;
     float *router_logits = nullptr, *expert_out = nullptr, *side_z = nullptr;

@@ -241,7 +241,7 @@ int mix_delta(xfthip_model *m, const PlanLayer &L, int store, const StepView &v,
     PlanState &p = *m->plan;
     const int act = p.act;
     int rc;
-    const DeltaBuffers b = {p.a, p.gates, p.dq, p.dk, p.dqk, p.dg, p.dv, p.dbeta, p.do_, p.ov, p.state[store], p.conv_state[store]};
+    const DeltaBuffers b = {p.a, p.gates, p.dq, p.dk, p.dqk, p.dg, p.dv, p.dbeta, p.do_, p.ov, p.state[store], p.conv_state[store], p.chunks};
     if (L.gates) {
         const int first = L.in_col + L.channels() + L.beta_cols();
         if ((rc = plan_gemm_heads(act, L.gates, v.T, (const char *)p.a + (size_t)first * p.esz, L.in_ld, L.gcols, L.rank, p.gates, 2 * L.gcols, XFTHIP_F32, st)))
@@ -1438,7 +1438,7 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
     const size_t T = max_tokens, e = p->esz, hidden = plan->hidden;
     bool normed_results = false;
     size_t a = 0, cq = 0, q = 0, qa = 0, ov = 0, h = 0, gates = 0, dk = 0, dqk = 0, dg = 0, dv = 0, heads = 0, fv = 0, u = 0, carry = 0;
-    size_t top = 0, experts = 0, routes = 0, eh = 0, eo = 0;
+    size_t chunks = 0, top = 0, experts = 0, routes = 0, eh = 0, eo = 0;
     for (const PlanLayer &L : p->layers) {
         const size_t H = L.s.heads;
         a = std::max(a, (size_t)L.in_ld), ov = std::max(ov, (size_t)L.out_ld);
@@ -1462,7 +1462,7 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
         } else {
             const size_t KH = L.s.kv_heads;
             gates = std::max(gates, (size_t)2 * L.gcols), dk = std::max(dk, KH * L.KD), dqk = std::max(dqk, KH), dg = std::max(dg, L.head_decay() ? H : H * L.KD);
-            dv = std::max(dv, H * L.VD), heads = std::max(heads, H);
+            dv = std::max(dv, H * L.VD), heads = std::max(heads, H), chunks = std::max(chunks, delta_chunk_floats(L, max_tokens, max_batch));
         }
     }
     alloc(&p->xn, std::max(T, (size_t)p->logit_rows) * hidden * e);
@@ -1561,6 +1561,9 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
         if (ok && fresh > ctx && hipMemGetInfo(&left, &device) == hipSuccess && left > ctx * row) ctx += std::min(fresh - ctx, (left - ctx * row) / 8 / row);
         alloc(&p->rows, ctx * rl * e, true), alloc(&p->kx, ctx * kx * e, true), alloc(&p->vx, ctx * vx * e, true), p->context_rows = (int)ctx;
     }
+    // (the delta rule's chunks alike: within an eighth of what is left, or not at all)
+    size_t left = 0, device = 0;
+    if (ok && chunks && hipMemGetInfo(&left, &device) == hipSuccess && chunks * 4 <= left / 8) alloc(&p->chunks, chunks * 4);
     if (!ok) {
         set_error("xfthip_model_create_from_plan: out of device memory");
         xfthip_model_destroy(m);
