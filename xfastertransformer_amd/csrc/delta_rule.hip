@@ -1,5 +1,5 @@
 // The gated delta-rule recurrence of layer plans: short convolutions, unit norms, decays and step sizes (delta_prepare), the
-// walk over the tokens with the state in registers (delta_scan), the gated per-head norm behind it (delta_output).
+// walk over the tokens with the state in registers (delta_scan), both 16 tokens at a time in long segments (delta_chunk, delta_chunk_scan), the gated per-head norm behind it (delta_output).
 // Everything between the projections' outputs and the output projection's input is fp32.
 #include <algorithm>
 #include <type_traits>
