@@ -262,23 +262,26 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
     }
     // Step k in weight set k % WSETS.  Four LDS tiles: the barrier that ends a step publishes the tile requested in the step before (everything but this step's own
     // requests and loads is in) and frees the one that this step read; the reads under way are of the next tile.  Two: it publishes the one requested in this step.
-    auto end_step = [&]() {
+    // Behind the loop nothing takes the weights that a step loads, and the compiler leaves the loads out: the count is that of the requests alone there.
+    auto end_step = [&](auto loads) {
         XFT_FENCE();
-        if constexpr (NBUF > 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(WREQS + ALOADS) : "memory");
+        if constexpr (NBUF > 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(loads() + ALOADS) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WREQS) : "memory");
         ++kt;
     };
-#define XFT_STEP(s)                                              \
+    constexpr std::integral_constant<int, WREQS> loaded;
+    constexpr std::integral_constant<int, 0> none;
+#define XFT_STEP(s, loads)                                       \
     {                                                            \
         step((s) % WSETS, ((s) + 1) % WSETS, (s) % WSETS, kt);   \
-        end_step();                                              \
+        end_step(loads);                                         \
     }
     if constexpr (FOUR) {
         auto one = [&]() { // (the next tile's registers are copied: 16 of them a step of 128 products)
 #pragma unroll
             for (int m = 0; m < RT; ++m) read_a((kt & 1) * TILEB, 0, m);
             step(0, 1, 1, kt);
-            end_step();
+            end_step(loaded);
 #pragma unroll
             for (int t = 0; t < CT; ++t) wreg[0][0][t] = wreg[1][0][t];
         };
@@ -297,17 +300,17 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
         }
     } else {
         while (kt + WSETS <= kt_n) {
-            XFT_STEP(0) XFT_STEP(1)
-            if constexpr (WSETS > 2) XFT_STEP(2)
-            if constexpr (WSETS > 3) XFT_STEP(3)
-            if constexpr (WSETS > 4) XFT_STEP(4)
-            if constexpr (WSETS > 5) XFT_STEP(5)
+            XFT_STEP(0, loaded) XFT_STEP(1, loaded)
+            if constexpr (WSETS > 2) XFT_STEP(2, loaded)
+            if constexpr (WSETS > 3) XFT_STEP(3, loaded)
+            if constexpr (WSETS > 4) XFT_STEP(4, loaded)
+            if constexpr (WSETS > 5) XFT_STEP(5, loaded)
         }
-        if (kt < kt_n) XFT_STEP(0)
-        if (WSETS > 2 && kt < kt_n) XFT_STEP(1)
-        if (WSETS > 3 && kt < kt_n) XFT_STEP(2)
-        if (WSETS > 4 && kt < kt_n) XFT_STEP(3)
-        if (WSETS > 5 && kt < kt_n) XFT_STEP(4)
+        if (kt < kt_n) XFT_STEP(0, none)
+        if (WSETS > 2 && kt < kt_n) XFT_STEP(1, none)
+        if (WSETS > 3 && kt < kt_n) XFT_STEP(2, none)
+        if (WSETS > 4 && kt < kt_n) XFT_STEP(3, none)
+        if (WSETS > 5 && kt < kt_n) XFT_STEP(4, none)
     }
 #undef XFT_STEP
 #undef XFT_FENCE
