@@ -193,7 +193,10 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
     constexpr int APG = FOUR ? 2 : (ALOADS + CT - 1) / CT; // requests a group that has some
     MFrag wcur_hi, wcur_lo;
     float rs[2] = {0.0f, 0.0f};
-    auto step = [&](int w_cur, int w_next, int w_load, int kt) {
+    constexpr int WREQS = CT * WPARTS; // weight loads a step, but for the steps behind the loop, whose loads nothing would take
+    constexpr std::integral_constant<int, WREQS> loaded;
+    constexpr std::integral_constant<int, 0> none;
+    auto step = [&](int w_cur, int w_next, int w_load, int kt, auto loads) {
         const int buf = (kt & (NBUF - 1)) * TILEB, buf_next = ((kt + 1) & (NBUF - 1)) * TILEB;
 #pragma unroll
         for (int ms = 0; ms < MICRO; ++ms) {
@@ -203,8 +206,8 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
 #pragma unroll
                 for (int i = q * APG; i < (q + 1) * APG; ++i)
                     if (i < ALOADS) request_a(kt + AHEAD, i);
-                if (FOUR && q >= ALOADS / 2 && q < ALOADS / 2 + CT) load_w(w_load, kt + WD, 0, q - ALOADS / 2);
-                if (KIND == XFTHIP_W_INT8 && ms == 1) load_w(w_load, kt + WD, 0, t); // (its codes have been widened a group ago)
+                if (FOUR && loads() && q >= ALOADS / 2 && q < ALOADS / 2 + CT) load_w(w_load, kt + WD, 0, q - ALOADS / 2);
+                if (KIND == XFTHIP_W_INT8 && loads() && ms == 1) load_w(w_load, kt + WD, 0, t); // (its codes have been widened a group ago)
                 MFrag nhi, nlo;
                 if (t + 1 < CT) widen(w_cur, ms, t + 1, nhi, nlo);
                 else if (ms + 1 < MICRO) widen(w_cur, ms + 1, 0, nhi, nlo);
@@ -232,11 +235,10 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
                 wcur_hi = nhi;
                 if constexpr (NF4) wcur_lo = nlo;
                 XFT_FENCE();
-                if constexpr (BF16) load_w(w_load, kt + WD, ms, t);
+                if (BF16 && loads()) load_w(w_load, kt + WD, ms, t);
             }
         }
     };
-    constexpr int WREQS = CT * WPARTS; // weight loads a step
     int kt = 0;
     // prologue: the weight and activation tiles that the first step does not send
 #pragma unroll
@@ -262,31 +264,39 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
     }
     // Step k in weight set k % WSETS.  Four LDS tiles: the barrier that ends a step publishes the tile requested in the step before (everything but this step's own
     // requests and loads is in) and frees the one that this step read; the reads under way are of the next tile.  Two: it publishes the one requested in this step.
-    // Behind the loop nothing takes the weights that a step loads, and the compiler leaves the loads out: the count is that of the requests alone there.
+    // The counts are those of a step's own requests and loads, so that they hold only while the compiler leaves none of these loads out: behind the k loop the registers
+    // that they fill are used once more, as far as it knows (kept).
     auto end_step = [&](auto loads) {
         XFT_FENCE();
         if constexpr (NBUF > 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(loads() + ALOADS) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WREQS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(loads()) : "memory");
         ++kt;
     };
-    constexpr std::integral_constant<int, WREQS> loaded;
-    constexpr std::integral_constant<int, 0> none;
-#define XFT_STEP(s, loads)                                       \
-    {                                                            \
-        step((s) % WSETS, ((s) + 1) % WSETS, (s) % WSETS, kt);   \
-        end_step(loads);                                         \
+    auto kept = [&](int sets) {
+#pragma unroll
+        for (int i = 0; i < sets; ++i)
+#pragma unroll
+            for (int part = 0; part < WPARTS; ++part)
+#pragma unroll
+                for (int t = 0; t < CT; ++t) asm volatile("" ::"v"(wreg[i][part][t]));
+    };
+#define XFT_STEP(s, loads)                                            \
+    {                                                                 \
+        step((s) % WSETS, ((s) + 1) % WSETS, (s) % WSETS, kt, loads); \
+        end_step(loads);                                              \
     }
     if constexpr (FOUR) {
-        auto one = [&]() { // (the next tile's registers are copied: 16 of them a step of 128 products)
+        auto one = [&](auto loads) { // (the next tile's registers are copied: 16 of them a step of 128 products)
 #pragma unroll
             for (int m = 0; m < RT; ++m) read_a((kt & 1) * TILEB, 0, m);
-            step(0, 1, 1, kt);
-            end_step(loaded);
+            step(0, 1, 1, kt, loads);
+            end_step(loads);
 #pragma unroll
-            for (int t = 0; t < CT; ++t) wreg[0][0][t] = wreg[1][0][t];
+            for (int t = 0; t < CT && loads(); ++t) wreg[0][0][t] = wreg[1][0][t];
         };
         const int whole = kt_n - (half_tail ? 1 : 0);
-        while (kt < whole) one();
+        while (kt < whole) one(loaded);
+        kept(1);
         if (half_tail) { // the last 64 k to their place, the k past the end count nothing
             for (int i = threadIdx.x & 255; i < ROWS * 8; i += 256) {
                 const int r = i >> 3, c = i & 7;
@@ -296,7 +306,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
                 *high = u32x4 {0u, 0u, 0u, 0u};
             }
             __syncthreads();
-            one();
+            one(none);
         }
     } else {
         while (kt + WSETS <= kt_n) {
@@ -319,6 +329,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
     // into an LDS patch of its own and walks it in 8-column chunks, consecutive lanes along a row (flush_rows)
     constexpr int OPITCH = 64 * CT + 16; // patch row pitch in bytes
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the requests past the last tile have landed
+    if constexpr (!FOUR) kept(WSETS);
     __syncthreads();                                 // every wave is past its last read of the activation tiles
     if constexpr (KG == 2) {
         // the second K group hands its accumulators over, 16 bytes a lane, from the start of LDS (at most the two groups' tiles), its row sums behind the tiles
