@@ -303,6 +303,13 @@ int xfthip_attention(xfthip_kvcache_t c, const void *q, int qStride, void *out, 
         int S, int qHeads, float scale, int past, const int *past_dev, xfthip_stream_t stream);
 
 /*
+ * Which form of the kernels xfthip_attention takes for `tokens` new tokens behind `past` in each of `batch` sequences on the current device (or on 256
+ * compute units where none is in use): 0 few (token, head) columns, 1 many, 2 many and long walks (another shape of the same MFMAs).  For tests of all
+ * of them, and for tuning.  No counterpart in the reference.
+ */
+int xfthip_attention_prefill_form(int cache_int8, int q_heads, int kv_heads, int batch, int tokens, int past, int *form);
+
+/*
  * xfthip_attention for callers that cannot allocate (code under HIP graph capture, serving loops
  * and harnesses that forbid hipMalloc): same arguments, same kernel and same split of the KV
  * sequence, but the partial results and tickets of the split merge live in a statically allocated
@@ -346,6 +353,8 @@ int xfthip_paged_attention_decode(void *out, const void *q, const void *k, const
 int xfthip_paged_attention_prefill(void *out, const void *q, const void *k, const void *v, int q_heads, int kv_heads,
         int head_size, int q_stride, int kv_stride, int o_stride, float scale, int batch, const int *token_lens_host,
         void *kcache, void *vcache, int block_num, int block_size, const int *slot_mapping, xfthip_stream_t stream);
+/* the form (xfthip_attention_prefill_form) of every sequence of such a call: forms[batch] */
+int xfthip_paged_attention_prefill_forms(int q_heads, int kv_heads, int batch, const int *token_lens_host, int *forms);
 
 /* ---- decoder layers and the model driver -------------------------------------------- */
 typedef struct xfthip_model *xfthip_model_t;

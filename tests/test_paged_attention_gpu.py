@@ -235,6 +235,7 @@ def test_paged_prefill_bands(xh, orc, qH, kvH, lens):
 @pytest.mark.parametrize("qH,kvH,lens", [(32, 8, [1700, 1103, 33, 701]), (24, 24, [2101, 1500])])
 def test_paged_prefill_that_fills_the_device(xh, orc, qH, kvH, lens):
     """Enough long walks for the form in 16 x 16 MFMAs, a short sequence beside them."""
+    assert xh.paged_attention_prefill_forms(qH, kvH, lens) == [0 if n < 100 else 2 for n in lens]
     test_paged_prefill_matches_oracle(xh, orc, qH, kvH, lens, 16)
 
 

@@ -138,10 +138,12 @@ def test_scores_at_the_ends_of_the_range(xh, orc, score):
     (12, 65, 0, 32, 32, "bf16", 4, 4),  # three
     (64, 2, 700, 128, 4, "bf16", 0, 0),
     (5, 129, 64, 28, 4, "bf16", 8, 0),
+    (5, 129, 500, 28, 4, "bf16", 8, 0),  # the same behind a walk long enough for 16 x 16 MFMAs
 ])
 @pytest.mark.parametrize("spread", [0, 1])
 def test_int8_cache(xh, orc, B, S, past, qh, kvh, kind, extra, skip, spread):
     """spread: the values' sizes go up and down by powers of ten from token to token and block to block, so that the scale they are taken relative to moves."""
+    assert xh.attention_prefill_form(qh, kvh, B, S, past, int8=True) == (2 if past + S // 2 >= 256 else 1)
     rng = np.random.default_rng(S * 37 + past)
     n = past + S
     k, v = (rng.standard_normal((B, n, kvh * D)).astype(np.float32) for _ in range(2))
@@ -219,10 +221,10 @@ def test_any_softmax_scale(xh, orc, scale, size, kind):
 ])
 @pytest.mark.parametrize("score,scale", [(None, SCALE), (-1e30, SCALE), (3000.0, SCALE), (None, 1e-4)])
 def test_launches_that_fill_the_device(xh, orc, B, S, past, qh, kvh, kind, extra, skip, score, scale):
-    """512 and more workgroups, 20480 and more (workgroup, 32-token block) pairs: the form in 16 x 16 MFMAs.  The first 40 tokens score as the others,
+    """Enough workgroups and (workgroup, 32-token block) pairs for the form in 16 x 16 MFMAs.  The first 40 tokens score as the others,
     minus infinity, or so high that the others' weights vanish."""
     rng = np.random.default_rng(S * 31 + past)
-    assert -(-S * (qh // kvh) // 128) * B * kvh >= 512 and -(-S * (qh // kvh) // 128) * B * kvh * ((past + S // 2) // 32) >= 20480
+    assert xh.attention_prefill_form(qh, kvh, B, S, past) == 2
     k, v = (rng.standard_normal((B, past + S, kvh * D)).astype(np.float32) for _ in range(2))
     q = orc.round_bf16(rng.standard_normal((B * S, qh * D)))
     if score is not None:

@@ -391,6 +391,13 @@ def attention(cache, q_dev, q_stride, out_dev, o_stride, out_dtype, B, S, q_head
                                C.c_float(scale), past, past_dev, stream))
 
 
+def attention_prefill_form(q_heads, kv_heads, batch, tokens, past=0, int8=False):
+    """Which form of the kernels a prompt takes (include/xft_hip.h); needs no device."""
+    form = C.c_int()
+    check(lib.xfthip_attention_prefill_form(int(int8), q_heads, kv_heads, batch, tokens, past, C.byref(form)))
+    return form.value
+
+
 def attention_static(cache, q_dev, q_stride, out_dev, o_stride, out_dtype, B, S, q_heads, scale, past, past_dev=None,
                      stream=None):
     """xfthip_attention through the statically allocated split workspace (allocates nothing)."""
@@ -676,6 +683,14 @@ def paged_attention_prefill(out_dev, q_dev, k_dev, v_dev, q_heads, kv_heads, hea
     check(lib.xfthip_paged_attention_prefill(out_dev, q_dev, k_dev, v_dev, q_heads, kv_heads, head, q_stride, kv_stride, o_stride,
                                              C.c_float(scale), len(lens), _hp(lens), kcache_dev, vcache_dev, block_num, block_size,
                                              slots_dev, stream))
+
+
+def paged_attention_prefill_forms(q_heads, kv_heads, token_lens):
+    """The form (attention_prefill_form) of every sequence of such a call; needs no device."""
+    lens = np.ascontiguousarray(token_lens, np.int32)
+    forms = np.empty(len(lens), np.int32)
+    check(lib.xfthip_paged_attention_prefill_forms(q_heads, kv_heads, len(lens), _hp(lens), _hp(forms)))
+    return forms.tolist()
 
 
 def argmax(logits_dev, rows, cols, stream=None):

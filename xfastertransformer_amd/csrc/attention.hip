@@ -161,16 +161,15 @@ int xfthip::attention_launch(xfthip_kvcache_t c, const void *q, int qStride, voi
     p.past = past;
     p.past_dev = past_dev;
     p.CG = (S * p.G + 15) / 16;
-    // Many columns per KV head (prefill, long chunks): the form in which a wave walks the whole visible sequence
-    // for its 32 columns through LDS blocks shared by its workgroup, taken once such waves fill the device.
+    // many columns per KV head (prefill, long chunks)
     {
-        const long waves1 = (long)B * c->kv.H * p.CG; // waves with one column tile each
-        if (S > 1 && waves1 >= 4L * device_cu_count()) {
+        const int form = attention_prefill_form(c->kv.int8, p.G, (long)B * c->kv.H, S, past);
+        if (form) {
             p.nsplit = 1;
             const int ncg = (S * p.G + 127) / 128, npairs = B * c->kv.H;
             const PrefillBands bands = prefill_bands((npairs + 7) / 8);
             dim3 grid(8 * ((npairs + 7) / 8) * ncg);
-            const bool fine = prefill_fine(c->kv.int8, (long)ncg * npairs, past + S / 2);
+            const bool fine = form == 2;
             if (c->kv.int8 && fine) hipLaunchKernelGGL((attn_prefill32_kernel<true, true>), grid, dim3(256), 0, stream, p, ncg, npairs, bands);
             else if (c->kv.int8) hipLaunchKernelGGL((attn_prefill32_kernel<true, false>), grid, dim3(256), 0, stream, p, ncg, npairs, bands);
             else if (fine) hipLaunchKernelGGL((attn_prefill32_kernel<false, true>), grid, dim3(256), 0, stream, p, ncg, npairs, bands);

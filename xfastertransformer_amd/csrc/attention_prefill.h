@@ -131,10 +131,16 @@ __host__ __device__ inline void prefill_band(const PrefillBands b, const int gro
 // (97, 1.4 workgroups a CU) 73 -> 73, 4 x 800 (40) 40 -> 42, 8 x 500 (30) 37 -> 40, 512 behind 8000, half a workgroup a CU, 153 -> 154.
 // INT8, mean tokens walked in brackets: 4 x 2000 (1000) 226 -> 217, 5 x 1500 (750) 157 -> 148, 2 x 3500, 32 / 32 (1750) 344 -> 322, 512 behind 8000 (8250) 295 -> 282,
 // 900 (450) 40.2 -> 39.4; but 8 x 400 (200) 37.0 -> 37.7, 12 x 200 (100) 28.7 -> 28.8.
-// walk: the tokens that a column sees on average
-inline bool prefill_fine(bool int8, long workgroups, long walk) {
+// walk: the tokens that a column sees on average; least: blocks a CU from which on FP16 takes it
+inline bool prefill_fine(bool int8, long workgroups, long walk, long least = 80) {
     const long cus = device_cu_count();
-    return int8 ? walk >= 256 : workgroups >= 2 * cus && workgroups * (walk / 32) >= 80 * cus;
+    return int8 ? walk >= 256 : workgroups >= 2 * cus && workgroups * (walk / 32) >= least * cus;
+}
+// S new tokens behind `past` for each of `pairs` (sequence, KV head) pairs, G query heads a KV head: 0 the form for few columns, 1 this one, 2 this one, FINE.  This one (a wave walks the
+// whole visible sequence for its 32 columns) is taken once waves of 16 columns would fill the device.
+inline int attention_prefill_form(bool int8, int G, long pairs, int S, int past) {
+    if (S <= 1 || pairs * ((S * G + 15) / 16) < 4L * device_cu_count()) return 0;
+    return prefill_fine(int8, pairs * ((S * G + 127) / 128), past + S / 2) ? 2 : 1;
 }
 
 constexpr int kRing = 4, kLook = kRing - 1, kRingBlock = 16384, kRingLds = kRing * kRingBlock;

@@ -443,6 +443,37 @@ int check_common(const void *out, const void *q, const void *k, const void *v, i
     return 0;
 }
 
+// Which form takes the sequences of a launch, the longest first: the first `many` that for many columns, `scaled` of them with queries that carry the scale's power of two
+struct SeqForms {
+    int scaled, many;
+    bool fine;
+};
+SeqForms seq_forms(const int *rows, int n, int G, int kv_heads) {
+    SeqForms f = {0, 0, false};
+    const long enough = 4L * device_cu_count();
+    long waves = 0; // of 16 columns, of those that attention_launch would not take to the form for many columns
+    for (int i = 0; i < n; ++i) {
+        const long w = (long)kv_heads * (((long)rows[i] * G + 15) / 16);
+        if (rows[i] > 1 && w >= enough) ++f.scaled;
+        else waves += w;
+    }
+    // Those that it would, and the others with them where they are enough together (12 x 200 tokens, 32 query / 8 KV heads 21 us against 52 in the form for few columns, 8 x 600,
+    // 16 / 4 heads 29 against 79), with their queries as they are, as the form that each would take alone has them
+    f.many = waves >= enough ? n : f.scaled;
+    long groups = 0, walks = 0; // column groups of a KV head, the tokens that their columns see on average
+    for (int i = 0; i < f.many; ++i) {
+        const long g = ((long)rows[i] * G + 127) / 128;
+        groups += g, walks += g * (rows[i] / 2);
+    }
+    // (Blocks a CU in brackets, 32 / 8 heads, us of the call in 32 x 32 and in 16 x 16 MFMAs: 6 sequences of 750 to 1500 tokens (120) 98.0 and 94.5, 3000 and 30 of 60 (135) 103.9 and 102.6, 1700, 1103, 701 (71)
+    // 71.0 and 68.9, 2 of 2500, 16 / 4 heads (96) 82.2 and 81.1, 4 of 900 (51) 51.1 and 50.8; but 1700 and 2 of 200 (45) 72.6 and 74.2, 1500 and 60 of 60 (37) 61.2 and 62.6, 1200 and 63 of 64 (26) 47.6 and
+    // 48.6.  By the longest sequence's walk the last two would be 120 and 92.)
+    f.fine = f.many > 0 && prefill_fine(false, groups * kv_heads, walks / groups, 50);
+    return f;
+}
+// sequences of a launch: at most kSeqs, and kGroups groups of 8 (sequence, KV head) pairs
+int seqs_per_launch(int kv_heads) { return std::max(1, std::min(kSeqs, kGroups * 8 / kv_heads - 1)); }
+
 } // namespace
 } // namespace xfthip
 
@@ -489,6 +520,31 @@ extern "C" int xfthip_paged_attention_decode(void *out, const void *q, const voi
     return 0;
 }
 
+extern "C" int xfthip_attention_prefill_form(int cache_int8, int q_heads, int kv_heads, int batch, int tokens, int past, int *form) {
+    XFT_REQUIRE(form && batch > 0 && tokens > 0 && past >= 0 && kv_heads > 0 && q_heads % kv_heads == 0, "xfthip_attention_prefill_form: bad argument");
+    *form = attention_prefill_form(cache_int8 != 0, q_heads / kv_heads, (long)batch * kv_heads, tokens, past);
+    return 0;
+}
+
+extern "C" int xfthip_paged_attention_prefill_forms(int q_heads, int kv_heads, int batch, const int *token_lens_host, int *forms) {
+    XFT_REQUIRE(forms && token_lens_host && batch > 0 && kv_heads > 0 && q_heads % kv_heads == 0, "xfthip_paged_attention_prefill_forms: bad argument");
+    std::vector<int> order(batch), rows;
+    for (int b = 0; b < batch; ++b) {
+        XFT_REQUIRE(token_lens_host[b] > 0, "xfthip_paged_attention_prefill_forms: sequence %d has %d tokens", b, token_lens_host[b]);
+        order[b] = b;
+    }
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return token_lens_host[x] > token_lens_host[y]; });
+    const int G = q_heads / kv_heads, per_launch = seqs_per_launch(kv_heads);
+    for (int b = 0; b < batch; b += per_launch) {
+        const int n = std::min(per_launch, batch - b);
+        rows.clear();
+        for (int i = 0; i < n; ++i) rows.push_back(token_lens_host[order[b + i]]);
+        const SeqForms f = seq_forms(rows.data(), n, G, kv_heads);
+        for (int i = 0; i < n; ++i) forms[order[b + i]] = n == 1 ? attention_prefill_form(false, G, kv_heads, rows[0], 0) : i >= f.many ? 0 : f.fine ? 2 : 1;
+    }
+    return 0;
+}
+
 extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const void *k, const void *v, int q_heads, int kv_heads,
         int head_size, int q_stride, int kv_stride, int o_stride, float scale, int batch, const int *token_lens_host, void *kcache,
         void *vcache, int block_num, int block_size, const int *slot_mapping, xfthip_stream_t stream) {
@@ -498,8 +554,8 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
     hipStream_t st = (hipStream_t)stream;
     for (int b = 0; b < batch; ++b)
         XFT_REQUIRE(token_lens_host[b] > 0, "xfthip_paged_attention_prefill: sequence %d has %d tokens", b, token_lens_host[b]);
-    // launches of up to kSeqs sequences (and kGroups groups of 8 (sequence, KV head) pairs), the longest first
-    const int per_launch = std::max(1, std::min(kSeqs, kGroups * 8 / kv_heads - 1));
+    // launches of several sequences, the longest first
+    const int per_launch = seqs_per_launch(kv_heads);
     std::vector<int> order(batch), first(batch);
     for (int b = 0, at = 0; b < batch; at += token_lens_host[b], ++b) order[b] = b, first[b] = at;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return token_lens_host[x] > token_lens_host[y]; });
@@ -536,14 +592,9 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
     for (int b = 0; b < batch; b += per_launch) {
         SeqBatch s = {};
         s.n = std::min(per_launch, batch - b);
-        int n_long = 0;
-        long waves = 0; // of 16 columns, the others
         for (int i = 0; i < s.n; ++i) {
             const int S = token_lens_host[order[b + i]];
             s.row0[i] = first[order[b + i]], s.rows[i] = S, s.blk0[i + 1] = s.blk0[i] + (S + 31) / 32;
-            const long w = (long)kv_heads * (((long)S * G + 15) / 16);
-            if (S > 1 && w >= 4L * device_cu_count()) ++n_long;
-            else waves += w;
         }
         const int blocks = s.blk0[s.n];
         KvView kv = {};
@@ -564,10 +615,8 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
         AttnParams p = {};
         p.kv = kv, p.q = (const uint16_t *)q, p.qStride = q_stride, p.out = out, p.oStride = o_stride, p.out_dtype = XFTHIP_BF16;
         p.B = 1, p.G = G, p.scale = scale, p.nsplit = 1;
-        // Those that attention_launch would take to the form for many columns, and the others with them where they are enough together (12 x 200
-        // tokens, 32 query / 8 KV heads 21 us against 52 in the form for few columns, 8 x 600, 16 / 4 heads 29 against 79), with their queries as they are,
-        // as the form that each would take alone has them
-        s.first = 0, s.scaled = n_long, s.many = waves >= 4L * device_cu_count() ? s.n : n_long;
+        const SeqForms forms = seq_forms(s.rows, s.n, G, kv_heads);
+        s.first = 0, s.scaled = forms.scaled, s.many = forms.many;
         const int groups = (s.many * kv_heads + 7) / 8;
         s.bands = prefill_bands(groups);
         auto levels = [&](int g) { return (int)(((long)s.rows[g * 8 / kv_heads] * G + 127) / 128); }; // (the sequences are sorted: the group's first pair belongs to its longest)
@@ -576,8 +625,7 @@ extern "C" int xfthip_paged_attention_prefill(void *out, const void *q, const vo
             prefill_band(s.bands, g, band, width);
             s.grp0[g + 1] = s.grp0[g] + (levels(g) - (g + 1 < band + width ? levels(g + 1) : 0)) * (g - band + 1);
         }
-        const bool fine = prefill_fine(false, 8L * s.grp0[groups], s.rows[0] / 2);
-        if (s.many > 0 && fine) hipLaunchKernelGGL(paged_prefill_attn_kernel<true>, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
+        if (s.many > 0 && forms.fine) hipLaunchKernelGGL(paged_prefill_attn_kernel<true>, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
         else if (s.many > 0) hipLaunchKernelGGL(paged_prefill_attn_kernel<false>, dim3(8 * s.grp0[groups]), dim3(256), 0, st, p, s);
         s.first = s.many, s.many = s.n - s.many;
         if (s.many > 0)
