@@ -691,6 +691,11 @@ size_t xfthip_plan_weight_bytes(xfthip_plan_t p);
 int xfthip_model_create_from_plan(xfthip_plan_t p, int act_dtype, int max_batch, int max_seq, int max_tokens, int pool_tokens,
         xfthip_model_t *out);
 /*
+ * Which segments of a step the delta rule takes 16 tokens at a time (forms[i] 1; 0: token by token) on the current device (or on 256 compute units where none is in use),
+ * for a layer of these heads, key and value widths and filter taps with a decay a head or a channel.  For tests of both, and for tuning.
+ */
+int xfthip_delta_forms(int heads, int dim, int vdim, int taps, int decay_per_head, int segments, const int *lens_host, int *forms);
+/*
  * One step of a batch of unequal parts: entry i brings the next lens_host[i] tokens of slot rows_host[i] (a prompt, a portion of
  * one or a single token; ids back to back in ids_host); a slot that holds no sequence starts one at position 0.  want_host: n_want
  * indices into the step's tokens, ascending or not, whose logits go to logits_host (fp32 [n_want, vocab]).  Models from a plan only.

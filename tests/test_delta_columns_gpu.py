@@ -41,11 +41,8 @@ def test_scan(dim, vdim, heads, decay):
 LONG, THEN = [1, 16, 17, 140, 15, 32, 47, 129], [130, 9, 33, 1, 16, 3, 31, 48]
 
 
-# (one tile of 16 columns a wave and, from 1024 tiles on 256 compute units, two; key widths of 64, 128 and 256)
-@pytest.mark.parametrize("dim,vdim,heads,few", [(128, 128, 16, 0), (128, 96, 4, 0), (64, 64, 4, 0), (50, 64, 64, 0), (200, 96, 6, 0), (256, 64, 32, 0), (128, 64, 2, 3)])
-@pytest.mark.parametrize("decay", ["channel", "head"])
-def test_scan_in_chunks(dim, vdim, heads, few, decay):
-    """few: that many of the sequences, beginning with the longest"""
+def held(dim, vdim, heads, decay, steps, forms, tokens=512):
+    """A layer over several steps.  steps: the tokens of every sequence, step by step; forms: what xh.delta_forms has to say of each of them"""
     from xfastertransformer_amd import capi as xh
     xh.init(0)
     kv = heads // 2
@@ -55,16 +52,50 @@ def test_scan_in_chunks(dim, vdim, heads, few, decay):
     else:
         u, ref = one_decay, duvadra_ref
         cfg = u.config([(u.windowed_delta(r_heads=heads, r_kv_heads=kv, r_dim=dim, r_vdim=vdim, left=0.0), None)])
+    for lens, form in zip(steps, forms):
+        assert set(xh.delta_forms(heads, dim, vdim, 4, decay == "head", lens)) == form
     bits = u.weights(cfg, 22)
-    case = u.Case(xh, u.build_plan(xh, cfg, bits), u.oracle_weights(bits), lambda w, t: ref.forward(cfg, w, t), "f32", 3e-5, 8, 384, 512)
+    n = len(steps[0])
+    case = u.Case(xh, u.build_plan(xh, cfg, bits), u.oracle_weights(bits), lambda w, t: ref.forward(cfg, w, t), "f32", 3e-5, n, 384, tokens, n * 384)
     rng = np.random.default_rng(dim + heads)
-    first, then = (LONG[3:3 + few], THEN[3:3 + few]) if few else (LONG, THEN)
-    texts = [rng.integers(0, cfg["vocab"], a + b) for a, b in zip(first, then)]
+    ends = np.cumsum([[0] * n] + [list(s) for s in steps], 0)
+    texts = [rng.integers(0, cfg["vocab"], e) for e in ends[-1]]
     want = [case.want(t) for t in texts]
-    for ends, begins, what in ((first, [0] * 8, "first step"), ([len(t) for t in texts], first, "second step")):
-        got = case.model.step([(i, t[b:e], list(range(e - b))) for i, (t, b, e) in enumerate(zip(texts, begins, ends))])
-        case.check(got, np.concatenate([w[b:e] for w, b, e in zip(want, begins, ends)]), what)
+    for k in range(len(steps)):
+        part = list(zip(ends[k], ends[k + 1]))
+        got = case.model.step([(i, t[b:e], list(range(e - b))) for i, (t, (b, e)) in enumerate(zip(texts, part))])
+        case.check(got, np.concatenate([w[b:e] for w, (b, e) in zip(want, part)]), f"step {k}")
     case.free()
+
+
+# (one tile of 16 columns a wave; key widths of 64, 128 and 256.  1024 tiles on 256 compute units are enough for each segment to go by its own length: those of 64 tokens and more
+# (128 with one decay a head) in chunks, the others token by token; the last case's values are too wide for the preparation that walks several tokens.)
+@pytest.mark.parametrize("dim,vdim,heads,few,forms", [(128, 128, 16, 0, {0, 1}), (128, 96, 4, 0, {1}), (64, 64, 4, 0, {1}), (50, 64, 64, 0, {0, 1}), (200, 96, 6, 0, {1}), (256, 64, 32, 0, {0, 1}), (128, 64, 2, 3, {1}),
+                                                     (64, 288, 8, 0, {0, 1})])
+@pytest.mark.parametrize("decay", ["channel", "head"])
+def test_scan_in_chunks(dim, vdim, heads, few, forms, decay):
+    """few: that many of the sequences, beginning with the longest"""
+    first, then = (LONG[3:3 + few], THEN[3:3 + few]) if few else (LONG, THEN)
+    held(dim, vdim, heads, decay, [first, then], [forms, forms])
+
+
+# (two tiles of 16 columns a wave; a few short segments go with the long ones)
+@pytest.mark.parametrize("dim,vdim,heads", [(128, 128, 16), (50, 64, 64), (256, 64, 32)])
+@pytest.mark.parametrize("decay", ["channel", "head"])
+def test_scan_in_chunks_two_tiles(dim, vdim, heads, decay):
+    held(dim, vdim, heads, decay, [[140, 129, 128, 131, 144, 150, 160, 133, 5], [129, 130, 145, 128, 160, 133, 131, 150, 1]], [{1}, {1}], 1200)
+
+
+@pytest.mark.parametrize("dim,vdim,heads", [(128, 128, 16), (64, 64, 32), (256, 64, 32)])
+@pytest.mark.parametrize("decay", ["channel", "head"])
+def test_prompts_beside_decoding_sequences(dim, vdim, heads, decay):
+    """Single tokens by the kernel for them beside prompts in chunks, which go on one token at a time while the next prompt comes."""
+    held(dim, vdim, heads, decay, [[3, 2, 1, 4, 5, 1, 2, 2, 130, 3], [1, 1, 140, 1, 1, 1, 1, 1, 1, 129], [1] * 10, [1, 130, 1, 1, 1, 1, 1, 1, 17, 1]], [{0, 1}, {0, 1}, {0}, {0, 1}])
+
+
+def test_more_segments_than_a_launch_names():
+    lens = [32 + i % 5 for i in range(131)]
+    held(64, 32, 4, "channel", [lens, lens[::-1]], [{1}, {1}], 4608)
 
 
 @pytest.mark.parametrize("at", [0, 7, 16, 37])

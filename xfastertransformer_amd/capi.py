@@ -669,6 +669,14 @@ class PlanModel(Model):
         return free.value, total.value
 
 
+def delta_forms(heads, dim, vdim, taps, decay_per_head, lens):
+    """Which segments of a step the delta rule takes 16 tokens at a time (include/xft_hip.h); needs no device."""
+    lens = np.ascontiguousarray(lens, np.int32)
+    forms = np.empty(len(lens), np.int32)
+    check(lib.xfthip_delta_forms(heads, dim, vdim, taps, int(decay_per_head), len(lens), _hp(lens), _hp(forms)))
+    return forms.tolist()
+
+
 def paged_attention_decode(out_dev, q_dev, k_dev, v_dev, q_heads, kv_heads, head, q_stride, kv_stride, o_stride, scale, batch,
                            kcache_dev, vcache_dev, block_num, block_size, tables_dev, table_stride, ctx_dev, slots_dev, max_context,
                            stream=None):

@@ -2,6 +2,7 @@
 // walk over the tokens with the state in registers (delta_scan), both 16 tokens at a time in long segments (delta_chunk, delta_chunk_scan), the gated per-head norm behind it (delta_output).
 // Everything between the projections' outputs and the output projection's input is fp32.
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "plan_dev.h"
@@ -18,6 +19,7 @@ __device__ inline float ldb(const void *p, size_t i) {
 
 struct PrepParams {
     StepView v;
+    int below; // of the walk token by token: segments of as many tokens are taken in chunks
     DeltaBuffers b;
     const float *conv, *decay, *dt_bias;
     int H, KH, KD, VD, taps, ld, channels, beta_col, decay_col, gcols; // decay_col: one decay a head, in the row (or -1)
@@ -33,6 +35,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(PrepParams p) {
     if (head >= p.H) return;
     constexpr int DT = BF16 ? XFTHIP_BF16 : XFTHIP_F32;
     const int seg = p.v.tok_seg[t], pos = p.v.tok_pos[t];
+    if (p.v.seg_len[seg] >= p.below) return;
     const int off = p.v.seg_off[seg], row = p.v.seg_row[seg];
     const bool alone = p.v.seg_len[seg] == 1;
     const int local = t - off;
@@ -102,7 +105,7 @@ template <bool BF16, int TAPS, int J> // J: turns of 128 channels that cover a h
 __global__ __launch_bounds__(256) void delta_prepare_tiled_kernel(PrepParams p) {
     const int lane = threadIdx.x & 63, head = blockIdx.y * 4 + (threadIdx.x >> 6), seg = blockIdx.z;
     const int n = p.v.seg_len[seg], i0 = blockIdx.x * kPrepTokens;
-    if (head >= p.H || i0 >= n) return;
+    if (head >= p.H || i0 >= n || n >= p.below) return;
     const int off = p.v.seg_off[seg], row = p.v.seg_row[seg], start = p.v.seg_pos[seg];
     const int cnt = n - i0 < kPrepTokens ? n - i0 : kPrepTokens;
     const bool qk_head = head < p.KH;
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(256) void conv_tail_kernel(TailParams p) {
 struct ScanParams {
     StepView v;
     DeltaBuffers b;
-    int H, KH, VD;
+    int H, KH, VD, below; // (as above)
 };
 
 // The state's columns (value channels) do not interact.  L lanes hold C neighbouring columns, 4 RV key rows each (KD = 4 L RV).
@@ -270,6 +273,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(ScanParams p) {
     __shared__ f32x4 sums[CT * COLS * L / 4]; // the lanes' parts of the read-outs: [token][c][column group][lane]
     const int seg = 2 * blockIdx.z < gridDim.z ? blockIdx.x : gridDim.x - 1 - blockIdx.x, head = blockIdx.y, kvh = head / (p.H / p.KH);
     const int n = p.v.seg_len[seg], off = p.v.seg_off[seg];
+    if (n >= p.below) return;
     const int li = threadIdx.x % L, lc = threadIdx.x / L * C;
     const int col0 = blockIdx.z * COLS, col = col0 + lc;
     const bool own = col < p.VD; // (VD is a multiple of 32: C neighbouring columns are in it or not together)
@@ -432,16 +436,21 @@ constexpr int kChunk = 16;
 __host__ __device__ constexpr size_t chunk_floats(int KD) { return (size_t)(3 * kChunk + 1) * KD + 2 * kChunk * kChunk; }
 // records in front of a segment's: ceil(n / 16) of every segment fit in floor((off + n) / 16) - floor(off / 16) + 1
 __device__ inline size_t chunk_of(int off, int seg) { return (size_t)(off / kChunk + seg); }
+// the segments of a launch
+constexpr int kChunkSegs = 128;
+struct ChunkSegs {
+    int seg[kChunkSegs];
+};
 
 // In place of delta_prepare for such segments: convolutions, norms and decays of a (chunk, head) by a workgroup of its own, two neighbouring channels of q, k, v or the decays a
 // thread, and what the scan needs of them.  Tokens past the segment's end have no keys, queries and step sizes.  A and B: thread (s, 1/16 of the key dims) carries k_s on from token to token,
 // 16 lanes add up.  Bound by the round trips of a workgroup, of which six share a CU (4 prompts of 1000 to 1500 tokens, 16 heads of 128 x 128: 110 us for 270 MB; delta_prepare, which
 // leaves the products to the scan, 85).
 template <int KD, bool ONE, bool BF16>
-__global__ __launch_bounds__(256) void delta_chunk_kernel(PrepParams p) {
+__global__ __launch_bounds__(256) void delta_chunk_kernel(PrepParams p, ChunkSegs segs) {
     constexpr int J = KD / 64, N = kChunk * KD / 4 / 256, P = KD + 4, SIZE = kChunk * P; // (rows of P: lanes that read a column of rows are on banks of their own)
     __shared__ __align__(16) float q[SIZE], k[SIZE], g[SIZE], A[kChunk * kChunk], B[kChunk * kChunk], beta[kChunk], one[kChunk];
-    const int tid = threadIdx.x, head = blockIdx.y, seg = blockIdx.z, H = p.H, kvh = head / (H / p.KH), c0 = blockIdx.x * kChunk;
+    const int tid = threadIdx.x, head = blockIdx.y, seg = segs.seg[blockIdx.z], H = p.H, kvh = head / (H / p.KH), c0 = blockIdx.x * kChunk;
     const int n = p.v.seg_len[seg], off = p.v.seg_off[seg], start = p.v.seg_pos[seg], taps = p.taps;
     if (c0 >= n) return;
     const size_t hist = (size_t)p.v.seg_row[seg] * (taps - 1) * p.channels;
@@ -607,11 +616,11 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(PrepParams p) {
 // 3000 1038 / 431, 16 of 400 816 / 441; with one decay a head, 32 of 128 x 128, 2 of 3000 784 / 468, 16 of 400 603 / 526.
 // A wave for all key rows: 213 us for the prompt of 1500, two 103, four 82 (85 with two sums of every product, for as small an error as the walk token by token has).  With the stores of a last, ragged chunk in the loop every wait was one for the stores before, too: 100.
 template <int KD, int NW, int C>
-__global__ __launch_bounds__(64 * NW + 64, KD / NW == 32 && C == 1 ? 4 : 2) void delta_chunk_scan_kernel(ScanParams p) {
+__global__ __launch_bounds__(64 * NW + 64, KD / NW == 32 && C == 1 ? 4 : 2) void delta_chunk_scan_kernel(ScanParams p, ChunkSegs segs) {
     constexpr int I = KD / 16 / NW, SETS = 2;
     __shared__ f32x4 parts[2][NW][2][C][64];
     // (segments of one place are handed to one XCD in turn, whose share should be long and short ones)
-    const int seg = (blockIdx.x + blockIdx.y + (blockIdx.y >> 1) + (blockIdx.y >> 2)) % gridDim.x, head = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int seg = segs.seg[(blockIdx.x + blockIdx.y + (blockIdx.y >> 1) + (blockIdx.y >> 2)) % gridDim.x], head = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, c = lane & 15, row0 = wave * 16 * I;
     const int n = p.v.seg_len[seg], off = p.v.seg_off[seg], last = (n - 1) / kChunk;
     // addresses: scalar ones that move with the chunks, and these of a lane (in bytes), which do not
@@ -812,7 +821,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(ScanParams p) {
     constexpr int KD = 8 * L, COLS = 256 / L;
     const int seg = blockIdx.x, head = blockIdx.y, kvh = head / (p.H / p.KH), t = p.v.seg_off[seg];
     const int li = threadIdx.x % L, col = blockIdx.z * COLS + threadIdx.x / L;
-    if (col >= p.VD) return; // (whole groups of L lanes)
+    if (col >= p.VD || p.v.seg_len[seg] >= p.below) return; // (whole groups of L lanes)
     float *state = p.b.state + (((size_t)p.v.seg_row[seg] * p.H + head) * p.VD + col) * KD;
     f32x4 s0 = *(const f32x4 *)(state + 4 * li), s1 = *(const f32x4 *)(state + 4 * (L + li));
     const float *q = p.b.q + ((size_t)t * p.KH + kvh) * KD + 4 * li, *k = p.b.k + ((size_t)t * p.KH + kvh) * KD + 4 * li;
@@ -993,7 +1002,7 @@ __global__ __launch_bounds__(1024) void delta_decode_kernel(PrepParams p, OutPar
 
 PrepParams prep_params(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b) {
     PrepParams p;
-    p.v = v, p.b = b;
+    p.v = v, p.b = b, p.below = INT_MAX;
     p.b.in = (char *)b.in + (size_t)L.in_col * (act == XFTHIP_BF16 ? 2 : 4);
     p.conv = L.conv, p.decay = L.decay, p.dt_bias = L.dt_bias;
     p.H = L.s.heads, p.KH = L.s.kv_heads, p.KD = L.KD, p.VD = L.VD, p.taps = L.s.taps;
@@ -1002,15 +1011,18 @@ PrepParams prep_params(int act, const PlanLayer &L, const StepView &v, const Del
     return p;
 }
 
-// Tiles of 16 columns of all states of a step: four waves each and more
-long chunk_tiles(const PlanLayer &L, const StepView &v) { return (long)v.B * L.s.heads * (L.VD / 16); }
+// tiles of 16 columns of the states of so many segments: four waves each and more
+long chunk_tiles(const PlanLayer &L, size_t segments) { return (long)segments * L.s.heads * (L.VD / 16); }
 
-// Segments kChunk tokens at a time?  From a whole chunk on, where the walk token by token leaves most of the device idle (16 heads of 128 x 128, one prompt of 16 / 32 tokens 26 / 31 us, so 21 / 22); where
-// it does not, from two chunks on (16 prompts of 16 / 24 / 32 tokens 39 / 46 / 51 and 37 / 46 / 46), with one decay a head, which saves that walk a third of its reads, from eight (32 heads, 16
-// prompts of 32 / 64 / 400 tokens 65 / 104 / 603 and 66 / 107 / 526).
-bool chunked(const PlanLayer &L, const StepView &v, const DeltaBuffers &b) {
-    const int from = chunk_tiles(L, v) < 4L * device_cu_count() ? kChunk : L.head_decay() ? 8 * kChunk : 2 * kChunk;
-    return b.chunks && v.longest >= from && L.KD >= 64 && L.KD <= 256 && L.s.taps >= 2 && L.s.taps <= 4;
+// launches over some of the segments: f(how many, which)
+template <typename F>
+void over_segments(const std::vector<int> &segments, F f) {
+    for (size_t at = 0; at < segments.size(); at += kChunkSegs) {
+        ChunkSegs s = {};
+        const size_t n = std::min<size_t>(kChunkSegs, segments.size() - at);
+        std::copy_n(segments.begin() + at, n, s.seg);
+        f((unsigned)n, s);
+    }
 }
 
 // row_in: the input product's rows, if the gate is in them
@@ -1031,16 +1043,43 @@ int launch_output(int act, const OutParams &p, int T, hipStream_t st) {
 
 } // namespace
 
-int delta_prepare(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st) {
-    const PrepParams p = prep_params(act, L, v, b);
+// Which segments kChunk tokens at a time?
+// Where all tiles of the step leave most of the device idle: all, from a longest of a whole chunk on (16 heads of 128 x 128, one prompt of 16 / 32 tokens 26 / 31 us token by token, so 21 / 22).
+// Else, with hardly any short ones, all from two chunks on (16 prompts of 16 / 24 / 32 tokens 39 / 46 / 51 and 37 / 46 / 46), with one decay a head, which saves the walk a third of its reads, from
+// eight (32 heads, 16 prompts of 32 / 64 / 400 tokens 65 / 104 / 603 and 66 / 107 / 526).
+// Else each by its own length, since a single token costs as much as a whole chunk there; two launches more, which segments of less than four (eight) chunks do not pay for.  All token by token / all in
+// chunks / so, us: one prompt of 64 / 128 / 500 tokens beside 50 decoding sequences 62 / 119 / 63, 83 / 168 / 58 and 196 / 467 / 84, beside 200 163 / 440 / 131, 222 / 624 / 137 and 249 / 1701 / 156; 4 of 300
+// beside 20 170 / 125 / 91; with one decay a head, 32 heads, 128 tokens beside 50 101 / 243 / 84.
+DeltaSplit delta_split(const PlanLayer &L, const StepView &v, const int *lens, bool chunks) {
+    DeltaSplit s;
+    s.rest = v.longest;
+    if (!chunks || v.longest < kChunk || L.KD < 64 || L.KD > 256 || L.s.taps < 2 || L.s.taps > 4) return s;
+    const long full = 4L * device_cu_count();
+    const bool idle = chunk_tiles(L, v.B) < full;
+    int from = idle ? kChunk : L.head_decay() ? 8 * kChunk : 2 * kChunk;
+    const bool all = idle || chunk_tiles(L, std::count_if(lens, lens + v.B, [&](int n) { return n < from; })) < full / 2;
+    if (!all) from = L.head_decay() ? 8 * kChunk : 4 * kChunk;
+    if (v.longest < from) return s;
+    s.rest = 0, s.longest = v.longest, s.below = from;
+    for (int i = 0; i < v.B; ++i) {
+        if (all || lens[i] >= from) s.by_chunks.push_back(i);
+        else s.rest = std::max(s.rest, lens[i]);
+    }
+    return s;
+}
+
+int delta_prepare(int act, const PlanLayer &L, const StepView &v, const DeltaSplit &split, const DeltaBuffers &b, hipStream_t st) {
+    PrepParams p = prep_params(act, L, v, b);
     const dim3 grid(v.T, (p.H + 3) / 4);
     const int width = p.KD > p.VD ? p.KD : p.VD;
     const bool tiled = p.taps >= 2 && p.taps <= 4 && width <= 256;
-    if (chunked(L, v, b)) {
-        const dim3 chunks((v.longest + kChunk - 1) / kChunk, p.H, v.B);
+    if (!split.by_chunks.empty()) {
         auto launch = [&](auto bf16, auto f32) {
-            if (act == XFTHIP_BF16) hipLaunchKernelGGL(bf16, chunks, dim3(256), 0, st, p);
-            else hipLaunchKernelGGL(f32, chunks, dim3(256), 0, st, p);
+            over_segments(split.by_chunks, [&](unsigned n, const ChunkSegs &segs) {
+                const dim3 chunks((split.longest + kChunk - 1) / kChunk, p.H, n);
+                if (act == XFTHIP_BF16) hipLaunchKernelGGL(bf16, chunks, dim3(256), 0, st, p, segs);
+                else hipLaunchKernelGGL(f32, chunks, dim3(256), 0, st, p, segs);
+            });
         };
         switch (L.KD + (L.head_decay() ? 1 : 0)) {
             case 64: launch(delta_chunk_kernel<64, false, true>, delta_chunk_kernel<64, false, false>); break;
@@ -1051,10 +1090,12 @@ int delta_prepare(int act, const PlanLayer &L, const StepView &v, const DeltaBuf
             default: launch(delta_chunk_kernel<256, true, true>, delta_chunk_kernel<256, true, false>); break;
         }
         XFT_CHECK_HIP(hipGetLastError());
-        return conv_tail(act, v, p.b.in, p.ld, p.channels, p.taps, b.conv_state, st, 1); // (several workgroups read the inputs of a key head: nobody shifts those of a single token in place)
+        p.below = split.below;
+        // (several workgroups read the inputs of a key head: nobody shifts those of a single token in place)
+        if (!split.rest) return conv_tail(act, v, p.b.in, p.ld, p.channels, p.taps, b.conv_state, st, 1);
     }
     if (tiled) {
-        const dim3 tiles((v.longest + kPrepTokens - 1) / kPrepTokens, (p.H + 3) / 4, v.B);
+        const dim3 tiles((split.rest + kPrepTokens - 1) / kPrepTokens, (p.H + 3) / 4, v.B);
         const int key = (act == XFTHIP_BF16 ? 0 : 10) + p.taps + (width > 128 ? 100 : 0);
         switch (key) {
             case 2: hipLaunchKernelGGL((delta_prepare_tiled_kernel<true, 2, 1>), tiles, dim3(256), 0, st, p); break;
@@ -1094,17 +1135,19 @@ size_t delta_chunk_floats(const PlanLayer &L, int tokens, int segments) {
     return (size_t)(tokens / kChunk + std::min(segments, tokens)) * L.s.heads * chunk_floats(L.KD);
 }
 
-int delta_scan(const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st) {
+int delta_scan(const PlanLayer &L, const StepView &v, const DeltaSplit &split, const DeltaBuffers &b, hipStream_t st) {
     ScanParams p;
-    p.v = v, p.b = b, p.H = L.s.heads, p.KH = L.s.kv_heads, p.VD = L.VD;
+    p.v = v, p.b = b, p.H = L.s.heads, p.KH = L.s.kv_heads, p.VD = L.VD, p.below = INT_MAX;
     const int lanes = L.KD / 8;
     const bool one = L.head_decay();
-    if (chunked(L, v, b)) {
+    if (!split.by_chunks.empty()) {
         // Two tiles a wave where a CU has several workgroups of one in turn: 16 heads of 128 x 128, one / two, 4 prompts of 1000 to 1500 tokens 255 / 262 us, 6 of 200 to 1000 239 / 270, 8 of
         // 800 342 / 308, 16 of 400 351 / 314; 64 x 64, whose workgroups are of half the waves, 16 of 400 134 / 140; 8 of 256 x 256, 8 of 800 484 / 439
-        const bool two = L.VD % 32 == 0 && chunk_tiles(L, v) >= (L.KD == 64 ? 8L : 4L) * device_cu_count();
+        const bool two = chunk_tiles(L, split.by_chunks.size()) >= (L.KD == 64 ? 8L : 4L) * device_cu_count(); // (value widths are whole 32s)
         auto scan = [&](auto one_tile, auto two_tiles, int waves) {
-            hipLaunchKernelGGL(two ? two_tiles : one_tile, dim3(v.B, p.H, L.VD / 16 / (two ? 2 : 1)), dim3(64 * waves + 64), 0, st, p);
+            over_segments(split.by_chunks, [&](unsigned n, const ChunkSegs &segs) {
+                hipLaunchKernelGGL(two ? two_tiles : one_tile, dim3(n, p.H, L.VD / 16 / (two ? 2 : 1)), dim3(64 * waves + 64), 0, st, p, segs);
+            });
         };
         switch (L.KD) {
             case 64: scan(delta_chunk_scan_kernel<64, 2, 1>, delta_chunk_scan_kernel<64, 2, 2>, 2); break;
@@ -1112,18 +1155,19 @@ int delta_scan(const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hip
             default: scan(delta_chunk_scan_kernel<256, 4, 1>, delta_chunk_scan_kernel<256, 4, 2>, 4); break;
         }
         XFT_CHECK_HIP(hipGetLastError());
-        return 0;
+        if (!split.rest) return 0;
+        p.below = split.below;
     }
     // Two columns a group of lanes where one would make four waves a SIMD or more: below, the columns' chains are better hidden by each other's waves.  16
     // heads of 128 x 128, one column / two: 4 prompts of 1500 tokens 350 / 407 us, 6 of 1000 308 / 368, 8 of 800 308 / 272, 24 of 500 650 / 510.
-    const bool two = v.longest > 1 && lanes >= 8 && L.VD % (512 / lanes) == 0 && (long)v.B * p.H * L.VD * lanes >= (long)device_cu_count() * 1024;
+    const bool two = split.rest > 1 && lanes >= 8 && L.VD % (512 / lanes) == 0 && (long)v.B * p.H * L.VD * lanes >= (long)device_cu_count() * 1024;
     const int cols = (two ? 512 : 256) / lanes;
     const dim3 grid(v.B, p.H, (L.VD + cols - 1) / cols);
     auto launch = [&](auto several, auto single) {
         if (one) hipLaunchKernelGGL(single, grid, dim3(256), 0, st, p);
         else hipLaunchKernelGGL(several, grid, dim3(256), 0, st, p);
     };
-    const int key = (v.longest == 1 ? 0 : two ? 2000 : 1000) + L.KD;
+    const int key = (split.rest == 1 ? 0 : two ? 2000 : 1000) + L.KD;
     switch (key) {
         case 32: launch(delta_step_kernel<4, false>, delta_step_kernel<4, true>); break;
         case 64: launch(delta_step_kernel<8, false>, delta_step_kernel<8, true>); break;

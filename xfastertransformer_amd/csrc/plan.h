@@ -282,8 +282,17 @@ int conv_tail(int act, const StepView &v, const void *in, int ld, int channels, 
 // steps of one token a sequence: all three of the following in one launch, where it takes the layer
 bool delta_decodes_at_once(const PlanLayer &L, const StepView &v);
 int delta_decode(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, float eps, hipStream_t st);
-int delta_prepare(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st);
-int delta_scan(const PlanLayer &L, const StepView &v, const DeltaBuffers &b, hipStream_t st);
+// which segments of a step are taken several tokens at a time
+struct DeltaSplit {
+    std::vector<int> by_chunks;
+    int longest = 0; // tokens of the longest of them
+    int rest = 0; // and of the longest of the others, which have fewer than `below`; 0: there are none
+    int below = 0;
+};
+// lens: tokens of the segments; chunks: whether DeltaBuffers::chunks is there
+DeltaSplit delta_split(const PlanLayer &L, const StepView &v, const int *lens, bool chunks);
+int delta_prepare(int act, const PlanLayer &L, const StepView &v, const DeltaSplit &split, const DeltaBuffers &b, hipStream_t st);
+int delta_scan(const PlanLayer &L, const StepView &v, const DeltaSplit &split, const DeltaBuffers &b, hipStream_t st);
 size_t delta_chunk_floats(const PlanLayer &L, int tokens, int segments);
 int delta_output(int act, const PlanLayer &L, const StepView &v, const DeltaBuffers &b, float eps, hipStream_t st);
 

@@ -248,8 +248,9 @@ int mix_delta(xfthip_model *m, const PlanLayer &L, int store, const StepView &v,
             return rc;
     }
     if (delta_decodes_at_once(L, v)) return delta_decode(act, L, v, b, m->cfg.rms_eps, st);
-    if ((rc = delta_prepare(act, L, v, b, st))) return rc;
-    if ((rc = delta_scan(L, v, b, st))) return rc;
+    const DeltaSplit split = delta_split(L, v, p.seg_len_host.data(), p.chunks != nullptr);
+    if ((rc = delta_prepare(act, L, v, split, b, st))) return rc;
+    if ((rc = delta_scan(L, v, split, b, st))) return rc;
     return delta_output(act, L, v, b, m->cfg.rms_eps, st);
 }
 
@@ -1570,6 +1571,23 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
         return 1;
     }
     *out = m;
+    return 0;
+}
+
+int xfthip_delta_forms(int heads, int dim, int vdim, int taps, int decay_per_head, int segments, const int *lens_host, int *forms) {
+    XFT_REQUIRE(lens_host && forms && segments > 0 && heads > 0 && dim > 0 && dim <= 256 && vdim > 0 && taps > 0, "xfthip_delta_forms: bad argument");
+    PlanLayer L;
+    L.s = {};
+    L.s.heads = heads, L.s.dim = dim, L.s.vdim = vdim, L.s.taps = taps, L.s.decay_rank = decay_per_head ? 0 : 1;
+    L.KD = 32, L.VD = pad32(vdim);
+    while (L.KD < dim) L.KD *= 2;
+    StepView v = {};
+    v.B = segments;
+    for (int i = 0; i < segments; ++i) {
+        XFT_REQUIRE(lens_host[i] > 0, "xfthip_delta_forms: segment %d has %d tokens", i, lens_host[i]);
+        v.longest = std::max(v.longest, lens_host[i]), forms[i] = 0;
+    }
+    for (int i : delta_split(L, v, lens_host, true).by_chunks) forms[i] = 1;
     return 0;
 }
 
