@@ -686,15 +686,23 @@ size_t xfthip_plan_weight_bytes(xfthip_plan_t p);
  * on the bf16 matrix units) or XFTHIP_F32 (everything in 32 bits).  max_batch: sequence slots; pool_tokens: tokens the page
  * pool holds over all sequences (0 = max_batch * max_seq).  max_tokens: tokens of a step, which its scratch memory is sized by; latent attention in bf16
  * also keeps heads * (dim + vdim) + kv_rank + rot_dim values for each of max_seq context tokens, and for up to max_tokens + 992 as far as an eighth of
- * the device memory left by everything else holds them.
+ * the device memory left by everything else holds them; the delta rule keeps records for long segments likewise (xfthip_model_delta_chunks).
  */
 int xfthip_model_create_from_plan(xfthip_plan_t p, int act_dtype, int max_batch, int max_seq, int max_tokens, int pool_tokens,
         xfthip_model_t *out);
 /*
  * Which segments of a step the delta rule takes 16 tokens at a time (forms[i] 1; 0: token by token) on the current device (or on 256 compute units where none is in use),
- * for a layer of these heads, key and value widths and filter taps with a decay a head or a channel.  For tests of both, and for tuning.
+ * for a layer of these heads, key and value widths and filter taps with a decay a head or a channel, in a model that holds the records for it (below).  For tests of
+ * both, and for tuning.
  */
 int xfthip_delta_forms(int heads, int dim, int vdim, int taps, int decay_per_head, int segments, const int *lens_host, int *forms);
+/*
+ * The records through which a model's delta rule layers take long segments 16 tokens at a time.  A model from a plan holds them if, when it is made, an eighth of the device
+ * memory left by everything else does; without them all segments go token by token, which takes longer and adds up in another order (within the rounding of 32-bit sums).
+ * use > 0: hold them from now on (an error if they do not fit), 0: give them back, < 0: as it is.  held (or NULL): whether they are held (never without such layers).
+ * Not beside a step of the same model.
+ */
+int xfthip_model_delta_chunks(xfthip_model_t m, int use, int *held);
 /*
  * One step of a batch of unequal parts: entry i brings the next lens_host[i] tokens of slot rows_host[i] (a prompt, a portion of
  * one or a single token; ids back to back in ids_host); a slot that holds no sequence starts one at position 0.  want_host: n_want

@@ -1,5 +1,5 @@
-"""The delta rule's scan with one and with two columns a group of lanes, full chunks of tokens and remainders, states that go on from a step before;
-one decay a key channel and one a head."""
+"""The delta rule token by token, with one and with two columns a group of lanes, full chunks of tokens and remainders, states that go on from a step before, and 16
+tokens at a time; one decay a key channel and one a head."""
 import numpy as np
 import pytest
 
@@ -28,6 +28,7 @@ def test_scan(dim, vdim, heads, decay):
         cfg = u.config([(u.windowed_delta(r_heads=heads, r_kv_heads=kv, r_dim=dim, r_vdim=vdim, left=0.0), None)])
     bits = u.weights(cfg, 21)
     case = u.Case(xh, u.build_plan(xh, cfg, bits), u.oracle_weights(bits), lambda w, t: ref.forward(cfg, w, t), "f32", 3e-5, 8, 128, 256)
+    assert not case.model.delta_chunks(False)  # token by token, whatever the lengths
     rng = np.random.default_rng(dim + heads)
     texts = [rng.integers(0, cfg["vocab"], a + b) for a, b in zip(FIRST, SECOND)]
     want = [case.want(t) for t in texts]
@@ -57,6 +58,7 @@ def held(dim, vdim, heads, decay, steps, forms, tokens=512):
     bits = u.weights(cfg, 22)
     n = len(steps[0])
     case = u.Case(xh, u.build_plan(xh, cfg, bits), u.oracle_weights(bits), lambda w, t: ref.forward(cfg, w, t), "f32", 3e-5, n, 384, tokens, n * 384)
+    assert case.model.delta_chunks()
     rng = np.random.default_rng(dim + heads)
     ends = np.cumsum([[0] * n] + [list(s) for s in steps], 0)
     texts = [rng.integers(0, cfg["vocab"], e) for e in ends[-1]]
@@ -110,6 +112,7 @@ def test_chunks_and_what_is_not_finite(at, what):
     sound = u.oracle_weights(bits)
     bits["embed"][5, 3] = what
     case = u.Case(xh, u.build_plan(xh, cfg, bits), sound, lambda w, t: ref.forward(cfg, w, t), "f32", 3e-5, 8, 384, 512)
+    assert case.model.delta_chunks() and xh.delta_forms(4, 128, 64, 4, False, [45, 45]) == [1, 1]
     rng = np.random.default_rng(at)
     texts = [rng.integers(6, cfg["vocab"], 45) for _ in range(2)]
     want = [case.want(t) for t in texts]
@@ -118,3 +121,32 @@ def test_chunks_and_what_is_not_finite(at, what):
     assert not np.isfinite(got[at:45]).any()
     case.check(np.concatenate([got[:at], got[45:]]), np.concatenate([want[0][:at], want[1]]), "the others")
     case.free()
+
+
+def test_records_given_back_and_held_again():
+    """A sequence that goes on in the other form from step to step, and back."""
+    from xfastertransformer_amd import capi as xh
+    xh.init(0)
+    u, ref = many_decays, pinepel_ref
+    cfg = u.config([u.delta(heads=4, kv_heads=2, dim=100, vdim=64, conv=3)])
+    bits = u.weights(cfg, 24)
+    case = u.Case(xh, u.build_plan(xh, cfg, bits), u.oracle_weights(bits), lambda w, t: ref.forward(cfg, w, t), "f32", 3e-5, 2, 384, 256)
+    text = np.random.default_rng(5).integers(0, cfg["vocab"], 200)
+    want, at = case.want(text), 0
+    for use, n in ((None, 40), (False, 35), (False, 20), (True, 33), (True, 50), (False, 1), (True, 21)):
+        assert case.model.delta_chunks(use) == (use is not False) == case.model.delta_chunks()
+        case.check(case.model.step([(1, text[at:at + n], list(range(n)))]), want[at:at + n], f"at {at}")
+        at += n
+    case.free()
+
+
+def test_models_without_such_layers_hold_none():
+    from xfastertransformer_amd import capi as xh
+    xh.init(0)
+    u = many_decays
+    cfg = u.config([u.delta(heads=2, kv_heads=2, dim=32, vdim=32, conv=4)])  # (keys too narrow)
+    plan = u.build_plan(xh, cfg, u.weights(cfg, 25))
+    model = xh.PlanModel(plan, xh.F32, 2, 64, 64)
+    assert not model.delta_chunks() and not model.delta_chunks(True) and not model.delta_chunks(False)
+    model.free()
+    plan.free()

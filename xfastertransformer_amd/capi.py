@@ -653,6 +653,12 @@ class PlanModel(Model):
                                     C.c_void_p(out.ctypes.data), stream))
         return out
 
+    def delta_chunks(self, use=None):
+        """Whether the delta rule's records for long segments are held (include/xft_hip.h); use: hold them, or give them back."""
+        held = C.c_int()
+        check(lib.xfthip_model_delta_chunks(self.h, -1 if use is None else int(bool(use)), C.byref(held)))
+        return bool(held.value)
+
     def trace_residual(self, enable):
         check(lib.xfthip_model_trace_residual(self.h, int(enable)))
 

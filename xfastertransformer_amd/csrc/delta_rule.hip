@@ -1131,7 +1131,7 @@ int conv_tail(int act, const StepView &v, const void *in, int ld, int channels, 
 }
 
 size_t delta_chunk_floats(const PlanLayer &L, int tokens, int segments) {
-    if (L.KD < 64 || L.KD > 256 || tokens < kChunk) return 0;
+    if (L.KD < 64 || L.KD > 256 || L.s.taps < 2 || L.s.taps > 4 || tokens < kChunk) return 0;
     return (size_t)(tokens / kChunk + std::min(segments, tokens)) * L.s.heads * chunk_floats(L.KD);
 }
 

@@ -393,6 +393,7 @@ struct PlanState {
     // scratch (activation type unless float)
     void *xn = nullptr, *a = nullptr, *cq = nullptr, *q = nullptr, *qa = nullptr, *oc = nullptr, *ov = nullptr, *h = nullptr, *u = nullptr;
     float *y = nullptr, *y2 = nullptr, *gates = nullptr, *dq = nullptr, *dk = nullptr, *dqk = nullptr, *dg = nullptr, *dv = nullptr, *dbeta = nullptr, *do_ = nullptr, *chunks = nullptr, *carry = nullptr;
+    size_t chunk_floats = 0; // of `chunks`, held or not
     int *last_token = nullptr; // [slots]
     void *xn2 = nullptr, *first_values = nullptr, *side = nullptr, *narrow = nullptr;
     float *router_logits = nullptr, *expert_out = nullptr, *side_z = nullptr;

@@ -1439,7 +1439,7 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
     const size_t T = max_tokens, e = p->esz, hidden = plan->hidden;
     bool normed_results = false;
     size_t a = 0, cq = 0, q = 0, qa = 0, ov = 0, h = 0, gates = 0, dk = 0, dqk = 0, dg = 0, dv = 0, heads = 0, fv = 0, u = 0, carry = 0;
-    size_t chunks = 0, top = 0, experts = 0, routes = 0, eh = 0, eo = 0;
+    size_t top = 0, experts = 0, routes = 0, eh = 0, eo = 0;
     for (const PlanLayer &L : p->layers) {
         const size_t H = L.s.heads;
         a = std::max(a, (size_t)L.in_ld), ov = std::max(ov, (size_t)L.out_ld);
@@ -1463,7 +1463,7 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
         } else {
             const size_t KH = L.s.kv_heads;
             gates = std::max(gates, (size_t)2 * L.gcols), dk = std::max(dk, KH * L.KD), dqk = std::max(dqk, KH), dg = std::max(dg, L.head_decay() ? H : H * L.KD);
-            dv = std::max(dv, H * L.VD), heads = std::max(heads, H), chunks = std::max(chunks, delta_chunk_floats(L, max_tokens, max_batch));
+            dv = std::max(dv, H * L.VD), heads = std::max(heads, H), p->chunk_floats = std::max(p->chunk_floats, delta_chunk_floats(L, max_tokens, max_batch));
         }
     }
     alloc(&p->xn, std::max(T, (size_t)p->logit_rows) * hidden * e);
@@ -1564,7 +1564,7 @@ int xfthip_model_create_from_plan(xfthip_plan_t plan, int act_dtype, int max_bat
     }
     // (the delta rule's chunks alike: within an eighth of what is left, or not at all)
     size_t left = 0, device = 0;
-    if (ok && chunks && hipMemGetInfo(&left, &device) == hipSuccess && chunks * 4 <= left / 8) alloc(&p->chunks, chunks * 4);
+    if (ok && p->chunk_floats && hipMemGetInfo(&left, &device) == hipSuccess && p->chunk_floats * 4 <= left / 8) alloc(&p->chunks, p->chunk_floats * 4);
     if (!ok) {
         set_error("xfthip_model_create_from_plan: out of device memory");
         xfthip_model_destroy(m);
@@ -1588,6 +1588,28 @@ int xfthip_delta_forms(int heads, int dim, int vdim, int taps, int decay_per_hea
         v.longest = std::max(v.longest, lens_host[i]), forms[i] = 0;
     }
     for (int i : delta_split(L, v, lens_host, true).by_chunks) forms[i] = 1;
+    return 0;
+}
+
+int xfthip_model_delta_chunks(xfthip_model_t m, int use, int *held) {
+    XFT_REQUIRE(m && m->plan, "xfthip_model_delta_chunks: only for models from a plan");
+    PlanState &p = *m->plan;
+    if (use > 0 && !p.chunks && p.chunk_floats) {
+        void *b = nullptr;
+        if (hipMalloc(&b, p.chunk_floats * 4 + 256) != hipSuccess) {
+            (void)hipGetLastError(); // (told here: the check behind the next launch would report it again)
+            set_error("xfthip_model_delta_chunks: out of device memory");
+            return 1;
+        }
+        p.owned.push_back(b);
+        p.chunks = (float *)b;
+    } else if (use == 0 && p.chunks) {
+        p.owned.erase(std::find(p.owned.begin(), p.owned.end(), (void *)p.chunks));
+        void *b = p.chunks;
+        p.chunks = nullptr;
+        XFT_CHECK_HIP(hipFree(b)); // (waits for the steps that use it)
+    }
+    if (held) *held = p.chunks != nullptr;
     return 0;
 }
 
