@@ -455,6 +455,13 @@ def test_ragged_k_in_one_sum(xh, M):
 @pytest.mark.parametrize("kind", ["uint4", "nf4"])
 @pytest.mark.parametrize("M,K,N,direct", [(2100, 192, 6160, 1), (2308, 320, 2512, 1), (2000, 1088, 4112, 1), (2129, 12352, 400, 1), (2100, 64, 6160, 0)])
 def test_four_bit_steps_of_half_a_tile_against_64_bits(xh, orc, kind, M, K, N, direct):
-    """4-bit weights, K an odd number of 64: the last step of the tiles with activations straight into LDS is half a packed tile (a single half is not theirs)."""
+    """4-bit weights, K an odd number of 64: the last step of the tiles with activations straight into LDS is half a packed tile (the last shape is another tile's)."""
     assert xh.gemm_form({"uint4": xh.W_UINT4, "nf4": xh.W_NF4}[kind], M, K, N, 0, kind == "uint4")[4] == direct
     test_mfma_every_tile_against_64_bits(xh, orc, kind, M, K, N)
+
+
+@pytest.mark.parametrize("kind,M,N,tile", [("uint4", 773, 18000, (128, 256)), ("uint4", 810, 14000, (96, 256)), ("nf4", 1437, 8192, (96, 256)), ("nf4", 3585, 10800, (128, 128))])
+def test_half_a_packed_tile_alone_against_64_bits(xh, orc, kind, M, N, tile):
+    """4-bit weights, K = 64: the only step of the tiles with activations straight into LDS is half a packed tile, in front of which there is nothing to request."""
+    assert xh.gemm_form({"uint4": xh.W_UINT4, "nf4": xh.W_NF4}[kind], M, 64, N, 0, kind == "uint4") == tile + (1, 1, 1)
+    test_mfma_every_tile_against_64_bits(xh, orc, kind, M, 64, N)

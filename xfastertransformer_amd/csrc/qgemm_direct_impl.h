@@ -121,7 +121,9 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
     uint32_t a_off[ALOADS]; // bytes
 #pragma unroll
     for (int i = 0; i < ALOADS; ++i) {
-        const int r = (64 / CPR) * (ALOADS * wave + i) + lane / CPR, chunk = (lane % CPR) ^ direct_swizzle<KSTEP>(r);
+        const int r = (64 / CPR) * (ALOADS * wave + i) + lane / CPR;
+        int chunk = (lane % CPR) ^ direct_swizzle<KSTEP>(r);
+        if (FOUR && p.K < KSTEP) chunk &= 7; // (64 k in all or in a part of K: both halves are those)
         int row = m0 + r;
         row = row < p.M ? row : p.M - 1;
         if constexpr (DEVROWS) row = p.a_rows ? p.a_rows[row] : row;
@@ -135,11 +137,12 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void qgemm_direct_kernel
     // request.  The compiler holds nothing in M0 across statements.)
     const uint32_t lds_tiles = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)tiles + ALOADS * 1024 * wave;
     const uint16_t *a_uniform = (const uint16_t *)(uintptr_t)uniform_address(p.A);
-    const int half_tail = FOUR ? __builtin_amdgcn_readfirstlane(p.K & 64) : 0; // 4-bit kinds: the last step has 64 k (K is not below 128); requested with the 64 in front of them
+    const int half_tail = FOUR ? __builtin_amdgcn_readfirstlane(p.K & 64) : 0; // 4-bit kinds: the last step has 64 k; requested with the 64 in front of them
+    const int back = p.K < KSTEP ? 0 : half_tail;
     auto request_a = [&](int kt_, int i) {
         const int kt = kt_ < kt_n ? kt_ : kt_n - 1;
         const uint32_t dst = lds_tiles + (kt_ & (NBUF - 1)) * TILEB + i * 1024;
-        const uint16_t *src = a_uniform + ((ptrdiff_t)kt * KSTEP - (kt == kt_n - 1 ? half_tail : 0));
+        const uint16_t *src = a_uniform + ((ptrdiff_t)kt * KSTEP - (kt == kt_n - 1 ? back : 0));
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(a_off[i]), "s"(src) : "memory");
     };
 

@@ -181,7 +181,7 @@ bool choose_staged_tile(SkinnyParams &p, int kind, int ktile, bool may_split) {
 void choose_tile(SkinnyParams &p, int kind, int ktile, bool own_sum, bool may_split = true) {
     const int cus = device_cu_count(), kt_n = (p.K + ktile - 1) / ktile, cls = kind == XFTHIP_W_BF16 ? 1 : kind == XFTHIP_W_NF4 ? 2 : kind == XFTHIP_W_UINT4 ? 3 : 0;
     // activations straight into LDS: steps of 64 k, byte offsets of 32 bits
-    const bool direct = p.K % 64 == 0 && p.K >= ktile && (size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32);
+    const bool direct = p.K % 64 == 0 && (size_t)p.M * (size_t)p.lda * 2 < ((size_t)1 << 32);
     p.tile = 2, p.kgroups = 1, p.direct = 0;
     if (!direct && !p.rows_dev && choose_staged_tile(p, kind, ktile, may_split)) return;
     auto blocks_of = [&](const int rows) { // row blocks
