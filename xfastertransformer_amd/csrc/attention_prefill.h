@@ -492,7 +492,7 @@ __device__ inline void attn_prefill_ring_unit(const AttnParams &p, const int kvh
     products(std::false_type {}, 0);
     // Where the loop begins in the 32 bytes that are fetched at a time is worth 6 % (512 tokens behind 8000, by the number of 4-byte steps behind a border: 156,
     // 150, 150, 146, 148, 152, 154, 152 us; 4 x 2000 tokens 144 to 146.5, 2 x 1000 with 16 / 4 heads 23.9 to 24.9; FINE 154, 161, 172, 163, 160, 172, 154, 155, INT8 at 0, 2, 4, 6
-    // steps 293, 306, 305, 294), so it is said.
+    // steps 293, 306, 305, 294), so it is said.  (As the compiler of ROCm 7.2 lays out the code in front of it.)
     if constexpr (INT8 && FINE) asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
     else if constexpr (!INT8 && FINE) asm volatile(".p2align 5");
     else if constexpr (!INT8) asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");

@@ -444,7 +444,7 @@ struct ChunkSegs {
 
 // In place of delta_prepare for such segments: convolutions, norms and decays of a (chunk, head) by a workgroup of its own, two neighbouring channels of q, k, v or the decays a
 // thread, and what the scan needs of them.  Tokens past the segment's end have no keys, queries and step sizes.  A and B: thread (s, 1/16 of the key dims) carries k_s on from token to token,
-// 16 lanes add up.  Bound by the round trips of a workgroup, of which six share a CU (4 prompts of 1000 to 1500 tokens, 16 heads of 128 x 128: 110 us for 270 MB; delta_prepare, which
+// 16 lanes add up.  Bound by the round trips of a workgroup, of which four share a CU (112 registers; LDS would take five; 4 prompts of 1000 to 1500 tokens, 16 heads of 128 x 128: 110 us for 270 MB; delta_prepare, which
 // leaves the products to the scan, 85).
 template <int KD, bool ONE, bool BF16>
 __global__ __launch_bounds__(256) void delta_chunk_kernel(PrepParams p, ChunkSegs segs) {

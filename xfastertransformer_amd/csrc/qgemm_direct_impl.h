@@ -11,7 +11,10 @@
 // twice as often: 1.83 against 1.64 PFLOP/s in a loop of MFMAs and operand reads alone, 2.09 against 1.80 in MFMAs alone (2.45 either on zeros).  2048 x 16384,
 // K = 4096 / 16384, against that form: INT8 230 / 825 -> 218 / 775 us (1.42 PFLOP/s), UINT4 233 / 788 -> 210 / 710 (1.55), BF16 239 / 906 -> 212 / 866 (1.27);
 // 2011 x 11008 x 4096 INT8 155 -> 148, a Mixtral-8x7B layer of 256 tokens 356 -> 333.  What is left beside the products are the bytes they come from: at a step of
-// 4 KB a wave the weights' way from L2 is a fifth of the time (INT8, left out: 835 -> 659), the activations' 8 %, the barriers nothing.
+// 4 KB a wave the weights' way from L2 is a fifth of the time (INT8, left out: 835 -> 659), the activations' 8 %, the barriers nothing; their way from memory is hidden: 2048 x 11008 x 4096 over
+// one weight / eight in turn INT8 153.5 / 155.5 us, UINT4 143.8 / 144.0, BF16 153 / 158.  (Behind an idle device the first 24 launches take 188, 180 and 186, the next 96 166, 158 and 166.)
+// Counters of these launches, each by itself: INT8 305,000 clocks at 1.94 GHz, matrix units busy 58 % of them, vector ALUs 42 % (the issue of MFMAs among it), LDS ports 16 %, waves waiting 14 % of their
+// time in counted waits; UINT4 329,000 clocks at 2.17 GHz, 54 %, 36 %, 15 %, 13 %.
 #pragma once
 #include "qgemm_mfma_common.h"
 

@@ -1,7 +1,7 @@
 // Dequant-fused weight-only GEMM for many activation rows (M > 32): the prefill shape.
 // Replaces MMHelper::compute* (reference src/utils/matmul_helper.h:565-1705) at large M, where
-// the reference switches to AMX (oneDNN) kernels.  The kernel lives in qgemm_mfma_impl.h; this
-// file picks the weight kind.
+// the reference switches to AMX (oneDNN) kernels.  The kernels live in qgemm_mfma_impl.h and
+// qgemm_direct_impl.h; this file picks the weight kind and the tile.
 #include <math.h>
 
 #include <algorithm>
@@ -104,8 +104,10 @@ __global__ __launch_bounds__(256) void qgemm_split_finish_kernel(SkinnyParams p)
 // A CU's blocks are those of the XCD with the most (band_rows); a partly filled round costs between the blocks of the fullest CU and
 // those of the average one, a partly filled device a little less a step than a full one.  The constants (microseconds) are a
 // least-squares fit to 35000 timings on weights that do not fit the Infinity Cache: 340 shapes of 1024 .. 28672 columns x 1024 .. 14336 deep,
-// 33 to 4096 rows, 1 to 8 parts, the five weight kinds.  What it takes is 1.01 to 1.02 times the best form's time on average over those
-// cells (1.33 at worst).  In words: the largest tile that gives most CUs a block, K split or taken in two groups where that takes it to
+// 33 to 4096 rows, 1 to 8 parts, the five weight kinds, of the 96- and 128-row tiles on 32 x 32 x 16 MFMAs: 1.01 to 1.02 times the best form's time on average over those
+// cells then (1.33 at worst).  On the kernels as they are, whose 128 x 128 tile gained the most, over 3200 to 4500 shapes a kind: INT8 1.023 on average, 1.12 for one in twenty, 1.65 at worst (87 x 22016 x 4096
+// 50 us, best 30); UINT4 1.009, 1.06, 1.41 (1593 x 11264 x 2048 90, 64); NF4 1.015, 1.10, 1.23; BF16 1.038, 1.19, 1.55 (390 x 2048 x 2048 20.5, 13.2); their times come out 14 to 29 % too
+// long (INT8).  In words: the largest tile that gives most CUs a block, K split or taken in two groups where that takes it to
 // about a block a CU, and for few rows parts of K until there are two or three 32- or 64-row blocks a CU.  Against thresholds on the rows
 // (which left 700 rows x 4096 columns on 64-row tiles and split 128 rows too little) and bands padded to 8 row blocks: INT8 1.15 times as
 // fast in the geometric mean over the cells, with zero points 1.17, UINT4 1.12, NF4 1.19, BF16 1.43; 900 x 4096 x 14336 INT8 142 -> 113 us,
